@@ -9,9 +9,9 @@
 
 #include "dcpse_hip.h"
 
-// Cell list and per-particle take masks of the last same-set, single-cut-off
-// support count; the fill that follows with the same arguments gathers its
-// rows from them instead of repeating the distance tests.
+// Cell list, sorted candidate lists and per-particle take masks of the last
+// same-set, single-cut-off support count; the fill that follows with the same
+// arguments writes its rows from them instead of repeating the distance tests.
 struct dcpse_support_cache {
     void* buf = nullptr;  // grow-only device buffer
     size_t cap = 0;

@@ -5,14 +5,15 @@
 // (VL_NON_SYMMETRIC | VL_SKIP_REF_PART: q != p, |x_p - x_q| < rCut), see
 // src/DCPSE/SupportBuilder.cuh:15-61. Unlike that builder (one thread per
 // particle, host-side serial prefix sum, size_t keys, 4 host round trips), the
-// whole CSR is built on the device: a cell grid by counting sort, one
-// wavefront per particle walking the 3^dim neighbour cells as one flattened
-// candidate list, ballot compaction into LDS and an in-LDS rank sort so every
-// row comes out in ascending particle index (deterministic, independent of
-// atomic ordering).
+// whole CSR is built on the device: a cell grid by counting sort, then one
+// wavefront per cell (one set, one cut-off) or per particle over the
+// neighbouring cells' particles, flattened into one candidate list and sorted
+// in registers, so every row comes out in ascending particle index
+// (deterministic, independent of atomic ordering).
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 #include "dcpse_common.hpp"
 #include "dcpse_internal.hpp"
@@ -466,32 +467,22 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_support_rows(
 // The candidates of a cell are its 3^dim neighbouring cells, scanned as
 // 3^(dim-1) rows along dimension 0 (contiguous in the cell order, split in two
 // where a periodic wrap cuts a row), flattened into one list. The count pass
-// (k_support_cells_count) copies them, CellCap at a time, into the wave's LDS
-// slice (particle index and position) and tests every particle of the cell
-// against each copy, so the cell's particles share the candidate setup and
-// global loads; it stores, per particle, which candidates it takes (one bit
-// each, nws 64-bit words at masks[slot * nws]). The fill pass
-// (k_support_cells_masked) stages only the candidate indices and gathers each
-// row by its mask, with no distance work. Cells with more than kCellMaxPart
-// particles or more candidates than the masks cover (nws * 64) are left to
+// (k_cell_pairs) keeps the candidates within the cut-off of the bounding box
+// of the cell's particles, sorts their indices once per cell, and tests every
+// particle of the cell against them: it stores the sorted candidate list of
+// the cell and, per particle, which of them it takes (one bit each). The fill
+// (k_cell_rows) writes a particle's row as the marked entries of its cell's
+// list, which are in ascending order as they stand: no distance work and no
+// sort per row. Cells with more candidates than the list holds are left to
 // k_support_cells, which tests each particle against positions (restaging
-// them per particle when they exceed one LDS copy). All three use the
-// distance formula of k_support_rows on the same position copies and write
-// rows in ascending order, so the results are the same.
+// them per particle when they exceed one LDS copy). All use the distance
+// formula of k_support_rows on the same positions (k_cell_pairs wherever FP32
+// leaves the outcome open), so the results are the same.
 constexpr int kCellWaves = 2;
-constexpr int kCellMaxPart = 2 * kWave;  // particles of a masked cell
 template <int DIM>
-struct CellCap {  // candidates per LDS copy with positions (384: 3.5 waves per SIMD in the count)
+struct CellCap {  // candidates per LDS copy of k_support_cells
     static constexpr int v = DIM == 3 ? 384 : 256;
 };
-template <int DIM>
-struct MaskCap {  // candidates a particle's mask covers at most
-    static constexpr int v = DIM == 3 ? 2048 : 1024;
-};
-
-__device__ __forceinline__ bool masked_cell(int np, int total, int mask_cap) {
-    return np <= kCellMaxPart && total <= mask_cap;
-}
 
 // Block b's cell range: consecutive logical blocks on one XCD (blocks are
 // dealt round-robin over the 8 XCDs), so neighbouring cells, which share most
@@ -501,19 +492,28 @@ __device__ __forceinline__ unsigned xcd_block() {
     return (G % 8u == 0u) ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
 }
 
+// Cell c's coordinates (cells number below 2^31, see make_grid).
+template <int DIM>
+__device__ __forceinline__ void cell_coords(const CellGrid& g, int64_t c, int (&cc)[3]) {
+    unsigned rem = (unsigned)c;
+    cc[0] = cc[1] = cc[2] = 0;
+#pragma unroll
+    for (int d = 0; d < DIM - 1; ++d) {
+        const unsigned q = rem / (unsigned)g.nc[d];
+        cc[d] = (int)(rem - q * (unsigned)g.nc[d]);
+        rem = q;
+    }
+    cc[DIM - 1] = (int)rem;
+}
+
 // The candidate segments of cell c: lane 2i (+1) gets row i of the 3^(dim-1)
 // rows of three cells along dimension 0 (its part past a periodic wrap), as
 // the first cell slot cst and the length ccnt (0 for no segment).
 template <int DIM>
 __device__ __forceinline__ void cell_segments(const CellGrid& g, const int64_t* __restrict__ cell_start, int64_t c,
                                               int lane, long long& cst, int& ccnt) {
-    int cc[3] = {0, 0, 0};
-    int64_t rem = c;
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-        cc[d] = (int)(rem % g.nc[d]);
-        rem /= g.nc[d];
-    }
+    int cc[3];
+    cell_coords<DIM>(g, c, cc);
     constexpr int ROWS = DIM == 3 ? 9 : 3;
     cst = 0;
     ccnt = 0;
@@ -608,137 +608,423 @@ __device__ __forceinline__ bool within_cut(const double* xp, const double* sx, i
     return within_cut_at<DIM>(xp, xq, g, r2);
 }
 
-// Count pass over the masked cells (see above): row lengths to counts[p] and
-// take masks. The other cells are appended to spill[1 ..] (spill[0] = their
-// number) for k_support_cells.
+// Candidates are handled in coordinates relative to the cell centre, in units
+// of the cut-off, in FP32: there |a - b|^2 is within 4e-6 of the FP64 value
+// for cells up to four cut-offs wide whose positions lie within kMaxOffset
+// cut-offs of the origin (FP64 then resolves 1e-9 cut-offs), so outside
+// 1 +- kPairTol it decides the pair and inside the FP64 formula does.
+constexpr float kPairTol = 2e-5f;
+constexpr double kMaxOffset = 1e7;
+constexpr int kPairWaves = 4;  // cells (wavefronts) per block
+
+// v of lane ^ X for the lane exchanges of the sorting network.
+template <int X>
+__device__ __forceinline__ int lane_xor_key(int v, int lane) {
+    if constexpr (X == 1 || X == 2 || X == 8) return lane_xor<X>(v, lane);
+    else if constexpr (X == 3) return __builtin_amdgcn_update_dpp(0, v, 0x1B, 0xF, 0xF, false);    // quad_perm 3,2,1,0
+    else if constexpr (X == 7) return __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);   // row_half_mirror
+    else if constexpr (X == 15) return __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false);  // row_mirror
+    else if constexpr (X == 4) return lane_xor_key<3>(lane_xor_key<7>(v, lane), lane);
+    else if constexpr (X == 31) return __builtin_amdgcn_ds_swizzle(v, 0x1F | (31 << 10));
+    else return __builtin_amdgcn_ds_bpermute((lane ^ X) << 2, v);
+}
+
+// The smaller of v and p in lanes with sel = INT_MIN, the larger with INT_MAX
+// (the median of three: one instruction).
+__device__ __forceinline__ int pick(int v, int p, int sel) { return max(min(v, p), min(max(v, p), sel)); }
+
+constexpr int log2_c(int x) { return x <= 1 ? 0 : 1 + log2_c(x / 2); }
+
+// Half-cleaner of stride S over elements e = lane * R + r (lower index keeps
+// the smaller), then the smaller strides.
+template <int R, int S>
+__device__ __forceinline__ void clean_keys(int (&v)[R], const int (&sel)[6], int lane) {
+    if constexpr (S >= R) {
+        constexpr int X = S / R;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if constexpr (X == 16) {  // both rows of a pair side by side in one exchange
+                const auto x = __builtin_amdgcn_permlane16_swap((unsigned)v[r], (unsigned)v[r], false, false);
+                v[r] = pick((int)x[0], (int)x[1], sel[4]);
+            } else {
+                v[r] = pick(v[r], lane_xor_key<X>(v[r], lane), sel[log2_c(X)]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if ((r & S) == 0) {
+                const int a = v[r], b = v[r | S];
+                v[r] = min(a, b);
+                v[r | S] = max(a, b);
+            }
+    }
+    if constexpr (S > 1) clean_keys<R, S / 2>(v, sel, lane);
+}
+
+// Ascending sort of R * 64 keys held as element lane * R + r: merges of
+// doubling blocks, each opened by a mirrored exchange (element i of the block
+// with SIZE - 1 - i) so that every comparison points the same way. With a
+// lane's R keys adjacent, the short strides, which are the most frequent,
+// stay in registers.
+template <int R, int SIZE>
+__device__ __forceinline__ void sort_keys(int (&v)[R], const int (&sel)[6], int lane) {
+    if constexpr (SIZE > 2) sort_keys<R, SIZE / 2>(v, sel, lane);
+    if constexpr (SIZE <= R) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int m = r ^ (SIZE - 1);
+            if (r < m) {
+                const int a = v[r], b = v[m];
+                v[r] = min(a, b);
+                v[m] = max(a, b);
+            }
+        }
+    } else {
+        constexpr int X = SIZE / R - 1;
+        int p[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) p[r] = lane_xor_key<X>(v[R - 1 - r], lane);
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = pick(v[r], p[r], sel[log2_c((X + 1) / 2)]);
+    }
+    if constexpr (SIZE >= 4) clean_keys<R, SIZE / 4>(v, sel, lane);
+}
+
+// Minimum and maximum over the 64 lanes, in every lane.
+__device__ __forceinline__ float wave_min_f(float v) {
+    auto d = [](float x, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    v = fminf(v, d(v, std::integral_constant<int, 0xB1>()));
+    v = fminf(v, d(v, std::integral_constant<int, 0x4E>()));
+    v = fminf(v, d(v, std::integral_constant<int, 0x141>()));
+    v = fminf(v, d(v, std::integral_constant<int, 0x140>()));
+    auto l = [&](int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); };
+    return fminf(fminf(l(0), l(16)), fminf(l(32), l(48)));
+}
+
+__device__ __forceinline__ float readlane_f(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// old with lane l's value replaced by the wave-uniform v (v_writelane).
+extern "C" __device__ int dcpse_writelane(int v, int l, int old) __asm("llvm.amdgcn.writelane.i32");
+
+// What a wave knows of its cell: centre, reciprocal cut-off, particles.
 template <int DIM>
-__global__ __launch_bounds__(kCellWaves * kWave) void k_support_cells_count(
+struct PairCell {
+    double ctr[3];
+    double ir;  // 1 / cut-off
+    double r2;
+    int64_t pst;
+    int np, total;  // particles; candidates kept
+};
+
+// Position x (component d) relative to the cell centre in units of the
+// cut-off: the image nearest to the centre in a periodic dimension. With at
+// least four cells per period the candidates' nearest images are the ones the
+// pair's minimum image takes wherever the pair is within the cut-off.
+template <int DIM>
+__device__ __forceinline__ float relative(const PairCell<DIM>& pc, const CellGrid& g, double x, int d) {
+    return (float)(min_image_r(x - pc.ctr[d], g.len[d], g.ilen[d], (g.periodic >> d) & 1u) * pc.ir);
+}
+
+// Sorts the cell's pc.total <= R * 64 candidate indices (in the wave's LDS
+// list), stores them to list[0 ..) and tests the cell's particles against them.
+template <int DIM, int R>
+__device__ __forceinline__ void pair_tests(const PairCell<DIM>& pc, const CellGrid& g, int64_t n,
+                                           const double* __restrict__ pos, const int32_t* __restrict__ cell_part,
+                                           const double* __restrict__ pos_cell, int32_t* keys,
+                                           int32_t* __restrict__ list, uint64_t* __restrict__ masks, int nws,
+                                           int32_t* __restrict__ counts, int32_t* __restrict__ overflow, int lane) {
+    int key[R];
+    int sel[6];
+#pragma unroll
+    for (int b = 0; b < 6; ++b) sel[b] = (lane >> b) & 1 ? INT_MAX : INT_MIN;
+#pragma unroll
+    for (int r = 0; r < R; ++r) key[r] = lane * R + r < pc.total ? keys[lane * R + r] : INT_MAX;
+    sort_keys<R, R * kWave>(key, sel, lane);
+    // to element r * 64 + lane, so that a mask word covers 64 consecutive entries
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < R; ++r) keys[lane * R + r] = key[r];
+    wave_lds_sync();
+    float cx[R][DIM];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        key[r] = keys[r * kWave + lane];
+        const bool have = r * kWave + lane < pc.total;
+        const int64_t q = have ? key[r] : 0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            const float x = relative<DIM>(pc, g, pos[d * n + q], d);
+            cx[r][d] = have ? x : 1e18f;  // padding is out of reach
+        }
+        if (have) list[r * kWave + lane] = key[r];
+    }
+    const int nw = (pc.total + kWave - 1) >> 6;
+    for (int i0 = 0; i0 < pc.np; i0 += kWave) {
+        const int m64 = min(kWave, pc.np - i0);
+        int pid = 0;
+        float xp[DIM];
+        if (lane < m64) pid = cell_part[pc.pst + i0 + lane];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
+            xp[d] = lane < m64 ? relative<DIM>(pc, g, pos_cell[d * n + pc.pst + i0 + lane], d) : 0.0f;
+        int cnt = 0;
+        constexpr int PER = kWave / R;  // particles whose mask words fill the lanes
+        for (int ib = 0; ib < m64; ib += PER) {
+            const int ie = min(PER, m64 - ib);
+            int wlo = 0, whi = 0;
+            for (int k = 0; k < ie; ++k) {
+                const int i = ib + k;
+                const int p = __builtin_amdgcn_readlane(pid, i);
+                float x[DIM];
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) x[d] = readlane_f(xp[d], i);
+                int nacc = 0;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    float d2 = 0.0f;
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) {
+                        const float t = cx[r][d] - x[d];
+                        d2 = fmaf(t, t, d2);
+                    }
+                    unsigned long long m = __ballot(d2 < 1.0f + kPairTol) & ~__ballot(key[r] == p);
+                    const unsigned long long open = m & __ballot(d2 > 1.0f - kPairTol);
+                    if (open) {  // rare: the FP64 formula on the positions themselves
+                        double a[3], b[3];
+                        const bool mine = (open >> lane) & 1u;
+                        const int64_t q = mine ? key[r] : p;
+#pragma unroll
+                        for (int d = 0; d < DIM; ++d) {
+                            a[d] = pos[d * n + p];
+                            b[d] = pos[d * n + q];
+                        }
+                        const bool near = within_cut_at<DIM>(a, b, g, pc.r2);
+                        m = (m & ~open) | (open & __ballot(near));
+                    }
+                    nacc += __popcll(m);
+                    wlo = dcpse_writelane((int)m, k * R + r, wlo);
+                    whi = dcpse_writelane((int)(m >> 32), k * R + r, whi);
+                }
+                cnt = dcpse_writelane(nacc, i, cnt);
+            }
+            if (lane < ie * R && lane % R < nw)
+                masks[(pc.pst + i0 + ib + lane / R) * nws + lane % R] = ((uint64_t)(unsigned)whi << 32) | (unsigned)wlo;
+        }
+        if (lane < m64) {
+            counts[pid] = cnt;
+            if (cnt > DCPSE_MAX_ROW) atomicOr(overflow, 1);
+        }
+    }
+}
+
+// Count pass: one wavefront per cell (see above); counts[p], the cell's
+// sorted candidates at list[c * nws * 64 ..] (ncand[c] of them) and the take
+// masks. Cells with more than nws * 64 candidates, and cells with a particle
+// far outside (which FP32 would resolve too coarsely), are appended to spill[1 ..] (spill[0] = their number, ncand -1) for
+// k_support_cells. RMAX * 64 >= nws * 64 bounds the registers.
+//
+// Bound by VALU issue: 342 candidates per cell of the 128^3 set with 10%
+// removed (rcut 2.4 spacings) shrink to about 170 within reach of the
+// particles' bounding box, are sorted in 200-odd instructions, and a pair
+// test costs 9 instructions per 64 pairs with the candidates in registers and
+// the particle in scalar registers. 0.55 ms there (1.89M particles); FP64
+// tests of every candidate from LDS took 1.14 ms, and with them the fill,
+// which then sorted every row, 0.96 ms instead of 0.22 ms (k_cell_rows).
+template <int DIM, int RMAX>
+__global__ __launch_bounds__(kPairWaves * kWave) void k_cell_pairs(
     int64_t n, const double* __restrict__ rcut, CellGrid g, const int64_t* __restrict__ cell_start,
-    const int32_t* __restrict__ cell_part, const double* __restrict__ pos_cell, int32_t* __restrict__ counts,
-    int32_t* __restrict__ overflow, uint64_t* __restrict__ masks, int nws, int32_t* __restrict__ spill) {
-    constexpr int CAP = CellCap<DIM>::v;
-    __shared__ int32_t sq[kCellWaves][CAP];
-    __shared__ double sx[kCellWaves][DIM * CAP];
-    __shared__ int32_t mark[kCellWaves][kWave];
-    __shared__ long long seg_cst[kCellWaves][kWave];
-    __shared__ int32_t seg_ex[kCellWaves][kWave];
+    const int32_t* __restrict__ cell_part, const double* __restrict__ pos_cell, const double* __restrict__ pos,
+    int32_t* __restrict__ counts, int32_t* __restrict__ overflow, int32_t* __restrict__ ncand,
+    int32_t* __restrict__ lists, uint64_t* __restrict__ masks, int nws, int32_t* __restrict__ spill) {
+    __shared__ __align__(16) int32_t kbuf[kPairWaves][RMAX * kWave];
     const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t c = (int64_t)xcd_block() * kPairWaves + wv;
+    if (c >= g.ncell) return;  // whole wavefront
+    PairCell<DIM> pc;
+    pc.pst = cell_start[c];
+    pc.np = (int)(cell_start[c + 1] - pc.pst);
+    if (pc.np == 0) return;  // never looked at by the fill either
+    int cc[3];
+    cell_coords<DIM>(g, c, cc);
     const double r = rcut[0];
-    const double r2 = r * r;
-    const unsigned G = gridDim.x;
-    for (int64_t c = (int64_t)xcd_block() * kCellWaves + wv; c < g.ncell; c += (int64_t)G * kCellWaves) {
-        const int64_t pst = cell_start[c];
-        const int np = (int)(cell_start[c + 1] - pst);
-        if (np == 0) continue;
+    pc.r2 = r * r;
+    pc.ir = 1.0 / r;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) pc.ctr[d] = g.lo[d] + (cc[d] + 0.5) * g.cs[d];
+    // bounding box of the cell's particles
+    float lo[DIM], hi[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) lo[d] = 1e30f, hi[d] = 1e30f;  // hi: of the negated coordinate
+    const double xmax = kMaxOffset * r;
+    bool wild = false;
+    for (int i0 = 0; i0 < pc.np; i0 += kWave) {
+        const bool have = i0 + lane < pc.np;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            const double xr = have ? pos_cell[d * n + pc.pst + i0 + lane] : 0.0;
+            wild |= fabs(xr) > xmax;
+            const float x = relative<DIM>(pc, g, xr, d);
+            lo[d] = fminf(lo[d], have ? x : 1e30f);
+            hi[d] = fminf(hi[d], have ? -x : 1e30f);
+        }
+    }
+    bool spilled = __ballot(wild) != 0;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        lo[d] = wave_min_f(lo[d]);
+        hi[d] = -wave_min_f(hi[d]);
+        const float far = 2.0f * (float)(g.cs[d] * pc.ir);
+        spilled |= !(lo[d] >= -far && hi[d] <= far);
+    }
+    int nacc = 0;
+    if (!spilled) {
         long long cst;
         int ccnt;
         cell_segments<DIM>(g, cell_start, c, lane, cst, ccnt);
         const int incl = wave_incl_scan(ccnt);
         const int total = __builtin_amdgcn_readlane(incl, 63);
-        if (!masked_cell(np, total, nws * kWave)) {
-            if (lane == 0) spill[1 + atomicAdd(spill, 1)] = (int32_t)c;
-            continue;
-        }
         const int excl = incl - ccnt;
-        seg_cst[wv][lane] = cst;
-        seg_ex[wv][lane] = excl;
-        // the cell's particles, one per lane in two rounds of 64
-        int pid0 = 0, pid1 = 0;
-        double x0[3] = {0.0, 0.0, 0.0}, x1[3] = {0.0, 0.0, 0.0};
-        if (lane < np) {
-            pid0 = cell_part[pst + lane];
+        const int delta = (int)cst - excl;  // slot of candidate k of this segment: k + delta
+        const unsigned long long segs = __ballot(ccnt > 0);
+        for (int base = 0; base < total; base += 4 * kWave) {
+            int off[4] = {0, 0, 0, 0};
+            for (unsigned long long m = segs; m; m &= m - 1) {
+                const int s = __builtin_ctzll(m);
+                const int ex = __builtin_amdgcn_readlane(excl, s);
+                const int dl = __builtin_amdgcn_readlane(delta, s);
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) x0[d] = pos_cell[d * n + pst + lane];
+                for (int j = 0; j < 4; ++j) off[j] = base + j * kWave + lane >= ex ? dl : off[j];
+            }
+            int q[4];
+            double x[4][DIM];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int k = base + j * kWave + lane;
+                const int64_t slot = k < total ? off[j] + k : 0;
+                q[j] = cell_part[slot];
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) x[j][d] = pos_cell[d * n + slot];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float d2 = 0.0f;  // squared distance to the box
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) {
+                    wild |= fabs(x[j][d]) > xmax;
+                    const float a = relative<DIM>(pc, g, x[j][d], d);
+                    const float t = fmaxf(fmaxf(lo[d] - a, a - hi[d]), 0.0f);
+                    d2 = fmaf(t, t, d2);
+                }
+                const bool keep = (base + j * kWave + lane < total) & (d2 < 1.0f + 4.0f * kPairTol);
+                const unsigned long long m = __ballot(keep);
+                const int at = nacc + lane_prefix(m);
+                if (keep && at < RMAX * kWave) kbuf[wv][at] = q[j];
+                nacc += __popcll(m);
+            }
         }
-        if (lane + kWave < np) {
-            pid1 = cell_part[pst + kWave + lane];
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) x1[d] = pos_cell[d * n + pst + kWave + lane];
+        spilled = nacc > nws * kWave || __ballot(wild) != 0;
+    }
+    if (spilled) {
+        if (lane == 0) {
+            spill[1 + atomicAdd(spill, 1)] = (int32_t)c;
+            ncand[c] = -1;
         }
-        int cnt0 = 0, cnt1 = 0;  // lane i: the row length of particle i (i + 64)
-        for (int c0 = 0; c0 < total; c0 += CAP) {
-            const int cn = min(CAP, total - c0);
-            if (c0 > 0) wave_lds_sync();
-            stage_candidates<DIM, true>(c0, cn, ccnt, excl, mark[wv], seg_cst[wv], seg_ex[wv], cell_part, pos_cell,
-                                        n, sq[wv], sx[wv], CAP, lane);
-            // particles i and i + 1 against the copy (each candidate read
-            // from LDS once for both): their take counts, and their mask words
-            // of the copy (lane w: word w), stored together. With `two` false
-            // only particle i.
-            auto test2 = [&](int i, int pa, const double* xa, int pb, const double* xb, bool two, int& na,
-                             int& nb) {
-                uint64_t mwa = 0, mwb = 0;
-                na = nb = 0;
-                for (int t0 = 0; t0 < cn; t0 += kWave) {
-                    const int t = min(t0 + lane, cn - 1);
-                    double xq[3];
+        return;
+    }
+    if (lane == 0) ncand[c] = nacc;
+    pc.total = nacc;
+    wave_lds_sync();
+    int32_t* list = lists + c * nws * kWave;
+    if (nacc <= RMAX / 4 * kWave)
+        pair_tests<DIM, RMAX / 4>(pc, g, n, pos, cell_part, pos_cell, kbuf[wv], list, masks, nws, counts, overflow,
+                                  lane);
+    else if (nacc <= RMAX / 2 * kWave)
+        pair_tests<DIM, RMAX / 2>(pc, g, n, pos, cell_part, pos_cell, kbuf[wv], list, masks, nws, counts, overflow,
+                                  lane);
+    else
+        pair_tests<DIM, RMAX>(pc, g, n, pos, cell_part, pos_cell, kbuf[wv], list, masks, nws, counts, overflow, lane);
+}
+
+// The rows of a cell's particles from its candidate list and the take masks.
+template <int R>
+__device__ __forceinline__ void pair_rows(int64_t pst, int np, int total, const int32_t* __restrict__ cell_part,
+                                          const int32_t* __restrict__ list, const uint64_t* __restrict__ masks, int nws,
+                                          int32_t* __restrict__ overflow, const int64_t* __restrict__ row_ptr,
+                                          int32_t* __restrict__ col, int lane) {
+    int key[R];
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) xq[d] = sx[wv][d * CAP + t];
-                    const int q = sq[wv][t];
-                    const bool valid = t0 + lane < cn;
-                    // evaluated without short-circuit: no branches in the loop
-                    const bool neara = within_cut_at<DIM>(xa, xq, g, r2);
-                    const bool nearb = within_cut_at<DIM>(xb, xq, g, r2);
-                    const unsigned long long ma = __ballot(valid & (q != pa) & neara);
-                    const unsigned long long mb = __ballot(valid & (q != pb) & nearb & two);
-                    if (lane == (t0 >> 6)) {
-                        mwa = ma;
-                        mwb = mb;
-                    }
-                    na += __popcll(ma);
-                    nb += __popcll(mb);
-                }
-                const int nw = (cn + kWave - 1) >> 6;
-                if (lane < nw) masks[(pst + i) * nws + (c0 >> 6) + lane] = mwa;
-                if (two && lane < nw) masks[(pst + i + 1) * nws + (c0 >> 6) + lane] = mwb;
-            };
-            // particle i of the cell: its index and position (lane i, or
-            // lane i - 64 of the second set)
-            auto part = [&](int i, int& pid, double* xp) {
-                if (i < kWave) {
-                    pid = __builtin_amdgcn_readlane(pid0, i);
+    for (int r = 0; r < R; ++r) key[r] = r * kWave + lane < total ? list[r * kWave + lane] : 0;
+    const int nw = (total + kWave - 1) >> 6;
+    constexpr int PER = kWave / R;
+    for (int i0 = 0; i0 < np; i0 += kWave) {
+        const int m64 = min(kWave, np - i0);
+        int64_t rs = 0;
+        int len = 0;
+        if (lane < m64) {
+            const int pid = cell_part[pst + i0 + lane];
+            rs = row_ptr[pid];
+            len = (int)(row_ptr[pid + 1] - rs);
+        }
+        for (int ib = 0; ib < m64; ib += PER) {
+            const int ie = min(PER, m64 - ib);
+            uint64_t mw = 0;
+            if (lane < ie * R && lane % R < nw) mw = masks[(pst + i0 + ib + lane / R) * nws + lane % R];
+            for (int k = 0; k < ie; ++k) {
+                const int64_t row = readlane_i64(rs, ib + k);
+                const int n = __builtin_amdgcn_readlane(len, ib + k);
+                uint64_t m[R];
+                int tot = 0;
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) xp[d] = readlane_d(x0[d], i);
-                } else {
-                    pid = __builtin_amdgcn_readlane(pid1, i - kWave);
+                for (int r = 0; r < R; ++r) {
+                    m[r] = (uint64_t)readlane_i64((int64_t)mw, k * R + r);
+                    tot += __popcll(m[r]);
+                }
+                if (tot != n) {  // counted on other positions
+                    if (lane == 0) atomicOr(overflow, 2);
+                    continue;
+                }
+                int32_t* out = col + row;
+                int at = 0;
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) xp[d] = readlane_d(x1[d], i - kWave);
-                }
-            };
-            for (int i = 0; i < np; i += 2) {
-                const bool two = i + 1 < np;
-                int pa, pb;
-                double xa[3] = {0.0, 0.0, 0.0}, xb[3] = {0.0, 0.0, 0.0};
-                part(i, pa, xa);
-                if (two) part(i + 1, pb, xb);
-                else pb = pa;
-                int na, nb;
-                test2(i, pa, xa, pb, xb, two, na, nb);
-                if (i < kWave) {
-                    if (lane == i) cnt0 += na;
-                } else if (lane == i - kWave) {
-                    cnt1 += na;
-                }
-                if (two) {
-                    if (i + 1 < kWave) {
-                        if (lane == i + 1) cnt0 += nb;
-                    } else if (lane == i + 1 - kWave) {
-                        cnt1 += nb;
-                    }
+                for (int r = 0; r < R; ++r) {
+                    if ((m[r] >> lane) & 1u) out[at + lane_prefix(m[r])] = key[r];
+                    at += __popcll(m[r]);
                 }
             }
         }
-        if (lane < np) {
-            counts[pid0] = cnt0;
-            if (cnt0 > DCPSE_MAX_ROW) atomicOr(overflow, 1);
-        }
-        if (lane + kWave < np) {
-            counts[pid1] = cnt1;
-            if (cnt1 > DCPSE_MAX_ROW) atomicOr(overflow, 1);
-        }
-        wave_lds_sync();
     }
+}
+
+// Fill pass over the cells that k_cell_pairs listed (its cell list, candidate
+// lists and masks): a wavefront per cell, four masked stores per row and
+// nothing else; bound by the stores and the instructions that address them.
+template <int RMAX>
+__global__ __launch_bounds__(kPairWaves * kWave) void k_cell_rows(
+    int64_t ncell, const int64_t* __restrict__ cell_start, const int32_t* __restrict__ cell_part,
+    const int32_t* __restrict__ ncand, const int32_t* __restrict__ lists, const uint64_t* __restrict__ masks, int nws,
+    int32_t* __restrict__ overflow, const int64_t* __restrict__ row_ptr, int32_t* __restrict__ col) {
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t c = (int64_t)xcd_block() * kPairWaves + wv;
+    if (c >= ncell) return;
+    const int64_t pst = cell_start[c];
+    const int np = (int)(cell_start[c + 1] - pst);
+    if (np == 0) return;
+    const int total = ncand[c];
+    if (total < 0) return;  // filled from positions
+    const int32_t* list = lists + c * nws * kWave;
+    if (total <= RMAX / 4 * kWave)
+        pair_rows<RMAX / 4>(pst, np, total, cell_part, list, masks, nws, overflow, row_ptr, col, lane);
+    else if (total <= RMAX / 2 * kWave)
+        pair_rows<RMAX / 2>(pst, np, total, cell_part, list, masks, nws, overflow, row_ptr, col, lane);
+    else
+        pair_rows<RMAX>(pst, np, total, cell_part, list, masks, nws, overflow, row_ptr, col, lane);
 }
 
 // Count (FILL = false: counts[p]) or fill (FILL = true: col[row_ptr[p] ..])
@@ -828,82 +1114,6 @@ __global__ __launch_bounds__(kCellWaves * kWave) void k_support_cells(
     }
 }
 
-// Fill pass over the masked cells from the masks of k_support_cells_count
-// (nws words per particle); the cell list must be the one that pass used.
-// Dynamic LDS: kCellWaves * nws * 64 candidate indices.
-template <int DIM>
-__global__ __launch_bounds__(kCellWaves * kWave) void k_support_cells_masked(
-    CellGrid g, const int64_t* __restrict__ cell_start, const int32_t* __restrict__ cell_part,
-    const uint64_t* __restrict__ masks, int nws, int32_t* __restrict__ overflow, const int64_t* __restrict__ row_ptr,
-    int32_t* __restrict__ col) {
-    constexpr int MCAP = MaskCap<DIM>::v;
-    extern __shared__ int32_t sq_dyn[];
-    __shared__ int32_t buf[kCellWaves][DCPSE_MAX_ROW];
-    __shared__ int32_t mark[kCellWaves][kWave];
-    __shared__ long long seg_cst[kCellWaves][kWave];
-    __shared__ int32_t seg_ex[kCellWaves][kWave];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    const unsigned G = gridDim.x;
-    const int mask_cap = min(nws * kWave, MCAP);
-    int32_t* sq = sq_dyn + wv * mask_cap;
-    for (int64_t c = (int64_t)xcd_block() * kCellWaves + wv; c < g.ncell; c += (int64_t)G * kCellWaves) {
-        const int64_t pst = cell_start[c];
-        const int np = (int)(cell_start[c + 1] - pst);
-        if (np == 0) continue;
-        long long cst;
-        int ccnt;
-        cell_segments<DIM>(g, cell_start, c, lane, cst, ccnt);
-        const int incl = wave_incl_scan(ccnt);
-        const int total = __builtin_amdgcn_readlane(incl, 63);
-        if (!masked_cell(np, total, mask_cap)) continue;  // filled from positions
-        const int excl = incl - ccnt;
-        seg_cst[wv][lane] = cst;
-        seg_ex[wv][lane] = excl;
-        stage_candidates<DIM, false>(0, total, ccnt, excl, mark[wv], seg_cst[wv], seg_ex[wv], cell_part, nullptr, 0,
-                                     sq, nullptr, 0, lane);
-        // row bounds of the cell's particles, one per lane in two rounds of 64
-        int64_t rs0 = 0, re0 = 0, rs1 = 0, re1 = 0;
-        if (lane < np) {
-            const int pid = cell_part[pst + lane];
-            rs0 = row_ptr[pid];
-            re0 = row_ptr[pid + 1];
-        }
-        if (lane + kWave < np) {
-            const int pid = cell_part[pst + kWave + lane];
-            rs1 = row_ptr[pid];
-            re1 = row_ptr[pid + 1];
-        }
-        const int nr = (total + kWave - 1) / kWave;
-        uint64_t mw = lane < nr ? masks[pst * nws + lane] : 0;
-        for (int i = 0; i < np; ++i) {
-            const bool second = i >= kWave;
-            const int il = i & (kWave - 1);
-            const int64_t rs = readlane_i64(second ? rs1 : rs0, il);
-            const int64_t re = readlane_i64(second ? re1 : re0, il);
-            const uint64_t cur = mw;
-            if (i + 1 < np) mw = lane < nr ? masks[(pst + i + 1) * nws + lane] : 0;
-            int nacc = 0;
-            for (int rr = 0; rr < nr; ++rr) {
-                const uint64_t m = (uint64_t)readlane_i64((int64_t)cur, rr);
-                const bool take = (m >> lane) & 1u;
-                const int at = nacc + lane_prefix(m);
-                if (take && at < DCPSE_MAX_ROW) buf[wv][at] = sq[rr * kWave + lane];
-                nacc += __popcll(m);
-            }
-            wave_lds_sync();
-            const int nn = min(nacc, DCPSE_MAX_ROW);
-            if ((int64_t)nacc != re - rs) {
-                if (lane == 0) atomicOr(overflow, 2);
-            } else {
-                store_ranked(buf[wv], nn, col + rs, lane);
-            }
-            wave_lds_sync();
-        }
-        wave_lds_sync();
-    }
-}
-
 // Cell edge about rmax / K: smaller cells than the cut-off shrink the scanned
 // volume around a particle ((2k+1)^dim cells of edge rmax/K instead of 3^dim
 // of edge rmax), and let particles with a smaller cut-off scan fewer cells.
@@ -971,6 +1181,20 @@ __global__ __launch_bounds__(kMinMaxThreads) void k_minmax(const double* __restr
     }
 }
 
+// Calls launch with the dimension and the register width of a mask of nws
+// words as compile-time values.
+template <typename F>
+static void launch_pairs(int dim, int nws, F launch) {
+    auto width = [&](auto D) {
+        if (nws <= 4) launch(D, std::integral_constant<int, 4>());
+        else if (nws <= 8) launch(D, std::integral_constant<int, 8>());
+        else if (nws <= 16) launch(D, std::integral_constant<int, 16>());
+        else launch(D, std::integral_constant<int, 32>());
+    };
+    if (dim == 2) width(std::integral_constant<int, 2>());
+    else width(std::integral_constant<int, 3>());
+}
+
 static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup, int64_t n_sup,
                                  const double* pos_dom, int64_t n_dom, const int32_t* dom_self,
                                  const double* rcut, int rcut_pp,
@@ -1027,30 +1251,37 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
     CellGrid g;
     dcpse_status st;
     // one particle set and one cut-off: a wavefront per cell of edge >= rcut
-    // while the mean candidate list of a cell is well inside what a mask
-    // covers; otherwise a wavefront per particle. Mask words per particle:
-    // about 1.3x the mean candidate count, at least one LDS copy's worth.
+    // while the mean candidate count of a cell leaves room to sort them in
+    // registers; otherwise a wavefront per particle
     bool by_cell = same && !rcut_pp && n_dom > 0;
-    int nws = 0;
+    bool paired = false;  // candidate lists and take masks (k_cell_pairs)
+    int nws = 0;          // words of a take mask
     if (by_cell) {
         if ((st = make_grid(ctx, dim, box_lo, box_hi, periodic, rmax, 1, &g))) return st;
         const double cand = (double)n_sup * (dim == 3 ? 27.0 : 9.0) / (double)g.ncell;
-        const int mcap = dim == 3 ? MaskCap<3>::v : MaskCap<2>::v;
-        const int ccap = dim == 3 ? CellCap<3>::v : CellCap<2>::v;
-        by_cell = cand <= 0.8 * mcap;
-        nws = std::min(mcap, std::max(ccap, (int)std::ceil(1.3 * cand) + kWave)) / kWave;
+        by_cell = cand <= (dim == 3 ? 1638.0 : 819.0);
+        // about half of the 3^dim cells' particles are within reach of the
+        // cell's own; lists of 0.84 of them leave room for uneven cells
+        nws = std::max(2, std::min(32, (int)std::ceil(0.84 * cand / kWave)));
+        paired = by_cell;
+        for (int d = 0; d < dim; ++d) {  // see kPairTol, relative()
+            paired = paired && g.cs[d] <= 4.0 * rmax && std::fabs(box_lo[d]) <= kMaxOffset * rmax &&
+                     std::fabs(box_hi[d]) <= kMaxOffset * rmax && (g.nc[d] >= 4 || !((periodic >> d) & 1u));
+        }
     }
     if (!by_cell && (st = make_grid(ctx, dim, box_lo, box_hi, periodic, rmax, K, &g))) return st;
     const int64_t cb = by_cell ? std::max<int64_t>(1, std::min<int64_t>((g.ncell + kCellWaves - 1) / kCellWaves,
                                                                          (int64_t)ctx->num_cus * 16))
                                : 0;
     const unsigned cell_blocks = (unsigned)(cb >= 8 ? cb / 8 * 8 : cb);
+    // one wavefront per cell, the blocks in whole rounds over the XCDs
+    const unsigned pair_blocks = (unsigned)((g.ncell + kPairWaves * 8 - 1) / (kPairWaves * 8) * 8);
 
-    // the same-set, single-cut-off fill reuses the cell list and take masks of
-    // the count just before it when the arguments match
+    // the same-set, single-cut-off fill reuses the cell list, candidate lists and
+    // take masks of the count just before it when the arguments match
     dcpse_support_cache& sc = ctx->sup;
     const bool count_pass = col == nullptr;
-    const bool cached = by_cell && !count_pass && sc.valid && sc.dim == dim && sc.pos == pos_sup &&
+    const bool cached = paired && !count_pass && sc.valid && sc.dim == dim && sc.pos == pos_sup &&
                         sc.n == n_sup && sc.rcut == rmax && sc.periodic == periodic && sc.nws == nws &&
                         std::equal(box_lo, box_lo + dim, sc.lo) && std::equal(box_hi, box_hi + dim, sc.hi);
     sc.valid = false;
@@ -1072,15 +1303,27 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
     hipStream_t s = ctx->stream;
 
     uint64_t* masks = nullptr;
-    int32_t* spill = nullptr;
-    bool use_cache = by_cell && (count_pass || cached);
+    int32_t *spill = nullptr, *ncand = nullptr, *lists = nullptr;
+    bool use_cache = paired && (count_pass || cached);
     if (use_cache) {
-        // cell list, masks and the list of cells left to the position kernel
-        // in the context's support cache
-        const size_t cap = (((size_t)(g.ncell + 1) * 8 + 255) & ~(size_t)255) +
-                           (((size_t)(n_sup + 1) * 4 + 255) & ~(size_t)255) +
-                           (((size_t)dim * (n_sup + 1) * 8 + 255) & ~(size_t)255) +
-                           (((size_t)(n_sup + 1) * nws * 8 + 255) & ~(size_t)255) + (size_t)(g.ncell + 2) * 4;
+        // cell list, candidate lists, masks and the list of cells left to the
+        // position kernel in the context's support cache
+        auto carve = [&](Workspace& cw) {
+            cell_start = cw.take<int64_t>(g.ncell + 1);
+            cell_part = cw.take<int32_t>(n_sup + 1);
+            pos_cell = cw.take<double>((size_t)dim * (n_sup + 1));
+            masks = cw.take<uint64_t>((size_t)(n_sup + 1) * nws);
+            ncand = cw.take<int32_t>(g.ncell + 1);
+            lists = cw.take<int32_t>((size_t)g.ncell * nws * kWave);
+            spill = cw.take<int32_t>(g.ncell + 2);
+        };
+        int64_t* own_start = cell_start;
+        int32_t* own_part = cell_part;
+        double* own_pos = pos_cell;
+        Workspace cw;
+        cw.cap = ~size_t(0) >> 1;
+        carve(cw);  // sizes only
+        const size_t cap = cw.used;
         if (count_pass && sc.cap < cap) {
             DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(s));
             if (sc.buf) (void)hipFree(sc.buf);
@@ -1089,24 +1332,22 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
             if (hipMalloc(&sc.buf, cap) == hipSuccess) {
                 sc.cap = cap;
             } else {
-                // no room for the masks: count from positions, and the fill
+                // no room for the lists: count from positions, and the fill
                 // (finding no matching cache) fills from positions too
                 (void)hipGetLastError();
                 sc.buf = nullptr;
                 use_cache = false;
+                cell_start = own_start, cell_part = own_part, pos_cell = own_pos;
+                masks = nullptr, spill = nullptr;
             }
         }
-    }
-    if (use_cache) {
-        Workspace cw;
-        cw.base = static_cast<char*>(sc.buf);
-        cw.cap = sc.cap;
-        cell_start = cw.take<int64_t>(g.ncell + 1);
-        cell_part = cw.take<int32_t>(n_sup + 1);
-        pos_cell = cw.take<double>((size_t)dim * (n_sup + 1));
-        masks = cw.take<uint64_t>((size_t)(n_sup + 1) * nws);
-        spill = cw.take<int32_t>(g.ncell + 2);
-        if (!spill) return fail(ctx, DCPSE_ERR_INVALID, "support cache sizing error");
+        if (use_cache) {
+            cw = Workspace();
+            cw.base = static_cast<char*>(sc.buf);
+            cw.cap = sc.cap;
+            carve(cw);
+            if (!spill) return fail(ctx, DCPSE_ERR_INVALID, "support cache sizing error");
+        }
     }
 
     fill_i32(s, flags, 64, 0);
@@ -1142,19 +1383,20 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
                     n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, nullptr, nullptr, nullptr);
             DCPSE_LAUNCH_CHECK(ctx);
         } else if (by_cell) {
-            // masked cells, then the listed others from positions
+            // candidate lists and masks, then the cells they do not cover from positions
             fill_i32(s, spill, 1, 0);
-            if (dim == 2) {
-                k_support_cells_count<2><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
-                    n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, masks, nws, spill);
+            launch_pairs(dim, nws, [&](auto D, auto R) {
+                k_cell_pairs<decltype(D)::value, decltype(R)::value><<<pair_blocks, kPairWaves * kWave, 0, s>>>(
+                    n_sup, rcut, g, cell_start, cell_part, pos_cell, pos_sup, counts, flags, ncand, lists, masks, nws,
+                    spill);
+            });
+            DCPSE_LAUNCH_CHECK(ctx);
+            if (dim == 2)
                 k_support_cells<2, false><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
                     n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, nullptr, nullptr, spill);
-            } else {
-                k_support_cells_count<3><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
-                    n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, masks, nws, spill);
+            else
                 k_support_cells<3, false><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
                     n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, nullptr, nullptr, spill);
-            }
             DCPSE_LAUNCH_CHECK(ctx);
         } else if (n_dom > 0) {
             if (dim == 2)
@@ -1198,17 +1440,14 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
         }
     } else {
         if (cached) {
-            const size_t lds = (size_t)kCellWaves * nws * kWave * sizeof(int32_t);
-            if (dim == 2)
-                k_support_cells_masked<2><<<cell_blocks, kCellWaves * kWave, lds, s>>>(g, cell_start, cell_part, masks,
-                                                                                        nws, flags, row_ptr, col);
-            else
-                k_support_cells_masked<3><<<cell_blocks, kCellWaves * kWave, lds, s>>>(g, cell_start, cell_part, masks,
-                                                                                        nws, flags, row_ptr, col);
+            launch_pairs(dim, nws, [&](auto, auto R) {
+                k_cell_rows<decltype(R)::value><<<pair_blocks, kPairWaves * kWave, 0, s>>>(
+                    g.ncell, cell_start, cell_part, ncand, lists, masks, nws, flags, row_ptr, col);
+            });
             DCPSE_LAUNCH_CHECK(ctx);
         }
         if (by_cell && (!cached || sc.spill)) {
-            // the cells the masks do not cover (cached), or all of them
+            // the cells the lists do not cover (cached), or all of them
             const int32_t* list = cached ? spill : nullptr;
             if (dim == 2)
                 k_support_cells<2, true><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
