@@ -10,17 +10,18 @@
 #include "dcpse_hip.h"
 
 // Cell list, sorted candidate lists and per-particle take masks of the last
-// same-set, single-cut-off support count; the fill that follows with the same
-// arguments writes its rows from them instead of repeating the distance tests.
+// support count of one set; the fill that follows with the same arguments
+// writes its rows from them instead of repeating the distance tests.
 struct dcpse_support_cache {
     void* buf = nullptr;  // grow-only device buffer
     size_t cap = 0;
     bool valid = false;
-    bool spill = false;   // some cells are left to the position kernel
+    bool spill = false;   // some particles are left to the position kernel
     int dim = 0;
     const double* pos = nullptr;
     int64_t n = 0;
-    double rcut = 0.0;
+    double rcut = 0.0, rmin = 0.0;  // largest and smallest cut-off
+    int rcut_pp = 0;      // a cut-off per particle
     double lo[3] = {0.0, 0.0, 0.0}, hi[3] = {0.0, 0.0, 0.0};
     unsigned periodic = 0;
     int nws = 0;          // mask words per particle

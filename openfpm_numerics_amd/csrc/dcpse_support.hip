@@ -184,37 +184,108 @@ __device__ __forceinline__ int cell_of(double x, int d, const CellGrid& g) {
     return v;
 }
 
+// A particle in cell order: position and index side by side, so that a
+// candidate is one 32-byte access, in the scattered write as in the reads
+// (a 1.89M-particle list: assignment and fill 115 us, 205 us with separate
+// arrays and a second atomic pass).
+struct __align__(16) CellRec {
+    double x[3];
+    int32_t id;
+    int32_t pad;
+};
+
 template <int DIM>
-__global__ void k_cell_assign(const double* __restrict__ pos, int64_t n, CellGrid g,
-                              int32_t* __restrict__ cell_id, int32_t* __restrict__ cell_cnt) {
+__device__ __forceinline__ int32_t cell_index(const double* x, const CellGrid& g) {
+    int64_t c = 0, stride = 1;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        c += stride * cell_of(x[d], d, g);
+        stride *= g.nc[d];
+    }
+    return (int32_t)c;
+}
+
+// Home groups of a set with a cut-off per particle: level l holds the
+// particles whose cut-off lies in (rtop / 2^(l+1), rtop / 2^l] (the last level
+// all smaller ones) on a grid of its own, of edge about kHomeEdge times the
+// level's largest cut-off; first[l] is the level's first cell in one numbering.
+// An edge of 0.85 cut-offs puts 8 to 70 particles into a group at 58
+// neighbours each: enough to share the candidates' setup, few enough that most
+// candidates are some particle's neighbours.
+constexpr int kMaxLevels = 6;
+constexpr double kHomeEdge = 0.85;
+struct HomeLevels {
+    int n;
+    double rtop;
+    CellGrid g[kMaxLevels];
+    int32_t first[kMaxLevels + 1];
+};
+
+// cell of every particle and its place within it (the order within a cell is
+// whatever the atomics give; nothing that leaves the builder depends on it).
+template <int DIM, bool HOME>
+__global__ void k_cell_assign(const double* __restrict__ pos, int64_t n, const double* __restrict__ rcut, CellGrid g,
+                              HomeLevels h, int32_t* __restrict__ cell_id, int32_t* __restrict__ rank,
+                              int32_t* __restrict__ cell_cnt, int32_t* __restrict__ home_id,
+                              int32_t* __restrict__ home_rank, int32_t* __restrict__ home_cnt) {
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
          q += (int64_t)gridDim.x * blockDim.x) {
-        int64_t c = 0, stride = 1;
+        double x[DIM];
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            c += stride * cell_of(pos[d * n + q], d, g);
-            stride *= g.nc[d];
+        for (int d = 0; d < DIM; ++d) x[d] = pos[d * n + q];
+        const int32_t c = cell_index<DIM>(x, g);
+        cell_id[q] = c;
+        rank[q] = atomicAdd(&cell_cnt[c], 1);
+        if constexpr (HOME) {
+            const double r = rcut[q];
+            int l = 0;
+            double below = 0.5 * h.rtop;
+            while (l + 1 < h.n && r <= below) {
+                ++l;
+                below *= 0.5;
+            }
+            int32_t k = 0;
+#pragma unroll
+            for (int i = 0; i < kMaxLevels; ++i)
+                if (i == l) k = h.first[i] + cell_index<DIM>(x, h.g[i]);
+            home_id[q] = k;
+            home_rank[q] = atomicAdd(&home_cnt[k], 1);
         }
-        cell_id[q] = (int32_t)c;
-        atomicAdd(&cell_cnt[c], 1);
     }
 }
 
-// cell_part[slot] = particle, and a copy of its position in cell order
-// (pos_cell[d * n + slot]) so the row kernels read candidate positions
-// contiguously per cell, without waiting for the particle index first.
-template <int DIM>
-__global__ void k_cell_fill(const int32_t* __restrict__ cell_id, int64_t n, const double* __restrict__ pos,
-                            const int64_t* __restrict__ cell_start, int32_t* __restrict__ cursor,
-                            int32_t* __restrict__ cell_part, double* __restrict__ pos_cell) {
+// The records of the particles in cell order (and in home order).
+template <int DIM, bool HOME>
+__global__ void k_cell_fill(const double* __restrict__ pos, int64_t n, const int32_t* __restrict__ cell_id,
+                            const int32_t* __restrict__ rank, const int64_t* __restrict__ cell_start,
+                            CellRec* __restrict__ rec, const int32_t* __restrict__ home_id,
+                            const int32_t* __restrict__ home_rank, const int64_t* __restrict__ home_start,
+                            CellRec* __restrict__ home_rec) {
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
          q += (int64_t)gridDim.x * blockDim.x) {
-        int32_t c = cell_id[q];
-        int64_t at = cell_start[c] + atomicAdd(&cursor[c], 1);
-        cell_part[at] = (int32_t)q;
+        CellRec r;
+        r.x[2] = 0.0;
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) pos_cell[d * n + at] = pos[d * n + q];
+        for (int d = 0; d < DIM; ++d) r.x[d] = pos[d * n + q];
+        r.id = (int32_t)q;
+        r.pad = 0;
+        rec[cell_start[cell_id[q]] + rank[q]] = r;
+        if constexpr (HOME) home_rec[home_start[home_id[q]] + home_rank[q]] = r;
     }
+}
+
+// flag[i] = whether cell i holds a particle
+__global__ void k_occupied(const int32_t* __restrict__ cnt, int64_t n, int32_t* __restrict__ flag) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        flag[i] = cnt[i] > 0;
+}
+
+// The occupied cells in order: group_cell[index[i]] = i (index: exclusive scan
+// of the flags).
+__global__ void k_group_cells(const int32_t* __restrict__ cnt, const int64_t* __restrict__ index, int64_t n,
+                              int32_t* __restrict__ group_cell) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        if (cnt[i] > 0) group_cell[index[i]] = (int32_t)i;
 }
 
 constexpr int kRowWaves = 4;  // wavefronts per block in the row kernels
@@ -324,7 +395,22 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_sort_long_rows(int64_t n_
     }
 }
 
-// One wavefront per domain particle. FILL = false: count the support of p into
+// The distance test of a candidate at xq against xp (the minimum image in
+// periodic dimensions): the one formula of every support kernel.
+template <int DIM>
+__device__ __forceinline__ bool within_cut(const double* xp, const double* xq, const CellGrid& g, double r2) {
+    double d[3];
+#pragma unroll
+    for (int dd = 0; dd < DIM; ++dd)
+        d[dd] = min_image_r(xp[dd] - xq[dd], g.len[dd], g.ilen[dd], (g.periodic >> dd) & 1u);
+    double d2 = d[DIM - 1] * d[DIM - 1];
+#pragma unroll
+    for (int dd = DIM - 2; dd >= 0; --dd) d2 = fma(d[dd], d[dd], d2);
+    return d2 < r2;
+}
+
+// One wavefront per domain particle, or with list != NULL per particle
+// list[1 ..] (list[0] = their number). FILL = false: count the support of p into
 // counts[p] (and raise *overflow if it exceeds DCPSE_MAX_ROW). FILL = true:
 // write the support of p, sorted ascending, to col[row_ptr[p] ..].
 // The cells within k_d = ceil(rcut_p / cell edge) of p's cell in each
@@ -335,19 +421,19 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_sort_long_rows(int64_t n_
 // lanes.
 template <int DIM, bool FILL>
 __global__ __launch_bounds__(kRowWaves * kWave) void k_support_rows(
-    const double* __restrict__ pos_sup, int64_t n_sup, const double* __restrict__ pos_dom,
-    int64_t n_dom, int same_set, const int32_t* __restrict__ dom_self, const double* __restrict__ rcut, int rcut_pp,
-    CellGrid g, const int64_t* __restrict__ cell_start, const int32_t* __restrict__ cell_part,
-    const double* __restrict__ pos_cell, int32_t* __restrict__ counts, int32_t* __restrict__ overflow,
-    const int64_t* __restrict__ row_ptr, int32_t* __restrict__ col) {
+    const double* __restrict__ pos_dom, int64_t n_dom, int same_set, const int32_t* __restrict__ dom_self, const double* __restrict__ rcut, int rcut_pp,
+    CellGrid g, const int64_t* __restrict__ cell_start, const CellRec* __restrict__ rec,
+    int32_t* __restrict__ counts, int32_t* __restrict__ overflow, const int64_t* __restrict__ row_ptr,
+    int32_t* __restrict__ col, const int32_t* __restrict__ list) {
     __shared__ int32_t buf[FILL ? kRowWaves : 1][FILL ? DCPSE_MAX_ROW : 1];
     __shared__ int32_t mark[kRowWaves][kWave];      // segment starting at a candidate of the round
     __shared__ long long seg_cst[kRowWaves][kWave];  // first cell slot of each segment
     __shared__ int32_t seg_ex[kRowWaves][kWave];     // candidates before each segment
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    for (int64_t p = (int64_t)blockIdx.x * kRowWaves + wv; p < n_dom;
-         p += (int64_t)gridDim.x * kRowWaves) {
+    const int64_t n_rows = list ? list[0] : n_dom;
+    for (int64_t pi = (int64_t)blockIdx.x * kRowWaves + wv; pi < n_rows; pi += (int64_t)gridDim.x * kRowWaves) {
+        const int64_t p = list ? list[1 + pi] : pi;
         double xp[3];
         int c[3] = {0, 0, 0};
 #pragma unroll
@@ -426,16 +512,9 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_support_rows(
                 const long long s_cst = seg_cst[wv][seg];
                 const int s_ex = seg_ex[wv][seg];
                 const int64_t slot = s_cst + (k - s_ex);
-                const int q = cell_part[slot];
-                double d[3];
-#pragma unroll
-                for (int dd = 0; dd < DIM; ++dd)
-                    d[dd] = min_image_r(xp[dd] - pos_cell[dd * n_sup + slot], g.len[dd], g.ilen[dd],
-                                        (g.periodic >> dd) & 1u);
-                double d2 = d[DIM - 1] * d[DIM - 1];
-#pragma unroll
-                for (int dd = DIM - 2; dd >= 0; --dd) d2 = fma(d[dd], d[dd], d2);
-                const bool take = (base + lane < total) && q != self_q && d2 < r2;
+                const CellRec cand = rec[slot];
+                const int q = cand.id;
+                const bool take = (base + lane < total) && q != self_q && within_cut<DIM>(xp, cand.x, g, r2);
                 const unsigned long long m = __ballot(take);
                 if (FILL) {
                     const int at = nacc + lane_prefix(m);
@@ -463,34 +542,23 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_support_rows(
     }
 }
 
-// ---- one set, one cut-off: a wavefront per cell of edge >= rcut -----------
-// The candidates of a cell are its 3^dim neighbouring cells, scanned as
-// 3^(dim-1) rows along dimension 0 (contiguous in the cell order, split in two
-// where a periodic wrap cuts a row), flattened into one list. The count pass
-// (k_cell_pairs) keeps the candidates within the cut-off of the bounding box
-// of the cell's particles, sorts their indices once per cell, and tests every
-// particle of the cell against them: it stores the sorted candidate list of
-// the cell and, per particle, which of them it takes (one bit each). The fill
-// (k_cell_rows) writes a particle's row as the marked entries of its cell's
-// list, which are in ascending order as they stand: no distance work and no
-// sort per row. Cells with more candidates than the list holds are left to
-// k_support_cells, which tests each particle against positions (restaging
-// them per particle when they exceed one LDS copy). All use the distance
-// formula of k_support_rows on the same positions (k_cell_pairs wherever FP32
-// leaves the outcome open), so the results are the same.
-constexpr int kCellWaves = 2;
-template <int DIM>
-struct CellCap {  // candidates per LDS copy of k_support_cells
-    static constexpr int v = DIM == 3 ? 384 : 256;
-};
-
-// Block b's cell range: consecutive logical blocks on one XCD (blocks are
-// dealt round-robin over the 8 XCDs), so neighbouring cells, which share most
-// candidates, meet in one L2.
-__device__ __forceinline__ unsigned xcd_block() {
-    const unsigned G = gridDim.x;
-    return (G % 8u == 0u) ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
-}
+// ---- one set: a wavefront per group of neighbouring particles --------------
+// A group is the particles of one home cell. With one cut-off the home cells
+// are the cells of the list (edge >= rcut) and a group's candidates those of
+// the 3^dim cells around it; with a cut-off per particle the home cells come
+// in levels by cut-off (HomeLevels) and the candidates from the cells within
+// the group's largest cut-off of its bounding box. Cells along dimension 0 are
+// consecutive in the cell order, so a row of cells is one contiguous segment of
+// candidates (two across a periodic wrap).
+// The count pass (k_group_pairs) keeps the candidates within reach of the
+// group's bounding box, sorts their indices once, and tests every particle of
+// the group against them: it stores the group's sorted candidate list and, per
+// particle, which of them it takes (one bit each). The fill (k_group_rows)
+// writes a particle's row as the marked entries of its group's list, which are
+// in ascending order as they stand: no distance work and no sort per row.
+// Particles of groups with more candidates than the list holds are left to
+// k_support_rows. All decide by within_cut (k_group_pairs wherever FP32 leaves
+// the outcome open), so the results are the same.
 
 // Cell c's coordinates (cells number below 2^31, see make_grid).
 template <int DIM>
@@ -510,10 +578,8 @@ __device__ __forceinline__ void cell_coords(const CellGrid& g, int64_t c, int (&
 // rows of three cells along dimension 0 (its part past a periodic wrap), as
 // the first cell slot cst and the length ccnt (0 for no segment).
 template <int DIM>
-__device__ __forceinline__ void cell_segments(const CellGrid& g, const int64_t* __restrict__ cell_start, int64_t c,
-                                              int lane, long long& cst, int& ccnt) {
-    int cc[3];
-    cell_coords<DIM>(g, c, cc);
+__device__ __forceinline__ void cell_segments(const CellGrid& g, const int64_t* __restrict__ cell_start,
+                                              const int (&cc)[3], int lane, int64_t& cst, int& ccnt) {
     constexpr int ROWS = DIM == 3 ? 9 : 3;
     cst = 0;
     ccnt = 0;
@@ -521,10 +587,10 @@ __device__ __forceinline__ void cell_segments(const CellGrid& g, const int64_t* 
     if (row >= ROWS) return;
     int cy = cc[1] + row % 3 - 1, cz = DIM == 3 ? cc[2] + row / 3 - 1 : 0;
     bool ok = true;
-    if ((g.periodic >> 1) & 1u) cy = (cy + g.nc[1]) % g.nc[1];
+    if ((g.periodic >> 1) & 1u) cy += cy < 0 ? g.nc[1] : cy >= g.nc[1] ? -g.nc[1] : 0;
     else ok &= cy >= 0 && cy < g.nc[1];
     if (DIM == 3) {
-        if ((g.periodic >> 2) & 1u) cz = (cz + g.nc[2]) % g.nc[2];
+        if ((g.periodic >> 2) & 1u) cz += cz < 0 ? g.nc[2] : cz >= g.nc[2] ? -g.nc[2] : 0;
         else ok &= cz >= 0 && cz < g.nc[2];
     }
     int xa = cc[0] - 1, xb = cc[0] + 1;
@@ -550,72 +616,16 @@ __device__ __forceinline__ void cell_segments(const CellGrid& g, const int64_t* 
     }
 }
 
-// Copies candidates [c0, c0 + cn) of a cell (c0 a multiple of 64) to the
-// wave's LDS slice: sq[k - c0] = particle, and with POS its position
-// sx[d * sx_stride + k - c0]. A candidate's segment is the last non-empty one
-// starting at or before it: the segment starts of each round of 64 are
-// marked, a prefix maximum spreads them, and the last one carries over.
-// seg_cst / seg_ex (each lane's segment start slot and candidates before it)
-// must be written before the call; ends with the slice readable.
-template <int DIM, bool POS>
-__device__ __forceinline__ void stage_candidates(int c0, int cn, int ccnt, int excl, int32_t* mark,
-                                                 const long long* seg_cst, const int32_t* seg_ex,
-                                                 const int32_t* __restrict__ cell_part,
-                                                 const double* __restrict__ pos_cell, int64_t n, int32_t* sq,
-                                                 double* sx, int sx_stride, int lane) {
-    int carry = 0;
-    for (int base = 0; base < c0 + cn; base += kWave) {
-        mark[lane] = -1;
-        wave_lds_sync();
-        if (ccnt > 0 && excl >= base && excl < base + kWave) mark[excl - base] = lane;
-        wave_lds_sync();
-        const int seg = max(wave_incl_max(mark[lane]), carry);
-        carry = __builtin_amdgcn_readlane(seg, 63);
-        const int k = base + lane;
-        if (base >= c0 && k < c0 + cn) {
-            const int64_t slot = seg_cst[seg] + (k - seg_ex[seg]);
-            sq[k - c0] = cell_part[slot];
-            if (POS) {
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) sx[d * sx_stride + k - c0] = pos_cell[d * n + slot];
-            }
-        }
-    }
-    wave_lds_sync();
-}
-
-// The distance test of a candidate at xq against xp (the minimum image in
-// periodic dimensions), as in k_support_rows.
-template <int DIM>
-__device__ __forceinline__ bool within_cut_at(const double* xp, const double* xq, const CellGrid& g, double r2) {
-    double d[3];
-#pragma unroll
-    for (int dd = 0; dd < DIM; ++dd)
-        d[dd] = min_image_r(xp[dd] - xq[dd], g.len[dd], g.ilen[dd], (g.periodic >> dd) & 1u);
-    double d2 = d[DIM - 1] * d[DIM - 1];
-#pragma unroll
-    for (int dd = DIM - 2; dd >= 0; --dd) d2 = fma(d[dd], d[dd], d2);
-    return d2 < r2;
-}
-
-// ... of candidate slot t of the LDS copy.
-template <int DIM>
-__device__ __forceinline__ bool within_cut(const double* xp, const double* sx, int sx_stride, int t, const CellGrid& g,
-                                           double r2) {
-    double xq[3];
-#pragma unroll
-    for (int dd = 0; dd < DIM; ++dd) xq[dd] = sx[dd * sx_stride + t];
-    return within_cut_at<DIM>(xp, xq, g, r2);
-}
-
-// Candidates are handled in coordinates relative to the cell centre, in units
-// of the cut-off, in FP32: there |a - b|^2 is within 4e-6 of the FP64 value
-// for cells up to four cut-offs wide whose positions lie within kMaxOffset
-// cut-offs of the origin (FP64 then resolves 1e-9 cut-offs), so outside
-// 1 +- kPairTol it decides the pair and inside the FP64 formula does.
+// Candidates are handled in coordinates relative to the group's centre, in
+// units of its largest cut-off, in FP32: there |a - b|^2 is within 4e-6 of the
+// FP64 value for particles up to kMaxReach from the centre whose positions lie
+// within kMaxOffset cut-offs of the origin (FP64 then resolves 1e-9 cut-offs),
+// so outside kPairTol around a particle's squared cut-off it decides the pair
+// and inside the FP64 formula does.
 constexpr float kPairTol = 2e-5f;
+constexpr float kMaxReach = 8.0f;
 constexpr double kMaxOffset = 1e7;
-constexpr int kPairWaves = 4;  // cells (wavefronts) per block
+constexpr int kPairWaves = 4;  // groups (wavefronts) per block
 
 // v of lane ^ X for the lane exchanges of the sorting network.
 template <int X>
@@ -691,7 +701,7 @@ __device__ __forceinline__ void sort_keys(int (&v)[R], const int (&sel)[6], int 
     if constexpr (SIZE >= 4) clean_keys<R, SIZE / 4>(v, sel, lane);
 }
 
-// Minimum and maximum over the 64 lanes, in every lane.
+// Minimum over the 64 lanes, in every lane.
 __device__ __forceinline__ float wave_min_f(float v) {
     auto d = [](float x, auto ctrl) {
         return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xF, 0xF, true));
@@ -711,39 +721,68 @@ __device__ __forceinline__ float readlane_f(float v, int lane) {
 // old with lane l's value replaced by the wave-uniform v (v_writelane).
 extern "C" __device__ int dcpse_writelane(int v, int l, int old) __asm("llvm.amdgcn.writelane.i32");
 
-// What a wave knows of its cell: centre, reciprocal cut-off, particles.
-template <int DIM>
-struct PairCell {
+// The groups of a pass and where its results go.
+struct Groups {
+    int64_t n;                   // particles
+    const double* pos;           // by particle
+    const double* rcut;          // one, or one per particle (PP)
+    CellGrid g;                  // candidate cells
+    const int64_t* cell_start;
+    const CellRec* rec;          // by candidate cell
+    const int64_t* home_start;   // by home cell
+    const CellRec* home;
+    const int32_t* group_cell;   // home cell of each group, or NULL: every home cell is a group
+    const int64_t* n_groups;     // on the device, or NULL: max_groups
+    int64_t max_groups;          // groups with a list; the others' particles are spilled
+    int32_t* counts;
+    int32_t* flags;
+    int32_t* ncand;              // candidates of a group, -1: spilled
+    int32_t* lists;              // nws * 64 entries per group
+    uint64_t* masks;             // nws words per home slot
+    int nws;
+    int32_t* spill;
+};
+
+// The group of this wavefront, -1 for none: consecutive groups, which share
+// most candidates, on one XCD (blocks are dealt round-robin over the 8 XCDs).
+__device__ __forceinline__ int64_t wave_group(const Groups& a) {
+    const int64_t ng = a.n_groups ? *a.n_groups : a.max_groups;
+    const int64_t per = (ng + 8 * kPairWaves - 1) / (8 * kPairWaves);  // blocks per XCD
+    const int64_t i = blockIdx.x >> 3;
+    if (i >= per) return -1;
+    const int64_t gi =
+        ((blockIdx.x & 7) * per + i) * kPairWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    return gi < ng ? gi : -1;
+}
+
+// What a wave knows of its group: centre, unit of length, particles.
+struct PairGroup {
     double ctr[3];
-    double ir;  // 1 / cut-off
-    double r2;
+    double unit, iunit;
     int64_t pst;
     int np, total;  // particles; candidates kept
 };
 
-// Position x (component d) relative to the cell centre in units of the
-// cut-off: the image nearest to the centre in a periodic dimension. With at
-// least four cells per period the candidates' nearest images are the ones the
-// pair's minimum image takes wherever the pair is within the cut-off.
-template <int DIM>
-__device__ __forceinline__ float relative(const PairCell<DIM>& pc, const CellGrid& g, double x, int d) {
-    return (float)(min_image_r(x - pc.ctr[d], g.len[d], g.ilen[d], (g.periodic >> d) & 1u) * pc.ir);
+// Position x (component d) relative to the group's centre: the image nearest
+// to it in a periodic dimension. The period exceeds the home cell and two
+// cut-offs, so wherever a pair is within the cut-off these images are the ones
+// its minimum image takes.
+__device__ __forceinline__ float relative(const PairGroup& pg, const CellGrid& g, double x, int d) {
+    return (float)(min_image_r(x - pg.ctr[d], g.len[d], g.ilen[d], (g.periodic >> d) & 1u) * pg.iunit);
 }
 
-// Sorts the cell's pc.total <= R * 64 candidate indices (in the wave's LDS
-// list), stores them to list[0 ..) and tests the cell's particles against them.
-template <int DIM, int R>
-__device__ __forceinline__ void pair_tests(const PairCell<DIM>& pc, const CellGrid& g, int64_t n,
-                                           const double* __restrict__ pos, const int32_t* __restrict__ cell_part,
-                                           const double* __restrict__ pos_cell, int32_t* keys,
-                                           int32_t* __restrict__ list, uint64_t* __restrict__ masks, int nws,
-                                           int32_t* __restrict__ counts, int32_t* __restrict__ overflow, int lane) {
+// Sorts the group's pg.total <= R * 64 candidate indices (in the wave's LDS
+// list), stores them and tests the group's particles against them.
+template <int DIM, int R, bool PP>
+__device__ __forceinline__ void pair_tests(const Groups& a, const PairGroup& pg, int64_t gi, int32_t* keys, int lane) {
+    const int64_t n = a.n;
+    int32_t* __restrict__ list = a.lists + gi * a.nws * kWave;
     int key[R];
     int sel[6];
 #pragma unroll
     for (int b = 0; b < 6; ++b) sel[b] = (lane >> b) & 1 ? INT_MAX : INT_MIN;
 #pragma unroll
-    for (int r = 0; r < R; ++r) key[r] = lane * R + r < pc.total ? keys[lane * R + r] : INT_MAX;
+    for (int r = 0; r < R; ++r) key[r] = lane * R + r < pg.total ? keys[lane * R + r] : INT_MAX;
     sort_keys<R, R * kWave>(key, sel, lane);
     // to element r * 64 + lane, so that a mask word covers 64 consecutive entries
     wave_lds_sync();
@@ -754,24 +793,32 @@ __device__ __forceinline__ void pair_tests(const PairCell<DIM>& pc, const CellGr
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         key[r] = keys[r * kWave + lane];
-        const bool have = r * kWave + lane < pc.total;
+        const bool have = r * kWave + lane < pg.total;
         const int64_t q = have ? key[r] : 0;
 #pragma unroll
         for (int d = 0; d < DIM; ++d) {
-            const float x = relative<DIM>(pc, g, pos[d * n + q], d);
+            const float x = relative(pg, a.g, a.pos[d * n + q], d);
             cx[r][d] = have ? x : 1e18f;  // padding is out of reach
         }
         if (have) list[r * kWave + lane] = key[r];
     }
-    const int nw = (pc.total + kWave - 1) >> 6;
-    for (int i0 = 0; i0 < pc.np; i0 += kWave) {
-        const int m64 = min(kWave, pc.np - i0);
+    const int nw = (pg.total + kWave - 1) >> 6;
+    for (int i0 = 0; i0 < pg.np; i0 += kWave) {
+        const int m64 = min(kWave, pg.np - i0);
         int pid = 0;
         float xp[DIM];
-        if (lane < m64) pid = cell_part[pc.pst + i0 + lane];
+        float t2 = 1.0f;  // squared cut-off
+        {
+            const CellRec h = a.home[pg.pst + i0 + min(lane, m64 - 1)];
+            pid = h.id;
 #pragma unroll
-        for (int d = 0; d < DIM; ++d)
-            xp[d] = lane < m64 ? relative<DIM>(pc, g, pos_cell[d * n + pc.pst + i0 + lane], d) : 0.0f;
+            for (int d = 0; d < DIM; ++d) xp[d] = relative(pg, a.g, h.x[d], d);
+            if (PP) {
+                const double rc = a.rcut[pid];
+                const float t = (float)(rc * pg.iunit);
+                t2 = rc > 0.0 ? t * t : -1.0f;
+            }
+        }
         int cnt = 0;
         constexpr int PER = kWave / R;  // particles whose mask words fill the lanes
         for (int ib = 0; ib < m64; ib += PER) {
@@ -783,28 +830,30 @@ __device__ __forceinline__ void pair_tests(const PairCell<DIM>& pc, const CellGr
                 float x[DIM];
 #pragma unroll
                 for (int d = 0; d < DIM; ++d) x[d] = readlane_f(xp[d], i);
+                const float t = PP ? readlane_f(t2, i) : 1.0f;
+                const float tin = t - kPairTol, tout = t + kPairTol;
                 int nacc = 0;
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     float d2 = 0.0f;
 #pragma unroll
                     for (int d = 0; d < DIM; ++d) {
-                        const float t = cx[r][d] - x[d];
-                        d2 = fmaf(t, t, d2);
+                        const float u = cx[r][d] - x[d];
+                        d2 = fmaf(u, u, d2);
                     }
-                    unsigned long long m = __ballot(d2 < 1.0f + kPairTol) & ~__ballot(key[r] == p);
-                    const unsigned long long open = m & __ballot(d2 > 1.0f - kPairTol);
+                    unsigned long long m = __ballot(d2 < tout) & ~__ballot(key[r] == p);
+                    const unsigned long long open = m & __ballot(d2 > tin);
                     if (open) {  // rare: the FP64 formula on the positions themselves
-                        double a[3], b[3];
+                        double xa[3], xb[3];
                         const bool mine = (open >> lane) & 1u;
                         const int64_t q = mine ? key[r] : p;
+                        const double rc = a.rcut[PP ? p : 0];
 #pragma unroll
                         for (int d = 0; d < DIM; ++d) {
-                            a[d] = pos[d * n + p];
-                            b[d] = pos[d * n + q];
+                            xa[d] = a.pos[d * n + p];
+                            xb[d] = a.pos[d * n + q];
                         }
-                        const bool near = within_cut_at<DIM>(a, b, g, pc.r2);
-                        m = (m & ~open) | (open & __ballot(near));
+                        m = (m & ~open) | (open & __ballot(within_cut<DIM>(xa, xb, a.g, rc * rc)));
                     }
                     nacc += __popcll(m);
                     wlo = dcpse_writelane((int)m, k * R + r, wlo);
@@ -813,20 +862,20 @@ __device__ __forceinline__ void pair_tests(const PairCell<DIM>& pc, const CellGr
                 cnt = dcpse_writelane(nacc, i, cnt);
             }
             if (lane < ie * R && lane % R < nw)
-                masks[(pc.pst + i0 + ib + lane / R) * nws + lane % R] = ((uint64_t)(unsigned)whi << 32) | (unsigned)wlo;
+                a.masks[(pg.pst + i0 + ib + lane / R) * a.nws + lane % R] =
+                    ((uint64_t)(unsigned)whi << 32) | (unsigned)wlo;
         }
         if (lane < m64) {
-            counts[pid] = cnt;
-            if (cnt > DCPSE_MAX_ROW) atomicOr(overflow, 1);
+            a.counts[pid] = cnt;
+            if (cnt > DCPSE_MAX_ROW) atomicOr(a.flags, 1);
         }
     }
 }
 
-// Count pass: one wavefront per cell (see above); counts[p], the cell's
-// sorted candidates at list[c * nws * 64 ..] (ncand[c] of them) and the take
-// masks. Cells with more than nws * 64 candidates, and cells with a particle
-// far outside (which FP32 would resolve too coarsely), are appended to spill[1 ..] (spill[0] = their number, ncand -1) for
-// k_support_cells. RMAX * 64 >= nws * 64 bounds the registers.
+// Count pass: one wavefront per group (see above). Groups beyond max_groups,
+// with more than nws * 64 candidates or with a particle that FP32 would
+// resolve too coarsely go to the spill list (spill[0] particles at spill[1 ..]).
+// RMAX * 64 >= nws * 64 bounds the registers.
 //
 // Bound by VALU issue: 342 candidates per cell of the 128^3 set with 10%
 // removed (rcut 2.4 spacings) shrink to about 170 within reach of the
@@ -834,129 +883,249 @@ __device__ __forceinline__ void pair_tests(const PairCell<DIM>& pc, const CellGr
 // test costs 9 instructions per 64 pairs with the candidates in registers and
 // the particle in scalar registers. 0.55 ms there (1.89M particles); FP64
 // tests of every candidate from LDS took 1.14 ms, and with them the fill,
-// which then sorted every row, 0.96 ms instead of 0.22 ms (k_cell_rows).
-template <int DIM, int RMAX>
-__global__ __launch_bounds__(kPairWaves * kWave) void k_cell_pairs(
-    int64_t n, const double* __restrict__ rcut, CellGrid g, const int64_t* __restrict__ cell_start,
-    const int32_t* __restrict__ cell_part, const double* __restrict__ pos_cell, const double* __restrict__ pos,
-    int32_t* __restrict__ counts, int32_t* __restrict__ overflow, int32_t* __restrict__ ncand,
-    int32_t* __restrict__ lists, uint64_t* __restrict__ masks, int nws, int32_t* __restrict__ spill) {
+// which then sorted every row, 0.96 ms instead of 0.22 ms (k_group_rows).
+// With a cut-off per particle (PP; 490,000 particles, spacing 4 : 1): 0.33 ms
+// and a fill of 0.11 ms, against 1.08 and 1.22 ms of k_support_rows, whose
+// wavefronts each flatten and test the candidates of one particle.
+template <int DIM, int RMAX, bool PP>
+__global__ __launch_bounds__(kPairWaves * kWave) void k_group_pairs(const Groups a, const HomeLevels h) {
     __shared__ __align__(16) int32_t kbuf[kPairWaves][RMAX * kWave];
+    __shared__ int32_t marks[PP ? kPairWaves : 1][PP ? 4 * kWave : 1];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t c = (int64_t)xcd_block() * kPairWaves + wv;
-    if (c >= g.ncell) return;  // whole wavefront
-    PairCell<DIM> pc;
-    pc.pst = cell_start[c];
-    pc.np = (int)(cell_start[c + 1] - pc.pst);
-    if (pc.np == 0) return;  // never looked at by the fill either
+    const int64_t gi = wave_group(a);
+    if (gi < 0) return;  // whole wavefront
+    const int64_t c = a.group_cell ? a.group_cell[gi] : gi;
+    const CellGrid& g = a.g;
+    PairGroup pg;
+    pg.pst = a.home_start[c];
+    pg.np = (int)(a.home_start[c + 1] - pg.pst);
+    if (pg.np == 0) return;  // never looked at by the fill either
     int cc[3];
-    cell_coords<DIM>(g, c, cc);
-    const double r = rcut[0];
-    pc.r2 = r * r;
-    pc.ir = 1.0 / r;
+    if constexpr (PP) {
+        int l = 0;
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) pc.ctr[d] = g.lo[d] + (cc[d] + 0.5) * g.cs[d];
-    // bounding box of the cell's particles
+        for (int i = 1; i < kMaxLevels; ++i)
+            if (i < h.n && c >= h.first[i]) l = i;
+        const CellGrid& hg = h.g[l];
+        cell_coords<DIM>(hg, c - h.first[l], cc);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) pg.ctr[d] = hg.lo[d] + (cc[d] + 0.5) * hg.cs[d];
+        float rm = 0.0f;
+        for (int i0 = 0; i0 < pg.np; i0 += kWave)
+            if (i0 + lane < pg.np) rm = fmaxf(rm, (float)a.rcut[a.home[pg.pst + i0 + lane].id]);
+        // a little above the largest cut-off: every particle's lies within the unit
+        pg.unit = fmax((double)(-wave_min_f(-rm)) * 1.0000005, 1e-6 * h.rtop);
+    } else {
+        cell_coords<DIM>(g, c, cc);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) pg.ctr[d] = g.lo[d] + (cc[d] + 0.5) * g.cs[d];
+        pg.unit = a.rcut[0];
+    }
+    pg.iunit = 1.0 / pg.unit;
+    const double xmax = kMaxOffset * pg.unit;
+    // bounding box of the group
     float lo[DIM], hi[DIM];
+    bool wild = gi >= a.max_groups;
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) lo[d] = 1e30f, hi[d] = 1e30f;  // hi: of the negated coordinate
-    const double xmax = kMaxOffset * r;
-    bool wild = false;
-    for (int i0 = 0; i0 < pc.np; i0 += kWave) {
-        const bool have = i0 + lane < pc.np;
+    for (int d = 0; d < DIM; ++d) lo[d] = hi[d] = 1e30f;  // hi: of the negated coordinate
+    for (int i0 = 0; i0 < pg.np; i0 += kWave) {
+        const CellRec r = a.home[pg.pst + min(i0 + lane, pg.np - 1)];
 #pragma unroll
         for (int d = 0; d < DIM; ++d) {
-            const double xr = have ? pos_cell[d * n + pc.pst + i0 + lane] : 0.0;
-            wild |= fabs(xr) > xmax;
-            const float x = relative<DIM>(pc, g, xr, d);
-            lo[d] = fminf(lo[d], have ? x : 1e30f);
-            hi[d] = fminf(hi[d], have ? -x : 1e30f);
+            wild |= fabs(r.x[d]) > xmax;
+            const float x = relative(pg, g, r.x[d], d);
+            lo[d] = fminf(lo[d], x);
+            hi[d] = fminf(hi[d], -x);
         }
     }
-    bool spilled = __ballot(wild) != 0;
 #pragma unroll
     for (int d = 0; d < DIM; ++d) {
         lo[d] = wave_min_f(lo[d]);
         hi[d] = -wave_min_f(hi[d]);
-        const float far = 2.0f * (float)(g.cs[d] * pc.ir);
-        spilled |= !(lo[d] >= -far && hi[d] <= far);
+        wild |= !(lo[d] >= -kMaxReach && hi[d] <= kMaxReach);
     }
     int nacc = 0;
+    // keeps those of four candidates per lane that are within reach of the box
+    auto take4 = [&](const int64_t (&slot)[4], const bool (&have)[4]) {
+        CellRec r[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[j] = a.rec[slot[j]];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float d2 = 0.0f;  // squared distance to the box
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) {
+                wild |= fabs(r[j].x[d]) > xmax;
+                const float x = relative(pg, g, r[j].x[d], d);
+                const float t = fmaxf(fmaxf(lo[d] - x, x - hi[d]), 0.0f);
+                d2 = fmaf(t, t, d2);
+            }
+            const bool keep = have[j] & (d2 < 1.0f + 4.0f * kPairTol);
+            const unsigned long long m = __ballot(keep);
+            const int at = nacc + lane_prefix(m);
+            if (keep && at < RMAX * kWave) kbuf[wv][at] = r[j].id;
+            nacc += __popcll(m);
+        }
+    };
+    bool spilled = __ballot(wild) != 0;
     if (!spilled) {
-        long long cst;
-        int ccnt;
-        cell_segments<DIM>(g, cell_start, c, lane, cst, ccnt);
-        const int incl = wave_incl_scan(ccnt);
-        const int total = __builtin_amdgcn_readlane(incl, 63);
-        const int excl = incl - ccnt;
-        const int delta = (int)cst - excl;  // slot of candidate k of this segment: k + delta
-        const unsigned long long segs = __ballot(ccnt > 0);
-        for (int base = 0; base < total; base += 4 * kWave) {
-            int off[4] = {0, 0, 0, 0};
-            for (unsigned long long m = segs; m; m &= m - 1) {
-                const int s = __builtin_ctzll(m);
-                const int ex = __builtin_amdgcn_readlane(excl, s);
-                const int dl = __builtin_amdgcn_readlane(delta, s);
+        if constexpr (PP) {
+            // cells within the cut-off of the box, a dimension at a time (unwrapped)
+            int ia[3] = {0, 0, 0}, ib[3] = {0, 0, 0};
+            bool whole[3] = {false, false, false};
 #pragma unroll
-                for (int j = 0; j < 4; ++j) off[j] = base + j * kWave + lane >= ex ? dl : off[j];
-            }
-            int q[4];
-            double x[4][DIM];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int k = base + j * kWave + lane;
-                const int64_t slot = k < total ? off[j] + k : 0;
-                q[j] = cell_part[slot];
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) x[j][d] = pos_cell[d * n + slot];
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float d2 = 0.0f;  // squared distance to the box
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) {
-                    wild |= fabs(x[j][d]) > xmax;
-                    const float a = relative<DIM>(pc, g, x[j][d], d);
-                    const float t = fmaxf(fmaxf(lo[d] - a, a - hi[d]), 0.0f);
-                    d2 = fmaf(t, t, d2);
+            for (int d = 0; d < DIM; ++d) {
+                const double ics = 1.0 / g.cs[d], at = pg.ctr[d] - g.lo[d];
+                ia[d] = (int)floor((at + ((double)lo[d] - 1.0001) * pg.unit) * ics);
+                ib[d] = (int)floor((at + ((double)hi[d] + 1.0001) * pg.unit) * ics);
+                if (!((g.periodic >> d) & 1u)) {
+                    ia[d] = min(max(ia[d], 0), g.nc[d] - 1);
+                    ib[d] = min(max(ib[d], 0), g.nc[d] - 1);
+                } else if (ib[d] - ia[d] + 1 >= g.nc[d]) {
+                    whole[d] = true;
+                    ia[d] = 0;
+                    ib[d] = g.nc[d] - 1;
                 }
-                const bool keep = (base + j * kWave + lane < total) & (d2 < 1.0f + 4.0f * kPairTol);
-                const unsigned long long m = __ballot(keep);
-                const int at = nacc + lane_prefix(m);
-                if (keep && at < RMAX * kWave) kbuf[wv][at] = q[j];
-                nacc += __popcll(m);
+            }
+            const int ny = ib[1] - ia[1] + 1;
+            const int rows = DIM == 3 ? ny * (ib[2] - ia[2] + 1) : ny;
+            // distance of the box from the slab of cell index v of dimension d
+            auto gap = [&](int v, int d) {
+                const double s0 = (g.lo[d] + v * g.cs[d] - pg.ctr[d]) * pg.iunit;
+                const float below = (float)(s0 - hi[d]), above = (float)(lo[d] - (s0 + g.cs[d] * pg.iunit));
+                float t = fmaxf(below, above) - 1e-4f;
+                if (!((g.periodic >> d) & 1u)) {  // the outermost cells hold what lies outside
+                    if (v == 0) t = above - 1e-4f;
+                    if (v == g.nc[d] - 1) t = v == 0 ? 0.0f : below - 1e-4f;
+                }
+                return whole[d] ? 0.0f : fmaxf(t, 0.0f);
+            };
+            for (int rb = 0; rb < rows; rb += kWave / 2) {
+                // lane 2i (+1): row rb + i (its part past a periodic wrap)
+                int64_t cst = 0;
+                int ccnt = 0;
+                const int row = rb + (lane >> 1), part = lane & 1;
+                if (row < rows) {
+                    const int oz = DIM == 3 ? (int)((unsigned)row / (unsigned)ny) : 0;
+                    int cy = ia[1] + row - oz * ny, cz = ia[2] + oz;
+                    const float gy = gap(cy, 1), gz = DIM == 3 ? gap(cz, 2) : 0.0f;
+                    const float rest = 1.0001f - fmaf(gy, gy, gz * gz);
+                    if (rest > 0.0f) {
+                        const double half = (double)sqrtf(rest) + 1e-4;
+                        const double at = pg.ctr[0] - g.lo[0], ics = 1.0 / g.cs[0];
+                        int xa = ia[0], xb = ib[0];
+                        if (!whole[0]) {  // (ia, ib are clamped in an open dimension: so are these)
+                            xa = min(max(xa, (int)floor((at + (lo[0] - half) * pg.unit) * ics)), ib[0]);
+                            xb = max(min(xb, (int)floor((at + (hi[0] + half) * pg.unit) * ics)), ia[0]);
+                        }
+                        if ((g.periodic >> 1) & 1u) cy += cy < 0 ? g.nc[1] : cy >= g.nc[1] ? -g.nc[1] : 0;
+                        if (DIM == 3 && ((g.periodic >> 2) & 1u))
+                            cz += cz < 0 ? g.nc[2] : cz >= g.nc[2] ? -g.nc[2] : 0;
+                        bool ok = xa <= xb;
+                        if (xa < 0) {  // wraps below: [xa + nc, nc) and [0, xb]
+                            if (xb < 0) xa += g.nc[0], xb += g.nc[0], ok &= part == 0;
+                            else if (part == 0) xa += g.nc[0], xb = g.nc[0] - 1;
+                            else xa = 0;
+                        } else if (xb >= g.nc[0]) {
+                            if (xa >= g.nc[0]) xa -= g.nc[0], xb -= g.nc[0], ok &= part == 0;
+                            else if (part == 0) xb = g.nc[0] - 1;
+                            else xa = 0, xb -= g.nc[0];
+                        } else {
+                            ok &= part == 0;
+                        }
+                        if (ok) {
+                            const int64_t lin = (int64_t)g.nc[0] * ((int64_t)cy + (int64_t)g.nc[1] * cz);
+                            cst = a.cell_start[lin + xa];
+                            ccnt = (int)(a.cell_start[lin + xb + 1] - cst);
+                        }
+                    }
+                }
+                const int incl = wave_incl_scan(ccnt);
+                const int total = __builtin_amdgcn_readlane(incl, 63);
+                const int excl = incl - ccnt;
+                const int delta = (int)cst - excl;  // slot of candidate k of this segment: k + delta
+                // segment of candidate k: the last non-empty one starting at or
+                // before it. Each round marks the starts inside its 256
+                // candidates, a prefix maximum spreads them, and the last one
+                // carries over.
+                int32_t* mark = marks[wv];
+                int carry = 0;
+                for (int base = 0; base < total; base += 4 * kWave) {
+                    wave_lds_sync();
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) mark[j * kWave + lane] = -1;
+                    wave_lds_sync();
+                    if (ccnt > 0 && excl >= base && excl < base + 4 * kWave) mark[excl - base] = lane;
+                    wave_lds_sync();
+                    int64_t slot[4];
+                    bool have[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int seg = max(wave_incl_max(mark[j * kWave + lane]), carry);
+                        carry = __builtin_amdgcn_readlane(seg, 63);
+                        const int k = base + j * kWave + lane;
+                        have[j] = k < total;
+                        const int dl = __builtin_amdgcn_ds_bpermute(seg << 2, delta);
+                        slot[j] = have[j] ? k + dl : 0;
+                    }
+                    take4(slot, have);
+                }
+            }
+        } else {
+            int64_t cst;
+            int ccnt;
+            cell_segments<DIM>(g, a.cell_start, cc, lane, cst, ccnt);
+            const int incl = wave_incl_scan(ccnt);
+            const int total = __builtin_amdgcn_readlane(incl, 63);
+            const int excl = incl - ccnt;
+            const int delta = (int)cst - excl;  // slot of candidate k of this segment: k + delta
+            const unsigned long long segs = __ballot(ccnt > 0);
+            for (int base = 0; base < total; base += 4 * kWave) {
+                int off[4] = {0, 0, 0, 0};
+                for (unsigned long long m = segs; m; m &= m - 1) {
+                    const int s = __builtin_ctzll(m);
+                    const int ex = __builtin_amdgcn_readlane(excl, s);
+                    const int dl = __builtin_amdgcn_readlane(delta, s);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) off[j] = base + j * kWave + lane >= ex ? dl : off[j];
+                }
+                int64_t slot[4];
+                bool have[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int k = base + j * kWave + lane;
+                    have[j] = k < total;
+                    slot[j] = have[j] ? k + off[j] : 0;
+                }
+                take4(slot, have);
             }
         }
-        spilled = nacc > nws * kWave || __ballot(wild) != 0;
+        spilled = nacc > a.nws * kWave || __ballot(wild) != 0;
     }
     if (spilled) {
+        int at = 0;
         if (lane == 0) {
-            spill[1 + atomicAdd(spill, 1)] = (int32_t)c;
-            ncand[c] = -1;
+            at = 1 + atomicAdd(a.spill, pg.np);
+            if (gi < a.max_groups) a.ncand[gi] = -1;
         }
+        at = __builtin_amdgcn_readfirstlane(at);
+        for (int i = lane; i < pg.np; i += kWave) a.spill[at + i] = a.home[pg.pst + i].id;
         return;
     }
-    if (lane == 0) ncand[c] = nacc;
-    pc.total = nacc;
+    if (lane == 0) a.ncand[gi] = nacc;
+    pg.total = nacc;
     wave_lds_sync();
-    int32_t* list = lists + c * nws * kWave;
-    if (nacc <= RMAX / 4 * kWave)
-        pair_tests<DIM, RMAX / 4>(pc, g, n, pos, cell_part, pos_cell, kbuf[wv], list, masks, nws, counts, overflow,
-                                  lane);
-    else if (nacc <= RMAX / 2 * kWave)
-        pair_tests<DIM, RMAX / 2>(pc, g, n, pos, cell_part, pos_cell, kbuf[wv], list, masks, nws, counts, overflow,
-                                  lane);
-    else
-        pair_tests<DIM, RMAX>(pc, g, n, pos, cell_part, pos_cell, kbuf[wv], list, masks, nws, counts, overflow, lane);
+    if (nacc <= RMAX / 4 * kWave) pair_tests<DIM, RMAX / 4, PP>(a, pg, gi, kbuf[wv], lane);
+    else if (nacc <= RMAX / 2 * kWave) pair_tests<DIM, RMAX / 2, PP>(a, pg, gi, kbuf[wv], lane);
+    else pair_tests<DIM, RMAX, PP>(a, pg, gi, kbuf[wv], lane);
 }
 
-// The rows of a cell's particles from its candidate list and the take masks.
+// The rows of a group's particles from its candidate list and the take masks.
 template <int R>
-__device__ __forceinline__ void pair_rows(int64_t pst, int np, int total, const int32_t* __restrict__ cell_part,
-                                          const int32_t* __restrict__ list, const uint64_t* __restrict__ masks, int nws,
-                                          int32_t* __restrict__ overflow, const int64_t* __restrict__ row_ptr,
-                                          int32_t* __restrict__ col, int lane) {
+__device__ __forceinline__ void pair_rows(const Groups& a, int64_t gi, int64_t pst, int np, int total,
+                                          const int64_t* __restrict__ row_ptr, int32_t* __restrict__ col, int lane) {
+    const int32_t* __restrict__ list = a.lists + gi * a.nws * kWave;
     int key[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) key[r] = r * kWave + lane < total ? list[r * kWave + lane] : 0;
@@ -967,14 +1136,14 @@ __device__ __forceinline__ void pair_rows(int64_t pst, int np, int total, const 
         int64_t rs = 0;
         int len = 0;
         if (lane < m64) {
-            const int pid = cell_part[pst + i0 + lane];
+            const int pid = a.home[pst + i0 + lane].id;
             rs = row_ptr[pid];
             len = (int)(row_ptr[pid + 1] - rs);
         }
         for (int ib = 0; ib < m64; ib += PER) {
             const int ie = min(PER, m64 - ib);
             uint64_t mw = 0;
-            if (lane < ie * R && lane % R < nw) mw = masks[(pst + i0 + ib + lane / R) * nws + lane % R];
+            if (lane < ie * R && lane % R < nw) mw = a.masks[(pst + i0 + ib + lane / R) * a.nws + lane % R];
             for (int k = 0; k < ie; ++k) {
                 const int64_t row = readlane_i64(rs, ib + k);
                 const int n = __builtin_amdgcn_readlane(len, ib + k);
@@ -986,7 +1155,7 @@ __device__ __forceinline__ void pair_rows(int64_t pst, int np, int total, const 
                     tot += __popcll(m[r]);
                 }
                 if (tot != n) {  // counted on other positions
-                    if (lane == 0) atomicOr(overflow, 2);
+                    if (lane == 0) atomicOr(a.flags, 2);
                     continue;
                 }
                 int32_t* out = col + row;
@@ -1001,117 +1170,25 @@ __device__ __forceinline__ void pair_rows(int64_t pst, int np, int total, const 
     }
 }
 
-// Fill pass over the cells that k_cell_pairs listed (its cell list, candidate
-// lists and masks): a wavefront per cell, four masked stores per row and
-// nothing else; bound by the stores and the instructions that address them.
+// Fill pass over the groups that k_group_pairs listed: a wavefront per group,
+// a masked store per 64 candidates of a row and nothing else; bound by the
+// stores and the instructions that address them.
 template <int RMAX>
-__global__ __launch_bounds__(kPairWaves * kWave) void k_cell_rows(
-    int64_t ncell, const int64_t* __restrict__ cell_start, const int32_t* __restrict__ cell_part,
-    const int32_t* __restrict__ ncand, const int32_t* __restrict__ lists, const uint64_t* __restrict__ masks, int nws,
-    int32_t* __restrict__ overflow, const int64_t* __restrict__ row_ptr, int32_t* __restrict__ col) {
+__global__ __launch_bounds__(kPairWaves * kWave) void k_group_rows(const Groups a,
+                                                                   const int64_t* __restrict__ row_ptr,
+                                                                   int32_t* __restrict__ col) {
     const int lane = threadIdx.x & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t c = (int64_t)xcd_block() * kPairWaves + wv;
-    if (c >= ncell) return;
-    const int64_t pst = cell_start[c];
-    const int np = (int)(cell_start[c + 1] - pst);
+    const int64_t gi = wave_group(a);
+    if (gi < 0 || gi >= a.max_groups) return;  // beyond: filled from positions
+    const int64_t c = a.group_cell ? a.group_cell[gi] : gi;
+    const int64_t pst = a.home_start[c];
+    const int np = (int)(a.home_start[c + 1] - pst);
     if (np == 0) return;
-    const int total = ncand[c];
+    const int total = a.ncand[gi];
     if (total < 0) return;  // filled from positions
-    const int32_t* list = lists + c * nws * kWave;
-    if (total <= RMAX / 4 * kWave)
-        pair_rows<RMAX / 4>(pst, np, total, cell_part, list, masks, nws, overflow, row_ptr, col, lane);
-    else if (total <= RMAX / 2 * kWave)
-        pair_rows<RMAX / 2>(pst, np, total, cell_part, list, masks, nws, overflow, row_ptr, col, lane);
-    else
-        pair_rows<RMAX>(pst, np, total, cell_part, list, masks, nws, overflow, row_ptr, col, lane);
-}
-
-// Count (FILL = false: counts[p]) or fill (FILL = true: col[row_ptr[p] ..])
-// from positions, one particle of the cell at a time: every cell, or with
-// spill != NULL the spill[0] cells listed at spill[1 ..].
-template <int DIM, bool FILL>
-__global__ __launch_bounds__(kCellWaves * kWave) void k_support_cells(
-    int64_t n, const double* __restrict__ rcut, CellGrid g, const int64_t* __restrict__ cell_start,
-    const int32_t* __restrict__ cell_part, const double* __restrict__ pos_cell, int32_t* __restrict__ counts,
-    int32_t* __restrict__ overflow, const int64_t* __restrict__ row_ptr, int32_t* __restrict__ col,
-    const int32_t* __restrict__ spill) {
-    constexpr int CAP = CellCap<DIM>::v;
-    __shared__ int32_t sq[kCellWaves][CAP];
-    __shared__ double sx[kCellWaves][DIM * CAP];
-    __shared__ int32_t buf[FILL ? kCellWaves : 1][FILL ? DCPSE_MAX_ROW : 1];
-    __shared__ int32_t mark[kCellWaves][kWave];
-    __shared__ long long seg_cst[kCellWaves][kWave];
-    __shared__ int32_t seg_ex[kCellWaves][kWave];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    const double r = rcut[0];
-    const double r2 = r * r;
-    const unsigned G = gridDim.x;
-    const int64_t ncells = spill ? (int64_t)spill[0] : g.ncell;
-    for (int64_t ci = (int64_t)xcd_block() * kCellWaves + wv; ci < ncells; ci += (int64_t)G * kCellWaves) {
-        const int64_t c = spill ? (int64_t)spill[1 + ci] : ci;
-        const int64_t pst = cell_start[c];
-        const int np = (int)(cell_start[c + 1] - pst);
-        if (np == 0) continue;
-        long long cst;
-        int ccnt;
-        cell_segments<DIM>(g, cell_start, c, lane, cst, ccnt);
-        const int incl = wave_incl_scan(ccnt);
-        const int total = __builtin_amdgcn_readlane(incl, 63);
-        const int excl = incl - ccnt;
-        seg_cst[wv][lane] = cst;
-        seg_ex[wv][lane] = excl;
-        const bool fits = total <= CAP;
-        if (fits)
-            stage_candidates<DIM, true>(0, total, ccnt, excl, mark[wv], seg_cst[wv], seg_ex[wv], cell_part, pos_cell,
-                                        n, sq[wv], sx[wv], CAP, lane);
-        for (int i = 0; i < np; ++i) {
-            const int64_t ps = pst + i;
-            const int pid = cell_part[ps];
-            double xp[3];
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) xp[d] = pos_cell[d * n + ps];
-            int nacc = 0;
-            for (int c0 = 0; c0 < total; c0 += CAP) {
-                const int cn = min(CAP, total - c0);
-                if (!fits) {
-                    wave_lds_sync();
-                    stage_candidates<DIM, true>(c0, cn, ccnt, excl, mark[wv], seg_cst[wv], seg_ex[wv], cell_part,
-                                                pos_cell, n, sq[wv], sx[wv], CAP, lane);
-                }
-                for (int t0 = 0; t0 < cn; t0 += kWave) {
-                    const int t = min(t0 + lane, cn - 1);
-                    const int q = sq[wv][t];
-                    const bool near = within_cut<DIM>(xp, sx[wv], CAP, t, g, r2);
-                    const bool take = (t0 + lane < cn) & (q != pid) & near;
-                    const unsigned long long m = __ballot(take);
-                    if (FILL) {
-                        const int at = nacc + lane_prefix(m);
-                        if (take && at < DCPSE_MAX_ROW) buf[wv][at] = q;
-                    }
-                    nacc += __popcll(m);
-                }
-            }
-            if (!FILL) {
-                if (lane == 0) {
-                    counts[pid] = nacc;
-                    if (nacc > DCPSE_MAX_ROW) atomicOr(overflow, 1);
-                }
-            } else {
-                wave_lds_sync();
-                const int64_t rs = row_ptr[pid];
-                const int nn = min(nacc, DCPSE_MAX_ROW);
-                if ((int64_t)nacc != row_ptr[pid + 1] - rs) {
-                    if (lane == 0) atomicOr(overflow, 2);
-                } else {
-                    store_ranked(buf[wv], nn, col + rs, lane);
-                }
-                wave_lds_sync();
-            }
-        }
-        wave_lds_sync();
-    }
+    if (total <= RMAX / 4 * kWave) pair_rows<RMAX / 4>(a, gi, pst, np, total, row_ptr, col, lane);
+    else if (total <= RMAX / 2 * kWave) pair_rows<RMAX / 2>(a, gi, pst, np, total, row_ptr, col, lane);
+    else pair_rows<RMAX>(a, gi, pst, np, total, row_ptr, col, lane);
 }
 
 // Cell edge about rmax / K: smaller cells than the cut-off shrink the scanned
@@ -1154,14 +1231,16 @@ static dcpse_status make_grid(dcpse_ctx* ctx, int dim, const double* box_lo, con
     return DCPSE_OK;
 }
 
-// out[0] = min and out[1] = max(0, max) of v[0..n) (NaNs ignored), one block.
-constexpr int kMinMaxThreads = 1024;
+// Per block: out[2b] = min and out[2b + 1] = max(0, max) of its share of
+// v[0..n) (NaNs ignored).
+constexpr int kMinMaxThreads = 256;
+constexpr int kMinMaxBlocks = 256;
 __global__ __launch_bounds__(kMinMaxThreads) void k_minmax(const double* __restrict__ v, int64_t n,
                                                           double* __restrict__ out) {
     __shared__ double smin[kMinMaxThreads], smax[kMinMaxThreads];
     const int t = threadIdx.x;
-    double lo = n > 0 ? v[0] : 0.0, hi = 0.0;
-    for (int64_t i = t; i < n; i += kMinMaxThreads) {
+    double lo = v[0], hi = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * kMinMaxThreads + t; i < n; i += (int64_t)gridDim.x * kMinMaxThreads) {
         lo = fmin(lo, v[i]);
         hi = fmax(hi, v[i]);
     }
@@ -1176,15 +1255,15 @@ __global__ __launch_bounds__(kMinMaxThreads) void k_minmax(const double* __restr
         __syncthreads();
     }
     if (t == 0) {
-        out[0] = smin[0];
-        out[1] = smax[0];
+        out[2 * blockIdx.x] = smin[0];
+        out[2 * blockIdx.x + 1] = smax[0];
     }
 }
 
 // Calls launch with the dimension and the register width of a mask of nws
 // words as compile-time values.
 template <typename F>
-static void launch_pairs(int dim, int nws, F launch) {
+static void launch_groups(int dim, int nws, F launch) {
     auto width = [&](auto D) {
         if (nws <= 4) launch(D, std::integral_constant<int, 4>());
         else if (nws <= 8) launch(D, std::integral_constant<int, 8>());
@@ -1193,6 +1272,42 @@ static void launch_pairs(int dim, int nws, F launch) {
     };
     if (dim == 2) width(std::integral_constant<int, 2>());
     else width(std::integral_constant<int, 3>());
+}
+
+// The home levels of a set with cut-offs in [rmin, rmax]: a level for every
+// halving, as long as their cells number a few per particle.
+static void make_levels(int dim, const double* box_lo, const double* box_hi, unsigned periodic, double rmin,
+                        double rmax, int64_t n, HomeLevels* h) {
+    h->n = 0;
+    h->rtop = rmax;
+    h->first[0] = 0;
+    double total = 0.0, edge = kHomeEdge * rmax, top = rmax;
+    for (int l = 0; l < kMaxLevels; ++l, edge *= 0.5, top *= 0.5) {
+        if (l > 0 && !(rmin <= top)) break;  // no particle is this small
+        CellGrid& g = h->g[l];
+        g.periodic = periodic;
+        double cells = 1.0;
+        for (int d = 0; d < 3; ++d) {
+            const double len = d < dim ? box_hi[d] - box_lo[d] : 1.0;
+            const double k = d < dim ? std::min(std::max(std::ceil(len / edge), 1.0), 1e6) : 1.0;
+            g.nc[d] = (int)k;
+            g.kmax[d] = 0;
+            g.lo[d] = d < dim ? box_lo[d] : 0.0;
+            g.len[d] = len;
+            g.ilen[d] = 1.0 / len;
+            g.cs[d] = len / k;
+            cells *= k;
+        }
+        if (total + cells > 4.0 * (double)n + 4096.0 && l > 0) break;
+        total += cells;
+        if (total > 1e9) {  // (level 0 of a sparse set: not worth grouping)
+            h->n = 0;
+            return;
+        }
+        g.ncell = (int64_t)cells;
+        h->n = l + 1;
+        h->first[l + 1] = (int32_t)total;
+    }
 }
 
 static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup, int64_t n_sup,
@@ -1222,104 +1337,120 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
         return DCPSE_OK;
     }
     if (!rcut) return fail(ctx, DCPSE_ERR_INVALID, "rcut is null");
+    hipStream_t s = ctx->stream;
     // the largest cut-off fixes the cell edge
     double rmax = 0.0, rmin = 0.0;
     if (rcut_pp) {
-        // reduced on the device; only the two extremes come back
+        // reduced on the device; only the blocks' extremes come back
         Workspace w0;
-        dcpse_status st0 = reserve_workspace(ctx, 1024, &w0);
+        dcpse_status st0 = reserve_workspace(ctx, kMinMaxBlocks * 2 * sizeof(double) + 256, &w0);
         if (st0) return st0;
-        double* mm = w0.take<double>(2);
-        k_minmax<<<1, kMinMaxThreads, 0, ctx->stream>>>(rcut, n_dom, mm);
+        double* mm = w0.take<double>(2 * kMinMaxBlocks);
+        if (!mm) return fail(ctx, DCPSE_ERR_INVALID, "workspace sizing error");
+        const int nb = (int)std::min<int64_t>(kMinMaxBlocks, (n_dom + kMinMaxThreads - 1) / kMinMaxThreads);
+        k_minmax<<<nb, kMinMaxThreads, 0, s>>>(rcut, n_dom, mm);
         DCPSE_LAUNCH_CHECK(ctx);
-        double h[2] = {0.0, 0.0};
-        DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(h, mm, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
-        DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-        rmin = h[0];
-        rmax = h[1];
+        double hv[2 * kMinMaxBlocks];
+        DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(hv, mm, 2 * nb * sizeof(double), hipMemcpyDeviceToHost, s));
+        DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(s));
+        rmin = hv[0];
+        for (int b = 0; b < nb; ++b) {
+            rmin = std::fmin(rmin, hv[2 * b]);
+            rmax = std::fmax(rmax, hv[2 * b + 1]);
+        }
     } else {
-        DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&rmax, rcut, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+        DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&rmax, rcut, sizeof(double), hipMemcpyDeviceToHost, s));
+        DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(s));
         rmin = rmax;
     }
-    // cells per cut-off: 2 (3D) or 4 (2D) for one cut-off; with a spread of
-    // cut-offs, about rmax / rmin so the smallest scan only their own
-    // neighbourhood (bounded: a wave handles 32 cell rows per round)
     const double spread = rmin > 0.0 ? rmax / rmin : 1.0;
-    const int K = dim == 3 ? std::min(4, std::max(2, (int)std::ceil(spread - 1e-9)))
-                           : std::min(8, std::max(4, (int)std::ceil(spread - 1e-9)));
     CellGrid g;
+    HomeLevels home;
+    home.n = 0;
     dcpse_status st;
-    // one particle set and one cut-off: a wavefront per cell of edge >= rcut
-    // while the mean candidate count of a cell leaves room to sort them in
-    // registers; otherwise a wavefront per particle
-    bool by_cell = same && !rcut_pp && n_dom > 0;
-    bool paired = false;  // candidate lists and take masks (k_cell_pairs)
-    int nws = 0;          // words of a take mask
-    if (by_cell) {
+    // One particle set goes by groups (k_group_pairs) where FP32 resolves the
+    // pairs (see kPairTol, relative()) and the candidates of a group leave room
+    // to sort them in registers; everything else a wavefront per particle.
+    bool grouped = same && rmax > 1e-30 && rmax < 1e30;
+    for (int d = 0; d < dim; ++d)
+        grouped = grouped && std::fabs(box_lo[d]) <= kMaxOffset * rmax && std::fabs(box_hi[d]) <= kMaxOffset * rmax;
+    int nws = 0;  // words of a take mask
+    if (grouped && !rcut_pp) {
+        // cells of edge >= rcut
         if ((st = make_grid(ctx, dim, box_lo, box_hi, periodic, rmax, 1, &g))) return st;
         const double cand = (double)n_sup * (dim == 3 ? 27.0 : 9.0) / (double)g.ncell;
-        by_cell = cand <= (dim == 3 ? 1638.0 : 819.0);
+        grouped = cand <= (dim == 3 ? 1638.0 : 819.0);
         // about half of the 3^dim cells' particles are within reach of the
         // cell's own; lists of 0.84 of them leave room for uneven cells
         nws = std::max(2, std::min(32, (int)std::ceil(0.84 * cand / kWave)));
-        paired = by_cell;
-        for (int d = 0; d < dim; ++d) {  // see kPairTol, relative()
-            paired = paired && g.cs[d] <= 4.0 * rmax && std::fabs(box_lo[d]) <= kMaxOffset * rmax &&
-                     std::fabs(box_hi[d]) <= kMaxOffset * rmax && (g.nc[d] >= 4 || !((periodic >> d) & 1u));
+        for (int d = 0; d < dim; ++d)
+            grouped = grouped && g.cs[d] <= 0.5 * kMaxReach * rmax && (g.nc[d] >= 4 || !((periodic >> d) & 1u));
+    } else if (grouped) {
+        // candidate cells of about half the smallest cut-off, at most a few
+        // per particle: coarser ones bring more candidates that the box test
+        // drops, finer ones more empty cells
+        make_levels(dim, box_lo, box_hi, periodic, rmin, rmax, n_sup, &home);
+        grouped = home.n > 0 && rmin > 0.0;
+        for (int d = 0; d < dim; ++d)
+            if ((periodic >> d) & 1u) grouped = grouped && box_hi[d] - box_lo[d] > (kHomeEdge + 2.1) * rmax;
+        int K = (int)std::min(dim == 3 ? 8.0 : 16.0, std::ceil(2.0 * spread - 1e-9));
+        for (; grouped && K >= 1; --K) {
+            if ((st = make_grid(ctx, dim, box_lo, box_hi, periodic, rmax, K, &g))) return st;
+            if (g.ncell <= 8 * n_sup + 4096 || K == 1) break;
         }
+        nws = dim == 3 ? 8 : 4;
     }
-    if (!by_cell && (st = make_grid(ctx, dim, box_lo, box_hi, periodic, rmax, K, &g))) return st;
-    const int64_t cb = by_cell ? std::max<int64_t>(1, std::min<int64_t>((g.ncell + kCellWaves - 1) / kCellWaves,
-                                                                         (int64_t)ctx->num_cus * 16))
-                               : 0;
-    const unsigned cell_blocks = (unsigned)(cb >= 8 ? cb / 8 * 8 : cb);
-    // one wavefront per cell, the blocks in whole rounds over the XCDs
-    const unsigned pair_blocks = (unsigned)((g.ncell + kPairWaves * 8 - 1) / (kPairWaves * 8) * 8);
+    if (!grouped) {
+        // cells per cut-off: 2 (3D) or 4 (2D) for one cut-off; with a spread of
+        // cut-offs, about rmax / rmin so the smallest scan only their own
+        // neighbourhood (bounded: a wave handles 32 cell rows per round)
+        const int K = dim == 3 ? std::min(4, std::max(2, (int)std::ceil(spread - 1e-9)))
+                               : std::min(8, std::max(4, (int)std::ceil(spread - 1e-9)));
+        if ((st = make_grid(ctx, dim, box_lo, box_hi, periodic, rmax, K, &g))) return st;
+    }
+    const bool pp = grouped && rcut_pp;
+    // home cells: the candidate cells, or the levels' cells
+    const int64_t n_home = pp ? home.first[home.n] : g.ncell;
+    // groups numbered over the occupied home cells where most are empty
+    const bool compact = grouped && (pp || n_home > 2 * n_sup);
+    const int64_t max_groups = !compact ? n_home : pp ? std::min(n_sup, n_sup / 4 + 4096) : n_sup;
 
-    // the same-set, single-cut-off fill reuses the cell list, candidate lists and
-    // take masks of the count just before it when the arguments match
+    // the fill of one set reuses the cell list, candidate lists and take masks
+    // of the count just before it when the arguments match
     dcpse_support_cache& sc = ctx->sup;
     const bool count_pass = col == nullptr;
-    const bool cached = paired && !count_pass && sc.valid && sc.dim == dim && sc.pos == pos_sup &&
-                        sc.n == n_sup && sc.rcut == rmax && sc.periodic == periodic && sc.nws == nws &&
+    const bool cached = grouped && !count_pass && sc.valid && sc.dim == dim && sc.pos == pos_sup &&
+                        sc.n == n_sup && sc.rcut == rmax && sc.rmin == rmin && sc.rcut_pp == rcut_pp &&
+                        sc.periodic == periodic && sc.nws == nws &&
                         std::equal(box_lo, box_lo + dim, sc.lo) && std::equal(box_hi, box_hi + dim, sc.hi);
     sc.valid = false;
 
-    Workspace w;
-    size_t need = (size_t)n_sup * 4 * 2 + (size_t)dim * (n_sup + 1) * 8 + (size_t)(g.ncell + 1) * 8 +
-                  (size_t)g.ncell * 4 * 2 + (size_t)n_dom * 4 + scan_workspace_bytes(std::max(g.ncell, n_dom)) +
-                  64 * 256;
-    if ((st = reserve_workspace(ctx, need, &w))) return st;
-    int32_t* cell_id = w.take<int32_t>(n_sup + 1);
-    int32_t* cell_part = w.take<int32_t>(n_sup + 1);
-    double* pos_cell = w.take<double>((size_t)dim * (n_sup + 1));
-    int32_t* cell_cnt = w.take<int32_t>(g.ncell + 1);
-    int64_t* cell_start = w.take<int64_t>(g.ncell + 1);
-    int32_t* counts = w.take<int32_t>(n_dom + 1);
-    int32_t* flags = w.take<int32_t>(64);
-    Workspace ws_scan = w;
-    if (!flags) return fail(ctx, DCPSE_ERR_INVALID, "workspace sizing error");
-    hipStream_t s = ctx->stream;
-
+    // Cell list, candidate lists, masks and the list of particles left to
+    // k_support_rows: in the context's support cache when grouped (a fill
+    // finds them there), the cell list alone in the workspace otherwise.
+    int64_t *cell_start = nullptr, *home_start = nullptr, *group_index = nullptr;
+    CellRec *rec = nullptr, *home_rec = nullptr;
+    int32_t *group_cell = nullptr, *ncand = nullptr, *lists = nullptr, *spill = nullptr;
     uint64_t* masks = nullptr;
-    int32_t *spill = nullptr, *ncand = nullptr, *lists = nullptr;
-    bool use_cache = paired && (count_pass || cached);
-    if (use_cache) {
-        // cell list, candidate lists, masks and the list of cells left to the
-        // position kernel in the context's support cache
-        auto carve = [&](Workspace& cw) {
-            cell_start = cw.take<int64_t>(g.ncell + 1);
-            cell_part = cw.take<int32_t>(n_sup + 1);
-            pos_cell = cw.take<double>((size_t)dim * (n_sup + 1));
-            masks = cw.take<uint64_t>((size_t)(n_sup + 1) * nws);
-            ncand = cw.take<int32_t>(g.ncell + 1);
-            lists = cw.take<int32_t>((size_t)g.ncell * nws * kWave);
-            spill = cw.take<int32_t>(g.ncell + 2);
-        };
-        int64_t* own_start = cell_start;
-        int32_t* own_part = cell_part;
-        double* own_pos = pos_cell;
+    auto carve_cells = [&](Workspace& cw) {
+        cell_start = cw.take<int64_t>(g.ncell + 1);
+        rec = cw.take<CellRec>(n_sup);
+    };
+    auto carve = [&](Workspace& cw) {
+        carve_cells(cw);
+        home_start = pp ? cw.take<int64_t>(n_home + 1) : cell_start;
+        home_rec = pp ? cw.take<CellRec>(n_sup) : rec;
+        if (compact) {
+            group_index = cw.take<int64_t>(n_home + 1);
+            group_cell = cw.take<int32_t>(std::min(n_home, n_sup) + 1);
+        }
+        masks = cw.take<uint64_t>((size_t)n_sup * nws);
+        ncand = cw.take<int32_t>(max_groups + 1);
+        lists = cw.take<int32_t>((size_t)max_groups * nws * kWave);
+        spill = cw.take<int32_t>(n_sup + 2);
+    };
+    bool groups_on = grouped && (count_pass || cached);
+    if (groups_on) {
         Workspace cw;
         cw.cap = ~size_t(0) >> 1;
         carve(cw);  // sizes only
@@ -1336,12 +1467,10 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
                 // (finding no matching cache) fills from positions too
                 (void)hipGetLastError();
                 sc.buf = nullptr;
-                use_cache = false;
-                cell_start = own_start, cell_part = own_part, pos_cell = own_pos;
-                masks = nullptr, spill = nullptr;
+                groups_on = false;
             }
         }
-        if (use_cache) {
+        if (groups_on) {
             cw = Workspace();
             cw.base = static_cast<char*>(sc.buf);
             cw.cap = sc.cap;
@@ -1349,73 +1478,120 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
             if (!spill) return fail(ctx, DCPSE_ERR_INVALID, "support cache sizing error");
         }
     }
+    const bool home_on = groups_on && pp;
+    Workspace w;
+    const size_t need = (size_t)n_sup * 4 * 4 + (size_t)g.ncell * 4 + (size_t)n_home * 8 + (size_t)n_dom * 4 +
+                        (groups_on ? 0 : (size_t)(g.ncell + 1) * 8 + (size_t)n_sup * sizeof(CellRec)) +
+                        scan_workspace_bytes(std::max(std::max(g.ncell, n_home), n_dom)) + 64 * 256;
+    if ((st = reserve_workspace(ctx, need, &w))) return st;
+    if (!groups_on) carve_cells(w);
+    int32_t* cell_id = w.take<int32_t>(n_sup + 1);
+    int32_t* rank = w.take<int32_t>(n_sup + 1);
+    int32_t* cell_cnt = w.take<int32_t>(g.ncell + 1);
+    int32_t *home_id = nullptr, *home_rank = nullptr, *home_cnt = cell_cnt, *occupied = nullptr;
+    if (home_on) {
+        home_id = w.take<int32_t>(n_sup + 1);
+        home_rank = w.take<int32_t>(n_sup + 1);
+        home_cnt = w.take<int32_t>(n_home + 1);
+    }
+    if (groups_on && compact) occupied = w.take<int32_t>(n_home + 1);
+    int32_t* counts = w.take<int32_t>(n_dom + 1);
+    int32_t* flags = w.take<int32_t>(64);
+    const Workspace ws_scan = w;
+    if (!flags) return fail(ctx, DCPSE_ERR_INVALID, "workspace sizing error");
 
     fill_i32(s, flags, 64, 0);
-    const int64_t tb = std::max<int64_t>(1, std::min<int64_t>((n_sup + 255) / 256, 16384));
+    auto blocks_for = [](int64_t n) {
+        return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 16384));
+    };
+    auto scan = [&](const int32_t* in, int64_t n, int64_t* out) {
+        Workspace ws = ws_scan;
+        return scan_counts(ctx, in, n, out, &ws);
+    };
     if (!cached) {
         fill_i32(s, cell_cnt, g.ncell + 1, 0);
-        if (n_sup > 0) {
-            if (dim == 2) k_cell_assign<2><<<(unsigned)tb, 256, 0, s>>>(pos_sup, n_sup, g, cell_id, cell_cnt);
-            else k_cell_assign<3><<<(unsigned)tb, 256, 0, s>>>(pos_sup, n_sup, g, cell_id, cell_cnt);
+        if (home_on) fill_i32(s, home_cnt, n_home + 1, 0);
+        const unsigned tb = blocks_for(n_sup);
+        auto cells = [&](auto D, auto H) {
+            constexpr int DIM = decltype(D)::value;
+            constexpr bool HOME = decltype(H)::value;
+            k_cell_assign<DIM, HOME><<<tb, 256, 0, s>>>(pos_sup, n_sup, rcut, g, home, cell_id, rank, cell_cnt,
+                                                       home_id, home_rank, home_cnt);
             DCPSE_LAUNCH_CHECK(ctx);
-        }
-        if ((st = scan_counts(ctx, cell_cnt, g.ncell, cell_start, &ws_scan))) return st;
-        fill_i32(s, cell_cnt, g.ncell + 1, 0);  // reuse as cursor
-        if (n_sup > 0) {
-            if (dim == 2)
-                k_cell_fill<2><<<(unsigned)tb, 256, 0, s>>>(cell_id, n_sup, pos_sup, cell_start, cell_cnt,
-                                                            cell_part, pos_cell);
-            else
-                k_cell_fill<3><<<(unsigned)tb, 256, 0, s>>>(cell_id, n_sup, pos_sup, cell_start, cell_cnt,
-                                                            cell_part, pos_cell);
+            dcpse_status sst;
+            if ((sst = scan(cell_cnt, g.ncell, cell_start))) return sst;
+            if (HOME && (sst = scan(home_cnt, n_home, home_start))) return sst;
+            k_cell_fill<DIM, HOME><<<tb, 256, 0, s>>>(pos_sup, n_sup, cell_id, rank, cell_start, rec, home_id,
+                                                     home_rank, home_start, home_rec);
+            DCPSE_LAUNCH_CHECK(ctx);
+            return DCPSE_OK;
+        };
+        auto by_home = [&](auto D) { return home_on ? cells(D, std::true_type()) : cells(D, std::false_type()); };
+        st = dim == 2 ? by_home(std::integral_constant<int, 2>()) : by_home(std::integral_constant<int, 3>());
+        if (st) return st;
+        if (occupied) {
+            k_occupied<<<blocks_for(n_home), 256, 0, s>>>(home_cnt, n_home, occupied);
+            DCPSE_LAUNCH_CHECK(ctx);
+            if ((st = scan(occupied, n_home, group_index))) return st;
+            k_group_cells<<<blocks_for(n_home), 256, 0, s>>>(home_cnt, group_index, n_home, group_cell);
             DCPSE_LAUNCH_CHECK(ctx);
         }
     }
-    const int64_t rb = std::max<int64_t>(1, std::min<int64_t>((n_dom + kRowWaves - 1) / kRowWaves,
-                                                              (int64_t)ctx->num_cus * 16));
+    Groups a;
+    a.n = n_sup;
+    a.pos = pos_sup;
+    a.rcut = rcut;
+    a.g = g;
+    a.cell_start = cell_start;
+    a.rec = rec;
+    a.home_start = home_start;
+    a.home = home_rec;
+    a.group_cell = group_cell;
+    a.n_groups = group_cell ? group_index + n_home : nullptr;
+    a.max_groups = max_groups;
+    a.counts = counts;
+    a.flags = flags;
+    a.ncand = ncand;
+    a.lists = lists;
+    a.masks = masks;
+    a.nws = nws;
+    a.spill = spill;
+    // a wavefront per group, the blocks in whole rounds over the XCDs
+    const int64_t launch_groups_n = compact ? std::min(n_home, n_sup) : n_home;
+    const unsigned group_blocks = (unsigned)((launch_groups_n + kPairWaves * 8 - 1) / (kPairWaves * 8) * 8);
+    const unsigned row_blocks = (unsigned)std::max<int64_t>(
+        1, std::min<int64_t>((n_dom + kRowWaves - 1) / kRowWaves, (int64_t)ctx->num_cus * 16));
+    // every row (list NULL) or the listed ones from positions
+    auto rows = [&](auto F, const int32_t* list) {
+        constexpr bool FILL = decltype(F)::value;
+        if (dim == 2)
+            k_support_rows<2, FILL><<<row_blocks, kRowWaves * kWave, 0, s>>>(
+                pos_dom, n_dom, same, dom_self, rcut, rcut_pp, g, cell_start, rec, counts, flags, row_ptr, col, list);
+        else
+            k_support_rows<3, FILL><<<row_blocks, kRowWaves * kWave, 0, s>>>(
+                pos_dom, n_dom, same, dom_self, rcut, rcut_pp, g, cell_start, rec, counts, flags, row_ptr, col, list);
+    };
     if (count_pass) {
-        if (by_cell && !use_cache) {
-            if (dim == 2)
-                k_support_cells<2, false><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
-                    n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, nullptr, nullptr, nullptr);
-            else
-                k_support_cells<3, false><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
-                    n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, nullptr, nullptr, nullptr);
-            DCPSE_LAUNCH_CHECK(ctx);
-        } else if (by_cell) {
-            // candidate lists and masks, then the cells they do not cover from positions
+        if (groups_on) {
+            // candidate lists and masks, then the particles they do not cover
             fill_i32(s, spill, 1, 0);
-            launch_pairs(dim, nws, [&](auto D, auto R) {
-                k_cell_pairs<decltype(D)::value, decltype(R)::value><<<pair_blocks, kPairWaves * kWave, 0, s>>>(
-                    n_sup, rcut, g, cell_start, cell_part, pos_cell, pos_sup, counts, flags, ncand, lists, masks, nws,
-                    spill);
+            launch_groups(dim, nws, [&](auto D, auto R) {
+                constexpr int DIM = decltype(D)::value, RM = decltype(R)::value;
+                if (pp) k_group_pairs<DIM, RM, true><<<group_blocks, kPairWaves * kWave, 0, s>>>(a, home);
+                else k_group_pairs<DIM, RM, false><<<group_blocks, kPairWaves * kWave, 0, s>>>(a, home);
             });
             DCPSE_LAUNCH_CHECK(ctx);
-            if (dim == 2)
-                k_support_cells<2, false><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
-                    n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, nullptr, nullptr, spill);
-            else
-                k_support_cells<3, false><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
-                    n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, nullptr, nullptr, spill);
-            DCPSE_LAUNCH_CHECK(ctx);
-        } else if (n_dom > 0) {
-            if (dim == 2)
-                k_support_rows<2, false><<<(unsigned)rb, kRowWaves * kWave, 0, s>>>(
-                    pos_sup, n_sup, pos_dom, n_dom, same, dom_self, rcut, rcut_pp, g, cell_start, cell_part, pos_cell, counts,
-                    flags, nullptr, nullptr);
-            else
-                k_support_rows<3, false><<<(unsigned)rb, kRowWaves * kWave, 0, s>>>(
-                    pos_sup, n_sup, pos_dom, n_dom, same, dom_self, rcut, rcut_pp, g, cell_start, cell_part, pos_cell, counts,
-                    flags, nullptr, nullptr);
-            DCPSE_LAUNCH_CHECK(ctx);
+            rows(std::false_type(), spill);
+        } else {
+            rows(std::false_type(), nullptr);
         }
-        Workspace ws2 = ws_scan;
-        if ((st = scan_counts(ctx, counts, n_dom, row_ptr, &ws2))) return st;
+        DCPSE_LAUNCH_CHECK(ctx);
+        if ((st = scan(counts, n_dom, row_ptr))) return st;
         int64_t nnz = 0;
         int32_t ovf = 0, n_spill = 0;
         DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&nnz, row_ptr + n_dom, sizeof(int64_t), hipMemcpyDeviceToHost, s));
         DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&ovf, flags, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        if (spill)
+        if (groups_on)
             DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&n_spill, spill, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(s));
         if (ovf & 1)
@@ -1424,13 +1600,15 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
         if (nnz >= ((int64_t)1 << 31) * 64)
             return fail(ctx, DCPSE_ERR_RANGE, "nnz out of range");
         if (nnz_out) *nnz_out = nnz;
-        if (use_cache) {
+        if (groups_on) {
             sc.valid = true;
             sc.spill = n_spill > 0;
             sc.dim = dim;
             sc.pos = pos_sup;
             sc.n = n_sup;
             sc.rcut = rmax;
+            sc.rmin = rmin;
+            sc.rcut_pp = rcut_pp;
             sc.periodic = periodic;
             sc.nws = nws;
             for (int d = 0; d < 3; ++d) {
@@ -1440,34 +1618,14 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
         }
     } else {
         if (cached) {
-            launch_pairs(dim, nws, [&](auto, auto R) {
-                k_cell_rows<decltype(R)::value><<<pair_blocks, kPairWaves * kWave, 0, s>>>(
-                    g.ncell, cell_start, cell_part, ncand, lists, masks, nws, flags, row_ptr, col);
+            launch_groups(dim, nws, [&](auto, auto R) {
+                k_group_rows<decltype(R)::value><<<group_blocks, kPairWaves * kWave, 0, s>>>(a, row_ptr, col);
             });
             DCPSE_LAUNCH_CHECK(ctx);
         }
-        if (by_cell && (!cached || sc.spill)) {
-            // the cells the lists do not cover (cached), or all of them
-            const int32_t* list = cached ? spill : nullptr;
-            if (dim == 2)
-                k_support_cells<2, true><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
-                    n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, row_ptr, col, list);
-            else
-                k_support_cells<3, true><<<cell_blocks, kCellWaves * kWave, 0, s>>>(
-                    n_sup, rcut, g, cell_start, cell_part, pos_cell, counts, flags, row_ptr, col, list);
+        if (!cached || sc.spill) {
+            rows(std::true_type(), cached ? spill : nullptr);
             DCPSE_LAUNCH_CHECK(ctx);
-        } else if (!by_cell && n_dom > 0) {
-            if (dim == 2)
-                k_support_rows<2, true><<<(unsigned)rb, kRowWaves * kWave, 0, s>>>(
-                    pos_sup, n_sup, pos_dom, n_dom, same, dom_self, rcut, rcut_pp, g, cell_start, cell_part, pos_cell, counts,
-                    flags, row_ptr, col);
-            else
-                k_support_rows<3, true><<<(unsigned)rb, kRowWaves * kWave, 0, s>>>(
-                    pos_sup, n_sup, pos_dom, n_dom, same, dom_self, rcut, rcut_pp, g, cell_start, cell_part, pos_cell, counts,
-                    flags, row_ptr, col);
-            DCPSE_LAUNCH_CHECK(ctx);
-        }
-        if (n_dom > 0) {
             const int64_t lb = std::max<int64_t>(
                 1, std::min<int64_t>((n_dom + kRowWaves * kWave - 1) / (kRowWaves * kWave), (int64_t)ctx->num_cus * 8));
             k_sort_long_rows<<<(unsigned)lb, kRowWaves * kWave, 0, s>>>(n_dom, row_ptr, col);
