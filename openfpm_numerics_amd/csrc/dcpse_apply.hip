@@ -246,8 +246,8 @@ __global__ __launch_bounds__(kApplyMaxBlock) void k_apply_v4(const ApplyArgs<flo
 // particle-major (fil[q * NF + b]), so a neighbour's NF values are one
 // contiguous 4 NF-byte read instead of NF separate gathers, and the col/W
 // streams are read once for all of them. Each field's sum runs over the
-// nonzeros in the order of k_apply_v4 (same lanes, same chunks, same
-// reduction), so the results equal the field-major kernel's bit for bit.
+// nonzeros in the order of k_apply_v4, so the results equal the field-major
+// kernel's bit for bit.
 template <int NF>
 __global__ __launch_bounds__(256) void k_interleave(int64_t n, const float* __restrict__ f, int64_t ld,
                                                     float* __restrict__ fil) {
@@ -265,97 +265,203 @@ __global__ __launch_bounds__(256) void k_interleave(int64_t n, const float* __re
 
 typedef float vf4a __attribute__((ext_vector_type(4)));
 
+// EL consecutive 4-byte elements of a stream, at any element offset.
+template <typename T, int EL>
+struct StreamVec {
+    typedef T type __attribute__((ext_vector_type(EL), aligned(4)));
+};
+template <typename T>
+struct StreamVec<T, 1> {
+    typedef T type;
+};
+
+// v of lane SRC of this lane's group of L lanes (L = 1, 2, 4).
+template <int L, int SRC>
+__device__ __forceinline__ int group_lane(int v) {
+    if constexpr (L == 1) return v;
+    else if constexpr (L == 2) return __builtin_amdgcn_update_dpp(0, v, SRC ? 0xF5 : 0xA0, 0xF, 0xF, true);
+    else return __builtin_amdgcn_update_dpp(0, v, SRC * 0x55, 0xF, 0xF, true);
+}
+
+// L = NF / 4 lanes per row, 4 fields each: a neighbour's NF values are read by
+// its row's lanes side by side, so one 16-byte load instruction serves 64 / L
+// neighbours with one cache line each. (With a lane per neighbour reading all
+// its NF values, every one of its 16-byte loads looked up 64 lines: 308 us
+// against 161 us forward, 395 against 175 us transposed, for 16 fields on
+// 1024^2 particles with 29 neighbours. The cache's lookup rate bounded that;
+// here the vector units and the address unit are busy two thirds of the time
+// each. Measured and not better: more waves (spilled registers), the next
+// chunk's gathers ahead of the sums (half the waves), 32-bit addresses.) The
+// row's lanes load a chunk of 4 nonzeros together and pass them round by DPP.
+// Each field's sum takes the order of k_apply_v4<G, NCH>, whose lane p of a
+// row sums the chunks p, p + G, ... and then the strided tail: the partial sums
+// are formed here one after another and added up as its lane exchanges do.
 template <int G, int NCH, int NF, int MODE>
-__global__ __launch_bounds__(kApplyMaxBlock) void k_apply_il(const ApplyArgs<float> a) {
-    static_assert(NF % 4 == 0, "fields in groups of 4");
+struct BatchRow {
+    static constexpr int L = NF / 4, EL = 4 / L;
+    typedef typename StreamVec<int32_t, EL>::type vq;
+    typedef typename StreamVec<float, EL>::type vw;
+    const ApplyArgs<float>& a;
+    int64_t rs;
+    int len, lenv;  // nonzeros; those taken in chunks of 4 (0: all by the tail)
+    int g;          // lane of the row's group
+    vf4a fp;
+    // the chunks' columns and weights, read ahead while they fit 32 registers
+    static constexpr bool AHEAD = 2 * EL * G * NCH <= 32;
+    vq q[AHEAD ? G * NCH : 1];
+    vw w[AHEAD ? G * NCH : 1];
+
+    template <int K>
+    __device__ __forceinline__ void element(int32_t qv, float wv, vf4a& f, double& wd) {
+        const int32_t qq = group_lane<L, K>(qv);
+        wd = (double)__int_as_float(group_lane<L, K>(__float_as_int(wv)));
+        f = *reinterpret_cast<const vf4a*>(a.f + ((int64_t)qq * NF + 4 * g));
+    }
+    static __device__ __forceinline__ int32_t part(const vq& v, int k) {
+        if constexpr (EL == 1) return v;
+        else return v[k];
+    }
+    static __device__ __forceinline__ float part(const vw& v, int k) {
+        if constexpr (EL == 1) return v;
+        else return v[k];
+    }
+    template <bool MASK>
+    __device__ __forceinline__ void add(const vf4a (&f)[4], const double (&wd)[4], const bool (&v)[4], double (&s)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const double d = MODE == kDiff ? (double)f[i][b] - (double)fp[b] : (double)f[i][b];
+                const double t = fma(wd[i], d, s[b]);
+                s[b] = MASK ? (v[i] ? t : s[b]) : t;
+            }
+    }
+    template <bool MASK>
+    __device__ __forceinline__ void four(const vq& qc, const vw& wc, const bool (&v)[4], double (&s)[4]) {
+        vf4a f[4];
+        double wd[4];
+        element<0 / EL>(part(qc, 0 % EL), part(wc, 0 % EL), f[0], wd[0]);
+        element<1 / EL>(part(qc, 1 % EL), part(wc, 1 % EL), f[1], wd[1]);
+        element<2 / EL>(part(qc, 2 % EL), part(wc, 2 % EL), f[2], wd[2]);
+        element<3 / EL>(part(qc, 3 % EL), part(wc, 3 % EL), f[3], wd[3]);
+        add<MASK>(f, wd, v, s);
+    }
+    // Column and weight of chunk C: lane g takes EL of its 4 nonzeros.
+    template <int C>
+    __device__ __forceinline__ void load(vq& qc, vw& wc) {
+        const int e = 4 * C + EL * g;
+        const int64_t at = lenv > 0 ? rs + min(e, lenv - 1) : 0;
+        qc = *reinterpret_cast<const vq*>(a.col + at);
+        wc = *reinterpret_cast<const vw*>(a.W[0] + at);
+    }
+    template <int C>
+    __device__ __forceinline__ void load_ahead() {
+        if constexpr (AHEAD) {
+            if (__ballot(4 * C < lenv)) load<C>(q[C], w[C]);
+            if constexpr (C + 1 < G * NCH) load_ahead<C + 1>();
+        }
+    }
+    template <int C>
+    __device__ __forceinline__ void chunk(double (&s)[4]) {
+        if (!__ballot(4 * C < lenv)) return;
+        const bool v[4] = {4 * C < lenv, 4 * C + 1 < lenv, 4 * C + 2 < lenv, 4 * C + 3 < lenv};
+        vq qc;
+        vw wc;
+        if constexpr (AHEAD) qc = q[C], wc = w[C];
+        else load<C>(qc, wc);
+        if (__ballot(!v[3])) four<true>(qc, wc, v, s);
+        else four<false>(qc, wc, v, s);
+    }
+    // Partial sum P: its chunks, then every G-th nonzero of the tail.
+    template <int P>
+    __device__ __forceinline__ void partial(double (&s)[4]) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) s[b] = 0.0;
+        chunk<P>(s);
+        if constexpr (NCH > 1) chunk<P + G>(s);
+        if constexpr (NCH > 2) chunk<P + 2 * G>(s);
+        const int tail = lenv > 0 ? 4 * G * NCH : 0;
+        for (int e = tail + P; __ballot(e < len); e += 4 * G) {
+            // the next four of the stride, EL per lane
+            int32_t qe[EL];
+            float we[EL];
+#pragma unroll
+            for (int k = 0; k < EL; ++k) {
+                const int at = e + G * (EL * g + k);
+                const int64_t j = at < len ? rs + at : 0;
+                qe[k] = a.col[j];
+                we[k] = a.W[0][j];
+            }
+            vq qv;
+            vw wv;
+            if constexpr (EL == 1) qv = qe[0], wv = we[0];
+            else
+#pragma unroll
+                for (int k = 0; k < EL; ++k) qv[k] = qe[k], wv[k] = we[k];
+            const bool v[4] = {e < len, e + G < len, e + 2 * G < len, e + 3 * G < len};
+            four<true>(qv, wv, v, s);
+        }
+    }
+    // The sum that lane P holds after exchanges at distances G/2 .. OFF.
+    template <int P, int OFF>
+    __device__ __forceinline__ void tree(double (&s)[4]) {
+        if constexpr (OFF == G) {
+            partial<P>(s);
+        } else {
+            tree<P, 2 * OFF>(s);
+            double t[4];
+            tree<P + OFF, 2 * OFF>(t);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                s[b] += t[b];
+                asm volatile("" : "+v"(s[b]));  // added here: not all partial sums kept to the end
+            }
+        }
+    }
+};
+
+constexpr int kBatchBlock = 256;
+template <int G, int NCH, int NF, int MODE>
+__global__ __launch_bounds__(kBatchBlock) void k_apply_batch(const ApplyArgs<float> a) {
+    typedef BatchRow<G, NCH, NF, MODE> Row;
     const int64_t hb = blockIdx.x;
     const int64_t lb = (hb & 7) * a.per_xcd + (hb >> 3);
     if (lb >= a.blocks_needed) return;
-    const int rows_per_block = blockDim.x / G;
-    const int gl = threadIdx.x % G;
-    const int64_t row = lb * rows_per_block + threadIdx.x / G;
-    if (row >= a.n_rows) return;
-    const int64_t rs = a.row_ptr[row];
-    const int64_t re = a.row_ptr[row + 1];
+    const int64_t at = (lb * kBatchBlock + threadIdx.x) / Row::L;
+    const bool live = at < a.n_rows;
+    if (!__ballot(live)) return;  // whole wavefront
+    const int64_t row = live ? at : a.n_rows - 1;
     const int64_t nnz_total = a.row_ptr[a.n_rows];
-    auto gather = [&](int64_t q, float* v) {
-        const vf4a* p = reinterpret_cast<const vf4a*>(a.f + q * NF);
+    const int64_t re = a.row_ptr[row + 1];
+    Row r{a};
+    r.rs = a.row_ptr[row];
+    r.len = (int)(re - r.rs);
+    // rows whose vector loads could pass the end of the arrays take the tail's
+    // single loads, as in k_apply_v4
+    r.lenv = re + 3 <= nnz_total ? r.len : 0;
+    r.g = threadIdx.x % Row::L;
+    r.fp = *reinterpret_cast<const vf4a*>(a.f + row * NF + 4 * r.g);
+    double s[4];
+    r.template load_ahead<0>();
+    r.template tree<0, 1>(s);
+    if (!live) return;
 #pragma unroll
-        for (int c = 0; c < NF / 4; ++c) {
-            const vf4a x = p[c];
-            v[4 * c] = x.x;
-            v[4 * c + 1] = x.y;
-            v[4 * c + 2] = x.z;
-            v[4 * c + 3] = x.w;
-        }
-    };
-    float fp[NF];
-    gather(row, fp);
-    double acc[NF];
-#pragma unroll
-    for (int b = 0; b < NF; ++b) acc[b] = 0.0;
-    int64_t jtail = rs + gl;
-    if (re > rs && re + 3 <= nnz_total) {
-        vi4u q[NCH];
-        vf4u w[NCH];
-        int64_t e0[NCH];
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            e0[c] = rs + 4 * (gl + c * G);
-            const int64_t ee = e0[c] < re ? e0[c] : re - 1;
-            q[c] = DCPSE_STREAM_LOAD((const vi4u*)(a.col + ee));
-            w[c] = DCPSE_STREAM_LOAD((const vf4u*)(a.W[0] + ee));
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int c = 0; c < NCH; ++c)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const bool v = e0[c] + i < re;
-                float fq[NF];
-                gather(q[c][i], fq);
-#pragma unroll
-                for (int b = 0; b < NF; ++b) {
-                    const double d = MODE == kDiff ? (double)fq[b] - (double)fp[b] : (double)fq[b];
-                    acc[b] = v ? fma((double)w[c][i], d, acc[b]) : acc[b];
-                }
-            }
-        jtail = rs + 4 * G * NCH + gl;
-    }
-    for (int64_t j = jtail; j < re; j += G) {
-        const int32_t qq = DCPSE_STREAM_LOAD(a.col + j);
-        const float ww = DCPSE_STREAM_LOAD(a.W[0] + j);
-        float fq[NF];
-        gather(qq, fq);
-#pragma unroll
-        for (int b = 0; b < NF; ++b) {
-            const double d = MODE == kDiff ? (double)fq[b] - (double)fp[b] : (double)fq[b];
-            acc[b] = fma((double)ww, d, acc[b]);
-        }
-    }
-#pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1)
-#pragma unroll
-        for (int b = 0; b < NF; ++b) acc[b] += __shfl_xor(acc[b], off, kWave);
-    if (gl == 0) {
-#pragma unroll
-        for (int b = 0; b < NF; ++b) {
-            double val = acc[b];
-            if (MODE == kExplicitDiag) val = fma((double)a.diag[row], (double)fp[b], val);
-            float* dst = a.out[0] + b * a.ld_out + row;
-            val *= (double)a.alpha;
-            if (a.beta != 0.0f) val = fma((double)a.beta, (double)*dst, val);
-            *dst = (float)val;
-        }
+    for (int b = 0; b < 4; ++b) {
+        double val = s[b];
+        if (MODE == kExplicitDiag) val = fma((double)a.diag[row], (double)r.fp[b], val);
+        float* dst = a.out[0] + (4 * r.g + b) * a.ld_out + row;
+        val *= (double)a.alpha;
+        if (a.beta != 0.0f) val = fma((double)a.beta, (double)*dst, val);
+        *dst = (float)val;
     }
 }
 
 template <int G, int NCH, int NF, int MODE>
-static void launch_apply_il(ApplyArgs<float> a, int block, hipStream_t s) {
-    const int rows_per_block = block / G;
+static void launch_apply_il(ApplyArgs<float> a, int, hipStream_t s) {
+    const int rows_per_block = kBatchBlock / (NF / 4);
     a.blocks_needed = (a.n_rows + rows_per_block - 1) / rows_per_block;
     a.per_xcd = (a.blocks_needed + 7) / 8;
-    k_apply_il<G, NCH, NF, MODE><<<(unsigned)(a.per_xcd * 8), block, 0, s>>>(a);
+    k_apply_batch<G, NCH, NF, MODE><<<(unsigned)(a.per_xcd * 8), kBatchBlock, 0, s>>>(a);
 }
 
 // The interleaved batch kernel for the shapes of the 16-byte-load kernel
