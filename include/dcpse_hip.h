@@ -402,12 +402,42 @@ dcpse_status dcpse_apply_transpose_bundle16_f32(dcpse_ctx* ctx, int64_t n, const
                                                 const int32_t* exc_col, const float* exc_W, int64_t n_exc,
                                                 const float* diag, const float* g, float* out, float alpha,
                                                 float beta);
+/* 16-bit columns shared by every operator of a Verlet list (one set of
+ * n < 2^30 particles): col16[n_slots] in slot order beside each operator's own
+ * weights (dcpse_sell_fill_weights_f32 / _f64). Slot j of slice s has a base
+ * for its 64 lanes, base[slice_ptr[s] / 64 + j] (n_slots / 64 of them), and a
+ * lane stores the offset q - p (modulo n into [-n/2, n/2)) less the base as an
+ * unsigned residual; 0xFFFF marks padding and the neighbours that do not fit,
+ * which are listed per lane with their slots. dcpse_sell_fill_col16 writes
+ * col16, base, exc_ptr[64*n_slices+1] (device) and *n_exc (host, synchronises);
+ * dcpse_sell_fill_col16_far then sell_row16 (sell_row with bit 30 set on lanes
+ * that have listed neighbours), exc_col[n_exc] and exc_slot[n_exc]. The apply
+ * (out = alpha * D f + beta * out, n_ops operators in one pass) equals
+ * dcpse_apply_sell_f32 / _f64 bit for bit where nothing is listed. */
+dcpse_status dcpse_sell_fill_col16(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
+                                   const int64_t* slice_ptr, const int32_t* sell_row, uint16_t* col16, int32_t* base,
+                                   int64_t* exc_ptr, int64_t* n_exc);
+dcpse_status dcpse_sell_fill_col16_far(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
+                                       const int64_t* slice_ptr, const int32_t* sell_row, const int32_t* base,
+                                       const int64_t* exc_ptr, int64_t n_exc, int32_t* sell_row16, int32_t* exc_col,
+                                       int32_t* exc_slot);
+dcpse_status dcpse_apply_col16_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                   const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                   const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                   int64_t n_exc, int32_t n_ops, const float* const* sell_W, const float* f,
+                                   float* const* out, float alpha, float beta);
+dcpse_status dcpse_apply_col16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                   const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                   const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                   int64_t n_exc, int32_t n_ops, const double* const* sell_W, const double* f,
+                                   double* const* out, double alpha, double beta);
 /* Software pipeline of the SELL apply: groups of 4 slots per batch (2 or 4)
  * and stages (2: the stream loads of one batch overlap the gathers and FMAs
  * of the other). Default (2, 2). */
 dcpse_status dcpse_set_sell_pipeline(dcpse_ctx* ctx, int32_t groups, int32_t depth);
 /* Accumulation of the FP32 sliced-ELL forward applies (dcpse_apply_sell_f32,
- * dcpse_apply_sell_bundle_f32, dcpse_apply_sell_bundle16_f32): 64 (default)
+ * dcpse_apply_sell_bundle_f32, dcpse_apply_sell_bundle16_f32,
+ * dcpse_apply_col16_f32): 64 (default)
  * sums the FP32 products (f_q - f_p) W_pq in FP64 and rounds each row once;
  * 32 does every operation in FP32, differences included, as the reference's
  * apply does for float properties (src/DCPSE/Dcpse.hpp:560-659). Transposed
@@ -445,7 +475,7 @@ dcpse_status dcpse_scale_rows_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t*
  * skipped when null; outputs may alias y_a/y_b but not u). Replaces the
  * per-stage vector kernels of src/OdeIntegrators/vector_algebra_ofp_gpu.hpp:13-362
  * that odeint's runge_kutta4 drives through src/OdeIntegrators/OdeIntegrators.hpp:63-135.
- * CSR (f32/f64) and sliced-ELL (f32) layouts as for the apply. */
+ * CSR and sliced-ELL layouts as for the apply. */
 dcpse_status dcpse_stage_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
                              const float* W, const float* u, float alpha, const float* y_a, float ca, float* out_a,
                              const float* y_b, float cb, float* out_b);
@@ -463,6 +493,27 @@ dcpse_status dcpse_stage_bundle16_f32(dcpse_ctx* ctx, int64_t n_rows, const int6
                                       const int64_t* exc_ptr, const int32_t* exc_col, const float* exc_W,
                                       int64_t n_exc, const float* u, float alpha, const float* y_a, float ca,
                                       float* out_a, const float* y_b, float cb, float* out_b);
+/* The FP64 stage on the sliced-ELL layouts, and the stage on 16-bit columns. */
+dcpse_status dcpse_stage_sell_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                  const int32_t* sell_row, const int32_t* sell_col, const double* sell_W,
+                                  const double* u, double alpha, const double* y_a, double ca, double* out_a,
+                                  const double* y_b, double cb, double* out_b);
+dcpse_status dcpse_stage_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
+                                      const int64_t* slice_ptr, const int32_t* sell_row16, const int32_t* bundle,
+                                      const int64_t* exc_ptr, const int32_t* exc_col, const double* exc_W,
+                                      int64_t n_exc, const double* u, double alpha, const double* y_a, double ca,
+                                      double* out_a, const double* y_b, double cb, double* out_b);
+dcpse_status dcpse_stage_col16_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                   const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                   const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                   int64_t n_exc, const float* sell_W, const float* u, float alpha, const float* y_a,
+                                   float ca, float* out_a, const float* y_b, float cb, float* out_b);
+dcpse_status dcpse_stage_col16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                   const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                   const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                   int64_t n_exc, const double* sell_W, const double* u, double alpha,
+                                   const double* y_a, double ca, double* out_a, const double* y_b, double cb,
+                                   double* out_b);
 /* n_steps classic RK4 steps of df/dt = alpha * D f (the integration of
  * src/OdeIntegrators/tests/OdeIntegratores_base_tests.cpp:478-577 with
  * runge_kutta4), state f updated in place; 4 stage launches per step.
@@ -478,6 +529,24 @@ dcpse_status dcpse_rk4_bundle16_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_
                                     const int64_t* slice_ptr, const int32_t* sell_row16, const int32_t* bundle,
                                     const int64_t* exc_ptr, const int32_t* exc_col, const float* exc_W,
                                     int64_t n_exc, float alpha, double dt, int64_t n_steps, float* f, float* work);
+dcpse_status dcpse_rk4_sell_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                const int32_t* sell_row, const int32_t* sell_col, const double* sell_W, double alpha,
+                                double dt, int64_t n_steps, double* f, double* work);
+dcpse_status dcpse_rk4_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
+                                    const int64_t* slice_ptr, const int32_t* sell_row16, const int32_t* bundle,
+                                    const int64_t* exc_ptr, const int32_t* exc_col, const double* exc_W,
+                                    int64_t n_exc, double alpha, double dt, int64_t n_steps, double* f,
+                                    double* work);
+dcpse_status dcpse_rk4_col16_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                 const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                 const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                 int64_t n_exc, const float* sell_W, float alpha, double dt, int64_t n_steps,
+                                 float* f, float* work);
+dcpse_status dcpse_rk4_col16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                 const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                 const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                 int64_t n_exc, const double* sell_W, double alpha, double dt, int64_t n_steps,
+                                 double* f, double* work);
 
 #ifdef __cplusplus
 }

@@ -26,6 +26,10 @@ _u32 = C.c_uint32
 _f32 = C.c_float
 _f64 = C.c_double
 
+# row_ptr .. exc_slot and n_exc of the 16-bit columns; u .. out_b of an FP64 stage
+_COL16 = [_vp] * 8 + [_i64]
+_STAGE64 = [_vp, _f64, _vp, _f64, _vp, _vp, _f64, _vp]
+
 # name -> (restype, argtypes); mirrors include/dcpse_hip.h one to one
 SIGNATURES = {
     "dcpse_version": (_i32, []),
@@ -99,6 +103,18 @@ SIGNATURES = {
     "dcpse_rk4_sell_f32": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _f32, _f64, _i64, _vp, _vp]),
     "dcpse_stage_bundle16_f32": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _f32, _vp, _f32,
                                         _vp, _vp, _f32, _vp]),
+    "dcpse_sell_fill_col16": (_i32, [_vp, _i64] + [_vp] * 8),
+    "dcpse_sell_fill_col16_far": (_i32, [_vp, _i64] + [_vp] * 6 + [_i64] + [_vp] * 3),
+    "dcpse_apply_col16_f32": (_i32, [_vp, _i64] + _COL16 + [_i32, _vp, _vp, _vp, _f32, _f32]),
+    "dcpse_apply_col16_f64": (_i32, [_vp, _i64] + _COL16 + [_i32, _vp, _vp, _vp, _f64, _f64]),
+    "dcpse_stage_sell_f64": (_i32, [_vp, _i64] + [_vp] * 5 + _STAGE64),
+    "dcpse_stage_bundle16_f64": (_i32, [_vp, _i64] + [_vp] * 7 + [_i64] + _STAGE64),
+    "dcpse_stage_col16_f32": (_i32, [_vp, _i64] + _COL16 + [_vp, _vp, _f32, _vp, _f32, _vp, _vp, _f32, _vp]),
+    "dcpse_stage_col16_f64": (_i32, [_vp, _i64] + _COL16 + [_vp] + _STAGE64),
+    "dcpse_rk4_sell_f64": (_i32, [_vp, _i64] + [_vp] * 5 + [_f64, _f64, _i64, _vp, _vp]),
+    "dcpse_rk4_bundle16_f64": (_i32, [_vp, _i64] + [_vp] * 7 + [_i64, _f64, _f64, _i64, _vp, _vp]),
+    "dcpse_rk4_col16_f32": (_i32, [_vp, _i64] + _COL16 + [_vp, _f32, _f64, _i64, _vp, _vp]),
+    "dcpse_rk4_col16_f64": (_i32, [_vp, _i64] + _COL16 + [_vp, _f64, _f64, _i64, _vp, _vp]),
     "dcpse_rk4_bundle16_f32": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _f32, _f64, _i64, _vp,
                                       _vp]),
 }

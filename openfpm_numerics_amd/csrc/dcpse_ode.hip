@@ -132,6 +132,51 @@ dcpse_status dcpse_rk4_bundle16_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_
     return DCPSE_OK;
 }
 
+dcpse_status dcpse_rk4_sell_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                const int32_t* sell_row, const int32_t* sell_col, const double* sell_W, double alpha,
+                                double dt, int64_t n_steps, double* f, double* work) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!f || !work || n_steps < 0 || n_rows < 0) return fail(ctx, DCPSE_ERR_INVALID, "null pointer or bad size");
+    DCPSE_RK4_STEPS(dcpse_stage_sell_f64, double, ctx, n_rows, row_ptr, slice_ptr, sell_row, sell_col, sell_W);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_rk4_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
+                                    const int64_t* slice_ptr, const int32_t* sell_row16, const int32_t* bundle,
+                                    const int64_t* exc_ptr, const int32_t* exc_col, const double* exc_W,
+                                    int64_t n_exc, double alpha, double dt, int64_t n_steps, double* f,
+                                    double* work) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!f || !work || n_steps < 0 || n_rows < 0) return fail(ctx, DCPSE_ERR_INVALID, "null pointer or bad size");
+    DCPSE_RK4_STEPS(dcpse_stage_bundle16_f64, double, ctx, n_rows, row_ptr, slice_ptr, sell_row16, bundle, exc_ptr,
+                    exc_col, exc_W, n_exc);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_rk4_col16_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                 const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                 const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                 int64_t n_exc, const float* sell_W, float alpha, double dt, int64_t n_steps,
+                                 float* f, float* work) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!f || !work || n_steps < 0 || n_rows < 0) return fail(ctx, DCPSE_ERR_INVALID, "null pointer or bad size");
+    DCPSE_RK4_STEPS(dcpse_stage_col16_f32, float, ctx, n_rows, row_ptr, slice_ptr, sell_row16, col16, base, exc_ptr,
+                    exc_col, exc_slot, n_exc, sell_W);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_rk4_col16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                 const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                 const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                 int64_t n_exc, const double* sell_W, double alpha, double dt, int64_t n_steps,
+                                 double* f, double* work) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!f || !work || n_steps < 0 || n_rows < 0) return fail(ctx, DCPSE_ERR_INVALID, "null pointer or bad size");
+    DCPSE_RK4_STEPS(dcpse_stage_col16_f64, double, ctx, n_rows, row_ptr, slice_ptr, sell_row16, col16, base, exc_ptr,
+                    exc_col, exc_slot, n_exc, sell_W);
+    return DCPSE_OK;
+}
+
 dcpse_status dcpse_rk4_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
                            const float* W, float alpha, double dt, int64_t n_steps, float* f, float* work) {
     if (!ctx) return DCPSE_ERR_INVALID;

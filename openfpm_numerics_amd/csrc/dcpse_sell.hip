@@ -372,6 +372,117 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16_f64(
     }
 }
 
+// 16-bit columns shared by every operator of a Verlet list (col16 beside the
+// operators' own weights in slot order; one set of n particles). Slot j of
+// slice s has one 32-bit base for its 64 lanes, base[slice_ptr[s] / 64 + j],
+// and a lane stores its offset q - p (modulo n, as above) less that base as an
+// unsigned 16-bit residual. The lanes' rows are consecutive particles, whose
+// j-th neighbours lie about as far away, so the residuals fit where the offsets
+// themselves, planes of a large set apart, do not: of the 60M neighbours of the
+// adaptive million-particle set EXC16 do not fit, against EXC0 of plain 16-bit
+// offsets. kFar16 marks neighbours that do not fit (listed per lane with their
+// slot, as for the bundle) and padding, so it is the apply's only mask.
+constexpr int kFar16 = 0xFFFF;
+
+// One block per slice through an LDS tile of 32 slots x 64 lanes, as in
+// k_sell_fill_bundle16; a wavefront then takes 4 slots at a time, the base from
+// the middle one of the lanes that have the slot. exc_count: neighbours of the
+// lane that do not fit.
+__global__ __launch_bounds__(256) void k_sell_fill_col16(int64_t n_rows, const int64_t* __restrict__ row_ptr,
+                                                         const int32_t* __restrict__ col,
+                                                         const int64_t* __restrict__ slice_ptr,
+                                                         const int32_t* __restrict__ sell_row,
+                                                         uint16_t* __restrict__ col16, int32_t* __restrict__ base,
+                                                         int32_t* __restrict__ exc_count) {
+    __shared__ int32_t tc[kB16Chunk * kB16Pitch];
+    __shared__ int32_t srow[64];
+    __shared__ int64_t srs[64];
+    __shared__ int32_t slen[64];
+    __shared__ int32_t cnt[256];
+    const int64_t n_slices = (n_rows + 63) / 64;
+    const int tid = threadIdx.x;
+    const int l = tid & 63, gsub = tid >> 6, e = tid & 31;
+    for (int64_t s = blockIdx.x; s < n_slices; s += gridDim.x) {
+        __syncthreads();  // the previous slice's lane table is consumed
+        if (tid < 64) {
+            const SliceLane r = slice_lane(row_ptr, sell_row, s * 64 + tid);
+            srow[tid] = r.row;
+            srs[tid] = r.rs;
+            slen[tid] = r.len;
+        }
+        __syncthreads();
+        const int len = slen[l];
+        const int64_t first = slice_ptr[s];
+        const int ng = (int)((slice_ptr[s + 1] - first) >> 8);
+        int far = 0;
+        for (int g0 = 0; g0 < ng; g0 += kB16Chunk / 4) {
+            const int j = 4 * g0 + e;
+            for (int it = 0; it < 8; ++it) {
+                const int ll = 16 * gsub + 2 * it + ((tid >> 5) & 1);
+                int32_t d = 0;
+                if (j < slen[ll]) d = (int32_t)col_offset(col[srs[ll] + j], srow[ll], n_rows);
+                tc[e * kB16Pitch + ll] = d;
+            }
+            __syncthreads();
+            const int gn = min(kB16Chunk / 4, ng - g0);
+            for (int gl = gsub; gl < gn; gl += 4) {
+                typedef uint16_t vu4 __attribute__((ext_vector_type(4)));
+                vu4 v;
+#pragma unroll
+                for (int jj = 0; jj < 4; ++jj) {
+                    const int jl = 4 * (g0 + gl) + jj;
+                    const int32_t d = tc[(4 * gl + jj) * kB16Pitch + l];
+                    const bool have = jl < len;
+                    const int n_have = __popcll(__ballot(have));  // the first lanes: rows by decreasing length
+                    const int32_t b = __builtin_amdgcn_readlane(d, n_have >> 1) - kFar16 / 2;
+                    const int32_t r = d - b;
+                    const bool fits = have && r >= 0 && r < kFar16;
+                    far += have && !fits;
+                    v[jj] = (uint16_t)(fits ? r : kFar16);
+                    if (l == 0) base[first / 64 + jl] = b;
+                }
+                *reinterpret_cast<vu4*>(col16 + first + (int64_t)(g0 + gl) * 256 + 4 * l) = v;
+            }
+            __syncthreads();
+        }
+        cnt[tid] = far;
+        __syncthreads();
+        if (gsub == 0) exc_count[s * 64 + l] = cnt[l] + cnt[64 + l] + cnt[128 + l] + cnt[192 + l];
+    }
+}
+
+// sell_row with the lanes that have listed neighbours marked, and the lists:
+// one thread per lane walks its row in order.
+__global__ void k_col16_exc(int64_t n_rows, const int64_t* __restrict__ row_ptr, const int32_t* __restrict__ col,
+                            const int64_t* __restrict__ slice_ptr, const int32_t* __restrict__ sell_row,
+                            const int32_t* __restrict__ base, const int64_t* __restrict__ exc_ptr,
+                            int32_t* __restrict__ sell_row16, int32_t* __restrict__ exc_col,
+                            int32_t* __restrict__ exc_slot) {
+    const int64_t n_lanes = ((n_rows + 63) / 64) * 64;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_lanes;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        int64_t e = exc_ptr[i];
+        const SliceLane r = slice_lane(row_ptr, sell_row, i);
+        const bool any = exc_ptr[i + 1] > e;
+        sell_row16[i] = any ? (r.row | kExcFlag) : r.row;
+        if (!any) continue;
+        const int64_t sb = slice_ptr[i / 64] / 64;
+        for (int j = 0; j < r.len; ++j) {
+            const int32_t q = col[r.rs + j];
+            const int64_t d = col_offset(q, r.row, n_rows) - base[sb + j];
+            if (d < 0 || d >= kFar16) {
+                exc_col[e] = q;
+                exc_slot[e] = j;
+                ++e;
+            }
+        }
+    }
+}
+
+// Column formats of the apply kernels: 32-bit columns (separate arrays or the
+// interleaved bundle), the 16-bit offsets of the bundle, and 16-bit residuals.
+enum SellCols { kCol32 = 0, kBundle16 = 1, kResid16 = 2 };
+
 struct SellArgs {
     int64_t n_rows;
     const int64_t* row_ptr;
@@ -383,6 +494,9 @@ struct SellArgs {
     const int32_t* exc_col;
     const float* exc_W;
     int64_t n_exc;
+    const uint16_t* col16;    // 16-bit residuals (see k_sell_fill_col16), their bases and
+    const int32_t* base;      // the slots of the far neighbours
+    const int32_t* exc_slot;
     const float* W[4];
     const float* f;
     const float* f_self;
@@ -437,9 +551,10 @@ __device__ __forceinline__ void sell_epilogue(const SellArgs& a, int32_t row, fl
     }
 }
 
-template <int NOPS, int UNR, bool C16 = false>
+template <int NOPS, int UNR, int COLS = kCol32>
 struct SellBatch {
-    typename std::conditional<C16, vs4a, vi4a>::type q[UNR];  // columns, or 16-bit offsets
+    typename std::conditional<COLS == kCol32, vi4a, vs4a>::type q[UNR];  // columns, or 16 bits each
+    vi4a base[COLS == kResid16 ? UNR : 1];                               // wave-uniform
     vf4a w[NOPS][UNR];
 };
 
@@ -449,18 +564,22 @@ struct SellBatch {
 // Every slot a lane can read is written by k_sell_fill: padding and the lanes
 // without a row hold column 0, so every gather stays inside f. The loaded
 // columns are used as they are (no select on them), so nothing waits for a
-// batch before its gathers are due.
-template <int NOPS, int UNR, bool C16 = false>
+// batch before its gathers are due. bp: the slice's bases (16-bit residuals),
+// ng its groups.
+template <int NOPS, int UNR, int COLS>
 __device__ __forceinline__ void sell_load(const int32_t* cp, const float* const* wp, int64_t gs, int g0, int len,
-                                          SellBatch<NOPS, UNR, C16>& b) {
+                                          const int32_t* bp, int ng, SellBatch<NOPS, UNR, COLS>& b) {
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
         const int g = g0 + u;
         const int64_t off = 4 * g < len ? (int64_t)g * gs : 0;
-        if constexpr (C16)  // cp points at this lane's 8 bytes of offsets
+        if constexpr (COLS == kBundle16)  // cp points at this lane's 8 bytes of offsets
             b.q[u] = *(const vs4a*)(reinterpret_cast<const int16_t*>(cp) + 2 * off);
+        else if constexpr (COLS == kResid16)
+            b.q[u] = *(const vs4a*)(reinterpret_cast<const int16_t*>(cp) + off);
         else
             b.q[u] = *(const vi4a*)(cp + off);
+        if constexpr (COLS == kResid16) b.base[u] = *(const vi4a*)(bp + 4 * min(g, ng - 1));
 #pragma unroll
         for (int o = 0; o < NOPS; ++o) b.w[o][u] = *(const vf4a*)(wp[o] + off);
     }
@@ -469,74 +588,85 @@ __device__ __forceinline__ void sell_load(const int32_t* cp, const float* const*
 // Where lane `lane` of slice s finds its columns and weights, and the element
 // stride between its consecutive slot groups: separate arrays (stride 256) or
 // the interleaved bundle (stride (1 + NOPS) * 256).
-template <int NOPS, bool C16 = false>
+template <int NOPS, int COLS>
 __device__ __forceinline__ int64_t sell_streams(const SellArgs& a, int64_t base, int lane, const int32_t*& cp,
                                                 const float* (&wp)[NOPS]) {
-    if constexpr (C16) {
+    if constexpr (COLS == kBundle16) {
         const int64_t blk = 128 + 256 * NOPS;
         const int32_t* bp = a.bundle + (base / 256) * blk;
         cp = bp + 2 * lane;  // 8 bytes of offsets per lane
 #pragma unroll
         for (int o = 0; o < NOPS; ++o) wp[o] = reinterpret_cast<const float*>(bp + 128 + o * 256) + 4 * lane;
         return blk;
-    }
-    if (a.bundle) {
-        const int32_t* bp = a.bundle + (int64_t)(1 + NOPS) * base + 4 * lane;
-        cp = bp;
+    } else {
+        if (COLS == kCol32 && a.bundle) {
+            const int32_t* bp = a.bundle + (int64_t)(1 + NOPS) * base + 4 * lane;
+            cp = bp;
 #pragma unroll
-        for (int o = 0; o < NOPS; ++o) wp[o] = reinterpret_cast<const float*>(bp + (1 + o) * 256);
-        return (int64_t)(1 + NOPS) * 256;
-    }
-    cp = a.sell_col + base + 4 * lane;
+            for (int o = 0; o < NOPS; ++o) wp[o] = reinterpret_cast<const float*>(bp + (1 + o) * 256);
+            return (int64_t)(1 + NOPS) * 256;
+        }
+        if constexpr (COLS == kResid16) cp = reinterpret_cast<const int32_t*>(a.col16 + base + 4 * lane);
+        else cp = a.sell_col + base + 4 * lane;
 #pragma unroll
-    for (int o = 0; o < NOPS; ++o) wp[o] = a.W[o] + base + 4 * lane;
-    return 256;
+        for (int o = 0; o < NOPS; ++o) wp[o] = a.W[o] + base + 4 * lane;
+        return 256;
+    }
 }
 
 // The f gathers of groups [g0, g0+UNR) (columns of a loaded batch).
-template <int UNR>
+template <int UNR, typename T = float>
 struct SellGathered {
-    float fq[UNR][4];
+    T fq[UNR][4];
+    vs4a r[UNR];  // 16-bit residuals with the groups past the row masked
 };
 
-// Column of a 16-bit offset d of row rb in a set of n particles.
-__device__ __forceinline__ int32_t sell_col16(int32_t rb, int16_t d, int32_t n) {
-    int32_t q = rb + (int32_t)d;
-    q += q < 0 ? n : 0;
-    q -= q >= n ? n : 0;
-    return q;
+// Column q in (-n, 2n) wrapped into a set of n < 2^30 particles.
+__device__ __forceinline__ int32_t wrap_col(int32_t q, int32_t n) {
+    const uint32_t a = min((uint32_t)q, (uint32_t)q + (uint32_t)n);  // a negative q is the larger unsigned one
+    return (int32_t)min(a, a - (uint32_t)n);
 }
 
-template <int NOPS, int UNR, bool C16 = false>
-__device__ __forceinline__ void sell_gather(const SellArgs& a, const SellBatch<NOPS, UNR, C16>& b,
-                                            SellGathered<UNR>& g, int32_t rb = 0) {
+// Column of a 16-bit offset d of row rb in a set of n particles.
+__device__ __forceinline__ int32_t sell_col16(int32_t rb, int16_t d, int32_t n) { return wrap_col(rb + (int32_t)d, n); }
+
+// ... of residual r over base b (any value for kFar16 and masked groups, kept inside the set).
+__device__ __forceinline__ int32_t sell_resid16(int32_t rb, int32_t b, int16_t r, int32_t n) {
+    return (int32_t)min((uint32_t)wrap_col(rb + b + (int32_t)(uint16_t)r, n), (uint32_t)(n - 1));
+}
+
+template <int UNR, int COLS, typename Batch, typename T>
+__device__ __forceinline__ void sell_gather(const T* __restrict__ f, int32_t n, const Batch& b, int g0, int len,
+                                            SellGathered<UNR, T>& g, int32_t rb) {
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
-        if constexpr (C16) {
-            const int32_t n = (int32_t)a.n_rows;
-            g.fq[u][0] = a.f[sell_col16(rb, b.q[u].x, n)];
-            g.fq[u][1] = a.f[sell_col16(rb, b.q[u].y, n)];
-            g.fq[u][2] = a.f[sell_col16(rb, b.q[u].z, n)];
-            g.fq[u][3] = a.f[sell_col16(rb, b.q[u].w, n)];
-        } else {
-            g.fq[u][0] = a.f[b.q[u].x];
-            g.fq[u][1] = a.f[b.q[u].y];
-            g.fq[u][2] = a.f[b.q[u].z];
-            g.fq[u][3] = a.f[b.q[u].w];
+        if constexpr (COLS == kResid16) {
+            const bool past = 4 * (g0 + u) >= len;
+            typedef int32_t vi2 __attribute__((ext_vector_type(2)));
+            vi2 w = __builtin_bit_cast(vi2, b.q[u]);
+            w.x = past ? -1 : w.x;
+            w.y = past ? -1 : w.y;
+            g.r[u] = __builtin_bit_cast(vs4a, w);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (COLS == kBundle16) g.fq[u][i] = f[sell_col16(rb, b.q[u][i], n)];
+            else if constexpr (COLS == kResid16) g.fq[u][i] = f[sell_resid16(rb, b.base[u][i], g.r[u][i], n)];
+            else g.fq[u][i] = f[b.q[u][i]];
         }
     }
 }
 
 // The FMAs of groups [g0, g0+UNR); slots past the row are masked. Acc is
 // double (default) or float (every operation in FP32).
-template <int NOPS, int UNR, int MODE, bool C16, typename Acc>
-__device__ __forceinline__ void sell_fma(int g0, int len, float fp, const SellBatch<NOPS, UNR, C16>& b,
-                                         const SellGathered<UNR>& g, Acc* acc) {
+template <int NOPS, int UNR, int MODE, int COLS, typename Acc, typename Batch, typename T>
+__device__ __forceinline__ void sell_fma(int g0, int len, T fp, const Batch& b, const SellGathered<UNR, T>& g,
+                                         Acc* acc) {
 #pragma unroll
     for (int u = 0; u < UNR; ++u)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const bool v = 4 * (g0 + u) + i < len;
+            const bool v = COLS == kResid16 ? (uint16_t)g.r[u][i] != kFar16 : 4 * (g0 + u) + i < len;
             const Acc d = MODE == 1 ? (Acc)g.fq[u][i] : (Acc)g.fq[u][i] - (Acc)fp;
 #pragma unroll
             for (int o = 0; o < NOPS; ++o) acc[o] = v ? fma((Acc)b.w[o][u][i], d, acc[o]) : acc[o];
@@ -549,153 +679,142 @@ __device__ __forceinline__ void sell_fma(int g0, int len, float fp, const SellBa
 // waiting for the gathers does not wait for the stream loads issued after
 // them: the next batch's col/W loads stay in flight across the FMAs, and its
 // gathers go out as soon as its columns arrive.
-template <int NOPS, int UNR, int MODE, bool C16 = false, bool ACC32 = false>
+template <int NOPS, int UNR, int MODE, int COLS = kCol32, bool ACC32 = false>
 __global__ __launch_bounds__(kSellWaves * kWave) void k_apply_sell(const SellArgs a) {
     using Acc = typename std::conditional<ACC32, float, double>::type;
     const int64_t hb = blockIdx.x;
     const int64_t lb = (hb & 7) * a.per_xcd + (hb >> 3);
     if (lb >= a.blocks_needed) return;
     const int lane = threadIdx.x & 63;
-    const int64_t s = lb * kSellWaves + (threadIdx.x >> 6);
+    const int64_t s = lb * kSellWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (s * 64 >= a.n_rows) return;  // whole wavefront
     const int32_t row_raw = a.sell_row[s * 64 + lane];
     const bool live = row_raw >= 0;
-    const bool has_exc = C16 && live && (row_raw & kExcFlag);
-    const int32_t row = C16 && live ? (row_raw & ~kExcFlag) : row_raw;
+    const bool has_exc = COLS != kCol32 && live && (row_raw & kExcFlag);
+    const int32_t row = COLS != kCol32 && live ? (row_raw & ~kExcFlag) : row_raw;
     const int len = live ? (int)(a.row_ptr[row + 1] - a.row_ptr[row]) : 0;
     const float fp = live ? a.f_self[row] : 0.0f;
     const int64_t base = a.slice_ptr[s];
     const int ng = (int)((a.slice_ptr[s + 1] - base) >> 8);  // groups of 4 slots
     const int32_t* cp;
     const float* wp[NOPS];
-    const int64_t gs = sell_streams<NOPS, C16>(a, base, lane, cp, wp);
+    const int64_t gs = sell_streams<NOPS, COLS>(a, base, lane, cp, wp);
+    const int32_t* bp = COLS == kResid16 ? a.base + base / 64 : nullptr;
     const int32_t rb = live ? row : 0;  // 16-bit offsets are relative to the lane's row
+    const int32_t n = (int32_t)a.n_rows;
     Acc acc[NOPS];
 #pragma unroll
     for (int o = 0; o < NOPS; ++o) acc[o] = 0;
     if (ng > 0) {  // a slice of empty rows has no slots to read
-        SellBatch<NOPS, UNR, C16> bA, bB;
+        SellBatch<NOPS, UNR, COLS> bA, bB;
         SellGathered<UNR> gA, gB;
-        sell_load<NOPS, UNR, C16>(cp, wp, gs, 0, len, bA);
+        sell_load<NOPS, UNR, COLS>(cp, wp, gs, 0, len, bp, ng, bA);
         for (int g0 = 0; g0 < ng; g0 += 2 * UNR) {
-            sell_gather<NOPS, UNR, C16>(a, bA, gA, rb);
+            sell_gather<UNR, COLS>(a.f, n, bA, g0, len, gA, rb);
             __builtin_amdgcn_sched_barrier(0);
-            sell_load<NOPS, UNR, C16>(cp, wp, gs, g0 + UNR, len, bB);
+            sell_load<NOPS, UNR, COLS>(cp, wp, gs, g0 + UNR, len, bp, ng, bB);
             __builtin_amdgcn_sched_barrier(0);
-            sell_fma<NOPS, UNR, MODE, C16, Acc>(g0, len, fp, bA, gA, acc);
+            sell_fma<NOPS, UNR, MODE, COLS, Acc>(g0, len, fp, bA, gA, acc);
             __builtin_amdgcn_sched_barrier(0);
-            sell_gather<NOPS, UNR, C16>(a, bB, gB, rb);
+            sell_gather<UNR, COLS>(a.f, n, bB, g0 + UNR, len, gB, rb);
             __builtin_amdgcn_sched_barrier(0);
-            sell_load<NOPS, UNR, C16>(cp, wp, gs, g0 + 2 * UNR, len, bA);
+            sell_load<NOPS, UNR, COLS>(cp, wp, gs, g0 + 2 * UNR, len, bp, ng, bA);
             __builtin_amdgcn_sched_barrier(0);
-            sell_fma<NOPS, UNR, MODE, C16, Acc>(g0 + UNR, len, fp, bB, gB, acc);
+            sell_fma<NOPS, UNR, MODE, COLS, Acc>(g0 + UNR, len, fp, bB, gB, acc);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    if constexpr (C16) {
+    if constexpr (COLS != kCol32) {
         if (has_exc) {  // the far neighbours of this row (rare; after every pipelined load)
             const int64_t i = s * 64 + lane;
             for (int64_t k = a.exc_ptr[i]; k < a.exc_ptr[i + 1]; ++k) {
                 const Acc d = MODE == 1 ? (Acc)a.f[a.exc_col[k]] : (Acc)a.f[a.exc_col[k]] - (Acc)fp;
+                const int j = COLS == kResid16 ? a.exc_slot[k] : 0;
 #pragma unroll
-                for (int o = 0; o < NOPS; ++o) acc[o] = fma((Acc)a.exc_W[o * a.n_exc + k], d, acc[o]);
+                for (int o = 0; o < NOPS; ++o) {
+                    const float w = COLS == kResid16 ? wp[o][(int64_t)(j >> 2) * 256 + (j & 3)] : a.exc_W[o * a.n_exc + k];
+                    acc[o] = fma((Acc)w, d, acc[o]);
+                }
             }
         }
     }
     if (live) sell_epilogue<NOPS, MODE>(a, row, fp, acc);
 }
 
-// FP64 forward apply from the sliced-ELL layout: the columns of the FP32
-// layout (sell_col) and FP64 weights in the same slot order. The pipeline is
-// that of k_apply_sell (two register batches; the gathers of the loaded batch
-// before the next batch's stream loads); a slot group is 16 bytes of columns
-// and 32 bytes of weights per operator and lane.
+// FP64 apply (MODE 0) and time-integration stage (MODE 2) from the sliced-ELL
+// layouts: the columns of the FP32 layouts and FP64 weights in the same slot
+// order. The pipeline is that of k_apply_sell (two register batches; the
+// gathers of the loaded batch before the next batch's stream loads); a slot
+// group is 16 bytes of columns (8 in 16 bits) and 32 bytes of weights per
+// operator and lane.
 typedef double vd4a __attribute__((ext_vector_type(4)));
 
 struct Sell64Args {
     int64_t n_rows;
     const int64_t* row_ptr;
     const int64_t* slice_ptr;
-    const int32_t* sell_row;  // 16-bit bundle: sell_row16 (bit 30: the lane has far neighbours)
+    const int32_t* sell_row;  // 16-bit columns: sell_row16 (bit 30: the lane has far neighbours)
     const int32_t* sell_col;
     const double* W[4];
     const int32_t* bundle;    // 16-bit bundle (k_sell_fill_bundle16_f64), or null
-    const int64_t* exc_ptr;   // 16-bit bundle: far neighbours per lane
+    const int64_t* exc_ptr;   // 16-bit columns: far neighbours per lane
     const int32_t* exc_col;
     const double* exc_W;
     int64_t n_exc;
+    const uint16_t* col16;    // as in SellArgs
+    const int32_t* base;
+    const int32_t* exc_slot;
     const double* f;
     const double* f_self;
     double* out[4];
     double alpha, beta;
+    const double* y_a;  // MODE 2, as in SellArgs
+    const double* y_b;
+    double* out_a;
+    double* out_b;
+    double ca, cb;
     int64_t blocks_needed, per_xcd;
 };
 
-template <int NOPS, int UNR, bool C16 = false>
+template <int NOPS, int UNR, int COLS>
 struct Sell64Batch {
-    typename std::conditional<C16, vs4a, vi4a>::type q[UNR];  // columns, or 16-bit offsets
+    typename std::conditional<COLS == kCol32, vi4a, vs4a>::type q[UNR];  // columns, or 16 bits each
+    vi4a base[COLS == kResid16 ? UNR : 1];                               // wave-uniform
     vd4a w[NOPS][UNR];
 };
 
 // gs: element stride between a lane's consecutive slot groups (the columns'
-// unit: int32 for the separate arrays, int16 for the bundle; weights double)
-template <int NOPS, int UNR, bool C16 = false>
+// unit: int32 for the 32-bit columns, int16 otherwise; weights double)
+template <int NOPS, int UNR, int COLS>
 __device__ __forceinline__ void sell64_load(const void* cp, const double* const* wp, int64_t gsc, int64_t gsw,
-                                            int g0, int len, Sell64Batch<NOPS, UNR, C16>& b) {
+                                            int g0, int len, const int32_t* bp, int ng,
+                                            Sell64Batch<NOPS, UNR, COLS>& b) {
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
         const int g = g0 + u;
         const int64_t gg = 4 * g < len ? (int64_t)g : 0;  // past the row: group 0 again
-        if constexpr (C16)
+        if constexpr (COLS != kCol32)
             b.q[u] = *(const vs4a*)(reinterpret_cast<const int16_t*>(cp) + gg * gsc);
         else
             b.q[u] = *(const vi4a*)(reinterpret_cast<const int32_t*>(cp) + gg * gsc);
+        if constexpr (COLS == kResid16) b.base[u] = *(const vi4a*)(bp + 4 * min(g, ng - 1));
 #pragma unroll
         for (int o = 0; o < NOPS; ++o) b.w[o][u] = *(const vd4a*)(wp[o] + gg * gsw);
     }
 }
 
-template <int NOPS, int UNR, bool C16 = false>
-__device__ __forceinline__ void sell64_gather(const Sell64Args& a, const Sell64Batch<NOPS, UNR, C16>& b,
-                                              double (&fq)[UNR][4], int32_t rb) {
-#pragma unroll
-    for (int u = 0; u < UNR; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if constexpr (C16) fq[u][i] = a.f[sell_col16(rb, b.q[u][i], (int32_t)a.n_rows)];
-            else fq[u][i] = a.f[b.q[u][i]];
-        }
-}
-
-template <int NOPS, int UNR, bool C16 = false>
-__device__ __forceinline__ void sell64_fma(int g0, int len, double fp, const Sell64Batch<NOPS, UNR, C16>& b,
-                                           const double (&fq)[UNR][4], double* acc) {
-#pragma unroll
-    for (int u = 0; u < UNR; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const bool v = 4 * (g0 + u) + i < len;
-            const double d = fq[u][i] - fp;
-#pragma unroll
-            for (int o = 0; o < NOPS; ++o) acc[o] = v ? fma(b.w[o][u][i], d, acc[o]) : acc[o];
-        }
-}
-
-// C16: the 16-bit bundle (k_sell_fill_bundle16_f64); offsets are relative to
-// the lane's row, and a lane flagged in sell_row16 adds its far neighbours
-// from the exception list after the slot loop.
-template <int NOPS, int UNR, bool C16 = false>
+template <int NOPS, int UNR, int COLS, int MODE>
 __global__ __launch_bounds__(kSellWaves * kWave) void k_apply_sell64(const Sell64Args a) {
     const int64_t hb = blockIdx.x;
     const int64_t lb = (hb & 7) * a.per_xcd + (hb >> 3);
     if (lb >= a.blocks_needed) return;
     const int lane = threadIdx.x & 63;
-    const int64_t s = lb * kSellWaves + (threadIdx.x >> 6);
+    const int64_t s = lb * kSellWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (s * 64 >= a.n_rows) return;  // whole wavefront
     const int32_t row_raw = a.sell_row[s * 64 + lane];
     const bool live = row_raw >= 0;
-    const bool has_exc = C16 && live && (row_raw & kExcFlag);
-    const int32_t row = C16 && live ? (row_raw & ~kExcFlag) : row_raw;
+    const bool has_exc = COLS != kCol32 && live && (row_raw & kExcFlag);
+    const int32_t row = COLS != kCol32 && live ? (row_raw & ~kExcFlag) : row_raw;
     const int len = live ? (int)(a.row_ptr[row + 1] - a.row_ptr[row]) : 0;
     const double fp = live ? a.f_self[row] : 0.0;
     const int64_t base = a.slice_ptr[s];
@@ -703,7 +822,7 @@ __global__ __launch_bounds__(kSellWaves * kWave) void k_apply_sell64(const Sell6
     const void* cp;
     const double* wp[NOPS];
     int64_t gsc, gsw;
-    if constexpr (C16) {
+    if constexpr (COLS == kBundle16) {
         const int64_t blk = 128 + 512 * NOPS;  // words per slot group
         const int32_t* bp = a.bundle + (base / 256) * blk;
         cp = reinterpret_cast<const int16_t*>(bp) + 4 * lane;
@@ -712,68 +831,86 @@ __global__ __launch_bounds__(kSellWaves * kWave) void k_apply_sell64(const Sell6
         gsc = 2 * blk;  // int16 units
         gsw = blk / 2;  // double units
     } else {
-        cp = a.sell_col + base + 4 * lane;
+        if constexpr (COLS == kResid16) cp = a.col16 + base + 4 * lane;
+        else cp = a.sell_col + base + 4 * lane;
 #pragma unroll
         for (int o = 0; o < NOPS; ++o) wp[o] = a.W[o] + base + 4 * lane;
         gsc = gsw = 256;
     }
+    const int32_t* bp = COLS == kResid16 ? a.base + base / 64 : nullptr;
     const int32_t rb = live ? row : 0;
+    const int32_t n = (int32_t)a.n_rows;
     double acc[NOPS];
 #pragma unroll
     for (int o = 0; o < NOPS; ++o) acc[o] = 0.0;
     if (ng > 0) {
-        Sell64Batch<NOPS, UNR, C16> bA, bB;
-        double gA[UNR][4], gB[UNR][4];
-        sell64_load<NOPS, UNR, C16>(cp, wp, gsc, gsw, 0, len, bA);
+        Sell64Batch<NOPS, UNR, COLS> bA, bB;
+        SellGathered<UNR, double> gA, gB;
+        sell64_load<NOPS, UNR, COLS>(cp, wp, gsc, gsw, 0, len, bp, ng, bA);
         for (int g0 = 0; g0 < ng; g0 += 2 * UNR) {
-            sell64_gather<NOPS, UNR, C16>(a, bA, gA, rb);
+            sell_gather<UNR, COLS>(a.f, n, bA, g0, len, gA, rb);
             __builtin_amdgcn_sched_barrier(0);
-            sell64_load<NOPS, UNR, C16>(cp, wp, gsc, gsw, g0 + UNR, len, bB);
+            sell64_load<NOPS, UNR, COLS>(cp, wp, gsc, gsw, g0 + UNR, len, bp, ng, bB);
             __builtin_amdgcn_sched_barrier(0);
-            sell64_fma<NOPS, UNR, C16>(g0, len, fp, bA, gA, acc);
+            sell_fma<NOPS, UNR, 0, COLS, double>(g0, len, fp, bA, gA, acc);
             __builtin_amdgcn_sched_barrier(0);
-            sell64_gather<NOPS, UNR, C16>(a, bB, gB, rb);
+            sell_gather<UNR, COLS>(a.f, n, bB, g0 + UNR, len, gB, rb);
             __builtin_amdgcn_sched_barrier(0);
-            sell64_load<NOPS, UNR, C16>(cp, wp, gsc, gsw, g0 + 2 * UNR, len, bA);
+            sell64_load<NOPS, UNR, COLS>(cp, wp, gsc, gsw, g0 + 2 * UNR, len, bp, ng, bA);
             __builtin_amdgcn_sched_barrier(0);
-            sell64_fma<NOPS, UNR, C16>(g0 + UNR, len, fp, bB, gB, acc);
+            sell_fma<NOPS, UNR, 0, COLS, double>(g0 + UNR, len, fp, bB, gB, acc);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    if constexpr (C16) {
+    if constexpr (COLS != kCol32) {
         if (has_exc) {  // the far neighbours of this row (rare; after every pipelined load)
             const int64_t i = s * 64 + lane;
             for (int64_t k = a.exc_ptr[i]; k < a.exc_ptr[i + 1]; ++k) {
                 const double d = a.f[a.exc_col[k]] - fp;
+                const int j = COLS == kResid16 ? a.exc_slot[k] : 0;
 #pragma unroll
-                for (int o = 0; o < NOPS; ++o) acc[o] = fma(a.exc_W[o * a.n_exc + k], d, acc[o]);
+                for (int o = 0; o < NOPS; ++o) {
+                    const double w =
+                        COLS == kResid16 ? wp[o][(int64_t)(j >> 2) * 256 + (j & 3)] : a.exc_W[o * a.n_exc + k];
+                    acc[o] = fma(w, d, acc[o]);
+                }
             }
         }
     }
     if (!live) return;
+    if constexpr (MODE == 2) {  // both inputs are read before either output is written
+        const double k = a.alpha * acc[0];
+        const double ya = a.out_a ? a.y_a[row] : 0.0;
+        const double yb = a.out_b ? a.y_b[row] : 0.0;
+        if (a.out_a) a.out_a[row] = fma(a.ca, k, ya);
+        if (a.out_b) a.out_b[row] = fma(a.cb, k, yb);
+    } else {
 #pragma unroll
-    for (int o = 0; o < NOPS; ++o) {
-        double val = acc[o] * a.alpha;
-        if (a.beta != 0.0) val = fma(a.beta, a.out[o][row], val);
-        a.out[o][row] = val;
+        for (int o = 0; o < NOPS; ++o) {
+            double val = acc[o] * a.alpha;
+            if (a.beta != 0.0) val = fma(a.beta, a.out[o][row], val);
+            a.out[o][row] = val;
+        }
     }
 }
 
-template <int NOPS, int UNR, bool C16 = false>
+// two slot groups per batch (437 us for the fused Laplacian + Dx at 128^3 on
+// 32-bit columns, one group 445 us; the CSR kernel takes 512 us)
+template <int NOPS, int COLS, int MODE>
 static void launch_sell64(Sell64Args a, hipStream_t st) {
     const int64_t n_slices = (a.n_rows + 63) / 64;
     a.blocks_needed = (n_slices + kSellWaves - 1) / kSellWaves;
     a.per_xcd = (a.blocks_needed + 7) / 8;
-    k_apply_sell64<NOPS, UNR, C16><<<(unsigned)(a.per_xcd * 8), kSellWaves * kWave, 0, st>>>(a);
+    k_apply_sell64<NOPS, 2, COLS, MODE><<<(unsigned)(a.per_xcd * 8), kSellWaves * kWave, 0, st>>>(a);
 }
 
-template <int UNR, bool C16 = false>
+template <int COLS>
 static bool dispatch_sell64(const Sell64Args& a, int nops, hipStream_t st) {
     switch (nops) {
-        case 1: launch_sell64<1, UNR, C16>(a, st); return true;
-        case 2: launch_sell64<2, UNR, C16>(a, st); return true;
-        case 3: launch_sell64<3, UNR, C16>(a, st); return true;
-        case 4: launch_sell64<4, UNR, C16>(a, st); return true;
+        case 1: launch_sell64<1, COLS, 0>(a, st); return true;
+        case 2: launch_sell64<2, COLS, 0>(a, st); return true;
+        case 3: launch_sell64<3, COLS, 0>(a, st); return true;
+        case 4: launch_sell64<4, COLS, 0>(a, st); return true;
     }
     return false;
 }
@@ -783,15 +920,15 @@ static void launch_sell(SellArgs a, hipStream_t st) {
     const int64_t n_slices = (a.n_rows + 63) / 64;
     a.blocks_needed = (n_slices + kSellWaves - 1) / kSellWaves;
     a.per_xcd = (a.blocks_needed + 7) / 8;
-    k_apply_sell<NOPS, UNR, MODE, false, ACC32><<<(unsigned)(a.per_xcd * 8), kSellWaves * kWave, 0, st>>>(a);
+    k_apply_sell<NOPS, UNR, MODE, kCol32, ACC32><<<(unsigned)(a.per_xcd * 8), kSellWaves * kWave, 0, st>>>(a);
 }
 
-template <int NOPS, int UNR, int MODE = 0, bool ACC32 = false>
+template <int NOPS, int UNR, int MODE = 0, bool ACC32 = false, int COLS = kBundle16>
 static void launch_sell16(SellArgs a, hipStream_t st) {
     const int64_t n_slices = (a.n_rows + 63) / 64;
     a.blocks_needed = (n_slices + kSellWaves - 1) / kSellWaves;
     a.per_xcd = (a.blocks_needed + 7) / 8;
-    k_apply_sell<NOPS, UNR, MODE, true, ACC32><<<(unsigned)(a.per_xcd * 8), kSellWaves * kWave, 0, st>>>(a);
+    k_apply_sell<NOPS, UNR, MODE, COLS, ACC32><<<(unsigned)(a.per_xcd * 8), kSellWaves * kWave, 0, st>>>(a);
 }
 
 // 16-bit-offset bundles: forward apply, two-stage pipeline (groups 2 or 4).
@@ -809,6 +946,18 @@ static bool dispatch_sell16_acc(const SellArgs& a, int nops, int unr, hipStream_
 
 static bool dispatch_sell16(const SellArgs& a, int nops, int unr, bool acc32, hipStream_t st) {
     return acc32 ? dispatch_sell16_acc<true>(a, nops, unr, st) : dispatch_sell16_acc<false>(a, nops, unr, st);
+}
+
+// 16-bit residuals: two groups per batch.
+template <bool ACC32>
+static bool dispatch_resid16(const SellArgs& a, int nops, hipStream_t st) {
+    switch (nops) {
+        case 1: launch_sell16<1, 2, 0, ACC32, kResid16>(a, st); return true;
+        case 2: launch_sell16<2, 2, 0, ACC32, kResid16>(a, st); return true;
+        case 3: launch_sell16<3, 2, 0, ACC32, kResid16>(a, st); return true;
+        case 4: launch_sell16<4, 2, 0, ACC32, kResid16>(a, st); return true;
+    }
+    return false;
 }
 
 template <int UNR, int MODE, bool ACC32 = false>
@@ -898,6 +1047,54 @@ static dcpse_status sell_count_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_
     DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     if (ovf) return fail(ctx, DCPSE_ERR_RANGE, "a row exceeds DCPSE_MAX_ROW=%d", DCPSE_MAX_ROW);
     if (n_slots) *n_slots = total;
+    return DCPSE_OK;
+}
+
+// The arguments of the 16-bit residual layout, shared by its entry points.
+template <typename Args, typename T>
+static dcpse_status col16_args(dcpse_ctx* ctx, Args& a, int64_t n_rows, const int64_t* row_ptr,
+                               const int64_t* slice_ptr, const int32_t* sell_row16, const uint16_t* col16,
+                               const int32_t* base, const int64_t* exc_ptr, const int32_t* exc_col,
+                               const int32_t* exc_slot, int64_t n_exc, int32_t n_ops, const T* const* sell_W,
+                               const T* f) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!row_ptr || !slice_ptr || !sell_row16 || !col16 || !base || !exc_ptr || !sell_W || !f || n_rows < 0 ||
+        n_ops < 1 || n_exc < 0 || (n_exc > 0 && (!exc_col || !exc_slot)))
+        return fail(ctx, DCPSE_ERR_INVALID, "null pointer or bad size");
+    if (n_ops > 4) return fail(ctx, DCPSE_ERR_UNSUPPORTED, "at most 4 operators per pass");
+    if (n_rows >= kExcFlag) return fail(ctx, DCPSE_ERR_RANGE, "too many particles for 16-bit columns");
+    for (int o = 0; o < n_ops; ++o)
+        if (!sell_W[o]) return fail(ctx, DCPSE_ERR_INVALID, "null operator pointer");
+    DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    a.n_rows = n_rows;
+    a.row_ptr = row_ptr;
+    a.slice_ptr = slice_ptr;
+    a.sell_row = sell_row16;
+    a.col16 = col16;
+    a.base = base;
+    a.exc_ptr = exc_ptr;
+    a.exc_col = exc_col;
+    a.exc_slot = exc_slot;
+    a.n_exc = n_exc;
+    for (int o = 0; o < n_ops; ++o) a.W[o] = sell_W[o];
+    a.f = a.f_self = f;
+    return DCPSE_OK;
+}
+
+// A time-integration stage's inputs and outputs.
+template <typename Args, typename T>
+static dcpse_status stage_args(dcpse_ctx* ctx, Args& a, const T* u, T alpha, const T* y_a, T ca, T* out_a,
+                               const T* y_b, T cb, T* out_b) {
+    if ((out_a && !y_a) || (out_b && !y_b)) return fail(ctx, DCPSE_ERR_INVALID, "an output without its input");
+    if (out_a == u || out_b == u) return fail(ctx, DCPSE_ERR_INVALID, "a stage output may not alias its input u");
+    a.f = a.f_self = u;
+    a.alpha = alpha;
+    a.y_a = y_a;
+    a.y_b = y_b;
+    a.out_a = out_a;
+    a.out_b = out_b;
+    a.ca = ca;
+    a.cb = cb;
     return DCPSE_OK;
 }
 
@@ -1008,9 +1205,7 @@ dcpse_status dcpse_apply_sell_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t*
     a.f_self = f_self ? f_self : f;
     a.alpha = alpha;
     a.beta = beta;
-    // two slot groups per batch (437 us for the fused Laplacian + Dx at 128^3,
-    // one group 445 us; the CSR kernel takes 512 us)
-    if (!dispatch_sell64<2>(a, n_ops, ctx->stream)) return fail(ctx, DCPSE_ERR_UNSUPPORTED, "no SELL kernel for %d operators", n_ops);
+    if (!dispatch_sell64<kCol32>(a, n_ops, ctx->stream)) return fail(ctx, DCPSE_ERR_UNSUPPORTED, "no SELL kernel for %d operators", n_ops);
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
 }
@@ -1075,7 +1270,7 @@ dcpse_status dcpse_apply_sell_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const
     a.f_self = f_self ? f_self : f;
     a.alpha = alpha;
     a.beta = beta;
-    if (!dispatch_sell64<2, true>(a, n_ops, ctx->stream))
+    if (!dispatch_sell64<kBundle16>(a, n_ops, ctx->stream))
         return fail(ctx, DCPSE_ERR_UNSUPPORTED, "no SELL kernel for %d operators", n_ops);
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
@@ -1366,6 +1561,178 @@ dcpse_status dcpse_apply_transpose_bundle16_f32(dcpse_ctx* ctx, int64_t n, const
     a.beta = beta;
     if (ctx->sell_groups == 4) launch_sell16<1, 4, 1>(a, ctx->stream);
     else launch_sell16<1, 2, 1>(a, ctx->stream);
+    DCPSE_LAUNCH_CHECK(ctx);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_sell_fill_col16(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
+                                   const int64_t* slice_ptr, const int32_t* sell_row, uint16_t* col16, int32_t* base,
+                                   int64_t* exc_ptr, int64_t* n_exc) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!row_ptr || !col || !slice_ptr || !sell_row || !col16 || !base || !exc_ptr || !n_exc || n_rows < 0)
+        return fail(ctx, DCPSE_ERR_INVALID, "null pointer or negative size");
+    if (n_rows >= kExcFlag) return fail(ctx, DCPSE_ERR_RANGE, "too many particles for 16-bit columns");
+    DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    const int64_t n_lanes = ((n_rows + 63) / 64) * 64;
+    Workspace w;
+    dcpse_status st = reserve_workspace(ctx, (size_t)(n_lanes + 1) * 4 + scan_workspace_bytes(n_lanes) + 1024, &w);
+    if (st) return st;
+    int32_t* counts = w.take<int32_t>(n_lanes + 1);
+    if (n_lanes > 0) {
+        const int64_t b = std::min<int64_t>(n_lanes / 64, 65536);
+        k_sell_fill_col16<<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, col, slice_ptr, sell_row, col16,
+                                                                base, counts);
+        DCPSE_LAUNCH_CHECK(ctx);
+    }
+    if ((st = scan_counts(ctx, counts, n_lanes, exc_ptr, &w))) return st;
+    int64_t total = 0;
+    DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&total, exc_ptr + n_lanes, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+    DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    *n_exc = total;
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_sell_fill_col16_far(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
+                                       const int64_t* slice_ptr, const int32_t* sell_row, const int32_t* base,
+                                       const int64_t* exc_ptr, int64_t n_exc, int32_t* sell_row16, int32_t* exc_col,
+                                       int32_t* exc_slot) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!row_ptr || !col || !slice_ptr || !sell_row || !base || !exc_ptr || !sell_row16 || n_rows < 0 || n_exc < 0 ||
+        (n_exc > 0 && (!exc_col || !exc_slot)))
+        return fail(ctx, DCPSE_ERR_INVALID, "null pointer or negative size");
+    if (n_rows >= kExcFlag) return fail(ctx, DCPSE_ERR_RANGE, "too many particles for 16-bit columns");
+    DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    if (n_rows == 0) return DCPSE_OK;
+    const int64_t b = std::min<int64_t>((n_rows + 63 + 255) / 256, 65536);
+    k_col16_exc<<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, col, slice_ptr, sell_row, base, exc_ptr,
+                                                      sell_row16, exc_col, exc_slot);
+    DCPSE_LAUNCH_CHECK(ctx);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_apply_col16_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                   const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                   const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                   int64_t n_exc, int32_t n_ops, const float* const* sell_W, const float* f,
+                                   float* const* out, float alpha, float beta) {
+    SellArgs a{};
+    dcpse_status st = col16_args(ctx, a, n_rows, row_ptr, slice_ptr, sell_row16, col16, base, exc_ptr, exc_col,
+                                 exc_slot, n_exc, n_ops, sell_W, f);
+    if (st) return st;
+    if (!out) return fail(ctx, DCPSE_ERR_INVALID, "out is null");
+    for (int o = 0; o < n_ops; ++o) {
+        if (!out[o]) return fail(ctx, DCPSE_ERR_INVALID, "null output pointer");
+        a.out[o] = out[o];
+    }
+    if (n_rows == 0) return DCPSE_OK;
+    a.alpha = alpha;
+    a.beta = beta;
+    if (ctx->apply_acc == 32) dispatch_resid16<true>(a, n_ops, ctx->stream);
+    else dispatch_resid16<false>(a, n_ops, ctx->stream);
+    DCPSE_LAUNCH_CHECK(ctx);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_apply_col16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                   const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                   const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                   int64_t n_exc, int32_t n_ops, const double* const* sell_W, const double* f,
+                                   double* const* out, double alpha, double beta) {
+    Sell64Args a{};
+    dcpse_status st = col16_args(ctx, a, n_rows, row_ptr, slice_ptr, sell_row16, col16, base, exc_ptr, exc_col,
+                                 exc_slot, n_exc, n_ops, sell_W, f);
+    if (st) return st;
+    if (!out) return fail(ctx, DCPSE_ERR_INVALID, "out is null");
+    for (int o = 0; o < n_ops; ++o) {
+        if (!out[o]) return fail(ctx, DCPSE_ERR_INVALID, "null output pointer");
+        a.out[o] = out[o];
+    }
+    if (n_rows == 0) return DCPSE_OK;
+    a.alpha = alpha;
+    a.beta = beta;
+    dispatch_sell64<kResid16>(a, n_ops, ctx->stream);
+    DCPSE_LAUNCH_CHECK(ctx);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_stage_col16_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                   const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                   const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                   int64_t n_exc, const float* sell_W, const float* u, float alpha, const float* y_a,
+                                   float ca, float* out_a, const float* y_b, float cb, float* out_b) {
+    SellArgs a{};
+    dcpse_status st = col16_args(ctx, a, n_rows, row_ptr, slice_ptr, sell_row16, col16, base, exc_ptr, exc_col,
+                                 exc_slot, n_exc, 1, &sell_W, u);
+    if (st || (st = stage_args(ctx, a, u, alpha, y_a, ca, out_a, y_b, cb, out_b))) return st;
+    if (n_rows == 0 || (!out_a && !out_b)) return DCPSE_OK;
+    launch_sell16<1, 2, 2, false, kResid16>(a, ctx->stream);
+    DCPSE_LAUNCH_CHECK(ctx);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_stage_col16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                   const int32_t* sell_row16, const uint16_t* col16, const int32_t* base,
+                                   const int64_t* exc_ptr, const int32_t* exc_col, const int32_t* exc_slot,
+                                   int64_t n_exc, const double* sell_W, const double* u, double alpha,
+                                   const double* y_a, double ca, double* out_a, const double* y_b, double cb,
+                                   double* out_b) {
+    Sell64Args a{};
+    dcpse_status st = col16_args(ctx, a, n_rows, row_ptr, slice_ptr, sell_row16, col16, base, exc_ptr, exc_col,
+                                 exc_slot, n_exc, 1, &sell_W, u);
+    if (st || (st = stage_args(ctx, a, u, alpha, y_a, ca, out_a, y_b, cb, out_b))) return st;
+    if (n_rows == 0 || (!out_a && !out_b)) return DCPSE_OK;
+    launch_sell64<1, kResid16, 2>(a, ctx->stream);
+    DCPSE_LAUNCH_CHECK(ctx);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_stage_sell_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int64_t* slice_ptr,
+                                  const int32_t* sell_row, const int32_t* sell_col, const double* sell_W,
+                                  const double* u, double alpha, const double* y_a, double ca, double* out_a,
+                                  const double* y_b, double cb, double* out_b) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!row_ptr || !slice_ptr || !sell_row || !sell_col || !sell_W || !u || n_rows < 0)
+        return fail(ctx, DCPSE_ERR_INVALID, "null pointer or negative size");
+    DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    Sell64Args a{};
+    a.n_rows = n_rows;
+    a.row_ptr = row_ptr;
+    a.slice_ptr = slice_ptr;
+    a.sell_row = sell_row;
+    a.sell_col = sell_col;
+    a.W[0] = sell_W;
+    dcpse_status st = stage_args(ctx, a, u, alpha, y_a, ca, out_a, y_b, cb, out_b);
+    if (st) return st;
+    if (n_rows == 0 || (!out_a && !out_b)) return DCPSE_OK;
+    launch_sell64<1, kCol32, 2>(a, ctx->stream);
+    DCPSE_LAUNCH_CHECK(ctx);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_stage_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
+                                      const int64_t* slice_ptr, const int32_t* sell_row16, const int32_t* bundle,
+                                      const int64_t* exc_ptr, const int32_t* exc_col, const double* exc_W,
+                                      int64_t n_exc, const double* u, double alpha, const double* y_a, double ca,
+                                      double* out_a, const double* y_b, double cb, double* out_b) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!row_ptr || !slice_ptr || !sell_row16 || !bundle || !exc_ptr || !u || n_rows < 0 || n_exc < 0 ||
+        (n_exc > 0 && (!exc_col || !exc_W)))
+        return fail(ctx, DCPSE_ERR_INVALID, "null pointer or bad size");
+    DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    Sell64Args a{};
+    a.n_rows = n_rows;
+    a.row_ptr = row_ptr;
+    a.slice_ptr = slice_ptr;
+    a.sell_row = sell_row16;
+    a.bundle = bundle;
+    a.exc_ptr = exc_ptr;
+    a.exc_col = exc_col;
+    a.exc_W = exc_W;
+    a.n_exc = n_exc;
+    dcpse_status st = stage_args(ctx, a, u, alpha, y_a, ca, out_a, y_b, cb, out_b);
+    if (st) return st;
+    if (n_rows == 0 || (!out_a && !out_b)) return DCPSE_OK;
+    launch_sell64<1, kBundle16, 2>(a, ctx->stream);
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
 }

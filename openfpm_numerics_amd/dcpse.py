@@ -37,10 +37,11 @@ AT_LEAST_N_PARTICLES = 3
 
 _FILE_MAGIC = b"DCPSEHIP"
 
-#: Single-field applies run on the sliced-ELL layouts: FP32 on the 16-bit-offset
-#: bundle (one operator on one particle set) or 32-bit columns, FP64 on 32-bit
-#: columns with FP64 weights (fused Laplacian + Dx at 128^3: 437 us against the
-#: CSR kernel's 512 us); set False to use the CSR kernels
+#: Single-field applies run on the sliced-ELL layouts: one operator on one
+#: particle set on its 16-bit-offset bundle, several operators, and lists whose
+#: neighbours lie too far apart for plain 16-bit offsets, on the list's 16-bit
+#: columns beside the operators' weights, two particle sets on 32-bit columns;
+#: set False to use the CSR kernels
 USE_SELL = True
 #: ... from an operator's SELL_AFTER-th such apply after its assembly on; the
 #: ones before run the CSR kernel. The default, 1, builds the copy at the first
@@ -53,8 +54,9 @@ USE_SELL = True
 SELL_AFTER = 1
 #: The 16-bit-offset bundle serves neighbours whose index offset does not fit
 #: 16 bits from a per-lane exception list; above this fraction of such
-#: neighbours (e.g. Morton-ordered particles: 6.7% at 128^3) the 32-bit
-#: sliced-ELL layout is faster and the automatic choice takes it.
+#: neighbours (e.g. Morton-ordered particles: 6.7% at 128^3) the automatic
+#: choice takes the list's 16-bit columns, and where more than this fraction
+#: does not fit those either, the 32-bit sliced-ELL layout.
 BUNDLE16_MAX_EXC = 0.01
 _FILE_VERSION = 1
 
@@ -203,8 +205,8 @@ class Dcpse:
     def sell_weights(self) -> torch.Tensor:
         """FP32 weights in the sliced-ELL layout of this operator's Verlet list."""
         if self._W.get("sell") is None:
-            self._W["sell"] = sell_weights(self.verletList.row_ptr, self._W[torch.float32], self.verletList.sell(),
-                                           self.verletList.n_rows)
+            self._W["sell"] = sell_weights(self.verletList.row_ptr, self._W[torch.float32],
+                                           self.verletList.sell_slices(), self.verletList.n_rows)
         return self._W["sell"]
 
     def sell_weights64(self) -> torch.Tensor:
@@ -212,7 +214,7 @@ class Dcpse:
         if self._W.get("sell64") is None:
             vl = self.verletList
             slice_ptr, sell_row, n_slots = vl.sell_slices()
-            sw = torch.empty(n_slots, dtype=torch.float64, device=vl.row_ptr.device)
+            sw = torch.empty(max(n_slots, 4), dtype=torch.float64, device=vl.row_ptr.device)
             _lib.context(vl.row_ptr.device.index or 0).call(
                 "dcpse_sell_fill_weights_f64", vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(self.weights(torch.float64)),
                 _lib.ptr(slice_ptr), _lib.ptr(sell_row), _lib.ptr(sw))
@@ -243,6 +245,12 @@ class Dcpse:
                 _lib.ptr(exc_ptr), n_exc.ctypes.data)
             vl._n_exc16 = int(n_exc[0])
         return vl._n_exc16 <= BUNDLE16_MAX_EXC * max(vl.nnz, 1)
+
+    def col16(self):
+        """The 16-bit columns of this operator's list (VerletList.col16) where it
+        is of one particle set and at most BUNDLE16_MAX_EXC of its neighbours
+        do not fit; else None."""
+        return self.verletList.col16(BUNDLE16_MAX_EXC) if self.same_set else None
 
     def computeDifferentialOperator(self, f: torch.Tensor, out: torch.Tensor | None = None,
                                     f_domain: torch.Tensor | None = None, alpha=1.0, beta=0.0):
@@ -611,6 +619,12 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
                  1, _lib.ptr(bundle), _lib.ptr(exc_ptr), _lib.ptr(exc_col), _lib.ptr(exc_W), ne, _lib.ptr(f2),
                  _lib.ptr(fd), _lib.ptr_array(outs), alpha, beta)
         return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
+    c16 = ops[0].col16() if use_sell and fd is None else None
+    if c16 is not None:
+        SW = [op.sell_weights() for op in ops]
+        ctx.call("dcpse_apply_col16_f32", n_rows, _lib.ptr(vl.row_ptr), *map(_lib.ptr, c16[:-1]), c16[-1], len(ops),
+                 _lib.ptr_array(SW), _lib.ptr(f2), _lib.ptr_array(outs), alpha, beta)
+        return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
     if use_sell:
         slice_ptr, sell_row, sell_col = vl.sell()
         SW = [op.sell_weights() for op in ops]
@@ -625,6 +639,12 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
             ctx.call("dcpse_apply_sell_bundle16_f64", n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr),
                      _lib.ptr(row16), 1, _lib.ptr(bundle), _lib.ptr(exc_ptr), _lib.ptr(exc_col), _lib.ptr(exc_W), ne,
                      _lib.ptr(f2), _lib.ptr(fd), _lib.ptr_array(outs), alpha, beta)
+            return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
+        c16 = ops[0].col16() if fd is None else None
+        if c16 is not None:
+            SW = [op.sell_weights64() for op in ops]
+            ctx.call("dcpse_apply_col16_f64", n_rows, _lib.ptr(vl.row_ptr), *map(_lib.ptr, c16[:-1]), c16[-1],
+                     len(ops), _lib.ptr_array(SW), _lib.ptr(f2), _lib.ptr_array(outs), alpha, beta)
             return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
         # FP64: the 32-bit-column layout with FP64 weights in its slot order
         slice_ptr, sell_row, sell_col = vl.sell()

@@ -13,7 +13,30 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from . import dcpse as _dcpse_module
 from .dcpse import Dcpse
+
+#: Stage applies in FP64 since assembly from which "auto" builds the sliced-ELL
+#: copy: it costs about 0.35 ms at 75^3 particles and saves some 25 us per stage
+SELL64_AFTER = 12
+
+
+def _layout(d: Dcpse, dtype, layout: str, stages: int) -> str:
+    """The layout a call of this many stages runs on."""
+    if dtype == torch.float32:
+        if layout != "auto":
+            return layout
+        d._n32["fwd"] += stages - 1
+        ready = d._count_apply32("fwd")
+    else:
+        if layout in ("bundle16", "col16", "sell", "csr"):
+            return layout
+        d._n32["stage64"] = d._n32.get("stage64", 0) + stages
+        ready = (d._n32["stage64"] >= max(SELL64_AFTER, _dcpse_module.SELL_AFTER) or d._W.get("bundle16_64") is not None
+                 or d._W.get("sell64") is not None)
+    if not ready or d.verletList.n_rows == 0:
+        return "csr"
+    return "bundle16" if d.bundle16_suits() else "col16" if d.col16() is not None else "sell"
 
 
 def _dcpse(op) -> Dcpse:
@@ -23,16 +46,41 @@ def _dcpse(op) -> Dcpse:
     return d
 
 
+_NAMES = {"bundle16": "bundle16_", "col16": "col16_", "sell": "sell_", "csr": ""}
+
+
+def _operator_args(d: Dcpse, dtype, layout: str):
+    """The library arguments that describe operator d on a layout, after n_rows."""
+    vl = d.verletList
+    p = _lib.ptr
+    if layout == "bundle16":
+        bundle, row16, exc_ptr, exc_col, exc_W, ne = d.sell_bundle16(dtype)
+        return p(vl.row_ptr), p(vl.sell_slices()[0]), p(row16), p(bundle), p(exc_ptr), p(exc_col), p(exc_W), ne
+    W = (d.sell_weights if dtype == torch.float32 else d.sell_weights64)
+    if layout == "col16":
+        c16 = d.col16()
+        if c16 is None:
+            raise ValueError("too many neighbours of this list do not fit 16-bit columns")
+        return (p(vl.row_ptr), *map(p, c16[:-1]), c16[-1], p(W()))
+    if layout == "sell":
+        return (p(vl.row_ptr), *map(p, vl.sell()), p(W()))
+    if layout == "csr":
+        return p(vl.row_ptr), p(vl.col), p(d.weights(dtype))
+    raise ValueError(f"unknown layout {layout!r}")
+
+
 def rk4(op, f: torch.Tensor, dt: float, n_steps: int, alpha: float = 1.0, layout: str = "auto",
         work: torch.Tensor | None = None) -> torch.Tensor:
     """Advances f (N,) in place by n_steps RK4 steps of df/dt = alpha * D f and returns it.
 
-    float32 state runs the FP32 kernels: layout "bundle16" (sliced-ELL with
-    16-bit column offsets, the fewest bytes), "sell" (32-bit columns), "csr",
-    or "auto": the 4 n_steps stage applies count towards the operator's
-    ``dcpse.SELL_AFTER`` and run on "bundle16" once it is reached (its copy is
-    then built; "sell" where too many neighbours fall outside 16-bit offsets,
-    ``dcpse.BUNDLE16_MAX_EXC``), on "csr" before. float64 state runs the FP64 CSR kernels.
+    float32 and float64 state run the kernels of their type on layout "bundle16"
+    (sliced-ELL with 16-bit column offsets, the fewest bytes), "col16" (the
+    list's 16-bit columns), "sell" (32-bit columns), "csr", or "auto": the
+    4 n_steps stage applies count towards the operator's ``dcpse.SELL_AFTER``
+    (FP64: ``SELL64_AFTER`` stages, or a copy that is there) and run on
+    "bundle16" once it is reached (its copy is then built; "col16", then "sell",
+    where too many neighbours do not fit, ``dcpse.BUNDLE16_MAX_EXC``), on "csr"
+    before.
     ``work`` (3N of f's dtype) may be passed to avoid an allocation per call.
     """
     d = _dcpse(op)
@@ -48,28 +96,12 @@ def rk4(op, f: torch.Tensor, dt: float, n_steps: int, alpha: float = 1.0, layout
         raise ValueError("work must be a contiguous tensor of 3N elements of f's dtype")
     ctx = _lib.context(f.device.index or 0)
     ctx.bind_current_stream()
-    if f.dtype == torch.float32 and layout == "auto":
-        d._n32["fwd"] += 4 * int(n_steps) - 1
-        layout = ("bundle16" if d.bundle16_suits() else "sell") if d._count_apply32("fwd") else "csr"
-    if f.dtype == torch.float64:
-        ctx.call("dcpse_rk4_f64", n, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), _lib.ptr(d.weights(torch.float64)),
-                 float(alpha), float(dt), int(n_steps), _lib.ptr(f), _lib.ptr(work))
-    elif layout == "bundle16":
-        slice_ptr = vl.sell_slices()[0]
-        bundle, row16, exc_ptr, exc_col, exc_W, ne = d.sell_bundle16()
-        ctx.call("dcpse_rk4_bundle16_f32", n, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr), _lib.ptr(row16),
-                 _lib.ptr(bundle), _lib.ptr(exc_ptr), _lib.ptr(exc_col), _lib.ptr(exc_W), ne, float(alpha),
-                 float(dt), int(n_steps), _lib.ptr(f), _lib.ptr(work))
-    elif layout == "sell":
-        slice_ptr, sell_row, sell_col = vl.sell()
-        ctx.call("dcpse_rk4_sell_f32", n, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr), _lib.ptr(sell_row),
-                 _lib.ptr(sell_col), _lib.ptr(d.sell_weights()), float(alpha), float(dt), int(n_steps), _lib.ptr(f),
-                 _lib.ptr(work))
-    elif layout == "csr":
-        ctx.call("dcpse_rk4_f32", n, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), _lib.ptr(d.weights(torch.float32)),
-                 float(alpha), float(dt), int(n_steps), _lib.ptr(f), _lib.ptr(work))
-    else:
-        raise ValueError(f"unknown layout {layout!r}")
+    layout = _layout(d, f.dtype, layout, 4 * int(n_steps))
+    p = _lib.ptr
+    t = "f32" if f.dtype == torch.float32 else "f64"
+    end = (float(alpha), float(dt), int(n_steps), p(f), p(work))
+    args = _operator_args(d, f.dtype, layout)
+    ctx.call(f"dcpse_rk4_{_NAMES[layout]}{t}", n, *args, *end)
     return f
 
 
@@ -83,26 +115,8 @@ def stage(op, u: torch.Tensor, alpha: float, y_a: torch.Tensor | None, ca: float
     ctx = _lib.context(u.device.index or 0)
     ctx.bind_current_stream()
     p = _lib.ptr
-    if u.dtype == torch.float32 and layout == "auto":
-        layout = ("bundle16" if d.bundle16_suits() else "sell") if d._count_apply32("fwd") else "csr"
-    if u.dtype == torch.float64:
-        ctx.call("dcpse_stage_f64", vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col),
-                 _lib.ptr(d.weights(torch.float64)), _lib.ptr(u), float(alpha), p(y_a), float(ca), p(out_a), p(y_b),
-                 float(cb), p(out_b))
-    elif layout == "bundle16":
-        slice_ptr = vl.sell_slices()[0]
-        bundle, row16, exc_ptr, exc_col, exc_W, ne = d.sell_bundle16()
-        ctx.call("dcpse_stage_bundle16_f32", vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr), _lib.ptr(row16),
-                 _lib.ptr(bundle), _lib.ptr(exc_ptr), _lib.ptr(exc_col), _lib.ptr(exc_W), ne, _lib.ptr(u),
-                 float(alpha), p(y_a), float(ca), p(out_a), p(y_b), float(cb), p(out_b))
-    elif layout == "sell":
-        slice_ptr, sell_row, sell_col = vl.sell()
-        ctx.call("dcpse_stage_sell_f32", vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr), _lib.ptr(sell_row),
-                 _lib.ptr(sell_col), _lib.ptr(d.sell_weights()), _lib.ptr(u), float(alpha), p(y_a), float(ca),
-                 p(out_a), p(y_b), float(cb), p(out_b))
-    elif layout == "csr":
-        ctx.call("dcpse_stage_f32", vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col),
-                 _lib.ptr(d.weights(torch.float32)), _lib.ptr(u), float(alpha), p(y_a), float(ca), p(out_a), p(y_b),
-                 float(cb), p(out_b))
-    else:
-        raise ValueError(f"unknown layout {layout!r}")
+    layout = _layout(d, u.dtype, layout, 1)
+    t = "f32" if u.dtype == torch.float32 else "f64"
+    args = _operator_args(d, u.dtype, layout)
+    ctx.call(f"dcpse_stage_{_NAMES[layout]}{t}", vl.n_rows, *args, p(u), float(alpha), p(y_a), float(ca), p(out_a),
+             p(y_b), float(cb), p(out_b))

@@ -94,6 +94,7 @@ class ParticleSet:
         vl._sell = None
         vl._slices = None
         vl._n_exc16 = None
+        vl._col16 = None
         return vl
 
 
@@ -192,6 +193,7 @@ class VerletList:
         self._sell = None
         self._slices = None
         self._n_exc16 = None
+        self._col16 = None
         self.map_ctr = -1
 
     @property
@@ -274,6 +276,36 @@ class VerletList:
                                                          n_slots))
         return self._sell
 
+    def col16(self, max_far: float):
+        """The 16-bit columns of the sliced-ELL layout (one particle set; see
+        dcpse_sell_fill_col16), shared by every operator on this list: the
+        arguments (slice_ptr, sell_row16, col16, base, exc_ptr, exc_col,
+        exc_slot, n_exc); None where more than the share max_far of the
+        neighbours would be listed as far. Built on first use."""
+        if getattr(self, "_col16", None) is None:
+            dev = self.row_ptr.device
+            ctx = _lib.context(dev.index or 0)
+            slice_ptr, sell_row, n_slots = self.sell_slices()
+            col16 = torch.empty(max(n_slots, 4), dtype=torch.int16, device=dev)
+            base = torch.empty(max(n_slots // 64, 4), dtype=torch.int32, device=dev)
+            exc_ptr = torch.empty(sell_row.numel() + 1, dtype=torch.int64, device=dev)
+            n_exc = np.zeros(1, np.int64)
+            ctx.call("dcpse_sell_fill_col16", self.n_rows, _lib.ptr(self.row_ptr), _lib.ptr(self.col),
+                     _lib.ptr(slice_ptr), _lib.ptr(sell_row), _lib.ptr(col16), _lib.ptr(base), _lib.ptr(exc_ptr),
+                     n_exc.ctypes.data)
+            ne = int(n_exc[0])
+            if ne > max_far * max(self.nnz, 1):
+                self._col16 = False
+            else:
+                sell_row16 = torch.empty_like(sell_row)
+                exc_col = torch.empty(max(ne, 1), dtype=torch.int32, device=dev)
+                exc_slot = torch.empty(max(ne, 1), dtype=torch.int32, device=dev)
+                ctx.call("dcpse_sell_fill_col16_far", self.n_rows, _lib.ptr(self.row_ptr), _lib.ptr(self.col),
+                         _lib.ptr(slice_ptr), _lib.ptr(sell_row), _lib.ptr(base), _lib.ptr(exc_ptr), ne,
+                         _lib.ptr(sell_row16), _lib.ptr(exc_col), _lib.ptr(exc_slot))
+                self._col16 = (slice_ptr, sell_row16, col16, base, exc_ptr, exc_col, exc_slot, ne)
+        return self._col16 or None
+
 
 def sell_slices(row_ptr: torch.Tensor, n_rows: int):
     """Slice structure of the sliced-ELL layout of a CSR: slices of 64 rows,
@@ -308,10 +340,12 @@ def sell_layout(row_ptr: torch.Tensor, col: torch.Tensor, n_rows: int):
 
 
 def sell_weights(row_ptr: torch.Tensor, W: torch.Tensor, layout, n_rows: int):
-    """FP32 weights W (CSR order) in the sliced-ELL layout (slice_ptr, sell_row, sell_col)."""
-    slice_ptr, sell_row, sell_col = layout
+    """FP32 weights W (CSR order) in the sliced-ELL layout: (slice_ptr, sell_row,
+    sell_col) or (slice_ptr, sell_row, n_slots)."""
+    slice_ptr, sell_row, last = layout
     ctx = _lib.context(row_ptr.device.index or 0)
-    out = torch.empty(sell_col.numel(), dtype=torch.float32, device=row_ptr.device)
+    n_slots = max(last, 4) if isinstance(last, int) else last.numel()
+    out = torch.empty(n_slots, dtype=torch.float32, device=row_ptr.device)
     if n_rows:
         ctx.call("dcpse_sell_fill_weights_f32", n_rows, _lib.ptr(row_ptr), _lib.ptr(W), _lib.ptr(slice_ptr),
                  _lib.ptr(sell_row), _lib.ptr(out))
