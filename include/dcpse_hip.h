@@ -385,6 +385,18 @@ dcpse_status dcpse_apply_sell_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const
                                            const int32_t* bundle, const int64_t* exc_ptr, const int32_t* exc_col,
                                            const double* exc_W, int64_t n_exc, const double* f,
                                            const double* f_self, double* const* out, double alpha, double beta);
+/* The FP64 copies straight from an operator's kernels K and eps^-|beta|
+ * (row_scale): the weights of dcpse_scale_rows_f64, bit for bit, without the
+ * pass that forms them in CSR order first. */
+dcpse_status dcpse_sell_fill_weights_scaled_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
+                                                const double* K, const double* row_scale, const int64_t* slice_ptr,
+                                                const int32_t* sell_row, double* sell_W);
+dcpse_status dcpse_sell_fill_bundle16_scaled_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
+                                                 const int32_t* col, int32_t n_ops, const double* const* K,
+                                                 const double* const* row_scale, const int64_t* slice_ptr,
+                                                 const int32_t* sell_row, const int64_t* exc_ptr, int64_t n_exc,
+                                                 int32_t* bundle, int32_t* sell_row16, int32_t* exc_col,
+                                                 double* exc_W);
 /* Same result as dcpse_apply_transpose_f32 with one field, from the SELL
  * layout of the transposed CSR (built with the three calls above). */
 dcpse_status dcpse_apply_transpose_sell_f32(dcpse_ctx* ctx, int64_t n_cols, const int64_t* rowT_ptr,

@@ -103,6 +103,8 @@ SIGNATURES = {
     "dcpse_rk4_sell_f32": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _f32, _f64, _i64, _vp, _vp]),
     "dcpse_stage_bundle16_f32": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _f32, _vp, _f32,
                                         _vp, _vp, _f32, _vp]),
+    "dcpse_sell_fill_weights_scaled_f64": (_i32, [_vp, _i64] + [_vp] * 6),
+    "dcpse_sell_fill_bundle16_scaled_f64": (_i32, [_vp, _i64, _vp, _vp, _i32] + [_vp] * 5 + [_i64] + [_vp] * 4),
     "dcpse_sell_fill_col16": (_i32, [_vp, _i64] + [_vp] * 8),
     "dcpse_sell_fill_col16_far": (_i32, [_vp, _i64] + [_vp] * 6 + [_i64] + [_vp] * 3),
     "dcpse_apply_col16_f32": (_i32, [_vp, _i64] + _COL16 + [_i32, _vp, _vp, _vp, _f32, _f32]),

@@ -62,11 +62,6 @@ __global__ __launch_bounds__(256) void k_sell_width(int64_t n_rows, const int64_
     }
 }
 
-// Thread layout of the layout builds: a block of 256 threads walks slices
-// (grid-stride); thread t takes lane t % 64 of the slice and its slot groups
-// t / 64, t / 64 + 4, ... (4 slots each), so the loads of a row's entries are
-// independent and every store is a 16-byte (or 8-byte) vector store at
-// consecutive addresses across the lanes.
 struct SliceLane {
     int32_t row;
     int64_t rs;
@@ -81,35 +76,64 @@ __device__ __forceinline__ SliceLane slice_lane(const int64_t* row_ptr, const in
     return r;
 }
 
-// Every slot is written, padding included, also for the lanes of the last
-// slice that have no row, so no slot of the layout is ever left
-// uninitialised.
-template <bool COLS, typename TW = float>
+// The layout builds run a block of 256 threads per slice (grid-stride) through
+// LDS tiles of 32 slots x 64 lanes: the four waves read 32 entries of two rows
+// at a time, coalesced along the row, then thread t writes lane t % 64's slot
+// groups t / 64 and t / 64 + 4 of the tile, 4 slots in one vector store at
+// consecutive addresses across the lanes. (Each lane reading its own row took
+// 151 us for FP64 weights on 23M neighbours and 368 us for FP32 weights on
+// 105M, 84 and 173 us this way.)
+constexpr int kTileSlots = 32;
+constexpr int kTilePitch = 65;  // in elements (no bank conflicts)
+
+// Values v (columns or weights, CSR order) in slot order; with SCALE times the
+// row's scale, one rounding each. Every slot is written, padding included, also
+// for the lanes of the last slice that have no row, so no slot of the layout is
+// ever left uninitialised.
+template <typename T, bool SCALE>
 __global__ __launch_bounds__(256) void k_sell_fill(int64_t n_rows, const int64_t* __restrict__ row_ptr,
-                                                   const int32_t* __restrict__ col, const TW* __restrict__ W,
+                                                   const T* __restrict__ v, const T* __restrict__ scale,
                                                    const int64_t* __restrict__ slice_ptr,
-                                                   const int32_t* __restrict__ sell_row,
-                                                   int32_t* __restrict__ sell_col, TW* __restrict__ sell_W) {
-    typedef TW vw4 __attribute__((ext_vector_type(4)));
+                                                   const int32_t* __restrict__ sell_row, T* __restrict__ sell_v) {
+    typedef T vt4 __attribute__((ext_vector_type(4)));
+    __shared__ T tile[kTileSlots * kTilePitch];
+    __shared__ int64_t srs[64];
+    __shared__ int32_t slen[64];
+    __shared__ T sscale[SCALE ? 64 : 1];
     const int64_t n_slices = (n_rows + 63) / 64;
-    const int l = threadIdx.x & 63, gsub = threadIdx.x >> 6;
+    const int tid = threadIdx.x;
+    const int l = tid & 63, gsub = tid >> 6, e = tid & 31;
     for (int64_t s = blockIdx.x; s < n_slices; s += gridDim.x) {
-        const SliceLane r = slice_lane(row_ptr, sell_row, s * 64 + l);
+        __syncthreads();  // the previous slice's lane table is consumed
+        if (tid < 64) {
+            const SliceLane r = slice_lane(row_ptr, sell_row, s * 64 + tid);
+            srs[tid] = r.rs;
+            slen[tid] = r.len;
+            if (SCALE) sscale[tid] = r.row >= 0 ? scale[r.row] : T(0);
+        }
+        __syncthreads();
         const int64_t base = slice_ptr[s];
         const int ng = (int)((slice_ptr[s + 1] - base) >> 8);
-        for (int g = gsub; g < ng; g += 4) {
-            const int64_t dst = base + (int64_t)g * 256 + 4 * l;
-            if constexpr (COLS) {
-                vi4a v;
+        for (int g0 = 0; g0 < ng; g0 += kTileSlots / 4) {
+            const int j = 4 * g0 + e;
+            T x[8];
 #pragma unroll
-                for (int jj = 0; jj < 4; ++jj) v[jj] = 4 * g + jj < r.len ? col[r.rs + 4 * g + jj] : 0;
-                *reinterpret_cast<vi4a*>(sell_col + dst) = v;
-            } else {
-                vw4 v;
-#pragma unroll
-                for (int jj = 0; jj < 4; ++jj) v[jj] = 4 * g + jj < r.len ? W[r.rs + 4 * g + jj] : TW(0);
-                *reinterpret_cast<vw4*>(sell_W + dst) = v;
+            for (int it = 0; it < 8; ++it) {
+                const int ll = 16 * gsub + 2 * it + ((tid >> 5) & 1);
+                x[it] = j < slen[ll] ? v[srs[ll] + j] : T(0);
+                if (SCALE) x[it] = sscale[ll] * x[it];
             }
+#pragma unroll
+            for (int it = 0; it < 8; ++it) tile[e * kTilePitch + 16 * gsub + 2 * it + ((tid >> 5) & 1)] = x[it];
+            __syncthreads();
+            const int gn = min(kTileSlots / 4, ng - g0);
+            for (int gl = gsub; gl < gn; gl += 4) {
+                vt4 y;
+#pragma unroll
+                for (int jj = 0; jj < 4; ++jj) y[jj] = tile[(4 * gl + jj) * kTilePitch + l];
+                *reinterpret_cast<vt4*>(sell_v + base + (int64_t)(g0 + gl) * 256 + 4 * l) = y;
+            }
+            __syncthreads();
         }
     }
 }
@@ -173,26 +197,25 @@ __device__ __forceinline__ int64_t col_offset(int32_t q, int32_t p, int64_t n) {
 
 __device__ __forceinline__ bool far16(int64_t d) { return d > 32767 || d < -32768; }
 
-// exc_count[i] = far neighbours of the row of lane i: the four threads of a
-// lane count their slot groups and the first adds the four counts.
+// exc_count[i] = far neighbours of the row of lane i: a wavefront takes 16
+// lanes' rows, two at a time, 32 entries of each per load.
 __global__ __launch_bounds__(256) void k_bundle16_count(int64_t n_rows, const int64_t* __restrict__ row_ptr,
                                                         const int32_t* __restrict__ col,
                                                         const int32_t* __restrict__ sell_row,
                                                         int32_t* __restrict__ exc_count) {
-    __shared__ int cnt[256];
     const int64_t n_slices = (n_rows + 63) / 64;
-    const int l = threadIdx.x & 63, gsub = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, half = lane >> 5, e = lane & 31;
     for (int64_t s = blockIdx.x; s < n_slices; s += gridDim.x) {
-        const SliceLane r = slice_lane(row_ptr, sell_row, s * 64 + l);
-        int c = 0;
-        for (int g = gsub; 4 * g < r.len; g += 4)
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj)
-                if (4 * g + jj < r.len) c += far16(col_offset(col[r.rs + 4 * g + jj], r.row, n_rows));
-        cnt[threadIdx.x] = c;
-        __syncthreads();
-        if (gsub == 0) exc_count[s * 64 + l] = cnt[l] + cnt[64 + l] + cnt[128 + l] + cnt[192 + l];
-        __syncthreads();
+        for (int it = 0; it < 8; ++it) {
+            const int64_t i = s * 64 + 16 * wv + 2 * it + half;
+            const SliceLane r = slice_lane(row_ptr, sell_row, i);
+            int c = 0;
+            for (int j = e; j < r.len; j += 32) c += far16(col_offset(col[r.rs + j], r.row, n_rows));
+#pragma unroll
+            for (int off = 16; off > 0; off >>= 1) c += __shfl_xor(c, off, kWave);
+            if (e == 0) exc_count[i] = c;
+        }
     }
 }
 
@@ -202,15 +225,13 @@ __global__ __launch_bounds__(256) void k_bundle16_count(int64_t n_rows, const in
 // thread writes its lane's slot groups of the tile to the bundle, 16-bit
 // column offsets (0 where the offset does not fit: the lane's exception list
 // holds that neighbour) and the weights, padding slots zero.
-constexpr int kB16Chunk = 32;  // slots per tile
-constexpr int kB16Pitch = 65;  // tile row pitch in words (no bank conflicts)
 __global__ __launch_bounds__(256) void k_sell_fill_bundle16(
     int64_t n_rows, const int64_t* __restrict__ row_ptr, const int32_t* __restrict__ col, int n_ops,
     const float* W0, const float* W1, const float* W2, const float* W3, const int64_t* __restrict__ slice_ptr,
     const int32_t* __restrict__ sell_row, const int64_t* __restrict__ exc_ptr, int32_t* __restrict__ bundle,
     int32_t* __restrict__ sell_row16) {
-    __shared__ int32_t tc[kB16Chunk * kB16Pitch];      // column offsets
-    __shared__ float tw[4][kB16Chunk * kB16Pitch];     // weights per operator
+    __shared__ int32_t tc[kTileSlots * kTilePitch];      // column offsets
+    __shared__ float tw[4][kTileSlots * kTilePitch];     // weights per operator
     __shared__ int32_t srow[64];
     __shared__ int64_t srs[64];
     __shared__ int32_t slen[64];
@@ -233,7 +254,7 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16(
         __syncthreads();
         const int64_t base = slice_ptr[s];
         const int ng = (int)((slice_ptr[s + 1] - base) >> 8);
-        for (int g0 = 0; g0 < ng; g0 += kB16Chunk / 4) {
+        for (int g0 = 0; g0 < ng; g0 += kTileSlots / 4) {
             // load: wave w takes lanes 16 w .. 16 w + 15, two rows at a time
             const int e = tid & 31;
             const int j = 4 * g0 + e;
@@ -246,22 +267,22 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16(
                     const int64_t dj = col_offset(col[rs + j], srow[ll], n_rows);
                     d = far16(dj) ? 0 : (int32_t)dj;
                 }
-                tc[e * kB16Pitch + ll] = d;
-                for (int o = 0; o < n_ops; ++o) tw[o][e * kB16Pitch + ll] = j < len ? W[o][rs + j] : 0.0f;
+                tc[e * kTilePitch + ll] = d;
+                for (int o = 0; o < n_ops; ++o) tw[o][e * kTilePitch + ll] = j < len ? W[o][rs + j] : 0.0f;
             }
             __syncthreads();
             // write: thread (lane l, gsub) writes the tile's groups gsub, gsub + 4
-            const int gn = min(kB16Chunk / 4, ng - g0);
+            const int gn = min(kTileSlots / 4, ng - g0);
             for (int gl = gsub; gl < gn; gl += 4) {
                 const int64_t gb = (base / 256 + g0 + gl) * blk;  // word offset of the slot group's block
                 vs4a dv;
 #pragma unroll
-                for (int jj = 0; jj < 4; ++jj) dv[jj] = (int16_t)tc[(4 * gl + jj) * kB16Pitch + l];
+                for (int jj = 0; jj < 4; ++jj) dv[jj] = (int16_t)tc[(4 * gl + jj) * kTilePitch + l];
                 *reinterpret_cast<vs4a*>(cols16 + 2 * gb + 4 * l) = dv;
                 for (int o = 0; o < n_ops; ++o) {
                     vi4a v;
 #pragma unroll
-                    for (int jj = 0; jj < 4; ++jj) v[jj] = __float_as_int(tw[o][(4 * gl + jj) * kB16Pitch + l]);
+                    for (int jj = 0; jj < 4; ++jj) v[jj] = __float_as_int(tw[o][(4 * gl + jj) * kTilePitch + l]);
                     *reinterpret_cast<vi4a*>(bundle + gb + 128 + o * 256 + 4 * l) = v;
                 }
             }
@@ -270,15 +291,25 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16(
     }
 }
 
+// The weights of a layout build: W[o] in CSR order, or kernels W[o] times
+// scale[o] of their row (one rounding, the pre-scaled weight bit for bit).
+template <typename T>
+struct FillWeights {
+    const T* W[4];
+    const T* scale[4];
+    __device__ __forceinline__ T at(int o, int64_t j, int32_t row) const {
+        return scale[o] ? scale[o][row] * W[o][j] : W[o][j];
+    }
+};
+
 // The exception lists: one thread per lane whose row has far neighbours
 // walks the row in order.
 template <typename WT>
 __global__ void k_bundle16_exc(int64_t n_rows, const int64_t* __restrict__ row_ptr, const int32_t* __restrict__ col,
-                               int n_ops, const WT* W0, const WT* W1, const WT* W2, const WT* W3,
-                               const int32_t* __restrict__ sell_row, const int64_t* __restrict__ exc_ptr,
-                               int64_t n_exc, int32_t* __restrict__ exc_col, WT* __restrict__ exc_W) {
+                               int n_ops, const FillWeights<WT> W, const int32_t* __restrict__ sell_row,
+                               const int64_t* __restrict__ exc_ptr, int64_t n_exc, int32_t* __restrict__ exc_col,
+                               WT* __restrict__ exc_W) {
     const int64_t n_lanes = ((n_rows + 63) / 64) * 64;
-    const WT* W[4] = {W0, W1, W2, W3};
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_lanes;
          i += (int64_t)gridDim.x * blockDim.x) {
         int64_t e = exc_ptr[i];
@@ -288,7 +319,7 @@ __global__ void k_bundle16_exc(int64_t n_rows, const int64_t* __restrict__ row_p
             const int32_t q = col[r.rs + j];
             if (far16(col_offset(q, r.row, n_rows))) {
                 exc_col[e] = q;
-                for (int o = 0; o < n_ops; ++o) exc_W[o * n_exc + e] = W[o][r.rs + j];
+                for (int o = 0; o < n_ops; ++o) exc_W[o * n_exc + e] = W.at(o, r.rs + j, r.row);
                 ++e;
             }
         }
@@ -304,16 +335,14 @@ __global__ void k_bundle16_exc(int64_t n_rows, const int64_t* __restrict__ row_p
 // along the rows and written 32 contiguous bytes per lane.
 __global__ __launch_bounds__(256) void k_sell_fill_bundle16_f64(
     int64_t n_rows, const int64_t* __restrict__ row_ptr, const int32_t* __restrict__ col, int n_ops,
-    const double* W0, const double* W1, const double* W2, const double* W3, const int64_t* __restrict__ slice_ptr,
-    const int32_t* __restrict__ sell_row, const int64_t* __restrict__ exc_ptr, int32_t* __restrict__ bundle,
-    int32_t* __restrict__ sell_row16) {
-    __shared__ int32_t tc[kB16Chunk * kB16Pitch];  // column offsets
-    __shared__ double tw[kB16Chunk * kB16Pitch];   // one operator's weights
+    const FillWeights<double> W, const int64_t* __restrict__ slice_ptr, const int32_t* __restrict__ sell_row,
+    const int64_t* __restrict__ exc_ptr, int32_t* __restrict__ bundle, int32_t* __restrict__ sell_row16) {
+    __shared__ int32_t tc[kTileSlots * kTilePitch];  // column offsets
+    __shared__ double tw[kTileSlots * kTilePitch];   // one operator's weights
     __shared__ int32_t srow[64];
     __shared__ int64_t srs[64];
     __shared__ int32_t slen[64];
     const int64_t n_slices = (n_rows + 63) / 64;
-    const double* W[4] = {W0, W1, W2, W3};
     const int64_t blk = 128 + 512 * (int64_t)n_ops;
     int16_t* cols16 = reinterpret_cast<int16_t*>(bundle);
     const int tid = threadIdx.x;
@@ -331,9 +360,9 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16_f64(
         __syncthreads();
         const int64_t base = slice_ptr[s];
         const int ng = (int)((slice_ptr[s + 1] - base) >> 8);
-        for (int g0 = 0; g0 < ng; g0 += kB16Chunk / 4) {
+        for (int g0 = 0; g0 < ng; g0 += kTileSlots / 4) {
             const int j = 4 * g0 + e;
-            const int gn = min(kB16Chunk / 4, ng - g0);
+            const int gn = min(kTileSlots / 4, ng - g0);
             for (int o = -1; o < n_ops; ++o) {  // -1: the column offsets
                 // load: wave w takes lanes 16 w .. 16 w + 15, two rows at a time
                 for (int it = 0; it < 8; ++it) {
@@ -346,9 +375,9 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16_f64(
                             const int64_t dj = col_offset(col[rs + j], srow[ll], n_rows);
                             d = far16(dj) ? 0 : (int32_t)dj;
                         }
-                        tc[e * kB16Pitch + ll] = d;
+                        tc[e * kTilePitch + ll] = d;
                     } else {
-                        tw[e * kB16Pitch + ll] = j < len ? W[o][rs + j] : 0.0;
+                        tw[e * kTilePitch + ll] = j < len ? W.at(o, rs + j, srow[ll]) : 0.0;
                     }
                 }
                 __syncthreads();
@@ -358,12 +387,12 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16_f64(
                     if (o < 0) {
                         vs4a dv;
 #pragma unroll
-                        for (int jj = 0; jj < 4; ++jj) dv[jj] = (int16_t)tc[(4 * gl + jj) * kB16Pitch + l];
+                        for (int jj = 0; jj < 4; ++jj) dv[jj] = (int16_t)tc[(4 * gl + jj) * kTilePitch + l];
                         *reinterpret_cast<vs4a*>(cols16 + 2 * gb + 4 * l) = dv;
                     } else {
                         double2* wb = reinterpret_cast<double2*>(bundle + gb + 128 + o * 512) + 2 * l;
-                        wb[0] = make_double2(tw[(4 * gl) * kB16Pitch + l], tw[(4 * gl + 1) * kB16Pitch + l]);
-                        wb[1] = make_double2(tw[(4 * gl + 2) * kB16Pitch + l], tw[(4 * gl + 3) * kB16Pitch + l]);
+                        wb[0] = make_double2(tw[(4 * gl) * kTilePitch + l], tw[(4 * gl + 1) * kTilePitch + l]);
+                        wb[1] = make_double2(tw[(4 * gl + 2) * kTilePitch + l], tw[(4 * gl + 3) * kTilePitch + l]);
                     }
                 }
                 __syncthreads();
@@ -379,8 +408,9 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16_f64(
 // unsigned 16-bit residual. The lanes' rows are consecutive particles, whose
 // j-th neighbours lie about as far away, so the residuals fit where the offsets
 // themselves, planes of a large set apart, do not: of the 60M neighbours of the
-// adaptive million-particle set EXC16 do not fit, against EXC0 of plain 16-bit
-// offsets. kFar16 marks neighbours that do not fit (listed per lane with their
+// adaptive million-particle set 43,000 do not fit, against 7.0M of plain 16-bit
+// offsets (an RK4 stage there: 104 us, 119 us with 32-bit columns; Laplacian
+// and d/dx of the 128^3 set: 246 us, 276 us). kFar16 marks neighbours that do not fit (listed per lane with their
 // slot, as for the bundle) and padding, so it is the apply's only mask.
 constexpr int kFar16 = 0xFFFF;
 
@@ -394,7 +424,7 @@ __global__ __launch_bounds__(256) void k_sell_fill_col16(int64_t n_rows, const i
                                                          const int32_t* __restrict__ sell_row,
                                                          uint16_t* __restrict__ col16, int32_t* __restrict__ base,
                                                          int32_t* __restrict__ exc_count) {
-    __shared__ int32_t tc[kB16Chunk * kB16Pitch];
+    __shared__ int32_t tc[kTileSlots * kTilePitch];
     __shared__ int32_t srow[64];
     __shared__ int64_t srs[64];
     __shared__ int32_t slen[64];
@@ -415,23 +445,23 @@ __global__ __launch_bounds__(256) void k_sell_fill_col16(int64_t n_rows, const i
         const int64_t first = slice_ptr[s];
         const int ng = (int)((slice_ptr[s + 1] - first) >> 8);
         int far = 0;
-        for (int g0 = 0; g0 < ng; g0 += kB16Chunk / 4) {
+        for (int g0 = 0; g0 < ng; g0 += kTileSlots / 4) {
             const int j = 4 * g0 + e;
             for (int it = 0; it < 8; ++it) {
                 const int ll = 16 * gsub + 2 * it + ((tid >> 5) & 1);
                 int32_t d = 0;
                 if (j < slen[ll]) d = (int32_t)col_offset(col[srs[ll] + j], srow[ll], n_rows);
-                tc[e * kB16Pitch + ll] = d;
+                tc[e * kTilePitch + ll] = d;
             }
             __syncthreads();
-            const int gn = min(kB16Chunk / 4, ng - g0);
+            const int gn = min(kTileSlots / 4, ng - g0);
             for (int gl = gsub; gl < gn; gl += 4) {
                 typedef uint16_t vu4 __attribute__((ext_vector_type(4)));
                 vu4 v;
 #pragma unroll
                 for (int jj = 0; jj < 4; ++jj) {
                     const int jl = 4 * (g0 + gl) + jj;
-                    const int32_t d = tc[(4 * gl + jj) * kB16Pitch + l];
+                    const int32_t d = tc[(4 * gl + jj) * kTilePitch + l];
                     const bool have = jl < len;
                     const int n_have = __popcll(__ballot(have));  // the first lanes: rows by decreasing length
                     const int32_t b = __builtin_amdgcn_readlane(d, n_have >> 1) - kFar16 / 2;
@@ -1145,8 +1175,8 @@ dcpse_status dcpse_sell_fill_cols(dcpse_ctx* ctx, int64_t n_rows, const int64_t*
     DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     if (n_rows == 0) return DCPSE_OK;
     const int64_t b = std::min<int64_t>((n_rows + 63) / 64, 65536);
-    k_sell_fill<true, float><<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, col, nullptr, slice_ptr, sell_row,
-                                                            sell_col, nullptr);
+    k_sell_fill<int32_t, false><<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, col, nullptr, slice_ptr,
+                                                                      sell_row, sell_col);
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
 }
@@ -1159,8 +1189,8 @@ dcpse_status dcpse_sell_fill_weights_f32(dcpse_ctx* ctx, int64_t n_rows, const i
     DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     if (n_rows == 0) return DCPSE_OK;
     const int64_t b = std::min<int64_t>((n_rows + 63) / 64, 65536);
-    k_sell_fill<false, float><<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, nullptr, W, slice_ptr, sell_row,
-                                                             nullptr, sell_W);
+    k_sell_fill<float, false><<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, W, nullptr, slice_ptr, sell_row,
+                                                                    sell_W);
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
 }
@@ -1173,8 +1203,23 @@ dcpse_status dcpse_sell_fill_weights_f64(dcpse_ctx* ctx, int64_t n_rows, const i
     DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     if (n_rows == 0) return DCPSE_OK;
     const int64_t b = std::min<int64_t>((n_rows + 63) / 64, 65536);
-    k_sell_fill<false, double><<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, nullptr, W, slice_ptr,
-                                                                     sell_row, nullptr, sell_W);
+    k_sell_fill<double, false><<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, W, nullptr, slice_ptr, sell_row,
+                                                                     sell_W);
+    DCPSE_LAUNCH_CHECK(ctx);
+    return DCPSE_OK;
+}
+
+dcpse_status dcpse_sell_fill_weights_scaled_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
+                                                const double* K, const double* row_scale, const int64_t* slice_ptr,
+                                                const int32_t* sell_row, double* sell_W) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!row_ptr || !K || !row_scale || !slice_ptr || !sell_row || !sell_W || n_rows < 0)
+        return fail(ctx, DCPSE_ERR_INVALID, "null pointer or negative size");
+    DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    if (n_rows == 0) return DCPSE_OK;
+    const int64_t b = std::min<int64_t>((n_rows + 63) / 64, 65536);
+    k_sell_fill<double, true><<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, K, row_scale, slice_ptr,
+                                                                    sell_row, sell_W);
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
 }
@@ -1210,35 +1255,57 @@ dcpse_status dcpse_apply_sell_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t*
     return DCPSE_OK;
 }
 
-dcpse_status dcpse_sell_fill_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
-                                          const int32_t* col, int32_t n_ops, const double* const* W,
-                                          const int64_t* slice_ptr, const int32_t* sell_row,
-                                          const int64_t* exc_ptr, int64_t n_exc, int32_t* bundle,
-                                          int32_t* sell_row16, int32_t* exc_col, double* exc_W) {
+static dcpse_status fill_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
+                                      int32_t n_ops, const double* const* W, const double* const* row_scale,
+                                      const int64_t* slice_ptr, const int32_t* sell_row, const int64_t* exc_ptr,
+                                      int64_t n_exc, int32_t* bundle, int32_t* sell_row16, int32_t* exc_col,
+                                      double* exc_W) {
     if (!ctx) return DCPSE_ERR_INVALID;
     if (!row_ptr || !col || !W || !slice_ptr || !sell_row || !exc_ptr || !bundle || !sell_row16 || n_rows < 0 ||
         n_exc < 0 || (n_exc > 0 && (!exc_col || !exc_W)))
         return fail(ctx, DCPSE_ERR_INVALID, "null pointer or negative size");
     if (n_ops < 1 || n_ops > 4) return fail(ctx, DCPSE_ERR_UNSUPPORTED, "1 to 4 operators per bundle");
-    for (int o = 0; o < n_ops; ++o)
-        if (!W[o]) return fail(ctx, DCPSE_ERR_INVALID, "null weight array");
+    FillWeights<double> w{};
+    for (int o = 0; o < n_ops; ++o) {
+        if (!W[o] || (row_scale && !row_scale[o])) return fail(ctx, DCPSE_ERR_INVALID, "null weight array");
+        w.W[o] = W[o];
+        w.scale[o] = row_scale ? row_scale[o] : nullptr;
+    }
     if (n_rows >= ((int64_t)1 << 30)) return fail(ctx, DCPSE_ERR_RANGE, "16-bit bundles need n_rows < 2^30");
     DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     if (n_rows == 0) return DCPSE_OK;
     const int64_t n_slices = (n_rows + 63) / 64;
     const int64_t b = std::min<int64_t>(n_slices, (int64_t)ctx->num_cus * 16);
-    k_sell_fill_bundle16_f64<<<(unsigned)b, 256, 0, ctx->stream>>>(
-        n_rows, row_ptr, col, n_ops, W[0], n_ops > 1 ? W[1] : nullptr, n_ops > 2 ? W[2] : nullptr,
-        n_ops > 3 ? W[3] : nullptr, slice_ptr, sell_row, exc_ptr, bundle, sell_row16);
+    k_sell_fill_bundle16_f64<<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, col, n_ops, w, slice_ptr,
+                                                                   sell_row, exc_ptr, bundle, sell_row16);
     DCPSE_LAUNCH_CHECK(ctx);
     if (n_exc > 0) {
         const int64_t be = std::min<int64_t>((n_rows + 63 + 255) / 256, 65536);
-        k_bundle16_exc<double><<<(unsigned)be, 256, 0, ctx->stream>>>(
-            n_rows, row_ptr, col, n_ops, W[0], n_ops > 1 ? W[1] : nullptr, n_ops > 2 ? W[2] : nullptr,
-            n_ops > 3 ? W[3] : nullptr, sell_row, exc_ptr, n_exc, exc_col, exc_W);
+        k_bundle16_exc<double><<<(unsigned)be, 256, 0, ctx->stream>>>(n_rows, row_ptr, col, n_ops, w, sell_row,
+                                                                      exc_ptr, n_exc, exc_col, exc_W);
     }
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
+}
+
+dcpse_status dcpse_sell_fill_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
+                                          const int32_t* col, int32_t n_ops, const double* const* W,
+                                          const int64_t* slice_ptr, const int32_t* sell_row,
+                                          const int64_t* exc_ptr, int64_t n_exc, int32_t* bundle,
+                                          int32_t* sell_row16, int32_t* exc_col, double* exc_W) {
+    return fill_bundle16_f64(ctx, n_rows, row_ptr, col, n_ops, W, nullptr, slice_ptr, sell_row, exc_ptr, n_exc,
+                             bundle, sell_row16, exc_col, exc_W);
+}
+
+dcpse_status dcpse_sell_fill_bundle16_scaled_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
+                                                 const int32_t* col, int32_t n_ops, const double* const* K,
+                                                 const double* const* row_scale, const int64_t* slice_ptr,
+                                                 const int32_t* sell_row, const int64_t* exc_ptr, int64_t n_exc,
+                                                 int32_t* bundle, int32_t* sell_row16, int32_t* exc_col,
+                                                 double* exc_W) {
+    if (!row_scale) return fail(ctx, DCPSE_ERR_INVALID, "row_scale is null");
+    return fill_bundle16_f64(ctx, n_rows, row_ptr, col, n_ops, K, row_scale, slice_ptr, sell_row, exc_ptr, n_exc,
+                             bundle, sell_row16, exc_col, exc_W);
 }
 
 dcpse_status dcpse_apply_sell_bundle16_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr,
@@ -1391,9 +1458,10 @@ dcpse_status dcpse_sell_fill_bundle16_f32(dcpse_ctx* ctx, int64_t n_rows, const 
     DCPSE_LAUNCH_CHECK(ctx);
     if (n_exc > 0) {
         const int64_t be = std::min<int64_t>((n_rows + 63 + 255) / 256, 65536);
-        k_bundle16_exc<float><<<(unsigned)be, 256, 0, ctx->stream>>>(
-            n_rows, row_ptr, col, n_ops, W[0], n_ops > 1 ? W[1] : nullptr, n_ops > 2 ? W[2] : nullptr,
-            n_ops > 3 ? W[3] : nullptr, sell_row, exc_ptr, n_exc, exc_col, exc_W);
+        FillWeights<float> w{};
+        for (int o = 0; o < n_ops; ++o) w.W[o] = W[o];
+        k_bundle16_exc<float><<<(unsigned)be, 256, 0, ctx->stream>>>(n_rows, row_ptr, col, n_ops, w, sell_row,
+                                                                     exc_ptr, n_exc, exc_col, exc_W);
     }
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;

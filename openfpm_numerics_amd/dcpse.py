@@ -215,9 +215,14 @@ class Dcpse:
             vl = self.verletList
             slice_ptr, sell_row, n_slots = vl.sell_slices()
             sw = torch.empty(max(n_slots, 4), dtype=torch.float64, device=vl.row_ptr.device)
-            _lib.context(vl.row_ptr.device.index or 0).call(
-                "dcpse_sell_fill_weights_f64", vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(self.weights(torch.float64)),
-                _lib.ptr(slice_ptr), _lib.ptr(sell_row), _lib.ptr(sw))
+            ctx = _lib.context(vl.row_ptr.device.index or 0)
+            if torch.float64 in self._W:
+                ctx.call("dcpse_sell_fill_weights_f64", vl.n_rows, _lib.ptr(vl.row_ptr),
+                         _lib.ptr(self.weights(torch.float64)), _lib.ptr(slice_ptr), _lib.ptr(sell_row), _lib.ptr(sw))
+            else:
+                ctx.call("dcpse_sell_fill_weights_scaled_f64", vl.n_rows, _lib.ptr(vl.row_ptr),
+                         _lib.ptr(self.calcKernels), _lib.ptr(self.localEpsInvPow), _lib.ptr(slice_ptr),
+                         _lib.ptr(sell_row), _lib.ptr(sw))
             self._W["sell64"] = sw
         return self._W["sell64"]
 
@@ -236,15 +241,7 @@ class Dcpse:
         if not self.same_set:
             return False
         vl = self.verletList
-        if getattr(vl, "_n_exc16", None) is None:
-            sell_row = vl.sell_slices()[1]
-            exc_ptr = torch.empty(sell_row.numel() + 1, dtype=torch.int64, device=vl.row_ptr.device)
-            n_exc = np.zeros(1, np.int64)
-            _lib.context(vl.row_ptr.device.index or 0).call(
-                "dcpse_sell_bundle16_count", vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), _lib.ptr(sell_row),
-                _lib.ptr(exc_ptr), n_exc.ctypes.data)
-            vl._n_exc16 = int(n_exc[0])
-        return vl._n_exc16 <= BUNDLE16_MAX_EXC * max(vl.nnz, 1)
+        return vl.far16()[1] <= BUNDLE16_MAX_EXC * max(vl.nnz, 1)
 
     def col16(self):
         """The 16-bit columns of this operator's list (VerletList.col16) where it
@@ -684,21 +681,18 @@ def sell_bundle16(ops, dtype=torch.float32):
     N) listed per lane."""
     if not all(op.same_set for op in ops):
         raise ValueError("16-bit column offsets need operators whose support and domain sets are the same")
+    if dtype == torch.float64 and not any(dtype in op._W for op in ops):
+        return bundle16(ops[0].verletList, [op.calcKernels for op in ops], [op.localEpsInvPow for op in ops])
     return bundle16(ops[0].verletList, [op.weights(dtype) for op in ops])
 
 
-def bundle16(vl: VerletList, Ws):
+def bundle16(vl: VerletList, Ws, scales=None):
     """sell_bundle16 of weight arrays Ws (all FP32 or all FP64) in the CSR
-    order of vl."""
+    order of vl, or of FP64 kernels Ws with a scale per row each."""
     slice_ptr, sell_row, n_slots = vl.sell_slices()
     dev = vl.row_ptr.device
     ctx = _lib.context(dev.index or 0)
-    n_lanes = sell_row.numel()
-    exc_ptr = torch.empty(n_lanes + 1, dtype=torch.int64, device=dev)
-    n_exc = np.zeros(1, np.int64)
-    ctx.call("dcpse_sell_bundle16_count", vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), _lib.ptr(sell_row),
-             _lib.ptr(exc_ptr), n_exc.ctypes.data)
-    ne = int(n_exc[0])
+    exc_ptr, ne = vl.far16()
     dt = Ws[0].dtype
     if dt not in (torch.float32, torch.float64) or any(W.dtype != dt for W in Ws):
         raise TypeError("bundle weights must be all float32 or all float64")
@@ -707,9 +701,13 @@ def bundle16(vl: VerletList, Ws):
     sell_row16 = torch.empty_like(sell_row)
     exc_col = torch.empty(max(ne, 1), dtype=torch.int32, device=dev)
     exc_W = torch.empty(max(len(Ws) * ne, 1), dtype=dt, device=dev)
-    ctx.call("dcpse_sell_fill_bundle16_f32" if dt == torch.float32 else "dcpse_sell_fill_bundle16_f64", vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), len(Ws),
-             _lib.ptr_array(Ws), _lib.ptr(slice_ptr), _lib.ptr(sell_row), _lib.ptr(exc_ptr), ne, _lib.ptr(bundle),
-             _lib.ptr(sell_row16), _lib.ptr(exc_col), _lib.ptr(exc_W))
+    name = "dcpse_sell_fill_bundle16_f32" if dt == torch.float32 else "dcpse_sell_fill_bundle16_f64"
+    W = (_lib.ptr_array(Ws),)
+    if scales is not None:
+        name, W = "dcpse_sell_fill_bundle16_scaled_f64", (*W, _lib.ptr_array(scales))
+    ctx.call(name, vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), len(Ws), *W, _lib.ptr(slice_ptr),
+             _lib.ptr(sell_row), _lib.ptr(exc_ptr), ne, _lib.ptr(bundle), _lib.ptr(sell_row16), _lib.ptr(exc_col),
+             _lib.ptr(exc_W))
     return bundle, sell_row16, exc_ptr, exc_col, exc_W, ne
 
 

@@ -93,7 +93,7 @@ class ParticleSet:
         vl.__dict__.update(fresh.__dict__)
         vl._sell = None
         vl._slices = None
-        vl._n_exc16 = None
+        vl._far16 = None
         vl._col16 = None
         return vl
 
@@ -192,7 +192,7 @@ class VerletList:
         self._host = None
         self._sell = None
         self._slices = None
-        self._n_exc16 = None
+        self._far16 = None
         self._col16 = None
         self.map_ctr = -1
 
@@ -275,6 +275,19 @@ class VerletList:
             self._sell = (slice_ptr, sell_row, sell_cols(self.row_ptr, self.col, self.n_rows, slice_ptr, sell_row,
                                                          n_slots))
         return self._sell
+
+    def far16(self):
+        """(exc_ptr, n_exc): the neighbours whose plain 16-bit offset does not fit,
+        per lane (see dcpse_sell_bundle16_count); counted on first use."""
+        if getattr(self, "_far16", None) is None:
+            sell_row = self.sell_slices()[1]
+            exc_ptr = torch.empty(sell_row.numel() + 1, dtype=torch.int64, device=self.row_ptr.device)
+            n_exc = np.zeros(1, np.int64)
+            _lib.context(self.row_ptr.device.index or 0).call(
+                "dcpse_sell_bundle16_count", self.n_rows, _lib.ptr(self.row_ptr), _lib.ptr(self.col),
+                _lib.ptr(sell_row), _lib.ptr(exc_ptr), n_exc.ctypes.data)
+            self._far16 = (exc_ptr, int(n_exc[0]))
+        return self._far16
 
     def col16(self, max_far: float):
         """The 16-bit columns of the sliced-ELL layout (one particle set; see
