@@ -349,7 +349,7 @@ dcpse_status dcpse_apply_sell_bundle_f32(dcpse_ctx* ctx, int64_t n_rows, const i
  * words (the 64 lanes' four 16-bit offsets, then each operator's weights)
  * starting at (128 + 256 * n_ops) * slice_ptr[s] / 256; bundle holds
  * (0.5 + n_ops) * n_slots words. Neighbours with |d| > 32767 are stored as
- * d = 0 and listed per lane instead: count writes exc_ptr[64*n_slices+1]
+ * d = 0 with weight 0 and listed per lane instead: count writes exc_ptr[64*n_slices+1]
  * (device) and *n_exc (host, synchronises); fill writes the bundle,
  * sell_row16 (sell_row with bit 30 set on lanes that have such neighbours),
  * exc_col[n_exc] and exc_W[n_ops*n_exc] (weights of operator o at

@@ -182,8 +182,8 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle(int64_t n_rows, const 
 // hold offset 0.
 // A neighbour further than 32767 positions (in a lattice-ordered periodic set,
 // the rare pairs whose offset combines a wrap with plane steps) is stored as
-// offset 0 - so in the gather it contributes W * (f_p - f_p) = 0 - and kept in
-// a per-lane exception list (exc_ptr over lanes, exc_col, exc_W[o * n_exc + k])
+// offset 0 (in FP32 with weight 0) - so in the gather it contributes
+// W * (f_p - f_p) = 0 - and kept in a per-lane exception list (exc_ptr over lanes, exc_col, exc_W[o * n_exc + k])
 // that the apply adds after the slot loop; lanes with exceptions are marked
 // in sell_row16 by kExcFlag.
 constexpr int32_t kExcFlag = 1 << 30;
@@ -263,12 +263,16 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16(
                 const int len = slen[ll];
                 const int64_t rs = srs[ll];
                 int32_t d = 0;
-                if (j < len) {
+                bool in = j < len;
+                if (in) {
                     const int64_t dj = col_offset(col[rs + j], srow[ll], n_rows);
-                    d = far16(dj) ? 0 : (int32_t)dj;
+                    in = !far16(dj);
+                    d = in ? (int32_t)dj : 0;
                 }
                 tc[e * kTilePitch + ll] = d;
-                for (int o = 0; o < n_ops; ++o) tw[o][e * kTilePitch + ll] = j < len ? W[o][rs + j] : 0.0f;
+                // a far neighbour's slot has no weight: the transposed apply adds
+                // W g_q without the difference that would cancel it
+                for (int o = 0; o < n_ops; ++o) tw[o][e * kTilePitch + ll] = in ? W[o][rs + j] : 0.0f;
             }
             __syncthreads();
             // write: thread (lane l, gsub) writes the tile's groups gsub, gsub + 4
