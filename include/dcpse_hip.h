@@ -470,6 +470,15 @@ dcpse_status dcpse_export_csr_f64(dcpse_ctx* ctx, int64_t n_rows, const int64_t*
 dcpse_status dcpse_export_csr_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
                                   const float* W, double sign, int64_t* out_row_ptr, int32_t* out_col,
                                   float* out_val);
+/* The same with the number of neighbours (row_ptr[n_rows]) known to the host,
+ * which picks the lanes per row; row_scale not NULL: W holds the kernels K and
+ * W_pq = row_scale[p] * K_pq, the weights of dcpse_scale_rows_f64 bit for bit. */
+dcpse_status dcpse_export_csr_nnz_f64(dcpse_ctx* ctx, int64_t n_rows, int64_t nnz, const int64_t* row_ptr,
+                                      const int32_t* col, const double* W, const double* row_scale, double sign,
+                                      int64_t* out_row_ptr, int32_t* out_col, double* out_val);
+dcpse_status dcpse_export_csr_nnz_f32(dcpse_ctx* ctx, int64_t n_rows, int64_t nnz, const int64_t* row_ptr,
+                                      const int32_t* col, const float* W, double sign, int64_t* out_row_ptr,
+                                      int32_t* out_col, float* out_val);
 
 /* FP64 pre-scaled weights W[j] = row_scale[p] * K[j] for every neighbour j of
  * row p, one rounding per weight: the W64 output of dcpse_assemble (bit for

@@ -93,6 +93,8 @@ SIGNATURES = {
                                              _f64, _f64]),
     "dcpse_export_csr_f64": (_i32, [_vp, _i64, _vp, _vp, _vp, _f64, _vp, _vp, _vp]),
     "dcpse_export_csr_f32": (_i32, [_vp, _i64, _vp, _vp, _vp, _f64, _vp, _vp, _vp]),
+    "dcpse_export_csr_nnz_f64": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _f64, _vp, _vp, _vp]),
+    "dcpse_export_csr_nnz_f32": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _f64, _vp, _vp, _vp]),
     "dcpse_scale_rows_f64": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp]),
     "dcpse_stage_f32": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _f32, _vp, _f32, _vp, _vp, _f32, _vp]),
     "dcpse_stage_f64": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _f64, _vp, _f64, _vp, _vp, _f64, _vp]),

@@ -293,9 +293,16 @@ class Dcpse:
         rp = torch.empty(n + 1, dtype=torch.int64, device=dev)
         col = torch.empty(vl.nnz + n, dtype=torch.int32, device=dev)
         val = torch.empty(vl.nnz + n, dtype=dtype, device=dev)
-        name = "dcpse_export_csr_f64" if dtype == torch.float64 else "dcpse_export_csr_f32"
-        _lib.context(dev.index or 0).call(name, n, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), _lib.ptr(self.weights(dtype)),
-                                          float(self.getSign()), _lib.ptr(rp), _lib.ptr(col), _lib.ptr(val))
+        p = _lib.ptr
+        if dtype == torch.float64 and dtype not in self._W and torch.float32 in self._W:
+            # FP64 weights not formed yet: from the kernels
+            name, W = "dcpse_export_csr_nnz_f64", (p(self.calcKernels), p(self.localEpsInvPow))
+        elif dtype == torch.float64:
+            name, W = "dcpse_export_csr_nnz_f64", (p(self.weights(dtype)), None)
+        else:
+            name, W = "dcpse_export_csr_nnz_f32", (p(self.weights(dtype)),)
+        _lib.context(dev.index or 0).call(name, n, vl.nnz, p(vl.row_ptr), p(vl.col), *W, float(self.getSign()), p(rp),
+                                          p(col), p(val))
         return rp, col, val
 
     def to_sparse_csr(self, dtype=torch.float64) -> torch.Tensor:
