@@ -163,6 +163,25 @@ dcpse_status dcpse_support_fill_subset(dcpse_ctx* ctx, int32_t dim,
                                        const double* rcut, int32_t rcut_per_particle,
                                        const double* box_lo, const double* box_hi, uint32_t periodic_mask,
                                        const int64_t* row_ptr, int32_t* col);
+/* dcpse_support_count (dom_ids NULL) or _count_subset for one cut-off whose
+ * value the host holds (rcut[0] on the device has it too): nothing is read
+ * back before the search. */
+dcpse_status dcpse_support_count_one(dcpse_ctx* ctx, int32_t dim,
+                                     const double* pos_sup, int64_t n_sup,
+                                     const double* pos_dom, const int32_t* dom_ids, int64_t n_dom,
+                                     const double* rcut, double rcut_value,
+                                     const double* box_lo, const double* box_hi, uint32_t periodic_mask,
+                                     int64_t* row_ptr, int64_t* nnz);
+/* dcpse_support_fill (dom_ids NULL) or _fill_subset as the next call on this
+ * context after the count with the same arguments and data: the extremes of
+ * the cut-offs are those of the count instead of being reduced and read back
+ * again. */
+dcpse_status dcpse_support_fill_counted(dcpse_ctx* ctx, int32_t dim,
+                                        const double* pos_sup, int64_t n_sup,
+                                        const double* pos_dom, const int32_t* dom_ids, int64_t n_dom,
+                                        const double* rcut, int32_t rcut_per_particle,
+                                        const double* box_lo, const double* box_hi, uint32_t periodic_mask,
+                                        const int64_t* row_ptr, int32_t* col);
 
 /* ---- kernel assembly (FP64) ------------------------------------------- */
 /* Assembles sum_k coeffs[k] * D^{beta_k} for n_sig signatures that share one

@@ -27,6 +27,11 @@ dcpse_status dcpse_ctx_create(dcpse_ctx** out, int32_t device) {
         delete ctx;
         return DCPSE_ERR_HIP;
     }
+    if (hipHostMalloc(reinterpret_cast<void**>(&ctx->host), kResults * sizeof(int64_t), hipHostMallocDefault) !=
+        hipSuccess) {
+        delete ctx;
+        return DCPSE_ERR_HIP;
+    }
     *out = ctx;
     return DCPSE_OK;
 }
@@ -37,6 +42,7 @@ dcpse_status dcpse_ctx_destroy(dcpse_ctx* ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->ws) (void)hipFree(ctx->ws);
     if (ctx->sup.buf) (void)hipFree(ctx->sup.buf);
+    if (ctx->host) (void)hipHostFree(ctx->host);
     delete ctx;
     return DCPSE_OK;
 }

@@ -25,6 +25,11 @@ struct dcpse_support_cache {
     double lo[3] = {0.0, 0.0, 0.0}, hi[3] = {0.0, 0.0, 0.0};
     unsigned periodic = 0;
     int nws = 0;          // mask words per particle
+    // extremes of the cut-offs of the last count, whatever kernels it ran
+    bool seen = false;
+    const double *seen_pos = nullptr, *seen_rcut = nullptr;
+    int64_t seen_n = 0;   // rows
+    double seen_max = 0.0, seen_min = 0.0;
 };
 
 struct dcpse_ctx {
@@ -50,6 +55,7 @@ struct dcpse_ctx {
     int asm_bucket = 0;    // > 0: batches bucketed by row length, this bucket width
     void* ws = nullptr;    // grow-only device workspace
     size_t ws_size = 0;
+    int64_t* host = nullptr;  // pinned: kResults numbers that kernels leave for the host
     void* scratch = nullptr;  // this device's static no-alloc scratch (device address)
     dcpse_support_cache sup;
     char err[1024] = {0};
@@ -92,8 +98,16 @@ struct Workspace {
 // Ensures ctx->ws holds at least `bytes`; waits for queued work before growing.
 dcpse_status reserve_workspace(dcpse_ctx* ctx, size_t bytes, Workspace* w);
 
+// Numbers that a pass leaves in ctx->host: a kernel stores them to pinned
+// memory, so the host waits once instead of copying each to pageable memory
+// (a blocking 15-25 us apiece).
+constexpr int kResults = 8;
+
 // Exclusive scan of n int32 counts into out[0..n] (int64), on ctx->stream.
-dcpse_status scan_counts(dcpse_ctx* ctx, const int32_t* in, int64_t n, int64_t* out, Workspace* w);
+// to_host: the last kernel also leaves the total in ctx->host[0] and, where
+// given, *extra0 and *extra1 in ctx->host[1] and [2].
+dcpse_status scan_counts(dcpse_ctx* ctx, const int32_t* in, int64_t n, int64_t* out, Workspace* w,
+                         bool to_host = false, const int32_t* extra0 = nullptr, const int32_t* extra1 = nullptr);
 size_t scan_workspace_bytes(int64_t n);
 
 // Looks up this device's address of the static scratch array of the no-alloc

@@ -1073,13 +1073,10 @@ static dcpse_status sell_count_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_
                                                                                         sell_row, flags);
         DCPSE_LAUNCH_CHECK(ctx);
     }
-    if ((st = scan_counts(ctx, counts, n_slices, slice_ptr, &w))) return st;
-    int64_t total = 0;
-    int32_t ovf = 0;
-    DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&total, slice_ptr + n_slices, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
-    DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&ovf, flags, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+    if ((st = scan_counts(ctx, counts, n_slices, slice_ptr, &w, true, flags))) return st;
     DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    if (ovf) return fail(ctx, DCPSE_ERR_RANGE, "a row exceeds DCPSE_MAX_ROW=%d", DCPSE_MAX_ROW);
+    const int64_t total = ctx->host[0];
+    if (ctx->host[1]) return fail(ctx, DCPSE_ERR_RANGE, "a row exceeds DCPSE_MAX_ROW=%d", DCPSE_MAX_ROW);
     if (n_slots) *n_slots = total;
     return DCPSE_OK;
 }
@@ -1432,11 +1429,9 @@ dcpse_status dcpse_sell_bundle16_count(dcpse_ctx* ctx, int64_t n_rows, const int
         k_bundle16_count<<<(unsigned)b, 256, 0, ctx->stream>>>(n_rows, row_ptr, col, sell_row, counts);
         DCPSE_LAUNCH_CHECK(ctx);
     }
-    if ((st = scan_counts(ctx, counts, n_lanes, exc_ptr, &w))) return st;
-    int64_t total = 0;
-    DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&total, exc_ptr + n_lanes, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+    if ((st = scan_counts(ctx, counts, n_lanes, exc_ptr, &w, true))) return st;
     DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    *n_exc = total;
+    *n_exc = ctx->host[0];
     return DCPSE_OK;
 }
 
@@ -1656,11 +1651,9 @@ dcpse_status dcpse_sell_fill_col16(dcpse_ctx* ctx, int64_t n_rows, const int64_t
                                                                 base, counts);
         DCPSE_LAUNCH_CHECK(ctx);
     }
-    if ((st = scan_counts(ctx, counts, n_lanes, exc_ptr, &w))) return st;
-    int64_t total = 0;
-    DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&total, exc_ptr + n_lanes, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+    if ((st = scan_counts(ctx, counts, n_lanes, exc_ptr, &w, true))) return st;
     DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    *n_exc = total;
+    *n_exc = ctx->host[0];
     return DCPSE_OK;
 }
 

@@ -73,7 +73,8 @@ __global__ __launch_bounds__(1024) void k_scan_tilesums(int64_t* tsum, int64_t n
 
 __global__ __launch_bounds__(kScanBlock) void k_scan_tiles(const int32_t* __restrict__ in, int64_t n,
                                                            const int64_t* __restrict__ tsum,
-                                                           int64_t* __restrict__ out) {
+                                                           int64_t* __restrict__ out, int64_t* host,
+                                                           const int32_t* extra0, const int32_t* extra1) {
     __shared__ long long buf[kScanBlock];
     const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
     long long v[kScanItems];
@@ -99,7 +100,20 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_tiles(const int32_t* __rest
         if (k < n) out[k] = run;
         run += v[i];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = tsum[gridDim.x];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        out[n] = tsum[gridDim.x];
+        if (host) {
+            host[0] = tsum[gridDim.x];
+            if (extra0) host[1] = *extra0;
+            if (extra1) host[2] = *extra1;
+            __threadfence_system();
+        }
+    }
+}
+
+__global__ void k_to_host(const int32_t* v, int64_t* host) {
+    *host = *v;
+    __threadfence_system();
 }
 
 size_t scan_workspace_bytes(int64_t n) {
@@ -107,7 +121,8 @@ size_t scan_workspace_bytes(int64_t n) {
     return (size_t)(nt + 1) * sizeof(int64_t) + 256;
 }
 
-dcpse_status scan_counts(dcpse_ctx* ctx, const int32_t* in, int64_t n, int64_t* out, Workspace* w) {
+dcpse_status scan_counts(dcpse_ctx* ctx, const int32_t* in, int64_t n, int64_t* out, Workspace* w, bool to_host,
+                         const int32_t* extra0, const int32_t* extra1) {
     int64_t nt = (n + kScanTile - 1) / kScanTile;
     if (nt == 0) nt = 1;
     int64_t* tsum = w->take<int64_t>((size_t)nt + 1);
@@ -116,7 +131,8 @@ dcpse_status scan_counts(dcpse_ctx* ctx, const int32_t* in, int64_t n, int64_t* 
     DCPSE_LAUNCH_CHECK(ctx);
     k_scan_tilesums<<<1, 1024, 0, ctx->stream>>>(tsum, nt);
     DCPSE_LAUNCH_CHECK(ctx);
-    k_scan_tiles<<<(unsigned)nt, kScanBlock, 0, ctx->stream>>>(in, n, tsum, out);
+    k_scan_tiles<<<(unsigned)nt, kScanBlock, 0, ctx->stream>>>(in, n, tsum, out, to_host ? ctx->host : nullptr, extra0,
+                                                               extra1);
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
 }
@@ -1314,7 +1330,8 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
                                  const double* pos_dom, int64_t n_dom, const int32_t* dom_self,
                                  const double* rcut, int rcut_pp,
                                  const double* box_lo, const double* box_hi, unsigned periodic,
-                                 int64_t* row_ptr, int32_t* col, int64_t* nnz_out) {
+                                 int64_t* row_ptr, int32_t* col, int64_t* nnz_out,
+                                 const double* rcut_host = nullptr, bool continues = false) {
     if (dim != 2 && dim != 3) return fail(ctx, DCPSE_ERR_UNSUPPORTED, "dim must be 2 or 3");
     // positions of an empty set may be null (a particle set without storage)
     if ((!pos_sup && n_sup > 0) || !row_ptr || !box_lo || !box_hi || n_sup < 0 || n_dom < 0)
@@ -1340,7 +1357,13 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
     hipStream_t s = ctx->stream;
     // the largest cut-off fixes the cell edge
     double rmax = 0.0, rmin = 0.0;
-    if (rcut_pp) {
+    dcpse_support_cache& sc = ctx->sup;
+    if (rcut_host && !rcut_pp) {
+        rmin = rmax = *rcut_host;
+    } else if (continues && sc.seen && sc.seen_pos == pos_sup && sc.seen_rcut == rcut && sc.seen_n == n_dom) {
+        rmax = sc.seen_max;
+        rmin = sc.seen_min;
+    } else if (rcut_pp) {
         // reduced on the device; only the blocks' extremes come back
         Workspace w0;
         dcpse_status st0 = reserve_workspace(ctx, kMinMaxBlocks * 2 * sizeof(double) + 256, &w0);
@@ -1363,6 +1386,12 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
         DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(s));
         rmin = rmax;
     }
+    sc.seen = col == nullptr;
+    sc.seen_pos = pos_sup;
+    sc.seen_rcut = rcut;
+    sc.seen_n = n_dom;
+    sc.seen_max = rmax;
+    sc.seen_min = rmin;
     const double spread = rmin > 0.0 ? rmax / rmin : 1.0;
     CellGrid g;
     HomeLevels home;
@@ -1417,7 +1446,6 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
 
     // the fill of one set reuses the cell list, candidate lists and take masks
     // of the count just before it when the arguments match
-    dcpse_support_cache& sc = ctx->sup;
     const bool count_pass = col == nullptr;
     const bool cached = grouped && !count_pass && sc.valid && sc.dim == dim && sc.pos == pos_sup &&
                         sc.n == n_sup && sc.rcut == rmax && sc.rmin == rmin && sc.rcut_pp == rcut_pp &&
@@ -1586,14 +1614,13 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
             rows(std::false_type(), nullptr);
         }
         DCPSE_LAUNCH_CHECK(ctx);
-        if ((st = scan(counts, n_dom, row_ptr))) return st;
-        int64_t nnz = 0;
-        int32_t ovf = 0, n_spill = 0;
-        DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&nnz, row_ptr + n_dom, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&ovf, flags, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        if (groups_on)
-            DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&n_spill, spill, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        {
+            Workspace ws = ws_scan;
+            if ((st = scan_counts(ctx, counts, n_dom, row_ptr, &ws, true, flags, groups_on ? spill : nullptr))) return st;
+        }
         DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(s));
+        const int64_t nnz = ctx->host[0];
+        const int32_t ovf = (int32_t)ctx->host[1], n_spill = groups_on ? (int32_t)ctx->host[2] : 0;
         if (ovf & 1)
             return fail(ctx, DCPSE_ERR_RANGE, "a support row exceeds DCPSE_MAX_ROW=%d neighbours",
                         DCPSE_MAX_ROW);
@@ -1631,9 +1658,10 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
             k_sort_long_rows<<<(unsigned)lb, kRowWaves * kWave, 0, s>>>(n_dom, row_ptr, col);
             DCPSE_LAUNCH_CHECK(ctx);
         }
-        int32_t ovf = 0;
-        DCPSE_HIP_CHECK(ctx, hipMemcpyAsync(&ovf, flags, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        k_to_host<<<1, 1, 0, s>>>(flags, ctx->host);
+        DCPSE_LAUNCH_CHECK(ctx);
         DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(s));
+        const int32_t ovf = (int32_t)ctx->host[0];
         if (ovf & 3)
             return fail(ctx, DCPSE_ERR_INVALID,
                         "support fill disagrees with row_ptr (positions or rcut changed since count?)");
@@ -1873,6 +1901,30 @@ dcpse_status dcpse_support_fill_subset(dcpse_ctx* ctx, int32_t dim, const double
     DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     return support_pass(ctx, dim, pos_sup, n_sup, pos_dom, n_dom, dom_ids, rcut, rcut_per_particle, box_lo, box_hi,
                         periodic_mask, const_cast<int64_t*>(row_ptr), col, nullptr);
+}
+
+dcpse_status dcpse_support_count_one(dcpse_ctx* ctx, int32_t dim, const double* pos_sup, int64_t n_sup,
+                                     const double* pos_dom, const int32_t* dom_ids, int64_t n_dom, const double* rcut,
+                                     double rcut_value, const double* box_lo, const double* box_hi,
+                                     uint32_t periodic_mask, int64_t* row_ptr, int64_t* nnz) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (dom_ids && !pos_dom) return fail(ctx, DCPSE_ERR_INVALID, "a subset needs pos_dom and dom_ids");
+    DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    return support_pass(ctx, dim, pos_sup, n_sup, pos_dom, n_dom, dom_ids, rcut, 0, box_lo, box_hi, periodic_mask,
+                        row_ptr, nullptr, nnz, &rcut_value);
+}
+
+dcpse_status dcpse_support_fill_counted(dcpse_ctx* ctx, int32_t dim, const double* pos_sup, int64_t n_sup,
+                                        const double* pos_dom, const int32_t* dom_ids, int64_t n_dom,
+                                        const double* rcut, int32_t rcut_per_particle, const double* box_lo,
+                                        const double* box_hi, uint32_t periodic_mask, const int64_t* row_ptr,
+                                        int32_t* col) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!col) return fail(ctx, DCPSE_ERR_INVALID, "col is null");
+    if (dom_ids && !pos_dom) return fail(ctx, DCPSE_ERR_INVALID, "a subset needs pos_dom and dom_ids");
+    DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    return support_pass(ctx, dim, pos_sup, n_sup, pos_dom, n_dom, dom_ids, rcut, rcut_per_particle, box_lo, box_hi,
+                        periodic_mask, const_cast<int64_t*>(row_ptr), col, nullptr, nullptr, true);
 }
 
 dcpse_status dcpse_transpose_count(dcpse_ctx* ctx, int64_t n_rows, int64_t n_cols, const int64_t* row_ptr,

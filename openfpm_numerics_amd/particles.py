@@ -207,7 +207,12 @@ class VerletList:
         dom = support if domain is None else domain
         if dom.dims != support.dims:
             raise ValueError("support and domain sets differ in dimension")
-        rc = torch.as_tensor(rCut, dtype=torch.float64, device=dev).reshape(-1).contiguous()
+        # one cut-off the host holds: nothing is copied either way
+        one = isinstance(rCut, (int, float, np.integer, np.floating))
+        if one:
+            rc = torch.full((1,), float(rCut), dtype=torch.float64, device=dev)
+        else:
+            rc = torch.as_tensor(rCut, dtype=torch.float64, device=dev).reshape(-1).contiguous()
         per = int(rc.numel() > 1)
         if per and rc.numel() != dom.size_local():
             raise ValueError("per-particle rCut needs one value per domain particle")
@@ -222,21 +227,22 @@ class VerletList:
         pdom = None if domain is None else _lib.ptr(dom.pos_soa)
         lo = np.ascontiguousarray(support.box_lo)
         hi = np.ascontiguousarray(support.box_hi)
+        ids = None
         if isinstance(domain, ParticleSubset):
             if domain.parent is not support:
                 raise ValueError("a subset domain must be a subset of the support set")
-            count, fill, dom_args = "dcpse_support_count_subset", "dcpse_support_fill_subset", (
-                pdom, _lib.ptr(domain.ids), n_dom)
+            ids = _lib.ptr(domain.ids)
+        sets = (support.dims, _lib.ptr(support.pos_soa), support.size_local(), pdom, ids, n_dom, _lib.ptr(rc))
+        box = (lo.ctypes.data, hi.ctypes.data, support.periodic_mask, _lib.ptr(row_ptr))
+        if one:
+            ctx.call("dcpse_support_count_one", *sets, float(rCut), *box, nnz.ctypes.data)
+        elif ids is not None:
+            ctx.call("dcpse_support_count_subset", *sets, per, *box, nnz.ctypes.data)
         else:
-            count, fill, dom_args = "dcpse_support_count", "dcpse_support_fill", (pdom, n_dom)
-        ctx.call(count, support.dims, _lib.ptr(support.pos_soa), support.size_local(),
-                 *dom_args, _lib.ptr(rc), per, lo.ctypes.data, hi.ctypes.data,
-                 support.periodic_mask, _lib.ptr(row_ptr), nnz.ctypes.data)
+            ctx.call("dcpse_support_count", *sets[:4], *sets[5:], per, *box, nnz.ctypes.data)
         col = torch.empty(max(int(nnz[0]), 1), dtype=torch.int32, device=dev)
         if int(nnz[0]) > 0:
-            ctx.call(fill, support.dims, _lib.ptr(support.pos_soa), support.size_local(),
-                     *dom_args, _lib.ptr(rc), per, lo.ctypes.data, hi.ctypes.data,
-                     support.periodic_mask, _lib.ptr(row_ptr), _lib.ptr(col))
+            ctx.call("dcpse_support_fill_counted", *sets, per, *box, _lib.ptr(col))
         col = col[: int(nnz[0])]
         vl = cls(row_ptr, col, support.size_local(), rc, domain)
         vl.map_ctr = support.map_ctr
