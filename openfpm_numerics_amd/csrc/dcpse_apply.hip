@@ -245,17 +245,17 @@ __global__ __launch_bounds__(kApplyMaxBlock) void k_apply_v4(const ApplyArgs<flo
 // Batches of FP32 fields on one set: the NF fields are first interleaved
 // particle-major (fil[q * NF + b]), so a neighbour's NF values are one
 // contiguous 4 NF-byte read instead of NF separate gathers, and the col/W
-// streams are read once for all of them. Each field's sum runs over the
-// nonzeros in the order of k_apply_v4, so the results equal the field-major
-// kernel's bit for bit.
+// streams are read once for all of them; nf <= NF fields, zeros for the rest.
+// Each field's sum runs over the nonzeros in the order of k_apply_v4, so the
+// results equal the field-major kernel's bit for bit.
 template <int NF>
-__global__ __launch_bounds__(256) void k_interleave(int64_t n, const float* __restrict__ f, int64_t ld,
+__global__ __launch_bounds__(256) void k_interleave(int64_t n, const float* __restrict__ f, int64_t ld, int nf,
                                                     float* __restrict__ fil) {
     __shared__ float t[NF][257];
     const int64_t q0 = (int64_t)blockIdx.x * 256;
     const int64_t q = q0 + threadIdx.x;
 #pragma unroll
-    for (int b = 0; b < NF; ++b) t[b][threadIdx.x] = q < n ? f[b * ld + q] : 0.0f;
+    for (int b = 0; b < NF; ++b) t[b][threadIdx.x] = q < n && b < nf ? f[b * ld + q] : 0.0f;
     __syncthreads();
     for (int k = threadIdx.x; k < 256 * NF; k += 256) {
         const int qq = k / NF, b = k % NF;
@@ -283,33 +283,38 @@ __device__ __forceinline__ int group_lane(int v) {
     else return __builtin_amdgcn_update_dpp(0, v, SRC * 0x55, 0xF, 0xF, true);
 }
 
-// L = NF / 4 lanes per row, 4 fields each: a neighbour's NF values are read by
-// its row's lanes side by side, so one 16-byte load instruction serves 64 / L
-// neighbours with one cache line each. (With a lane per neighbour reading all
-// its NF values, every one of its 16-byte loads looked up 64 lines: 308 us
-// against 161 us forward, 395 against 175 us transposed, for 16 fields on
-// 1024^2 particles with 29 neighbours. The cache's lookup rate bounded that;
-// here the vector units and the address unit are busy two thirds of the time
-// each. Measured and not better: more waves (spilled registers), the next
-// chunk's gathers ahead of the sums (half the waves), 32-bit addresses.) The
-// row's lanes load a chunk of 4 nonzeros together and pass them round by DPP.
-// Each field's sum takes the order of k_apply_v4<G, NCH>, whose lane p of a
-// row sums the chunks p, p + G, ... and then the strided tail: the partial sums
-// are formed here one after another and added up as its lane exchanges do.
-template <int G, int NCH, int NF, int MODE>
+// R = 4 or 8 lanes per row: L = NF / 4 of them side by side hold 4 fields each,
+// so one 16-byte load instruction serves 64 / L neighbours with one cache line
+// each, and H = R / L such parts share the row's partial sums. (With a lane per
+// neighbour reading all its NF values, every one of its 16-byte loads looked up
+// 64 lines: 308 us against 161 us forward, 395 against 175 us transposed, for
+// 16 fields on 1024^2 particles with 29 neighbours. The cache's lookup rate
+// bounded that; here the vector units and the address unit are busy two thirds
+// of the time each. Measured and not better: more waves (spilled registers),
+// the next chunk's gathers ahead of the sums (half the waves), 32-bit
+// addresses; and for 4 and 8 fields one part of 1 and 2 lanes per row, whose
+// partial sums follow one another: 100 us against the 56 us of a lane per
+// neighbour for 6 fields on 512^2 particles.) A part's lanes load a chunk of 4
+// nonzeros together and pass them round by DPP. Each field's sum takes the
+// order of k_apply_v4<G, NCH>, whose lane p of a row sums the chunks p, p + G,
+// ... and then the strided tail: part h forms the partial sums h, h + H, ...
+// one after another, and all are added up as that kernel's lane exchanges do,
+// the last exchanges between the parts.
+template <int G, int NCH, int NF, int MODE, int R>
 struct BatchRow {
-    static constexpr int L = NF / 4, EL = 4 / L;
+    static constexpr int L = NF / 4, EL = 4 / L, H = R / L, GP = G / H;
+    static_assert(H <= G, "a part has at least one partial sum");
     typedef typename StreamVec<int32_t, EL>::type vq;
     typedef typename StreamVec<float, EL>::type vw;
     const ApplyArgs<float>& a;
     int64_t rs;
     int len, lenv;  // nonzeros; those taken in chunks of 4 (0: all by the tail)
-    int g;          // lane of the row's group
+    int g, h;       // lane of its part, part
     vf4a fp;
     // the chunks' columns and weights, read ahead while they fit 32 registers
-    static constexpr bool AHEAD = 2 * EL * G * NCH <= 32;
-    vq q[AHEAD ? G * NCH : 1];
-    vw w[AHEAD ? G * NCH : 1];
+    static constexpr bool AHEAD = 2 * EL * GP * NCH <= 48;
+    vq q[AHEAD ? GP * NCH : 1];
+    vw w[AHEAD ? GP * NCH : 1];
 
     template <int K>
     __device__ __forceinline__ void element(int32_t qv, float wv, vf4a& f, double& wd) {
@@ -346,10 +351,15 @@ struct BatchRow {
         element<3 / EL>(part(qc, 3 % EL), part(wc, 3 % EL), f[3], wd[3]);
         add<MASK>(f, wd, v, s);
     }
-    // Column and weight of chunk C: lane g takes EL of its 4 nonzeros.
+    // First nonzero of the part's C-th chunk.
+    template <int C>
+    __device__ __forceinline__ int first() const {
+        return H == 1 ? 4 * C : 4 * (C * H + h);
+    }
+    // Column and weight of that chunk: lane g takes EL of its 4 nonzeros.
     template <int C>
     __device__ __forceinline__ void load(vq& qc, vw& wc) {
-        const int e = 4 * C + EL * g;
+        const int e = first<C>() + EL * g;
         const int64_t at = lenv > 0 ? rs + min(e, lenv - 1) : 0;
         qc = *reinterpret_cast<const vq*>(a.col + at);
         wc = *reinterpret_cast<const vw*>(a.W[0] + at);
@@ -357,14 +367,15 @@ struct BatchRow {
     template <int C>
     __device__ __forceinline__ void load_ahead() {
         if constexpr (AHEAD) {
-            if (__ballot(4 * C < lenv)) load<C>(q[C], w[C]);
-            if constexpr (C + 1 < G * NCH) load_ahead<C + 1>();
+            if (__ballot(first<C>() < lenv)) load<C>(q[C], w[C]);
+            if constexpr (C + 1 < GP * NCH) load_ahead<C + 1>();
         }
     }
     template <int C>
     __device__ __forceinline__ void chunk(double (&s)[4]) {
-        if (!__ballot(4 * C < lenv)) return;
-        const bool v[4] = {4 * C < lenv, 4 * C + 1 < lenv, 4 * C + 2 < lenv, 4 * C + 3 < lenv};
+        const int e = first<C>();
+        if (!__ballot(e < lenv)) return;
+        const bool v[4] = {e < lenv, e + 1 < lenv, e + 2 < lenv, e + 3 < lenv};
         vq qc;
         vw wc;
         if constexpr (AHEAD) qc = q[C], wc = w[C];
@@ -372,40 +383,51 @@ struct BatchRow {
         if (__ballot(!v[3])) four<true>(qc, wc, v, s);
         else four<false>(qc, wc, v, s);
     }
-    // Partial sum P: its chunks, then every G-th nonzero of the tail.
+    // EL of the four nonzeros e, e + G, ... of the tail.
+    __device__ __forceinline__ void load_tail(int e, vq& qv, vw& wv) {
+        int32_t qe[EL];
+        float we[EL];
+#pragma unroll
+        for (int k = 0; k < EL; ++k) {
+            const int at = e + G * (EL * g + k);
+            const int64_t j = at < len ? rs + at : 0;
+            qe[k] = a.col[j];
+            we[k] = a.W[0][j];
+        }
+        if constexpr (EL == 1) qv = qe[0], wv = we[0];
+        else
+#pragma unroll
+            for (int k = 0; k < EL; ++k) qv[k] = qe[k], wv[k] = we[k];
+    }
+    // The part's P-th partial sum: its chunks, then every G-th nonzero of the
+    // tail, whose columns and weights are read one step ahead.
     template <int P>
     __device__ __forceinline__ void partial(double (&s)[4]) {
 #pragma unroll
         for (int b = 0; b < 4; ++b) s[b] = 0.0;
+        int e = (lenv > 0 ? 4 * G * NCH : 0) + (H == 1 ? P : P * H + h);
+        vq qt, qn;
+        vw wt, wn;
+        bool more = __ballot(e < len) != 0;
+        if (more) load_tail(e, qt, wt);
         chunk<P>(s);
-        if constexpr (NCH > 1) chunk<P + G>(s);
-        if constexpr (NCH > 2) chunk<P + 2 * G>(s);
-        const int tail = lenv > 0 ? 4 * G * NCH : 0;
-        for (int e = tail + P; __ballot(e < len); e += 4 * G) {
-            // the next four of the stride, EL per lane
-            int32_t qe[EL];
-            float we[EL];
-#pragma unroll
-            for (int k = 0; k < EL; ++k) {
-                const int at = e + G * (EL * g + k);
-                const int64_t j = at < len ? rs + at : 0;
-                qe[k] = a.col[j];
-                we[k] = a.W[0][j];
-            }
-            vq qv;
-            vw wv;
-            if constexpr (EL == 1) qv = qe[0], wv = we[0];
-            else
-#pragma unroll
-                for (int k = 0; k < EL; ++k) qv[k] = qe[k], wv[k] = we[k];
+        if constexpr (NCH > 1) chunk<P + GP>(s);
+        if constexpr (NCH > 2) chunk<P + 2 * GP>(s);
+        while (more) {
+            more = __ballot(e + 4 * G < len) != 0;
+            if (more) load_tail(e + 4 * G, qn, wn);
             const bool v[4] = {e < len, e + G < len, e + 2 * G < len, e + 3 * G < len};
-            four<true>(qv, wv, v, s);
+            four<true>(qt, wt, v, s);
+            e += 4 * G;
+            qt = qn;
+            wt = wn;
         }
     }
-    // The sum that lane P holds after exchanges at distances G/2 .. OFF.
+    // The sum that lane P * H + h of k_apply_v4's row holds after exchanges at
+    // distances G/2 .. OFF * H.
     template <int P, int OFF>
     __device__ __forceinline__ void tree(double (&s)[4]) {
-        if constexpr (OFF == G) {
+        if constexpr (OFF == GP) {
             partial<P>(s);
         } else {
             tree<P, 2 * OFF>(s);
@@ -421,13 +443,14 @@ struct BatchRow {
 };
 
 constexpr int kBatchBlock = 256;
-template <int G, int NCH, int NF, int MODE>
-__global__ __launch_bounds__(kBatchBlock) void k_apply_batch(const ApplyArgs<float> a) {
-    typedef BatchRow<G, NCH, NF, MODE> Row;
+constexpr int kBatchMin = 3;  // fields that go particle-major
+template <int G, int NCH, int NF, int MODE, int R>
+__global__ __launch_bounds__(kBatchBlock) void k_apply_batch(const ApplyArgs<float> a, int nf) {
+    typedef BatchRow<G, NCH, NF, MODE, R> Row;
     const int64_t hb = blockIdx.x;
     const int64_t lb = (hb & 7) * a.per_xcd + (hb >> 3);
     if (lb >= a.blocks_needed) return;
-    const int64_t at = (lb * kBatchBlock + threadIdx.x) / Row::L;
+    const int64_t at = (lb * kBatchBlock + threadIdx.x) / R;
     const bool live = at < a.n_rows;
     if (!__ballot(live)) return;  // whole wavefront
     const int64_t row = live ? at : a.n_rows - 1;
@@ -440,13 +463,22 @@ __global__ __launch_bounds__(kBatchBlock) void k_apply_batch(const ApplyArgs<flo
     // single loads, as in k_apply_v4
     r.lenv = re + 3 <= nnz_total ? r.len : 0;
     r.g = threadIdx.x % Row::L;
+    r.h = threadIdx.x % R / Row::L;
     r.fp = *reinterpret_cast<const vf4a*>(a.f + row * NF + 4 * r.g);
     double s[4];
     r.template load_ahead<0>();
     r.template tree<0, 1>(s);
+    // the parts' sums: lane ^ 4, ^ 2, ^ 1 of the row's
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        if constexpr (R == 8) s[b] += __shfl_xor(s[b], 4, kWave);
+        if constexpr (Row::L <= 2 && R >= 4) s[b] += dpp_d<0x4E>(s[b]);
+        if constexpr (Row::L == 1) s[b] += dpp_d<0xB1>(s[b]);
+    }
     if (!live) return;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
+        if (r.h != (Row::H <= 4 ? b * Row::H / 4 : b) || 4 * r.g + b >= nf) continue;  // another part's, or none
         double val = s[b];
         if (MODE == kExplicitDiag) val = fma((double)a.diag[row], (double)r.fp[b], val);
         float* dst = a.out[0] + (4 * r.g + b) * a.ld_out + row;
@@ -456,12 +488,26 @@ __global__ __launch_bounds__(kBatchBlock) void k_apply_batch(const ApplyArgs<flo
     }
 }
 
-template <int G, int NCH, int NF, int MODE>
-static void launch_apply_il(ApplyArgs<float> a, int, hipStream_t s) {
-    const int rows_per_block = kBatchBlock / (NF / 4);
+template <int G, int NCH, int NF, int MODE, int R>
+static void launch_batch(ApplyArgs<float> a, int nf, hipStream_t s) {
+    const int rows_per_block = kBatchBlock / R;
     a.blocks_needed = (a.n_rows + rows_per_block - 1) / rows_per_block;
     a.per_xcd = (a.blocks_needed + 7) / 8;
-    k_apply_batch<G, NCH, NF, MODE><<<(unsigned)(a.per_xcd * 8), kBatchBlock, 0, s>>>(a);
+    k_apply_batch<G, NCH, NF, MODE, R><<<(unsigned)(a.per_xcd * 8), kBatchBlock, 0, s>>>(a, nf);
+}
+
+// Eight lanes per row where rows are long or few, four otherwise (us, 4 / 8
+// lanes; B16: 16 fields, B4: 4). Few rows leave waves to spare: 91,000 rows of
+// 62 B16 48 / 41, of 93 65 / 53; 131,000 of 29 35 / 33. Long ones: 729,000 of 93
+// B16 438 / 342, B4 195 / 173; 512,000 of 62 202 / 171, 85 / 84; 490,000 of 51
+// 142 / 127 but B4 54 / 57; 1,049,000 of 29 187 / 198, 89 / 106.
+template <int G, int NCH, int NF, int MODE>
+static void launch_apply_il(const ApplyArgs<float>& a, int nf, double mean, hipStream_t s) {
+    if constexpr (G == 8) {
+        if (a.n_rows <= 131072 || mean > (NF == 16 ? 40.0 : 56.0))
+            return launch_batch<G, NCH, NF, MODE, 8>(a, nf, s);
+    }
+    launch_batch<G, NCH, NF, MODE, 4>(a, nf, s);
 }
 
 // The interleaved batch kernel for the shapes of the 16-byte-load kernel
@@ -471,14 +517,14 @@ static bool il_shape(int G, int epl) {
            (G == 16 && (epl == 4 || epl == 8)) || (G == 32 && epl == 4);
 }
 template <int MODE, int NF>
-static bool dispatch_il(const ApplyArgs<float>& a, int G, int epl, int block, hipStream_t s) {
-    if (G == 4 && epl == 8) return launch_apply_il<4, 2, NF, MODE>(a, block, s), true;
-    if (G == 8 && epl == 4) return launch_apply_il<8, 1, NF, MODE>(a, block, s), true;
-    if (G == 8 && epl == 8) return launch_apply_il<8, 2, NF, MODE>(a, block, s), true;
-    if (G == 8 && epl == 12) return launch_apply_il<8, 3, NF, MODE>(a, block, s), true;
-    if (G == 16 && epl == 4) return launch_apply_il<16, 1, NF, MODE>(a, block, s), true;
-    if (G == 16 && epl == 8) return launch_apply_il<16, 2, NF, MODE>(a, block, s), true;
-    if (G == 32 && epl == 4) return launch_apply_il<32, 1, NF, MODE>(a, block, s), true;
+static bool dispatch_il(const ApplyArgs<float>& a, int G, int epl, int nf, double mean, hipStream_t s) {
+    if (G == 4 && epl == 8) return launch_apply_il<4, 2, NF, MODE>(a, nf, mean, s), true;
+    if (G == 8 && epl == 4) return launch_apply_il<8, 1, NF, MODE>(a, nf, mean, s), true;
+    if (G == 8 && epl == 8) return launch_apply_il<8, 2, NF, MODE>(a, nf, mean, s), true;
+    if (G == 8 && epl == 12) return launch_apply_il<8, 3, NF, MODE>(a, nf, mean, s), true;
+    if (G == 16 && epl == 4) return launch_apply_il<16, 1, NF, MODE>(a, nf, mean, s), true;
+    if (G == 16 && epl == 8) return launch_apply_il<16, 2, NF, MODE>(a, nf, mean, s), true;
+    if (G == 32 && epl == 4) return launch_apply_il<32, 1, NF, MODE>(a, nf, mean, s), true;
     return false;
 }
 
@@ -553,29 +599,33 @@ static bool dispatch_group_v4(const ApplyArgs<float>& a, int G, int epl, int nop
 
 struct ApplyShape {
     int G, epl, vec;
+    double mean;  // row length, 0: not looked up
 };
 
 // Launch shape from the mean row length (16-byte loads, 8 lanes per row): up
-// to 24 nonzeros 4 per lane, otherwise 8 per lane (longer rows finish in the
-// strided tail; covering them with a third chunk measured slower). The mean is read once per
+// to 24 nonzeros 4 per lane, up to 72 8 per lane, beyond 12 (rows of 93: one
+// field 56 us against 47, 16 fields 255 against 205 with the strided tail from
+// the 65th on, 343,000 rows; FP64 keeps 8). The mean is read once per
 // (row_ptr, n_rows) and cached in the context, so repeated applies of one
 // operator never synchronise the stream. dcpse_set_apply_config overrides it.
 static ApplyShape auto_shape(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr) {
-    if (ctx->apply_group > 0) return {ctx->apply_group, ctx->apply_epl, ctx->apply_vec};
-    if (ctx->grp_rows == row_ptr && ctx->grp_n == n_rows) return {ctx->grp_g, ctx->grp_epl, ctx->grp_vec};
+    if (ctx->apply_group > 0) return {ctx->apply_group, ctx->apply_epl, ctx->apply_vec, 0.0};
+    if (ctx->grp_rows == row_ptr && ctx->grp_n == n_rows) return {ctx->grp_g, ctx->grp_epl, ctx->grp_vec, ctx->grp_mean};
     int64_t nnz = 0;
-    ApplyShape sh{8, 8, 4};
+    ApplyShape sh{8, 8, 4, 0.0};
     if (n_rows > 0 &&
         hipMemcpyAsync(&nnz, row_ptr + n_rows, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream) == hipSuccess &&
         hipStreamSynchronize(ctx->stream) == hipSuccess) {
-        double mean = (double)nnz / (double)n_rows;
-        if (mean <= 24) sh = {8, 4, 4};
+        sh.mean = (double)nnz / (double)n_rows;
+        if (sh.mean <= 24) sh.epl = 4;
+        else if (sh.mean > 72) sh.epl = 12;
     }
     ctx->grp_rows = row_ptr;
     ctx->grp_n = n_rows;
     ctx->grp_g = sh.G;
     ctx->grp_epl = sh.epl;
     ctx->grp_vec = sh.vec;
+    ctx->grp_mean = sh.mean;
     return sh;
 }
 
@@ -605,7 +655,8 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
         if (!W[o] || !out[o]) return fail(ctx, DCPSE_ERR_INVALID, "null operator pointer");
     if (n_rows == 0) return DCPSE_OK;
     DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
-    const ApplyShape sh = auto_shape(ctx, n_rows, row_ptr);
+    ApplyShape sh = auto_shape(ctx, n_rows, row_ptr);
+    if (!std::is_same<T, float>::value && ctx->apply_group <= 0 && sh.epl == 12) sh.epl = 8;
     const int block = ctx->apply_block;
     if (block % sh.G != 0 || block < 64 || block > kApplyMaxBlock)
         return fail(ctx, DCPSE_ERR_INVALID, "block %d incompatible with group %d", block, sh.G);
@@ -625,30 +676,31 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
     }
     int b0 = 0;
     if constexpr (std::is_same<T, float>::value) {
-        // batches of 4 or more fields on one set (columns and rows index the
-        // same n_rows particles): interleaved 16 (8, 4) at a time through the
-        // workspace (the col/W streams read once per group)
-        if (nops == 1 && nfields >= 4 && sh.vec == 4 && il_shape(sh.G, sh.epl) &&
+        // batches of several fields on one set (columns and rows index the
+        // same n_rows particles): interleaved 16 at a time through the
+        // workspace (the col/W streams read once per group), the last ones in
+        // the smallest of 4, 8 or 16 that holds them
+        if (nops == 1 && nfields >= kBatchMin && sh.vec == 4 && il_shape(sh.G, sh.epl) &&
             (!f_self || (f_self == f && ld_self == ld_f))) {
             Workspace ws;
             dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(float) + 256, &ws);
             if (st) return st;
             float* fil = ws.take<float>((size_t)n_rows * 16);
             if (!fil) return fail(ctx, DCPSE_ERR_INVALID, "apply workspace sizing error");
-            while (nfields - b0 >= 4) {
-                const int nf = nfields - b0 >= 16 ? 16 : (nfields - b0 >= 8 ? 8 : 4);
+            while (nfields - b0 >= kBatchMin) {
+                const int nf = std::min(nfields - b0, 16);
                 const unsigned ib = (unsigned)((n_rows + 255) / 256);
                 const float* fb = f + (int64_t)b0 * ld_f;
-                if (nf == 16) k_interleave<16><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, fil);
-                else if (nf == 8) k_interleave<8><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, fil);
-                else k_interleave<4><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, fil);
+                if (nf > 8) k_interleave<16><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
+                else if (nf > 4) k_interleave<8><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
+                else k_interleave<4><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
                 DCPSE_LAUNCH_CHECK(ctx);
                 a.f = fil;
                 a.f_self = fil;
                 a.out[0] = out[0] + (int64_t)b0 * ld_out;
-                const bool ok = nf == 16 ? dispatch_il<MODE, 16>(a, sh.G, sh.epl, block, ctx->stream)
-                                : nf == 8 ? dispatch_il<MODE, 8>(a, sh.G, sh.epl, block, ctx->stream)
-                                          : dispatch_il<MODE, 4>(a, sh.G, sh.epl, block, ctx->stream);
+                const bool ok = nf > 8   ? dispatch_il<MODE, 16>(a, sh.G, sh.epl, nf, sh.mean, ctx->stream)
+                                : nf > 4 ? dispatch_il<MODE, 8>(a, sh.G, sh.epl, nf, sh.mean, ctx->stream)
+                                         : dispatch_il<MODE, 4>(a, sh.G, sh.epl, nf, sh.mean, ctx->stream);
                 if (!ok) return fail(ctx, DCPSE_ERR_UNSUPPORTED, "no batched apply kernel for group=%d x %d", sh.G,
                                      sh.epl);
                 DCPSE_LAUNCH_CHECK(ctx);

@@ -48,6 +48,7 @@ struct dcpse_ctx {
     int grp_g = 8;
     int grp_epl = 8;
     int grp_vec = 4;
+    double grp_mean = 0.0;
     int asm_wpb = 1;       // waves per block in the assembly kernel
     int asm_ppb = 18;      // particles per batch (one wavefront walks a batch)
     int asm_chunk = 64;    // neighbours staged per LDS round (32 or 64)

@@ -1,0 +1,47 @@
+"""Batched FP32 applies whose fields do not fill a pass and whose rows are
+shared by four or eight lanes: every batch size around the passes of 4, 8 and
+16 fields, bit for bit against one single-field pass per field.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# mean rows below 24, below 40, 40 to 56, 56 to 72 and above 72 (the launch
+# shapes), each with rows shorter and longer than a pass covers
+LENGTHS = {"short": (0, 40), "middle": (0, 70), "mean_48": (30, 67), "mean_64": (1, 128), "long": (70, 131)}
+
+
+@pytest.mark.parametrize("few", [True, False])
+@pytest.mark.parametrize("name", list(LENGTHS))
+def test_batch_parts(cuda, name, few):
+    from openfpm_numerics_amd import _lib
+
+    rng = np.random.default_rng(len(name))
+    n = 999 if few else 140_001  # eight lanes per row up to 131,072 rows
+    lens = rng.integers(*LENGTHS[name], n)
+    rp = torch.as_tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int64, device=cuda)
+    nnz = int(lens.sum())
+    col = torch.as_tensor(rng.integers(0, n, nnz), dtype=torch.int32, device=cuda)
+    W = torch.as_tensor(rng.standard_normal(nnz), dtype=torch.float32, device=cuda)
+    diag = torch.as_tensor(rng.standard_normal(n), dtype=torch.float32, device=cuda)
+    f = torch.as_tensor(rng.standard_normal((19, n)), dtype=torch.float32, device=cuda)
+    ctx, p = _lib.context(cuda.index or 0), _lib.ptr
+
+    def forward(nb, src, dst):
+        ctx.call("dcpse_apply_f32", n, p(rp), p(col), 1, _lib.ptr_array([W]), p(src), n, nb, None, n,
+                 _lib.ptr_array([dst]), n, 1.0, 0.5)
+
+    def transposed(nb, src, dst):
+        ctx.call("dcpse_apply_transpose_f32", n, p(rp), p(col), p(W), p(diag), p(src), n, nb, p(dst), n, 1.0, 0.5)
+
+    for run in (forward, transposed):
+        want = torch.ones_like(f)
+        for b in range(len(f)):
+            run(1, f[b], want[b])
+        for nb in ((2, 3, 4, 5, 7, 8, 9, 12, 13, 16, 17, 18, 19) if few else (3, 6, 13, 19)):
+            got = torch.ones_like(f)
+            run(nb, f, got)
+            assert torch.equal(got[:nb], want[:nb]), (run.__name__, nb)
+            assert bool((got[nb:] == 1).all()), (run.__name__, nb)  # fields beyond the batch are not written
