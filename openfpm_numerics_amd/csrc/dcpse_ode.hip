@@ -15,7 +15,7 @@
 //     stage 2: u2  = f + dt/2 k2      acc = acc + dt/3 k2      (u = u1)
 //     stage 3: u1  = f + dt   k3      acc = acc + dt/3 k3      (u = u2)
 //     stage 4:                        f   = acc + dt/6 k4      (u = u1)
-#include <algorithm>
+#include <type_traits>
 
 #include "dcpse_common.hpp"
 #include "dcpse_internal.hpp"
@@ -37,24 +37,42 @@ struct StageArgs {
     T ca, cb;
 };
 
-constexpr int kStageLanes = 8;  // lanes per CSR row
-
-// G lanes per row stride the row, then reduce; one operator, difference form.
-template <typename T, int G>
+// G lanes per row, U nonzeros each at a time; one operator, difference form.
+// Small sets are bound by the chain of dependent reads (row bounds, columns,
+// gathered values; 64 nonzeros go through it at once) and the launch.
+template <typename T, int G, int U>
 __global__ __launch_bounds__(256) void k_stage_csr(const StageArgs<T> a) {
     const int64_t row = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G;
     const int gl = threadIdx.x % G;
     if (row >= a.n_rows) return;  // whole G-lane groups leave together
-    const int64_t rs = a.row_ptr[row], re = a.row_ptr[row + 1];
+    const int64_t rs = a.row_ptr[row];
+    const int len = (int)(a.row_ptr[row + 1] - rs);
     const double up = a.u[row];
+    // before the gathers, so that the epilogue finds them (either may be the output)
+    const double ya = a.out_a ? (double)a.y_a[row] : 0.0;
+    const double yb = a.out_b ? (double)a.y_b[row] : 0.0;
     double acc = 0.0;  // FP64 accumulation for both value types
-    for (int64_t j = rs + gl; j < re; j += G) acc = fma((double)a.W[j], (double)a.u[a.col[j]] - up, acc);
+    for (int j0 = gl; j0 < len; j0 += G * U) {
+        int32_t q[U];
+        T w[U], uq[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const int64_t j = rs + min(j0 + G * k, len - 1);
+            q[k] = a.col[j];
+            w[k] = a.W[j];
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k) uq[k] = a.u[q[k]];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const double t = fma((double)w[k], (double)uq[k] - up, acc);
+            acc = j0 + G * k < len ? t : acc;
+        }
+    }
 #pragma unroll
     for (int off = G / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kWave);
     if (gl == 0) {
         const double k = (double)a.alpha * acc;
-        const double ya = a.out_a ? (double)a.y_a[row] : 0.0;
-        const double yb = a.out_b ? (double)a.y_b[row] : 0.0;
         if (a.out_a) a.out_a[row] = (T)fma((double)a.ca, k, ya);
         if (a.out_b) a.out_b[row] = (T)fma((double)a.cb, k, yb);
     }
@@ -71,9 +89,17 @@ static dcpse_status stage_csr(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row
     DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     if (n_rows == 0 || (!out_a && !out_b)) return DCPSE_OK;
     StageArgs<T> a{n_rows, row_ptr, col, W, u, alpha, y_a, y_b, out_a, out_b, ca, cb};
-    const int64_t rows_per_block = 256 / kStageLanes;
-    const int64_t blocks = (n_rows + rows_per_block - 1) / rows_per_block;
-    k_stage_csr<T, kStageLanes><<<(unsigned)blocks, 256, 0, ctx->stream>>>(a);
+    auto launch = [&](auto lanes, auto per) {
+        constexpr int G = decltype(lanes)::value;
+        const int64_t rows_per_block = 256 / G;
+        const int64_t blocks = (n_rows + rows_per_block - 1) / rows_per_block;
+        k_stage_csr<T, G, decltype(per)::value><<<(unsigned)blocks, 256, 0, ctx->stream>>>(a);
+    };
+    // us per stage (FP64) of 8 lanes one nonzero at a time / 8 lanes by 4 / 16
+    // by 4: 3,687 rows of 55 5.0 / 3.4 / 3.0, 14,000 5.4 / 3.9 / 3.9, 32,400 of
+    // 29 4.8 / 4.1 / 5.5, 236,000 of 56 45 / 29 / 29
+    if (n_rows <= 8192) launch(std::integral_constant<int, 16>(), std::integral_constant<int, 4>());
+    else launch(std::integral_constant<int, 8>(), std::integral_constant<int, 4>());
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
 }
