@@ -174,6 +174,8 @@ class Context:
         if st != DCPSE_OK:
             raise DcpseError(f"dcpse_ctx_create(device={device}) failed with status {st}")
         self.h = h
+        self._raw_stream = torch._C._cuda_getCurrentRawStream
+        self._set_stream = self.lib.dcpse_ctx_set_stream
 
     def __del__(self):
         h = getattr(self, "h", None)
@@ -185,10 +187,7 @@ class Context:
             self.h = None
 
     def bind_current_stream(self):
-        import torch
-
-        s = torch.cuda.current_stream(self.device)
-        self.lib.dcpse_ctx_set_stream(self.h, C.c_void_p(s.cuda_stream))
+        self._set_stream(self.h, self._raw_stream(self.device))
 
     def check(self, status: int, what: str):
         if status != DCPSE_OK:

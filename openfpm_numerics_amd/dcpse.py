@@ -19,6 +19,7 @@ sum_d D^{2 e_d} as one operator.
 """
 from __future__ import annotations
 
+import ctypes as C
 import math
 import os
 import struct
@@ -129,7 +130,7 @@ class Dcpse:
         self.info = None
         self._W = {}
         self._T = {}
-        self._n32 = {"fwd": 0, "adj": 0, "fwd64": 0}  # single-field applies since assembly
+        self._renew()
         self.update_ctr = particles.map_ctr
         if opt != LOAD:
             self.initializeStaticSize(self.particlesSupport, self.particlesDomain)
@@ -147,13 +148,13 @@ class Dcpse:
                              check: bool = True):
         assemble_together([self], particlesSupport, particlesDomain, check=check)
 
-    def _outputs(self, n_dom: int, dev):
+    def _outputs(self, n_dom: int, dev, info):
         nnz = self.verletList.nnz
         return (torch.empty(n_dom, dtype=torch.float64, device=dev), torch.empty(n_dom, dtype=torch.float64, device=dev),
                 torch.empty(max(nnz, 1), dtype=torch.float64, device=dev),
                 torch.empty(max(nnz, 1), dtype=torch.float32, device=dev),
                 None,  # FP64 pre-scaled weights: derived at the first FP64 use (weights)
-                torch.empty(n_dom, dtype=torch.int32, device=dev))
+                info)
 
     def _adopt(self, out, map_ctr):
         eps, eip, K64, W32, W64, info = out
@@ -162,9 +163,18 @@ class Dcpse:
         self.calcKernels = K64[:nnz]
         self._W = {torch.float32: W32[:nnz]}
         self._T = {}
-        self._n32 = {"fwd": 0, "adj": 0, "fwd64": 0}
+        self._renew()
         self.info = info
         self.update_ctr = map_ctr
+
+    def _renew(self):
+        """New kernels: nothing prepared from the old ones counts any more."""
+        self._n32 = {"fwd": 0, "adj": 0, "fwd64": 0}  # single-field applies since assembly
+        self._plans = {}  # apply plans (_SellPlan) by value type and the operators beside this one
+        self._gen = object()  # token of these kernels
+
+    def __getstate__(self):
+        return {**self.__dict__, "_plans": {}}  # a copy makes its own plans
 
     def check_info(self):
         """Raises like the reference on the first particle whose assembly failed."""
@@ -452,7 +462,7 @@ class Dcpse:
         W64 = self.calcKernels * self.localEpsInvPow[rows]
         self._W = {torch.float64: W64, torch.float32: W64.to(torch.float32)}
         self._T = {}
-        self._n32 = {"fwd": 0, "adj": 0, "fwd64": 0}
+        self._renew()
         self.info = torch.zeros(n, dtype=torch.int32, device=dev)
         self.update_ctr = self.particlesSupport.map_ctr
 
@@ -549,7 +559,8 @@ def assemble_together(ops, particlesSupport: ParticleSet | None = None, particle
     n_dom = dom.size_local()
     if vl.n_rows != n_dom:
         raise ValueError(f"Verlet list has {vl.n_rows} rows, domain has {n_dom} particles")
-    outs = [d._outputs(n_dom, dev) for d in ops]
+    infos = torch.empty((len(ops), n_dom), dtype=torch.int32, device=dev)
+    outs = [d._outputs(n_dom, dev, info) for d, info in zip(ops, infos)]
     if n_dom == 0:  # an empty domain: no rows to assemble
         for d, o in zip(ops, outs):
             d._adopt(o, sup.map_ctr)
@@ -570,9 +581,68 @@ def assemble_together(ops, particlesSupport: ParticleSet | None = None, particle
              arrays[0], arrays[1], arrays[2], arrays[3], arrays[4], arrays[5])
     for d, o in zip(ops, outs):
         d._adopt(o, sup.map_ctr)
-    if check:
+    if check and bool(infos.any()):  # one wait for every operator
         for d in ops:
             d.check_info()
+
+
+class _SellPlan:
+    """A single-field apply of operators of one list on their sliced-ELL layout:
+    the library function and its arguments up to the field, and the tensors
+    they point into. It counts as long as the kernels, the list and the module's
+    settings are those it was made from (tokens: an assembly, a load and a new
+    list bring new ones; the other operators' are part of its key)."""
+
+    def __init__(self, ops, vl, dtype, n_domain: bool):
+        p = _lib.ptr
+        t = "f32" if dtype == torch.float32 else "f64"
+        self.tokens = (vl._gen, ops[0]._gen)
+        self.max_exc = BUNDLE16_MAX_EXC
+        self.device = vl.row_ptr.device
+        self.ctx = _lib.context(self.device.index or 0)
+        self.n, self.n_rows = vl.n_cols, vl.n_rows
+        self.outs_type = C.c_void_p * len(ops)
+        self.domain = True  # the function takes the field on the domain
+        c16 = None
+        if len(ops) == 1 and ops[0].bundle16_suits():
+            # one operator: its 16-bit-offset bundle, built once per assembly
+            *keep, ne = ops[0].sell_bundle16(dtype)
+            slice_ptr = vl.sell_slices()[0]
+            bundle, row16, exc_ptr, exc_col, exc_W = keep
+            name, keep = "dcpse_apply_sell_bundle16_", [vl.row_ptr, slice_ptr, *keep]
+            args = (p(vl.row_ptr), p(slice_ptr), p(row16), 1, p(bundle), p(exc_ptr), p(exc_col), p(exc_W), ne)
+        else:
+            W = [op.sell_weights() if dtype == torch.float32 else op.sell_weights64() for op in ops]
+            c16 = None if n_domain else ops[0].col16()
+            self.W = _lib.ptr_array(W)
+            if c16 is not None:
+                name, keep, self.domain = "dcpse_apply_col16_", [vl.row_ptr, *c16[:-1], *W], False
+                args = (p(vl.row_ptr), *map(p, c16[:-1]), c16[-1], len(ops), self.W)
+            else:  # 32-bit columns
+                name, keep = "dcpse_apply_sell_", [vl.row_ptr, *vl.sell(), *W]
+                args = (*map(p, keep[:4]), len(ops), self.W)
+        self.name = name + t
+        self.keep = keep
+        self.fn = getattr(self.ctx.lib, self.name)
+        self.args = (self.ctx.h, self.n_rows, *args)
+
+    def counts_for(self, ops, vl) -> bool:
+        tokens = self.tokens
+        return (tokens[0] is vl._gen and self.max_exc == BUNDLE16_MAX_EXC
+                and ops[0]._gen is tokens[1])
+
+    def __call__(self, f, fd, outs, alpha, beta):
+        self.ctx.bind_current_stream()
+        o = self.outs_type(*[t.data_ptr() for t in outs])
+        if self.domain:
+            st = self.fn(*self.args, f.data_ptr(), fd, o, alpha, beta)
+        else:
+            st = self.fn(*self.args, f.data_ptr(), o, alpha, beta)
+        if st:
+            self.ctx.check(st, self.name)
+
+
+_FWD = {torch.float32: "fwd", torch.float64: "fwd64"}
 
 
 def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = None, alpha=1.0, beta=0.0):
@@ -587,11 +657,22 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
     for op in ops[1:]:
         if op.verletList is not vl:
             raise ValueError("fused operators must share one Verlet list")
-    if f.dtype not in (torch.float32, torch.float64):
+    if f.dtype not in _FWD:
         raise TypeError("fields must be float32 or float64")
     for op in ops:
         if op.update_ctr != op.particlesSupport.map_ctr:
             raise RuntimeError("particles moved since assembly: call update()/initializeUpdate() first")
+    # an apply like the one the first operator's plan was made for
+    key = (f.dtype, *[op._gen for op in ops[1:]])
+    plan = ops[0]._plans.get(key)
+    if (plan is not None and outs is None and f_domain is None and USE_SELL and type(f) is torch.Tensor
+            and f.dim() == 1 and f.is_contiguous() and f.shape[0] == plan.n and f.device == plan.device
+            and plan.counts_for(ops, vl) and all([op._n32[_FWD[f.dtype]] + 1 >= SELL_AFTER for op in ops])):
+        for op in ops:
+            op._n32[_FWD[f.dtype]] += 1
+        outs = [torch.empty_like(f) for _ in ops]
+        plan(f, None, outs, alpha, beta)
+        return outs
     f2 = _batch2d(f).contiguous()
     nb, n = f2.shape
     if n != vl.n_cols:
@@ -612,50 +693,13 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
     if n_rows == 0:  # an empty domain: nothing to compute
         return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
     ctx = _lib.context(f.device.index or 0)
-    use_sell = False
-    if f.dtype == torch.float32 and nb == 1 and USE_SELL:
-        use_sell = all([op._count_apply32("fwd") for op in ops])
-    if use_sell and len(ops) == 1 and ops[0].bundle16_suits():
-        # one operator: its 16-bit-offset bundle, built once per assembly
-        slice_ptr = vl.sell_slices()[0]
-        bundle, row16, exc_ptr, exc_col, exc_W, ne = ops[0].sell_bundle16()
-        ctx.call("dcpse_apply_sell_bundle16_f32", n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr), _lib.ptr(row16),
-                 1, _lib.ptr(bundle), _lib.ptr(exc_ptr), _lib.ptr(exc_col), _lib.ptr(exc_W), ne, _lib.ptr(f2),
-                 _lib.ptr(fd), _lib.ptr_array(outs), alpha, beta)
-        return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
-    c16 = ops[0].col16() if use_sell and fd is None else None
-    if c16 is not None:
-        SW = [op.sell_weights() for op in ops]
-        ctx.call("dcpse_apply_col16_f32", n_rows, _lib.ptr(vl.row_ptr), *map(_lib.ptr, c16[:-1]), c16[-1], len(ops),
-                 _lib.ptr_array(SW), _lib.ptr(f2), _lib.ptr_array(outs), alpha, beta)
-        return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
-    if use_sell:
-        slice_ptr, sell_row, sell_col = vl.sell()
-        SW = [op.sell_weights() for op in ops]
-        ctx.call("dcpse_apply_sell_f32", n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr), _lib.ptr(sell_row),
-                 _lib.ptr(sell_col), len(ops), _lib.ptr_array(SW), _lib.ptr(f2), _lib.ptr(fd), _lib.ptr_array(outs), alpha, beta)
-        return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
-    if f.dtype == torch.float64 and nb == 1 and USE_SELL and all([op._count_apply32("fwd64") for op in ops]):
-        if len(ops) == 1 and ops[0].bundle16_suits():
-            # one operator: its FP64 16-bit-offset bundle (18 bytes per neighbour)
-            slice_ptr = vl.sell_slices()[0]
-            bundle, row16, exc_ptr, exc_col, exc_W, ne = ops[0].sell_bundle16(torch.float64)
-            ctx.call("dcpse_apply_sell_bundle16_f64", n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr),
-                     _lib.ptr(row16), 1, _lib.ptr(bundle), _lib.ptr(exc_ptr), _lib.ptr(exc_col), _lib.ptr(exc_W), ne,
-                     _lib.ptr(f2), _lib.ptr(fd), _lib.ptr_array(outs), alpha, beta)
-            return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
-        c16 = ops[0].col16() if fd is None else None
-        if c16 is not None:
-            SW = [op.sell_weights64() for op in ops]
-            ctx.call("dcpse_apply_col16_f64", n_rows, _lib.ptr(vl.row_ptr), *map(_lib.ptr, c16[:-1]), c16[-1],
-                     len(ops), _lib.ptr_array(SW), _lib.ptr(f2), _lib.ptr_array(outs), alpha, beta)
-            return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
-        # FP64: the 32-bit-column layout with FP64 weights in its slot order
-        slice_ptr, sell_row, sell_col = vl.sell()
-        SW = [op.sell_weights64() for op in ops]
-        ctx.call("dcpse_apply_sell_f64", n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr), _lib.ptr(sell_row),
-                 _lib.ptr(sell_col), len(ops), _lib.ptr_array(SW), _lib.ptr(f2), _lib.ptr(fd), _lib.ptr_array(outs),
-                 alpha, beta)
+    if nb == 1 and USE_SELL and all([op._count_apply32(_FWD[f.dtype]) for op in ops]):
+        plan = _SellPlan(ops, vl, f.dtype, fd is not None)
+        if fd is None and ops[0].same_set:
+            if len(ops[0]._plans) >= 8:
+                ops[0]._plans.clear()
+            ops[0]._plans[key] = plan
+        plan(f2, _lib.ptr(fd), outs, alpha, beta)
         return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
     W = [op.weights(f.dtype) for op in ops]
     name = "dcpse_apply_f32" if f.dtype == torch.float32 else "dcpse_apply_f64"

@@ -194,6 +194,7 @@ class VerletList:
         self._slices = None
         self._far16 = None
         self._col16 = None
+        self._gen = object()  # token of these neighbours
         self.map_ctr = -1
 
     @property
