@@ -1587,6 +1587,16 @@ int32_t dcpse_rhs(int32_t dim, const uint32_t* beta, uint32_t order, double* b, 
     return B.m;
 }
 
+// Particles per wavefront. The chip holds about 2048 wavefronts of the large
+// kernels: few particles go to as many of them as there are groups of three,
+// which are factored together; more share a wavefront to spread its start-up
+// and the first neighbours' latency. us with 3 / 6 / 12 / 18 per wavefront:
+// Laplacian + d/dx in 3D of 3,687 particles 39 / 40 / 56 / 78, 14,000 55 / 64 /
+// 74 / 85, 45,600 138 / 144 / 146 / 174, 126,800 363 / 361 / 372 / 363, 380,000
+// 1071 / 1042 / 1026 / 1032; the Laplacian in 2D of 6,226 27 / 28 / 36 / 51,
+// 59,000 96 / 87 / 90 / 112, 472,000 671 / 595 / 588 / 594.
+static int default_ppb(int64_t n) { return n <= 16384 ? 3 : n <= 131072 ? 6 : n <= 524288 ? 12 : 18; }
+
 static dcpse_status assemble_ops(dcpse_ctx* ctx, int32_t dim, const double* pos_sup, int64_t n_sup,
                                  const double* pos_dom, int64_t n_dom, const double* box_lo, const double* box_hi,
                                  uint32_t periodic_mask, const int64_t* row_ptr, const int32_t* col, int32_t n_ops,
@@ -1650,7 +1660,9 @@ static dcpse_status assemble_ops(dcpse_ctx* ctx, int32_t dim, const double* pos_
     args.refine = (flags & DCPSE_ASM_REFINE) ? 1 : 0;
     // one lane per particle of a batch; the static grid also reads the row
     // start of the particle after the last from lane ppb, so at most 63
-    args.ppb = std::min(ctx->asm_persistent ? 64 : 63, std::max(1, ctx->asm_ppb));
+    args.ppb = std::min(ctx->asm_persistent ? 64 : 63, ctx->asm_ppb > 0      ? ctx->asm_ppb
+                                                            : ctx->asm_persistent ? 18
+                                                                                  : default_ppb(n_dom));
     if (n_dom == 0) return DCPSE_OK;
     args.n_batches = (n_dom + args.ppb - 1) / args.ppb;
     const int ch = ctx->asm_chunk;
