@@ -71,12 +71,30 @@ __global__ __launch_bounds__(1024) void k_scan_tilesums(int64_t* tsum, int64_t n
     if (threadIdx.x == 0) tsum[nt] = carry;
 }
 
-__global__ __launch_bounds__(kScanBlock) void k_scan_tiles(const int32_t* __restrict__ in, int64_t n,
-                                                           const int64_t* __restrict__ tsum,
-                                                           int64_t* __restrict__ out, int64_t* host,
-                                                           const int32_t* extra0, const int32_t* extra1) {
-    __shared__ long long buf[kScanBlock];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
+// Sum over the block of one value per thread, in every thread.
+template <int BLOCK>
+__device__ __forceinline__ long long block_sum(long long v) {
+    __shared__ long long red[BLOCK / kWave];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    long long t = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / kWave; ++w) t += red[w];
+    __syncthreads();
+    return t;
+}
+
+// One tile per block. tsum: the tiles' sums (scanned: their exclusive scan),
+// or null where there is one tile.
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_scan_tiles(const int32_t* __restrict__ in, int64_t n,
+                                                      const int64_t* __restrict__ tsum, bool scanned,
+                                                      int64_t* __restrict__ out, int64_t* host,
+                                                      const int32_t* extra0, const int32_t* extra1) {
+    __shared__ long long wsum[BLOCK / kWave];
+    const int64_t base = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) * kScanItems;
     long long v[kScanItems];
     long long tot = 0;
 #pragma unroll
@@ -85,15 +103,29 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_tiles(const int32_t* __rest
         v[i] = k < n ? in[k] : 0;
         tot += v[i];
     }
-    buf[threadIdx.x] = tot;
-    __syncthreads();
-    for (int off = 1; off < kScanBlock; off <<= 1) {
-        long long t = threadIdx.x >= (unsigned)off ? buf[threadIdx.x - off] : 0;
-        __syncthreads();
-        buf[threadIdx.x] += t;
-        __syncthreads();
+    long long before = 0;
+    if (scanned) {
+        before = tsum[blockIdx.x];
+    } else if (tsum) {
+        for (int64_t i = threadIdx.x; i < (int64_t)blockIdx.x; i += BLOCK) before += tsum[i];
+        before = block_sum<BLOCK>(before);
     }
-    long long run = tsum[blockIdx.x] + buf[threadIdx.x] - tot;
+    // inclusive over the wavefront, then the wavefronts before this one
+    long long incl = tot;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const long long t = __shfl_up(incl, off, kWave);
+        if ((int)(threadIdx.x & 63) >= off) incl += t;
+    }
+    if ((threadIdx.x & 63) == 63) wsum[threadIdx.x >> 6] = incl;
+    __syncthreads();
+    long long all = before;
+#pragma unroll
+    for (int w = 0; w < BLOCK / kWave; ++w) {
+        if (w < (int)(threadIdx.x >> 6)) before += wsum[w];
+        all += wsum[w];
+    }
+    long long run = before + incl - tot;
 #pragma unroll
     for (int i = 0; i < kScanItems; ++i) {
         int64_t k = base + i;
@@ -101,9 +133,9 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_tiles(const int32_t* __rest
         run += v[i];
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
-        out[n] = tsum[gridDim.x];
+        out[n] = all;
         if (host) {
-            host[0] = tsum[gridDim.x];
+            host[0] = all;
             if (extra0) host[1] = *extra0;
             if (extra1) host[2] = *extra1;
             __threadfence_system();
@@ -123,16 +155,28 @@ size_t scan_workspace_bytes(int64_t n) {
 
 dcpse_status scan_counts(dcpse_ctx* ctx, const int32_t* in, int64_t n, int64_t* out, Workspace* w, bool to_host,
                          const int32_t* extra0, const int32_t* extra1) {
-    int64_t nt = (n + kScanTile - 1) / kScanTile;
-    if (nt == 0) nt = 1;
+    int64_t* host = to_host ? ctx->host : nullptr;
+    // one launch up to a block of 1024 threads; then the tiles' sums first, each
+    // block adding up those before its own (4.8 us a launch: lists of 2,500
+    // particles ran six of these kernels, now two or three), scanned by a
+    // kernel of their own where that would be long
+    if (n <= 1024 * kScanItems) {
+        k_scan_tiles<1024><<<1, 1024, 0, ctx->stream>>>(in, n, nullptr, false, out, host, extra0, extra1);
+        DCPSE_LAUNCH_CHECK(ctx);
+        return DCPSE_OK;
+    }
+    const int64_t nt = (n + kScanTile - 1) / kScanTile;
     int64_t* tsum = w->take<int64_t>((size_t)nt + 1);
     if (!tsum) return fail(ctx, DCPSE_ERR_INVALID, "scan: workspace too small");
     k_scan_tilesum<<<(unsigned)nt, kScanBlock, 0, ctx->stream>>>(in, n, tsum);
     DCPSE_LAUNCH_CHECK(ctx);
-    k_scan_tilesums<<<1, 1024, 0, ctx->stream>>>(tsum, nt);
-    DCPSE_LAUNCH_CHECK(ctx);
-    k_scan_tiles<<<(unsigned)nt, kScanBlock, 0, ctx->stream>>>(in, n, tsum, out, to_host ? ctx->host : nullptr, extra0,
-                                                               extra1);
+    const bool scanned = nt > 4096;
+    if (scanned) {
+        k_scan_tilesums<<<1, 1024, 0, ctx->stream>>>(tsum, nt);
+        DCPSE_LAUNCH_CHECK(ctx);
+    }
+    k_scan_tiles<kScanBlock><<<(unsigned)nt, kScanBlock, 0, ctx->stream>>>(in, n, tsum, scanned, out, host, extra0,
+                                                                          extra1);
     DCPSE_LAUNCH_CHECK(ctx);
     return DCPSE_OK;
 }
@@ -147,6 +191,18 @@ void fill_i32(hipStream_t s, int32_t* p, int64_t n, int32_t v) {
     if (n <= 0) return;
     int64_t blocks = std::min<int64_t>((n + 255) / 256, 65536);
     k_fill_i32<<<(unsigned)blocks, 256, 0, s>>>(p, n, v);
+}
+
+// Zeroes up to four ranges in one launch.
+struct ClearRanges {
+    int32_t* p[4];
+    int64_t n[4];
+};
+__global__ void k_clear(const ClearRanges r) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < r.n[k]; i += (int64_t)gridDim.x * blockDim.x)
+            r.p[k][i] = 0;
 }
 
 __global__ void k_fill_i64(int64_t* p, int64_t n, int64_t v) {
@@ -1528,7 +1584,6 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
     const Workspace ws_scan = w;
     if (!flags) return fail(ctx, DCPSE_ERR_INVALID, "workspace sizing error");
 
-    fill_i32(s, flags, 64, 0);
     auto blocks_for = [](int64_t n) {
         return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 16384));
     };
@@ -1536,9 +1591,12 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
         Workspace ws = ws_scan;
         return scan_counts(ctx, in, n, out, &ws);
     };
+    const ClearRanges zero = {{flags, cell_cnt, home_cnt, spill},
+                              {64, cached ? 0 : g.ncell + 1, home_on && !cached ? n_home + 1 : 0,
+                               count_pass && groups_on ? 1 : 0}};
+    k_clear<<<blocks_for(std::max<int64_t>(64, cached ? 0 : std::max(g.ncell, home_on ? n_home : 0))), 256, 0, s>>>(zero);
+    DCPSE_LAUNCH_CHECK(ctx);
     if (!cached) {
-        fill_i32(s, cell_cnt, g.ncell + 1, 0);
-        if (home_on) fill_i32(s, home_cnt, n_home + 1, 0);
         const unsigned tb = blocks_for(n_sup);
         auto cells = [&](auto D, auto H) {
             constexpr int DIM = decltype(D)::value;
@@ -1602,7 +1660,6 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
     if (count_pass) {
         if (groups_on) {
             // candidate lists and masks, then the particles they do not cover
-            fill_i32(s, spill, 1, 0);
             launch_groups(dim, nws, [&](auto D, auto R) {
                 constexpr int DIM = decltype(D)::value, RM = decltype(R)::value;
                 if (pp) k_group_pairs<DIM, RM, true><<<group_blocks, kPairWaves * kWave, 0, s>>>(a, home);
