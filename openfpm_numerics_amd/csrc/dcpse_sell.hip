@@ -198,7 +198,7 @@ __device__ __forceinline__ int64_t col_offset(int32_t q, int32_t p, int64_t n) {
 __device__ __forceinline__ bool far16(int64_t d) { return d > 32767 || d < -32768; }
 
 // exc_count[i] = far neighbours of the row of lane i: a wavefront takes 16
-// lanes' rows, two at a time, 32 entries of each per load.
+// lanes' rows, 32 entries of two of them per load, eight loads at once.
 __global__ __launch_bounds__(256) void k_bundle16_count(int64_t n_rows, const int64_t* __restrict__ row_ptr,
                                                         const int32_t* __restrict__ col,
                                                         const int32_t* __restrict__ sell_row,
@@ -206,15 +206,32 @@ __global__ __launch_bounds__(256) void k_bundle16_count(int64_t n_rows, const in
     const int64_t n_slices = (n_rows + 63) / 64;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, half = lane >> 5, e = lane & 31;
     for (int64_t s = blockIdx.x; s < n_slices; s += gridDim.x) {
+        // lanes 0 .. 15: the rows' bounds, handed round
+        const SliceLane mine = slice_lane(row_ptr, sell_row, s * 64 + 16 * wv + (lane & 15));
+        int mx = mine.len;
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) mx = max(mx, __shfl_xor(mx, off, kWave));
+        int32_t row[8], len[8], c[8];
+        int64_t rs[8];
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
-            const int64_t i = s * 64 + 16 * wv + 2 * it + half;
-            const SliceLane r = slice_lane(row_ptr, sell_row, i);
-            int c = 0;
-            for (int j = e; j < r.len; j += 32) c += far16(col_offset(col[r.rs + j], r.row, n_rows));
+            row[it] = __shfl(mine.row, 2 * it + half, kWave);
+            rs[it] = __shfl(mine.rs, 2 * it + half, kWave);
+            len[it] = __shfl(mine.len, 2 * it + half, kWave);
+            c[it] = 0;
+        }
+        for (int j = e; j < mx; j += 32) {
+            int32_t q[8];
 #pragma unroll
-            for (int off = 16; off > 0; off >>= 1) c += __shfl_xor(c, off, kWave);
-            if (e == 0) exc_count[i] = c;
+            for (int it = 0; it < 8; ++it) q[it] = j < len[it] ? col[rs[it] + j] : row[it];
+#pragma unroll
+            for (int it = 0; it < 8; ++it) c[it] += far16(col_offset(q[it], row[it], n_rows));
+        }
+#pragma unroll
+        for (int it = 0; it < 8; ++it) {
+#pragma unroll
+            for (int off = 16; off > 0; off >>= 1) c[it] += __shfl_xor(c[it], off, kWave);
+            if (e == 0) exc_count[s * 64 + 16 * wv + 2 * it + half] = c[it];
         }
     }
 }
@@ -258,21 +275,26 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16(
             // load: wave w takes lanes 16 w .. 16 w + 15, two rows at a time
             const int e = tid & 31;
             const int j = 4 * g0 + e;
+            int32_t q[8];
+            float w[8];
+            bool in[8];
+#pragma unroll
             for (int it = 0; it < 8; ++it) {
                 const int ll = 16 * gsub + 2 * it + ((tid >> 5) & 1);
-                const int len = slen[ll];
-                const int64_t rs = srs[ll];
-                int32_t d = 0;
-                bool in = j < len;
-                if (in) {
-                    const int64_t dj = col_offset(col[rs + j], srow[ll], n_rows);
-                    in = !far16(dj);
-                    d = in ? (int32_t)dj : 0;
-                }
-                tc[e * kTilePitch + ll] = d;
+                in[it] = j < slen[ll];
+                q[it] = in[it] ? col[srs[ll] + j] : 0;
+                w[it] = in[it] ? W0[srs[ll] + j] : 0.0f;
+            }
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                const int ll = 16 * gsub + 2 * it + ((tid >> 5) & 1);
+                const int64_t dj = col_offset(q[it], srow[ll], n_rows);
+                in[it] = in[it] && !far16(dj);
+                tc[e * kTilePitch + ll] = in[it] ? (int32_t)dj : 0;
                 // a far neighbour's slot has no weight: the transposed apply adds
                 // W g_q without the difference that would cancel it
-                for (int o = 0; o < n_ops; ++o) tw[o][e * kTilePitch + ll] = in ? W[o][rs + j] : 0.0f;
+                tw[0][e * kTilePitch + ll] = in[it] ? w[it] : 0.0f;
+                for (int o = 1; o < n_ops; ++o) tw[o][e * kTilePitch + ll] = in[it] ? W[o][srs[ll] + j] : 0.0f;
             }
             __syncthreads();
             // write: thread (lane l, gsub) writes the tile's groups gsub, gsub + 4
@@ -343,6 +365,7 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16_f64(
     const int64_t* __restrict__ exc_ptr, int32_t* __restrict__ bundle, int32_t* __restrict__ sell_row16) {
     __shared__ int32_t tc[kTileSlots * kTilePitch];  // column offsets
     __shared__ double tw[kTileSlots * kTilePitch];   // one operator's weights
+    __shared__ double sscale[4][64];
     __shared__ int32_t srow[64];
     __shared__ int64_t srs[64];
     __shared__ int32_t slen[64];
@@ -359,6 +382,8 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16_f64(
             srow[tid] = r.row;
             srs[tid] = r.rs;
             slen[tid] = r.len;
+            for (int o = 0; o < n_ops; ++o)
+                sscale[o][tid] = W.scale[o] && r.row >= 0 ? W.scale[o][r.row] : 0.0;
             sell_row16[i] = r.row < 0 ? r.row : (exc_ptr[i + 1] > exc_ptr[i] ? (r.row | kExcFlag) : r.row);
         }
         __syncthreads();
@@ -367,37 +392,39 @@ __global__ __launch_bounds__(256) void k_sell_fill_bundle16_f64(
         for (int g0 = 0; g0 < ng; g0 += kTileSlots / 4) {
             const int j = 4 * g0 + e;
             const int gn = min(kTileSlots / 4, ng - g0);
-            for (int o = -1; o < n_ops; ++o) {  // -1: the column offsets
+            for (int o = 0; o < n_ops; ++o) {  // the column offsets with the first operator's weights
                 // load: wave w takes lanes 16 w .. 16 w + 15, two rows at a time
+                int32_t q[8];
+                double w[8];
+#pragma unroll
                 for (int it = 0; it < 8; ++it) {
                     const int ll = 16 * gsub + 2 * it + ((tid >> 5) & 1);
-                    const int len = slen[ll];
-                    const int64_t rs = srs[ll];
-                    if (o < 0) {
-                        int32_t d = 0;
-                        if (j < len) {
-                            const int64_t dj = col_offset(col[rs + j], srow[ll], n_rows);
-                            d = far16(dj) ? 0 : (int32_t)dj;
-                        }
-                        tc[e * kTilePitch + ll] = d;
-                    } else {
-                        tw[e * kTilePitch + ll] = j < len ? W.at(o, rs + j, srow[ll]) : 0.0;
+                    const bool in = j < slen[ll];
+                    if (o == 0) q[it] = in ? col[srs[ll] + j] : srow[ll];
+                    w[it] = in ? W.W[o][srs[ll] + j] : 0.0;
+                }
+#pragma unroll
+                for (int it = 0; it < 8; ++it) {
+                    const int ll = 16 * gsub + 2 * it + ((tid >> 5) & 1);
+                    if (o == 0) {
+                        const int64_t dj = col_offset(q[it], srow[ll], n_rows);
+                        tc[e * kTilePitch + ll] = far16(dj) ? 0 : (int32_t)dj;
                     }
+                    tw[e * kTilePitch + ll] = W.scale[o] ? sscale[o][ll] * w[it] : w[it];
                 }
                 __syncthreads();
                 // write: thread (lane l, gsub) writes the tile's groups gsub, gsub + 4
                 for (int gl = gsub; gl < gn; gl += 4) {
                     const int64_t gb = (base / 256 + g0 + gl) * blk;  // word offset of the slot group's block
-                    if (o < 0) {
+                    if (o == 0) {
                         vs4a dv;
 #pragma unroll
                         for (int jj = 0; jj < 4; ++jj) dv[jj] = (int16_t)tc[(4 * gl + jj) * kTilePitch + l];
                         *reinterpret_cast<vs4a*>(cols16 + 2 * gb + 4 * l) = dv;
-                    } else {
-                        double2* wb = reinterpret_cast<double2*>(bundle + gb + 128 + o * 512) + 2 * l;
-                        wb[0] = make_double2(tw[(4 * gl) * kTilePitch + l], tw[(4 * gl + 1) * kTilePitch + l]);
-                        wb[1] = make_double2(tw[(4 * gl + 2) * kTilePitch + l], tw[(4 * gl + 3) * kTilePitch + l]);
                     }
+                    double2* wb = reinterpret_cast<double2*>(bundle + gb + 128 + o * 512) + 2 * l;
+                    wb[0] = make_double2(tw[(4 * gl) * kTilePitch + l], tw[(4 * gl + 1) * kTilePitch + l]);
+                    wb[1] = make_double2(tw[(4 * gl + 2) * kTilePitch + l], tw[(4 * gl + 3) * kTilePitch + l]);
                 }
                 __syncthreads();
             }
@@ -451,11 +478,16 @@ __global__ __launch_bounds__(256) void k_sell_fill_col16(int64_t n_rows, const i
         int far = 0;
         for (int g0 = 0; g0 < ng; g0 += kTileSlots / 4) {
             const int j = 4 * g0 + e;
+            int32_t q[8];
+#pragma unroll
             for (int it = 0; it < 8; ++it) {
                 const int ll = 16 * gsub + 2 * it + ((tid >> 5) & 1);
-                int32_t d = 0;
-                if (j < slen[ll]) d = (int32_t)col_offset(col[srs[ll] + j], srow[ll], n_rows);
-                tc[e * kTilePitch + ll] = d;
+                q[it] = j < slen[ll] ? col[srs[ll] + j] : srow[ll];
+            }
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                const int ll = 16 * gsub + 2 * it + ((tid >> 5) & 1);
+                tc[e * kTilePitch + ll] = (int32_t)col_offset(q[it], srow[ll], n_rows);
             }
             __syncthreads();
             const int gn = min(kTileSlots / 4, ng - g0);
