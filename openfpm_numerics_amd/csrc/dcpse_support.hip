@@ -840,7 +840,9 @@ struct PairGroup {
 // cut-offs, so wherever a pair is within the cut-off these images are the ones
 // its minimum image takes.
 __device__ __forceinline__ float relative(const PairGroup& pg, const CellGrid& g, double x, int d) {
-    return (float)(min_image_r(x - pg.ctr[d], g.len[d], g.ilen[d], (g.periodic >> d) & 1u) * pg.iunit);
+    // an open dimension has period 0: no select per lane
+    const bool wraps = (g.periodic >> d) & 1u;
+    return (float)(min_image_r(x - pg.ctr[d], wraps ? g.len[d] : 0.0, wraps ? g.ilen[d] : 0.0, true) * pg.iunit);
 }
 
 // Sorts the group's pg.total <= R * 64 candidate indices (in the wave's LDS
@@ -907,6 +909,7 @@ __device__ __forceinline__ void pair_tests(const Groups& a, const PairGroup& pg,
                 int nacc = 0;
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
+                    if (r > R / 2 && r >= nw) break;  // the last words are often empty
                     float d2 = 0.0f;
 #pragma unroll
                     for (int d = 0; d < DIM; ++d) {
@@ -1019,12 +1022,15 @@ __global__ __launch_bounds__(kPairWaves * kWave) void k_group_pairs(const Groups
     }
     int nacc = 0;
     // keeps those of four candidates per lane that are within reach of the box
-    auto take4 = [&](const int64_t (&slot)[4], const bool (&have)[4]) {
+    // (left of them: the last ones past the end of a list are skipped)
+    auto take4 = [&](const int64_t (&slot)[4], const bool (&have)[4], int left) {
         CellRec r[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = a.rec[slot[j]];
+        for (int j = 0; j < 4; ++j)
+            if (j * kWave < left) r[j] = a.rec[slot[j]];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+            if (j * kWave >= left) break;
             float d2 = 0.0f;  // squared distance to the box
 #pragma unroll
             for (int d = 0; d < DIM; ++d) {
@@ -1141,7 +1147,7 @@ __global__ __launch_bounds__(kPairWaves * kWave) void k_group_pairs(const Groups
                         const int dl = __builtin_amdgcn_ds_bpermute(seg << 2, delta);
                         slot[j] = have[j] ? k + dl : 0;
                     }
-                    take4(slot, have);
+                    take4(slot, have, total - base);
                 }
             }
         } else {
@@ -1170,7 +1176,7 @@ __global__ __launch_bounds__(kPairWaves * kWave) void k_group_pairs(const Groups
                     have[j] = k < total;
                     slot[j] = have[j] ? k + off[j] : 0;
                 }
-                take4(slot, have);
+                take4(slot, have, total - base);
             }
         }
         spilled = nacc > a.nws * kWave || __ballot(wild) != 0;
