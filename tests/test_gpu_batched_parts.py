@@ -45,3 +45,43 @@ def test_batch_parts(cuda, name, few):
             run(nb, f, got)
             assert torch.equal(got[:nb], want[:nb]), (run.__name__, nb)
             assert bool((got[nb:] == 1).all()), (run.__name__, nb)  # fields beyond the batch are not written
+
+
+@pytest.mark.parametrize("few", [True, False])
+@pytest.mark.parametrize("name", ["short", "mean_64", "long"])
+def test_fp64_batches(cuda, name, few):
+    """FP64 batches against FP64 single fields: the same terms in another order."""
+    from openfpm_numerics_amd import _lib
+
+    rng = np.random.default_rng(7 + few)
+    n = 999 if few else 40_003
+    lens = rng.integers(*LENGTHS[name], n)
+    lens[[0, n // 2, n - 1]] = 0
+    rp = torch.as_tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int64, device=cuda)
+    nnz = int(lens.sum())
+    col = torch.as_tensor(rng.integers(0, n, nnz), dtype=torch.int32, device=cuda)
+    W = torch.as_tensor(rng.standard_normal(nnz), device=cuda)
+    diag = torch.as_tensor(rng.standard_normal(n), device=cuda)
+    f = torch.as_tensor(rng.standard_normal((19, n)), device=cuda)
+    ctx, p = _lib.context(cuda.index or 0), _lib.ptr
+    # |terms| of a row: at most sum |W| (|f_q| + |f_p|) + |diag| |f|, two orders differ by a few ulp of that
+    mag = torch.zeros(n, dtype=torch.float64, device=cuda).index_add_(
+        0, torch.repeat_interleave(torch.arange(n, device=cuda), rp[1:] - rp[:-1]), W.abs())
+    bound = 140 * 2.0 ** -52 * (2 * mag + diag.abs() + 1) * float(f.abs().max())
+
+    def forward(nb, src, dst):
+        ctx.call("dcpse_apply_f64", n, p(rp), p(col), 1, _lib.ptr_array([W]), p(src), n, nb, None, n,
+                 _lib.ptr_array([dst]), n, 0.75, 0.5)
+
+    def transposed(nb, src, dst):
+        ctx.call("dcpse_apply_transpose_f64", n, p(rp), p(col), p(W), p(diag), p(src), n, nb, p(dst), n, 0.75, 0.5)
+
+    for run in (forward, transposed):
+        want = torch.ones_like(f)
+        for b in range(len(f)):
+            run(1, f[b], want[b])
+        for nb in (2, 3, 4, 5, 8, 9, 16, 17, 19):
+            got = torch.ones_like(f)
+            run(nb, f, got)
+            assert bool(((got[:nb] - want[:nb]).abs() <= bound).all()), (run.__name__, nb)
+            assert bool((got[nb:] == 1).all()), (run.__name__, nb)
