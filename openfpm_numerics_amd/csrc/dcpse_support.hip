@@ -293,6 +293,23 @@ struct HomeLevels {
     int32_t first[kMaxLevels + 1];
 };
 
+// cnt[c] += 1, returning the place taken: lanes side by side with the same c
+// (particles next to each other in memory mostly share a cell) take theirs with
+// one atomic. Called by the first `active` lanes of the wavefront.
+__device__ __forceinline__ int32_t take_place(int32_t* cnt, int32_t c, int active) {
+    const int lane = threadIdx.x & 63;
+    const int prev = __shfl_up(c, 1, kWave);
+    const bool head = lane == 0 || prev != c;
+    const unsigned long long heads = __ballot(head);
+    const unsigned long long upto = (2ull << lane) - 1;
+    const int first = 63 - __builtin_clzll(heads & upto);
+    const unsigned long long after = heads & ~upto;
+    const int end = after ? __builtin_ctzll(after) : active;
+    int32_t base = 0;
+    if (head) base = atomicAdd(&cnt[c], end - lane);
+    return __shfl(base, first, kWave) + lane - first;
+}
+
 // cell of every particle and its place within it (the order within a cell is
 // whatever the atomics give; nothing that leaves the builder depends on it).
 template <int DIM, bool HOME>
@@ -307,7 +324,8 @@ __global__ void k_cell_assign(const double* __restrict__ pos, int64_t n, const d
         for (int d = 0; d < DIM; ++d) x[d] = pos[d * n + q];
         const int32_t c = cell_index<DIM>(x, g);
         cell_id[q] = c;
-        rank[q] = atomicAdd(&cell_cnt[c], 1);
+        const int active = (int)min((int64_t)kWave, n - (q - (threadIdx.x & 63)));
+        rank[q] = take_place(cell_cnt, c, active);
         if constexpr (HOME) {
             const double r = rcut[q];
             int l = 0;
@@ -321,7 +339,7 @@ __global__ void k_cell_assign(const double* __restrict__ pos, int64_t n, const d
             for (int i = 0; i < kMaxLevels; ++i)
                 if (i == l) k = h.first[i] + cell_index<DIM>(x, h.g[i]);
             home_id[q] = k;
-            home_rank[q] = atomicAdd(&home_cnt[k], 1);
+            home_rank[q] = take_place(home_cnt, k, active);
         }
     }
 }
