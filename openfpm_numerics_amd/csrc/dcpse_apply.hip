@@ -512,12 +512,17 @@ static void launch_apply_il(const ApplyArgs<float>& a, int nf, double mean, hipS
 
 // FP64 batches: eight lanes per row, NF / 2 of them side by side with two
 // fields each (one 16-byte load per lane, a neighbour's NF values in one line),
-// the row's nonzeros dealt to the 16 / NF parts, four at a time. (us per apply,
-// 4 fields at a time field-major / so: 262,000 rows of 29 B4 53 / 33, B16
-// 207 / 92; 729,000 of 93 B4 321 / 319, B16 1287 / 920.)
-template <int NF, int MODE>
+// the row's nonzeros dealt to the H = 16 / NF parts. Nonzero j belongs to
+// partial sum j % G, as in k_apply<double, G, EPL> whose lanes' exchanges add
+// them up: part h holds the sums h, h + H, ..., so every field equals the
+// single-field CSR kernel bit for bit. (us per apply, 4 fields at a time
+// field-major / so: 262,000 rows of 29 B4 53 / 33, B16 207 / 92; 729,000 of 93
+// B4 321 / 319, B16 1287 / 920.)
+template <int NF, int G, int MODE>
 __global__ __launch_bounds__(kBatchBlock) void k_apply_batch64(const ApplyArgs<double> a, int nf) {
-    constexpr int L = NF / 2, H = 8 / L, U = 4;
+    constexpr int L = NF / 2, H = 8 / L, S = G / H, U = S < 4 ? 4 : S < 8 ? S : 8;
+    static_assert(S % U == 0 || U % S == 0, "a step takes whole turns of the partial sums");
+    constexpr int STEP = S > U ? S : U;  // of the part's nonzeros
     const int64_t hb = blockIdx.x;
     const int64_t lb = (hb & 7) * a.per_xcd + (hb >> 3);
     if (lb >= a.blocks_needed) return;
@@ -528,38 +533,52 @@ __global__ __launch_bounds__(kBatchBlock) void k_apply_batch64(const ApplyArgs<d
     const int64_t rs = a.row_ptr[row];
     const int len = live ? (int)(a.row_ptr[row + 1] - rs) : 0;
     const double2 fp = *reinterpret_cast<const double2*>(a.f + row * NF + 2 * g);
-    double sx = 0.0, sy = 0.0;
-    for (int j0 = h; j0 < len; j0 += H * U) {
-        int32_t q[U];
-        double w[U];
-        double2 f[U];
+    double sx[S], sy[S];
 #pragma unroll
-        for (int k = 0; k < U; ++k) {
-            const int64_t j = rs + min(j0 + H * k, len - 1);
-            q[k] = a.col[j];
-            w[k] = a.W[0][j];
-        }
+    for (int i = 0; i < S; ++i) sx[i] = sy[i] = 0.0;
+    for (int j0 = h; j0 < len; j0 += H * STEP) {
 #pragma unroll
-        for (int k = 0; k < U; ++k) f[k] = *reinterpret_cast<const double2*>(a.f + (int64_t)q[k] * NF + 2 * g);
+        for (int k0 = 0; k0 < STEP; k0 += U) {
+            int32_t q[U];
+            double w[U];
+            double2 f[U];
 #pragma unroll
-        for (int k = 0; k < U; ++k) {
-            const bool in = j0 + H * k < len;
-            const double tx = fma(w[k], MODE == kDiff ? f[k].x - fp.x : f[k].x, sx);
-            const double ty = fma(w[k], MODE == kDiff ? f[k].y - fp.y : f[k].y, sy);
-            sx = in ? tx : sx;
-            sy = in ? ty : sy;
+            for (int k = 0; k < U; ++k) {
+                const int64_t j = rs + min(j0 + H * (k0 + k), len - 1);
+                q[k] = a.col[j];
+                w[k] = a.W[0][j];
+            }
+#pragma unroll
+            for (int k = 0; k < U; ++k) f[k] = *reinterpret_cast<const double2*>(a.f + (int64_t)q[k] * NF + 2 * g);
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                const bool in = j0 + H * (k0 + k) < len;
+                const int i = (k0 + k) % S;
+                const double tx = fma(w[k], MODE == kDiff ? f[k].x - fp.x : f[k].x, sx[i]);
+                const double ty = fma(w[k], MODE == kDiff ? f[k].y - fp.y : f[k].y, sy[i]);
+                sx[i] = in ? tx : sx[i];
+                sy[i] = in ? ty : sy[i];
+            }
         }
     }
+    // distances G/2 .. H inside the part, H/2 .. 1 between the parts
+#pragma unroll
+    for (int off = S / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int i = 0; i < off; ++i) {
+            sx[i] += sx[i + off];
+            sy[i] += sy[i + off];
+        }
 #pragma unroll
     for (int off = 4; off >= L; off >>= 1) {
-        sx += __shfl_xor(sx, off, kWave);
-        sy += __shfl_xor(sy, off, kWave);
+        sx[0] += __shfl_xor(sx[0], off, kWave);
+        sy[0] += __shfl_xor(sy[0], off, kWave);
     }
     if (!live || h >= 2) return;
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
         if ((H > 1 && b != h % 2) || 2 * g + b >= nf) continue;  // the other part's field, or none
-        double val = b ? sy : sx;
+        double val = b ? sy[0] : sx[0];
         if (MODE == kExplicitDiag) val = fma(a.diag[row], b ? fp.y : fp.x, val);
         double* dst = a.out[0] + (2 * g + b) * a.ld_out + row;
         val *= a.alpha;
@@ -569,11 +588,13 @@ __global__ __launch_bounds__(kBatchBlock) void k_apply_batch64(const ApplyArgs<d
 }
 
 template <int NF, int MODE>
-static void launch_batch64(ApplyArgs<double> a, int nf, hipStream_t s) {
+static void launch_batch64(ApplyArgs<double> a, int nf, int G, hipStream_t s) {
     const int rows_per_block = kBatchBlock / 8;
     a.blocks_needed = (a.n_rows + rows_per_block - 1) / rows_per_block;
     a.per_xcd = (a.blocks_needed + 7) / 8;
-    k_apply_batch64<NF, MODE><<<(unsigned)(a.per_xcd * 8), kBatchBlock, 0, s>>>(a, nf);
+    const unsigned grid = (unsigned)(a.per_xcd * 8);
+    if (G == 16) k_apply_batch64<NF, 16, MODE><<<grid, kBatchBlock, 0, s>>>(a, nf);
+    else k_apply_batch64<NF, 8, MODE><<<grid, kBatchBlock, 0, s>>>(a, nf);
 }
 
 // The interleaved batch kernel for the shapes of the 16-byte-load kernel
@@ -775,7 +796,9 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
         }
     }
     if constexpr (std::is_same<T, double>::value) {
-        // FP64 batches likewise
+        // FP64 batches likewise (rows short enough for epl 4 run k_apply<16, 4>
+        // field by field)
+        const int lanes = sh.epl == 4 ? 16 : 8;
         if (nops == 1 && nfields >= kBatchMin && ctx->apply_group <= 0 && (!f_self || (f_self == f && ld_self == ld_f))) {
             Workspace ws;
             dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(double) + 256, &ws);
@@ -792,9 +815,9 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
                 DCPSE_LAUNCH_CHECK(ctx);
                 a.f = a.f_self = fil;
                 a.out[0] = out[0] + (int64_t)b0 * ld_out;
-                if (nf > 8) launch_batch64<16, MODE>(a, nf, ctx->stream);
-                else if (nf > 4) launch_batch64<8, MODE>(a, nf, ctx->stream);
-                else launch_batch64<4, MODE>(a, nf, ctx->stream);
+                if (nf > 8) launch_batch64<16, MODE>(a, nf, lanes, ctx->stream);
+                else if (nf > 4) launch_batch64<8, MODE>(a, nf, lanes, ctx->stream);
+                else launch_batch64<4, MODE>(a, nf, lanes, ctx->stream);
                 DCPSE_LAUNCH_CHECK(ctx);
                 b0 += nf;
             }
