@@ -59,6 +59,10 @@ SELL_AFTER = 1
 #: choice takes the list's 16-bit columns, and where more than this fraction
 #: does not fit those either, the 32-bit sliced-ELL layout.
 BUNDLE16_MAX_EXC = 0.01
+#: Neighbours above which several operators in one pass take the list's 16-bit
+#: columns: below, the 32-bit ones are as fast (8.2 and 8.4 us a stage with 3.8M
+#: neighbours, caches hold them) and 35 us quicker to build.
+COL16_MIN = 4_000_000
 _FILE_VERSION = 1
 
 
@@ -613,7 +617,7 @@ class _SellPlan:
             args = (p(vl.row_ptr), p(slice_ptr), p(row16), 1, p(bundle), p(exc_ptr), p(exc_col), p(exc_W), ne)
         else:
             W = [op.sell_weights() if dtype == torch.float32 else op.sell_weights64() for op in ops]
-            c16 = None if n_domain else ops[0].col16()
+            c16 = None if n_domain or (vl.nnz <= COL16_MIN and not vl._col16) else ops[0].col16()
             self.W = _lib.ptr_array(W)
             if c16 is not None:
                 name, keep, self.domain = "dcpse_apply_col16_", [vl.row_ptr, *c16[:-1], *W], False

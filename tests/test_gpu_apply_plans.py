@@ -108,3 +108,19 @@ def test_planned_apply_in_a_graph(cuda):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, lap(f)), k
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_columns_by_list_size(cuda, dtype, monkeypatch):
+    from openfpm_numerics_amd import Derivative_x, Laplacian, dcpse, fused
+
+    ps, rc, rng = _set(cuda, 5)
+    f = torch.as_tensor(rng.standard_normal(ps.size_local()), dtype=dtype, device=cuda)
+    got = []
+    for least in (dcpse.COL16_MIN, 0):
+        monkeypatch.setattr(dcpse, "COL16_MIN", least)
+        vl = ps.getVerlet(rc)
+        got.append(fused(Laplacian(ps, vl, 2, rc), Derivative_x(ps, vl, 2, rc), f=f))
+        assert bool(vl._col16) == (least == 0) and (vl._sell is None) == (least == 0)
+    for a, b in zip(*got):
+        assert float((a - b).abs().max()) <= 2 * torch.finfo(dtype).eps * float(a.abs().max())
