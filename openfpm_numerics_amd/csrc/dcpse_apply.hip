@@ -726,6 +726,16 @@ static int field_chunk(int remaining, int nops, int epl) {
     return 1;
 }
 
+// Whether a graph is being captured on the stream. A captured batch runs field
+// by field (the same bits): a graph outlives the workspace of the particle-major
+// copies, which a later call may replace by a larger one.
+static bool captured(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (!s || hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
 template <typename T, int MODE>
 static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
                                int nops, const T* const* W, const T* f, int64_t ld_f, int nfields,
@@ -768,7 +778,7 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
         // workspace (the col/W streams read once per group), the last ones in
         // the smallest of 4, 8 or 16 that holds them
         if (nops == 1 && nfields >= kBatchMin && sh.vec == 4 && il_shape(sh.G, sh.epl) &&
-            (!f_self || (f_self == f && ld_self == ld_f))) {
+            (!f_self || (f_self == f && ld_self == ld_f)) && !captured(ctx->stream)) {
             Workspace ws;
             dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(float) + 256, &ws);
             if (st) return st;
@@ -799,7 +809,8 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
         // FP64 batches likewise (rows short enough for epl 4 run k_apply<16, 4>
         // field by field)
         const int lanes = sh.epl == 4 ? 16 : 8;
-        if (nops == 1 && nfields >= kBatchMin && ctx->apply_group <= 0 && (!f_self || (f_self == f && ld_self == ld_f))) {
+        if (nops == 1 && nfields >= kBatchMin && ctx->apply_group <= 0 &&
+            (!f_self || (f_self == f && ld_self == ld_f)) && !captured(ctx->stream)) {
             Workspace ws;
             dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(double) + 256, &ws);
             if (st) return st;

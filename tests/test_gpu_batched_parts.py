@@ -80,3 +80,35 @@ def test_fp64_batches(cuda, name, few):
             run(nb, f, got)
             assert torch.equal(got[:nb], want[:nb]), (run.__name__, nb)
             assert bool((got[nb:] == 1).all()), (run.__name__, nb)
+
+
+@pytest.mark.parametrize("direction", ["forward", "transposed"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("nb", [3, 13])
+def test_captured_batches(cuda, nb, dtype, direction):
+    """A captured batch keeps no workspace: lists that outgrow it come between
+    capture and replay."""
+    from openfpm_numerics_amd import Laplacian, ParticleSet
+
+    rng = np.random.default_rng(nb)
+
+    def lattice(n):
+        g = (np.arange(n) + 0.5) / n
+        pos = np.stack(np.meshgrid(g, g, indexing="ij"), -1).reshape(-1, 2)
+        return ParticleSet(np.mod(pos + rng.uniform(-0.1 / n, 0.1 / n, pos.shape), 1.0), [0.0] * 2, [1.0] * 2, bc=[1, 1],
+                           device=cuda)
+
+    ps = lattice(48)
+    d = Laplacian(ps, ps.getVerlet(3.1 / 48), 2, 3.1 / 48).dcpse
+    f = torch.as_tensor(rng.standard_normal((nb, ps.size_local())), dtype=dtype, device=cuda)
+    run = d if direction == "forward" else d.applyTranspose
+    run(f)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run(f)
+    lattice(700).getVerlet(3.1 / 700)
+    for k in range(3):
+        f.copy_(torch.as_tensor(rng.standard_normal(f.shape), dtype=dtype))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, run(f)), k
