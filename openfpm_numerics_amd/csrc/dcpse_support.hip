@@ -974,10 +974,10 @@ __device__ __forceinline__ void pair_tests(const Groups& a, const PairGroup& pg,
 // removed (rcut 2.4 spacings) shrink to about 170 within reach of the
 // particles' bounding box, are sorted in 200-odd instructions, and a pair
 // test costs 9 instructions per 64 pairs with the candidates in registers and
-// the particle in scalar registers. 0.55 ms there (1.89M particles); FP64
+// the particle in scalar registers. 0.51 ms there (1.89M particles); FP64
 // tests of every candidate from LDS took 1.14 ms, and with them the fill,
 // which then sorted every row, 0.96 ms instead of 0.22 ms (k_group_rows).
-// With a cut-off per particle (PP; 490,000 particles, spacing 4 : 1): 0.33 ms
+// With a cut-off per particle (PP; 490,000 particles, spacing 4 : 1): 0.27 ms
 // and a fill of 0.11 ms, against 1.08 and 1.22 ms of k_support_rows, whose
 // wavefronts each flatten and test the candidates of one particle.
 template <int DIM, int RMAX, bool PP>
