@@ -73,7 +73,10 @@ int32_t dcpse_version(void);
 dcpse_status dcpse_ctx_create(dcpse_ctx** ctx, int32_t device);
 dcpse_status dcpse_ctx_destroy(dcpse_ctx* ctx);
 /* Orders all further work of ctx on hip_stream, a caller-owned hipStream_t
- * (NULL = the device's default stream, which is also the initial binding). */
+ * (NULL = the device's default stream, which is also the initial binding). Work
+ * already queued on another stream goes on; where a later call needs the
+ * context's workspace that such work still uses, its stream waits for it (not
+ * while it is being captured). The caller's own arrays are the caller's to order. */
 dcpse_status dcpse_ctx_set_stream(dcpse_ctx* ctx, void* hip_stream);
 void* dcpse_ctx_get_stream(dcpse_ctx* ctx);
 const char* dcpse_last_error(const dcpse_ctx* ctx);

@@ -726,16 +726,6 @@ static int field_chunk(int remaining, int nops, int epl) {
     return 1;
 }
 
-// Whether a graph is being captured on the stream. A captured batch runs field
-// by field (the same bits): a graph outlives the workspace of the particle-major
-// copies, which a later call may replace by a larger one.
-static bool captured(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (!s || hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
-    (void)hipGetLastError();
-    return false;
-}
-
 template <typename T, int MODE>
 static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
                                int nops, const T* const* W, const T* f, int64_t ld_f, int nfields,
@@ -776,12 +766,15 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
         // batches of several fields on one set (columns and rows index the
         // same n_rows particles): interleaved 16 at a time through the
         // workspace (the col/W streams read once per group), the last ones in
-        // the smallest of 4, 8 or 16 that holds them
+        // the smallest of 4, 8 or 16 that holds them. A captured batch runs
+        // field by field (the same bits): a graph outlives the workspace, which
+        // a later call may replace by a larger one.
         if (nops == 1 && nfields >= kBatchMin && sh.vec == 4 && il_shape(sh.G, sh.epl) &&
             (!f_self || (f_self == f && ld_self == ld_f)) && !captured(ctx->stream)) {
             Workspace ws;
             dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(float) + 256, &ws);
             if (st) return st;
+            const WorkspaceUse use(ctx);
             float* fil = ws.take<float>((size_t)n_rows * 16);
             if (!fil) return fail(ctx, DCPSE_ERR_INVALID, "apply workspace sizing error");
             while (nfields - b0 >= kBatchMin) {
@@ -814,6 +807,7 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
             Workspace ws;
             dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(double) + 256, &ws);
             if (st) return st;
+            const WorkspaceUse use(ctx);
             double* fil = ws.take<double>((size_t)n_rows * 16);
             if (!fil) return fail(ctx, DCPSE_ERR_INVALID, "apply workspace sizing error");
             while (nfields - b0 >= kBatchMin) {

@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <optional>
 #include <vector>
 
 #include "dcpse_common.hpp"
@@ -1724,6 +1725,7 @@ static dcpse_status assemble_ops(dcpse_ctx* ctx, int32_t dim, const double* pos_
     const int bw = persistent ? ctx->asm_bucket : 0;  // the static grid runs index order
     const int nb = bw > 0 ? std::max(1, (DCPSE_MAX_ROW + bw) / bw) : 0;
     const int64_t n_tiles = (n_dom + kBucketTile - 1) / kBucketTile;
+    std::optional<WorkspaceUse> use;
     if (persistent || bw > 0) {
         Workspace w;
         const size_t need = 64 * 4 + (bw > 0 ? (size_t)n_dom * 4 + ((size_t)nb * n_tiles + 1) * 12 +
@@ -1731,6 +1733,7 @@ static dcpse_status assemble_ops(dcpse_ctx* ctx, int32_t dim, const double* pos_
                                              : 0) + 1024;
         dcpse_status st = reserve_workspace(ctx, need, &w);
         if (st) return st;
+        use.emplace(ctx);
         unsigned* queues = w.take<unsigned>(64);
         if (!queues) return fail(ctx, DCPSE_ERR_INVALID, "assembly workspace sizing error");
         if (persistent) {

@@ -32,6 +32,11 @@ dcpse_status dcpse_ctx_create(dcpse_ctx** out, int32_t device) {
         delete ctx;
         return DCPSE_ERR_HIP;
     }
+    if (hipEventCreateWithFlags(&ctx->ws_event, hipEventDisableTiming) != hipSuccess) {
+        (void)hipHostFree(ctx->host);
+        delete ctx;
+        return DCPSE_ERR_HIP;
+    }
     *out = ctx;
     return DCPSE_OK;
 }
@@ -40,9 +45,11 @@ dcpse_status dcpse_ctx_destroy(dcpse_ctx* ctx) {
     if (!ctx) return DCPSE_OK;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->ws_queued) (void)hipEventSynchronize(ctx->ws_event);
     if (ctx->ws) (void)hipFree(ctx->ws);
     if (ctx->sup.buf) (void)hipFree(ctx->sup.buf);
     if (ctx->host) (void)hipHostFree(ctx->host);
+    if (ctx->ws_event) (void)hipEventDestroy(ctx->ws_event);
     delete ctx;
     return DCPSE_OK;
 }

@@ -311,6 +311,7 @@ dcpse_status dcpse_operator_diagnostics(dcpse_ctx* ctx, int32_t dim, const doubl
                         6 * 256;
     dcpse_status st = reserve_workspace(ctx, need, &w);
     if (st) return st;
+    const WorkspaceUse use(ctx);
     uint32_t* d_ex = w.take<uint32_t>((size_t)M * dim);
     double* d_b = w.take<double>((size_t)M);
     double* r_ws = w.take<double>((size_t)std::max<int64_t>(n_dom, 1));

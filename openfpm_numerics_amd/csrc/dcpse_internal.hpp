@@ -56,6 +56,10 @@ struct dcpse_ctx {
     int asm_bucket = 0;    // > 0: batches bucketed by row length, this bucket width
     void* ws = nullptr;    // grow-only device workspace
     size_t ws_size = 0;
+    // the last work queued on ws by a call that did not wait for it, and its stream
+    hipEvent_t ws_event = nullptr;
+    hipStream_t ws_stream = nullptr;
+    bool ws_queued = false;
     int64_t* host = nullptr;  // pinned: kResults numbers that kernels leave for the host
     void* scratch = nullptr;  // this device's static no-alloc scratch (device address)
     dcpse_support_cache sup;
@@ -96,8 +100,24 @@ struct Workspace {
     }
 };
 
+// Whether a graph is being captured on the stream.
+bool captured(hipStream_t s);
+
 // Ensures ctx->ws holds at least `bytes`; waits for queued work before growing.
+// Work that an earlier call left queued on ws from another stream is done
+// before what this call queues (a captured stream, which may not wait for it,
+// excepted).
 dcpse_status reserve_workspace(dcpse_ctx* ctx, size_t bytes, Workspace* w);
+
+// Held from reserve_workspace on by a call that returns without waiting for its
+// stream: the workspace's next user on another stream waits for what the call
+// queued.
+struct WorkspaceUse {
+    dcpse_ctx* ctx;
+    explicit WorkspaceUse(dcpse_ctx* c) : ctx(c) {}
+    WorkspaceUse(const WorkspaceUse&) = delete;
+    ~WorkspaceUse();
+};
 
 // Numbers that a pass leaves in ctx->host: a kernel stores them to pinned
 // memory, so the host waits once instead of copying each to pageable memory

@@ -217,8 +217,29 @@ static void fill_i64(hipStream_t s, int64_t* p, int64_t n, int64_t v) {
     k_fill_i64<<<(unsigned)blocks, 256, 0, s>>>(p, n, v);
 }
 
+bool captured(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (!s || hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
+WorkspaceUse::~WorkspaceUse() {
+    if (captured(ctx->stream)) return;  // nothing runs before the graph is launched
+    if (hipEventRecord(ctx->ws_event, ctx->stream) == hipSuccess) {
+        ctx->ws_stream = ctx->stream;
+        ctx->ws_queued = true;
+    } else {  // no event to wait for later: wait now
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(ctx->stream);
+    }
+}
+
 dcpse_status reserve_workspace(dcpse_ctx* ctx, size_t bytes, Workspace* w) {
+    if (ctx->ws_queued && ctx->ws_stream != ctx->stream && !captured(ctx->stream))
+        DCPSE_HIP_CHECK(ctx, hipStreamWaitEvent(ctx->stream, ctx->ws_event, 0));
     if (ctx->ws_size < bytes) {
+        if (ctx->ws_queued) DCPSE_HIP_CHECK(ctx, hipEventSynchronize(ctx->ws_event));
         DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->ws) DCPSE_HIP_CHECK(ctx, hipFree(ctx->ws));
         ctx->ws = nullptr;
@@ -2020,6 +2041,7 @@ dcpse_status dcpse_transpose_count(dcpse_ctx* ctx, int64_t n_rows, int64_t n_col
     Workspace w;
     dcpse_status st = reserve_workspace(ctx, (size_t)(n_cols + 1) * 4 + scan_workspace_bytes(n_cols) + 1024, &w);
     if (st) return st;
+    const WorkspaceUse use(ctx);
     int32_t* cnt = w.take<int32_t>(n_cols + 1);
     fill_i32(ctx->stream, cnt, n_cols + 1, 0);
     if (nnz > 0) {
