@@ -763,14 +763,15 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
     }
     int b0 = 0;
     if constexpr (std::is_same<T, float>::value) {
-        // batches of several fields on one set (columns and rows index the
-        // same n_rows particles): interleaved 16 at a time through the
+        // batches of several fields on one set (no f_self: columns and rows
+        // index the same n_rows particles; f_self == f may also be a domain
+        // that leads its support set, with columns past the rows): interleaved 16 at a time through the
         // workspace (the col/W streams read once per group), the last ones in
         // the smallest of 4, 8 or 16 that holds them. A captured batch runs
         // field by field (the same bits): a graph outlives the workspace, which
         // a later call may replace by a larger one.
-        if (nops == 1 && nfields >= kBatchMin && sh.vec == 4 && il_shape(sh.G, sh.epl) &&
-            (!f_self || (f_self == f && ld_self == ld_f)) && !captured(ctx->stream)) {
+        if (nops == 1 && nfields >= kBatchMin && sh.vec == 4 && il_shape(sh.G, sh.epl) && !f_self &&
+            !captured(ctx->stream)) {
             Workspace ws;
             dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(float) + 256, &ws);
             if (st) return st;
@@ -802,8 +803,7 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
         // FP64 batches likewise (rows short enough for epl 4 run k_apply<16, 4>
         // field by field)
         const int lanes = sh.epl == 4 ? 16 : 8;
-        if (nops == 1 && nfields >= kBatchMin && ctx->apply_group <= 0 &&
-            (!f_self || (f_self == f && ld_self == ld_f)) && !captured(ctx->stream)) {
+        if (nops == 1 && nfields >= kBatchMin && ctx->apply_group <= 0 && !f_self && !captured(ctx->stream)) {
             Workspace ws;
             dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(double) + 256, &ws);
             if (st) return st;
