@@ -239,8 +239,9 @@ dcpse_status dcpse_assemble_multi(dcpse_ctx* ctx, int32_t dim,
  * one set (f_self NULL) are copied particle-major into the context's workspace
  * (16 x n_rows values, grown on first use) and applied up to 16 fields per
  * pass; each field's result equals its single-field apply bit for bit. While
- * the stream is being captured they run field by field. The same holds for
- * dcpse_apply_transpose_f32 and _f64. */
+ * the stream is being captured they run field by field (the _nnz entry points
+ * below have no such limit). The same holds for dcpse_apply_transpose_f32 and
+ * _f64. */
 dcpse_status dcpse_apply_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
                              int32_t n_ops, const float* const* W,
                              const float* f, int64_t ld_f, int32_t n_fields,
@@ -276,6 +277,32 @@ dcpse_status dcpse_apply_transpose_f64(dcpse_ctx* ctx, int64_t n_cols, const int
                                        const int32_t* colT, const double* WT, const double* diag,
                                        const double* g, int64_t ld_g, int32_t n_fields,
                                        double* out, int64_t ld_out, double alpha, double beta);
+
+/* The same applies with what the host knows of the list and memory of the
+ * caller's: nnz (row_ptr[n_rows]) picks the launch shape, so nothing is read
+ * back; scratch (device, 16-byte aligned, scratch_bytes long, NULL for none)
+ * takes the particle-major copies of a batch instead of the context's
+ * workspace: n_rows values per field of a pass, which has 4, 8 or 16 fields,
+ * the smallest that holds the batch serving it best. With less, passes are
+ * narrower; without room for 4 the batch runs field by field. Same results bit
+ * for bit. The call's work uses scratch in stream order, so a graph being
+ * captured may hold it as long as it is replayed. */
+dcpse_status dcpse_apply_nnz_f32(dcpse_ctx* ctx, int64_t n_rows, int64_t nnz, const int64_t* row_ptr,
+                                 const int32_t* col, int32_t n_ops, const float* const* W, const float* f, int64_t ld_f,
+                                 int32_t n_fields, const float* f_self, int64_t ld_self, float* const* out,
+                                 int64_t ld_out, float alpha, float beta, void* scratch, size_t scratch_bytes);
+dcpse_status dcpse_apply_nnz_f64(dcpse_ctx* ctx, int64_t n_rows, int64_t nnz, const int64_t* row_ptr,
+                                 const int32_t* col, int32_t n_ops, const double* const* W, const double* f, int64_t ld_f,
+                                 int32_t n_fields, const double* f_self, int64_t ld_self, double* const* out,
+                                 int64_t ld_out, double alpha, double beta, void* scratch, size_t scratch_bytes);
+dcpse_status dcpse_apply_transpose_nnz_f32(dcpse_ctx* ctx, int64_t n_cols, int64_t nnz, const int64_t* rowT_ptr,
+                                           const int32_t* colT, const float* WT, const float* diag, const float* g,
+                                           int64_t ld_g, int32_t n_fields, float* out, int64_t ld_out, float alpha,
+                                           float beta, void* scratch, size_t scratch_bytes);
+dcpse_status dcpse_apply_transpose_nnz_f64(dcpse_ctx* ctx, int64_t n_cols, int64_t nnz, const int64_t* rowT_ptr,
+                                           const int32_t* colT, const double* WT, const double* diag, const double* g,
+                                           int64_t ld_g, int32_t n_fields, double* out, int64_t ld_out, double alpha,
+                                           double beta, void* scratch, size_t scratch_bytes);
 
 /* ---- diagnostics -------------------------------------------------------- */
 /* Per-particle diagnostics of an assembled operator (any argument of

@@ -25,6 +25,7 @@ _i64 = C.c_int64
 _u32 = C.c_uint32
 _f32 = C.c_float
 _f64 = C.c_double
+_sz = C.c_size_t
 
 # row_ptr .. exc_slot and n_exc of the 16-bit columns; u .. out_b of an FP64 stage
 _COL16 = [_vp] * 8 + [_i64]
@@ -93,6 +94,14 @@ SIGNATURES = {
     "dcpse_sell_fill_bundle16_f64": (_i32, [_vp, _i64, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp]),
     "dcpse_apply_sell_bundle16_f64": (_i32, [_vp, _i64, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp,
                                              _f64, _f64]),
+    "dcpse_apply_nnz_f32": (_i32, [_vp, _i64, _i64, _vp, _vp, _i32, _vp, _vp, _i64, _i32, _vp, _i64, _vp, _i64,
+                                   _f32, _f32, _vp, _sz]),
+    "dcpse_apply_nnz_f64": (_i32, [_vp, _i64, _i64, _vp, _vp, _i32, _vp, _vp, _i64, _i32, _vp, _i64, _vp, _i64,
+                                   _f64, _f64, _vp, _sz]),
+    "dcpse_apply_transpose_nnz_f32": (_i32, [_vp, _i64, _i64] + [_vp] * 5 + [_i64, _i32, _vp, _i64, _f32, _f32, _vp,
+                                                                             _sz]),
+    "dcpse_apply_transpose_nnz_f64": (_i32, [_vp, _i64, _i64] + [_vp] * 5 + [_i64, _i32, _vp, _i64, _f64, _f64, _vp,
+                                                                             _sz]),
     "dcpse_export_csr_f64": (_i32, [_vp, _i64, _vp, _vp, _vp, _f64, _vp, _vp, _vp]),
     "dcpse_export_csr_f32": (_i32, [_vp, _i64, _vp, _vp, _vp, _f64, _vp, _vp, _vp]),
     "dcpse_export_csr_nnz_f64": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _f64, _vp, _vp, _vp]),

@@ -16,6 +16,8 @@
 // remapped so that each XCD walks one contiguous slice of rows, keeping the
 // f halo of a slice in that XCD's L2.
 #include <algorithm>
+#include <cstdint>
+#include <optional>
 #include <type_traits>
 
 #include "dcpse_common.hpp"
@@ -692,9 +694,16 @@ struct ApplyShape {
 // Launch shape from the mean row length (16-byte loads, 8 lanes per row): up
 // to 24 nonzeros 4 per lane, up to 72 8 per lane, beyond 12 (rows of 93: one
 // field 56 us against 47, 16 fields 255 against 205 with the strided tail from
-// the 65th on, 343,000 rows; FP64 keeps 8). The mean is read once per
-// (row_ptr, n_rows) and cached in the context, so repeated applies of one
-// operator never synchronise the stream. dcpse_set_apply_config overrides it.
+// the 65th on, 343,000 rows; FP64 keeps 8). dcpse_set_apply_config overrides it.
+static ApplyShape shape_of(dcpse_ctx* ctx, int64_t n_rows, int64_t nnz) {
+    if (ctx->apply_group > 0) return {ctx->apply_group, ctx->apply_epl, ctx->apply_vec, 0.0};
+    const double mean = n_rows > 0 ? (double)nnz / (double)n_rows : 0.0;
+    return {8, mean <= 24 ? 4 : mean > 72 ? 12 : 8, 4, mean};
+}
+
+// The same where the caller gives no nnz: read once per (row_ptr, n_rows) and
+// cached in the context, so repeated applies of one operator never synchronise
+// the stream.
 static ApplyShape auto_shape(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr) {
     if (ctx->apply_group > 0) return {ctx->apply_group, ctx->apply_epl, ctx->apply_vec, 0.0};
     if (ctx->grp_rows == row_ptr && ctx->grp_n == n_rows) return {ctx->grp_g, ctx->grp_epl, ctx->grp_vec, ctx->grp_mean};
@@ -702,11 +711,8 @@ static ApplyShape auto_shape(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_
     ApplyShape sh{8, 8, 4, 0.0};
     if (n_rows > 0 &&
         hipMemcpyAsync(&nnz, row_ptr + n_rows, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream) == hipSuccess &&
-        hipStreamSynchronize(ctx->stream) == hipSuccess) {
-        sh.mean = (double)nnz / (double)n_rows;
-        if (sh.mean <= 24) sh.epl = 4;
-        else if (sh.mean > 72) sh.epl = 12;
-    }
+        hipStreamSynchronize(ctx->stream) == hipSuccess)
+        sh = shape_of(ctx, n_rows, nnz);
     ctx->grp_rows = row_ptr;
     ctx->grp_n = n_rows;
     ctx->grp_g = sh.G;
@@ -726,13 +732,27 @@ static int field_chunk(int remaining, int nops, int epl) {
     return 1;
 }
 
+// What a caller of the *_nnz entry points adds: the number of neighbours, which
+// picks the launch shape, and device memory for the particle-major copies.
+struct Counted {
+    int64_t nnz;
+    void* scratch;
+    size_t bytes;
+};
+
+// Fields of a pass: the smallest of 4, 8 and 16 that holds nf.
+static int pass_width(int nf) { return nf > 8 ? 16 : nf > 4 ? 8 : 4; }
+
 template <typename T, int MODE>
 static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,
                                int nops, const T* const* W, const T* f, int64_t ld_f, int nfields,
                                const T* f_self, int64_t ld_self, const T* diag, T* const* out, int64_t ld_out,
-                               T alpha, T beta) {
+                               T alpha, T beta, const Counted* given = nullptr) {
+    constexpr bool F32 = std::is_same<T, float>::value;
     if (!row_ptr || !col || !W || !f || !out || n_rows < 0 || nfields < 1 || nops < 1)
         return fail(ctx, DCPSE_ERR_INVALID, "null pointer or bad size");
+    if (given && (given->nnz < 0 || (reinterpret_cast<uintptr_t>(given->scratch) & 15)))
+        return fail(ctx, DCPSE_ERR_INVALID, "negative nnz or scratch not 16-byte aligned");
     if (nops > kMaxOps) return fail(ctx, DCPSE_ERR_UNSUPPORTED, "at most %d operators per pass", kMaxOps);
     if (nops > 1 && nfields > 1)
         return fail(ctx, DCPSE_ERR_UNSUPPORTED, "several operators and several fields in one pass");
@@ -742,8 +762,8 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
         if (!W[o] || !out[o]) return fail(ctx, DCPSE_ERR_INVALID, "null operator pointer");
     if (n_rows == 0) return DCPSE_OK;
     DCPSE_HIP_CHECK(ctx, hipSetDevice(ctx->device));
-    ApplyShape sh = auto_shape(ctx, n_rows, row_ptr);
-    if (!std::is_same<T, float>::value && ctx->apply_group <= 0 && sh.epl == 12) sh.epl = 8;
+    ApplyShape sh = given ? shape_of(ctx, n_rows, given->nnz) : auto_shape(ctx, n_rows, row_ptr);
+    if (!F32 && ctx->apply_group <= 0 && sh.epl == 12) sh.epl = 8;
     const int block = ctx->apply_block;
     if (block % sh.G != 0 || block < 64 || block > kApplyMaxBlock)
         return fail(ctx, DCPSE_ERR_INVALID, "block %d incompatible with group %d", block, sh.G);
@@ -762,71 +782,56 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
         a.out[o] = nullptr;
     }
     int b0 = 0;
-    if constexpr (std::is_same<T, float>::value) {
-        // batches of several fields on one set (no f_self: columns and rows
-        // index the same n_rows particles; f_self == f may also be a domain
-        // that leads its support set, with columns past the rows): interleaved 16 at a time through the
-        // workspace (the col/W streams read once per group), the last ones in
-        // the smallest of 4, 8 or 16 that holds them. A captured batch runs
-        // field by field (the same bits): a graph outlives the workspace, which
-        // a later call may replace by a larger one.
-        if (nops == 1 && nfields >= kBatchMin && sh.vec == 4 && il_shape(sh.G, sh.epl) && !f_self &&
-            !captured(ctx->stream)) {
-            Workspace ws;
-            dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(float) + 256, &ws);
-            if (st) return st;
-            const WorkspaceUse use(ctx);
-            float* fil = ws.take<float>((size_t)n_rows * 16);
-            if (!fil) return fail(ctx, DCPSE_ERR_INVALID, "apply workspace sizing error");
-            while (nfields - b0 >= kBatchMin) {
-                const int nf = std::min(nfields - b0, 16);
-                const unsigned ib = (unsigned)((n_rows + 255) / 256);
-                const float* fb = f + (int64_t)b0 * ld_f;
-                if (nf > 8) k_interleave<16><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
-                else if (nf > 4) k_interleave<8><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
-                else k_interleave<4><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
-                DCPSE_LAUNCH_CHECK(ctx);
-                a.f = fil;
-                a.f_self = fil;
-                a.out[0] = out[0] + (int64_t)b0 * ld_out;
-                const bool ok = nf > 8   ? dispatch_il<MODE, 16>(a, sh.G, sh.epl, nf, sh.mean, ctx->stream)
-                                : nf > 4 ? dispatch_il<MODE, 8>(a, sh.G, sh.epl, nf, sh.mean, ctx->stream)
-                                         : dispatch_il<MODE, 4>(a, sh.G, sh.epl, nf, sh.mean, ctx->stream);
-                if (!ok) return fail(ctx, DCPSE_ERR_UNSUPPORTED, "no batched apply kernel for group=%d x %d", sh.G,
-                                     sh.epl);
-                DCPSE_LAUNCH_CHECK(ctx);
-                b0 += nf;
-            }
-        }
+    // Batches of several fields on one set (no f_self: columns and rows index
+    // the same n_rows particles; f_self == f may also be a domain that leads
+    // its support set, with columns past the rows): interleaved up to 16 at a
+    // time (the col/W streams read once per pass), the last ones in the
+    // smallest of 4, 8 or 16 that holds them. The copy lies in the caller's
+    // scratch, which a graph being captured may keep, or in the context's
+    // workspace, which it may not (a later call can replace it): a captured
+    // batch without scratch runs field by field, with the same bits.
+    const bool particle_major = nops == 1 && nfields >= kBatchMin && !f_self &&
+                                (F32 ? sh.vec == 4 && il_shape(sh.G, sh.epl) : ctx->apply_group <= 0);
+    T* fil = nullptr;
+    int width = 0;  // fields that the copy has room for
+    std::optional<WorkspaceUse> use;
+    if (particle_major && given) {
+        const size_t room = given->scratch ? given->bytes / ((size_t)n_rows * sizeof(T)) : 0;
+        fil = static_cast<T*>(given->scratch);
+        width = room >= 16 ? 16 : room >= 8 ? 8 : room >= 4 ? 4 : 0;
+    } else if (particle_major && !captured(ctx->stream)) {
+        Workspace ws;
+        dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(T) + 256, &ws);
+        if (st) return st;
+        use.emplace(ctx);
+        fil = ws.take<T>((size_t)n_rows * 16);
+        if (!fil) return fail(ctx, DCPSE_ERR_INVALID, "apply workspace sizing error");
+        width = 16;
     }
-    if constexpr (std::is_same<T, double>::value) {
-        // FP64 batches likewise (rows short enough for epl 4 run k_apply<16, 4>
-        // field by field)
-        const int lanes = sh.epl == 4 ? 16 : 8;
-        if (nops == 1 && nfields >= kBatchMin && ctx->apply_group <= 0 && !f_self && !captured(ctx->stream)) {
-            Workspace ws;
-            dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(double) + 256, &ws);
-            if (st) return st;
-            const WorkspaceUse use(ctx);
-            double* fil = ws.take<double>((size_t)n_rows * 16);
-            if (!fil) return fail(ctx, DCPSE_ERR_INVALID, "apply workspace sizing error");
-            while (nfields - b0 >= kBatchMin) {
-                const int nf = std::min(nfields - b0, 16);
-                const unsigned ib = (unsigned)((n_rows + 255) / 256);
-                const double* fb = f + (int64_t)b0 * ld_f;
-                if (nf > 8) k_interleave<16><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
-                else if (nf > 4) k_interleave<8><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
-                else k_interleave<4><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
-                DCPSE_LAUNCH_CHECK(ctx);
-                a.f = a.f_self = fil;
-                a.out[0] = out[0] + (int64_t)b0 * ld_out;
-                if (nf > 8) launch_batch64<16, MODE>(a, nf, lanes, ctx->stream);
-                else if (nf > 4) launch_batch64<8, MODE>(a, nf, lanes, ctx->stream);
-                else launch_batch64<4, MODE>(a, nf, lanes, ctx->stream);
-                DCPSE_LAUNCH_CHECK(ctx);
-                b0 += nf;
-            }
+    while (width > 0 && nfields - b0 >= kBatchMin) {
+        const int nf = std::min(nfields - b0, width), pass = pass_width(nf);
+        const unsigned ib = (unsigned)((n_rows + 255) / 256);
+        const T* fb = f + (int64_t)b0 * ld_f;
+        if (pass == 16) k_interleave<16><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
+        else if (pass == 8) k_interleave<8><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
+        else k_interleave<4><<<ib, 256, 0, ctx->stream>>>(n_rows, fb, ld_f, nf, fil);
+        DCPSE_LAUNCH_CHECK(ctx);
+        a.f = a.f_self = fil;
+        a.out[0] = out[0] + (int64_t)b0 * ld_out;
+        bool ok = true;
+        if constexpr (F32) {
+            ok = pass == 16  ? dispatch_il<MODE, 16>(a, sh.G, sh.epl, nf, sh.mean, ctx->stream)
+                 : pass == 8 ? dispatch_il<MODE, 8>(a, sh.G, sh.epl, nf, sh.mean, ctx->stream)
+                             : dispatch_il<MODE, 4>(a, sh.G, sh.epl, nf, sh.mean, ctx->stream);
+        } else {
+            const int lanes = sh.epl == 4 ? 16 : 8;  // of the single-field kernel
+            if (pass == 16) launch_batch64<16, MODE>(a, nf, lanes, ctx->stream);
+            else if (pass == 8) launch_batch64<8, MODE>(a, nf, lanes, ctx->stream);
+            else launch_batch64<4, MODE>(a, nf, lanes, ctx->stream);
         }
+        if (!ok) return fail(ctx, DCPSE_ERR_UNSUPPORTED, "no batched apply kernel for group=%d x %d", sh.G, sh.epl);
+        DCPSE_LAUNCH_CHECK(ctx);
+        b0 += nf;
     }
     while (b0 < nfields) {
         const int nf = field_chunk(nfields - b0, nops, sh.epl);
@@ -914,6 +919,52 @@ dcpse_status dcpse_apply_transpose_f64(dcpse_ctx* ctx, int64_t n_cols, const int
     double* Op[1] = {out};
     return apply_impl<double, kExplicitDiag>(ctx, n_cols, rowT_ptr, colT, 1, Wp, g, ld_g, n_fields, nullptr, ld_g,
                                              diag, Op, ld_out, alpha, beta);
+}
+
+dcpse_status dcpse_apply_nnz_f32(dcpse_ctx* ctx, int64_t n_rows, int64_t nnz, const int64_t* row_ptr,
+                                 const int32_t* col, int32_t n_ops, const float* const* W, const float* f, int64_t ld_f,
+                                 int32_t n_fields, const float* f_self, int64_t ld_self, float* const* out,
+                                 int64_t ld_out, float alpha, float beta, void* scratch, size_t scratch_bytes) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    const Counted given{nnz, scratch, scratch_bytes};
+    return apply_impl<float, kDiff>(ctx, n_rows, row_ptr, col, n_ops, W, f, ld_f, n_fields, f_self, ld_self, nullptr,
+                                  out, ld_out, alpha, beta, &given);
+}
+
+dcpse_status dcpse_apply_transpose_nnz_f32(dcpse_ctx* ctx, int64_t n_cols, int64_t nnz, const int64_t* rowT_ptr,
+                                           const int32_t* colT, const float* WT, const float* diag, const float* g,
+                                           int64_t ld_g, int32_t n_fields, float* out, int64_t ld_out, float alpha,
+                                           float beta, void* scratch, size_t scratch_bytes) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!diag) return fail(ctx, DCPSE_ERR_INVALID, "diag is null");
+    const float* Wp[1] = {WT};
+    float* Op[1] = {out};
+    const Counted given{nnz, scratch, scratch_bytes};
+    return apply_impl<float, kExplicitDiag>(ctx, n_cols, rowT_ptr, colT, 1, Wp, g, ld_g, n_fields, nullptr, ld_g, diag,
+                                          Op, ld_out, alpha, beta, &given);
+}
+
+dcpse_status dcpse_apply_nnz_f64(dcpse_ctx* ctx, int64_t n_rows, int64_t nnz, const int64_t* row_ptr,
+                                 const int32_t* col, int32_t n_ops, const double* const* W, const double* f, int64_t ld_f,
+                                 int32_t n_fields, const double* f_self, int64_t ld_self, double* const* out,
+                                 int64_t ld_out, double alpha, double beta, void* scratch, size_t scratch_bytes) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    const Counted given{nnz, scratch, scratch_bytes};
+    return apply_impl<double, kDiff>(ctx, n_rows, row_ptr, col, n_ops, W, f, ld_f, n_fields, f_self, ld_self, nullptr,
+                                  out, ld_out, alpha, beta, &given);
+}
+
+dcpse_status dcpse_apply_transpose_nnz_f64(dcpse_ctx* ctx, int64_t n_cols, int64_t nnz, const int64_t* rowT_ptr,
+                                           const int32_t* colT, const double* WT, const double* diag, const double* g,
+                                           int64_t ld_g, int32_t n_fields, double* out, int64_t ld_out, double alpha,
+                                           double beta, void* scratch, size_t scratch_bytes) {
+    if (!ctx) return DCPSE_ERR_INVALID;
+    if (!diag) return fail(ctx, DCPSE_ERR_INVALID, "diag is null");
+    const double* Wp[1] = {WT};
+    double* Op[1] = {out};
+    const Counted given{nnz, scratch, scratch_bytes};
+    return apply_impl<double, kExplicitDiag>(ctx, n_cols, rowT_ptr, colT, 1, Wp, g, ld_g, n_fields, nullptr, ld_g, diag,
+                                          Op, ld_out, alpha, beta, &given);
 }
 
 dcpse_status dcpse_axpby_f32(dcpse_ctx* ctx, int64_t n, float alpha, const float* x, float beta, float* y) {

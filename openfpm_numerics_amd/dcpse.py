@@ -401,9 +401,10 @@ class Dcpse:
             ctx.call("dcpse_apply_transpose_sell_f32", n, _lib.ptr(rowT), _lib.ptr(slice_ptr), _lib.ptr(sell_rowT),
                      _lib.ptr(sell_colT), _lib.ptr(sell_WT), _lib.ptr(diag), _lib.ptr(g2), _lib.ptr(o), alpha, beta)
             return o.reshape(g.shape)
-        name = "dcpse_apply_transpose_f32" if g.dtype == torch.float32 else "dcpse_apply_transpose_f64"
-        ctx.call(name, n, _lib.ptr(rowT), _lib.ptr(colT), _lib.ptr(WT), _lib.ptr(diag), _lib.ptr(g2), n, nb,
-                 _lib.ptr(o), n, alpha, beta)
+        name = "dcpse_apply_transpose_nnz_f32" if g.dtype == torch.float32 else "dcpse_apply_transpose_nnz_f64"
+        scratch = _batch_scratch(g2)
+        ctx.call(name, n, self.verletList.nnz, _lib.ptr(rowT), _lib.ptr(colT), _lib.ptr(WT), _lib.ptr(diag),
+                 _lib.ptr(g2), n, nb, _lib.ptr(o), n, alpha, beta, _lib.ptr(scratch), _nbytes(scratch))
         return o.reshape(g.shape)
 
     # ---- persistence (Dcpse.hpp:302-379) -------------------------------------------
@@ -649,6 +650,25 @@ class _SellPlan:
 _FWD = {torch.float32: "fwd", torch.float64: "fwd64"}
 
 
+def _batch_scratch(f2: torch.Tensor):
+    """Memory for the particle-major copies of a batch (B, N) of 3 or more
+    fields, as wide as its widest pass (4, 8 or 16 fields); None for fewer, or
+    where there is no room, and the batch then runs field by field. It comes
+    from torch's allocator, so each stream, and a graph being captured, has
+    its own."""
+    nb, n = f2.shape
+    if nb < 3:
+        return None
+    try:
+        return torch.empty((4 if nb <= 4 else 8 if nb <= 8 else 16) * n, dtype=f2.dtype, device=f2.device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
+def _nbytes(t) -> int:
+    return 0 if t is None else t.numel() * t.element_size()
+
+
 def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = None, alpha=1.0, beta=0.0):
     """Applies several operators that share one Verlet list in a single pass.
 
@@ -706,13 +726,14 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
         plan(f2, _lib.ptr(fd), outs, alpha, beta)
         return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
     W = [op.weights(f.dtype) for op in ops]
-    name = "dcpse_apply_f32" if f.dtype == torch.float32 else "dcpse_apply_f64"
+    name = "dcpse_apply_nnz_f32" if f.dtype == torch.float32 else "dcpse_apply_nnz_f64"
     if len(ops) > 1 and nb > 1:
         res = [apply_ops([op], f, [o], f_domain, alpha, beta)[0] for op, o in zip(ops, outs)]
         return [r.reshape(*f.shape[:-1], n_rows) for r in res]
-    ctx.call(name, n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), len(ops), _lib.ptr_array(W),
+    scratch = _batch_scratch(f2) if fd is None else None
+    ctx.call(name, n_rows, vl.nnz, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), len(ops), _lib.ptr_array(W),
              _lib.ptr(f2), n, nb, _lib.ptr(fd), n_rows if fd is not None else n, _lib.ptr_array(outs), n_rows,
-             alpha, beta)
+             alpha, beta, _lib.ptr(scratch), _nbytes(scratch))
     return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
 
 
@@ -816,11 +837,14 @@ class PreparedApply:
             self.args = (self.ctx.h, vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr), _lib.ptr(sell_row),
                          _lib.ptr(sell_col), len(ops), self.W, _lib.ptr(f2), None, self.O, alpha, beta)
         else:
-            self._keep = (ops, f, outs, [op.weights(f.dtype) for op in ops])
-            self.fn = self.ctx.lib.dcpse_apply_f32 if f.dtype == torch.float32 else self.ctx.lib.dcpse_apply_f64
+            scratch = _batch_scratch(f2) if len(ops) == 1 else None
+            self._keep = (ops, f, outs, [op.weights(f.dtype) for op in ops], scratch)
+            self.fn = (self.ctx.lib.dcpse_apply_nnz_f32 if f.dtype == torch.float32
+                       else self.ctx.lib.dcpse_apply_nnz_f64)
             self.W = _lib.ptr_array(self._keep[3])
-            self.args = (self.ctx.h, vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), len(ops), self.W,
-                         _lib.ptr(f2), n, nb, None, n, self.O, vl.n_rows, alpha, beta)
+            self.args = (self.ctx.h, vl.n_rows, vl.nnz, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), len(ops), self.W,
+                         _lib.ptr(f2), n, nb, None, n, self.O, vl.n_rows, alpha, beta, _lib.ptr(scratch),
+                         _nbytes(scratch))
         lib = self.ctx.lib
         self.layout = next((name for fn, name in ((lib.dcpse_apply_sell_f32, "sell"),
                                                   (lib.dcpse_apply_sell_bundle_f32, "sell_bundle"),
