@@ -237,9 +237,10 @@ dcpse_status dcpse_assemble_multi(dcpse_ctx* ctx, int32_t dim,
  * is the leading part of its support set passes f_self = f and ld_self = ld_f.
  * beta == 0 never reads out. Batches of 3 or more fields of one operator on
  * one set (f_self NULL) are copied particle-major into the context's workspace
- * (16 x n_rows values, grown on first use) and applied up to 16 fields per
- * pass; each field's result equals its single-field apply bit for bit. While
- * the stream is being captured they run field by field (the _nnz entry points
+ * (n_rows values for each of the 4, 8 or 16 fields of a pass, grown on first
+ * use) and applied up to 16 fields per pass; each field's result equals its
+ * single-field apply bit for bit. Where that memory cannot be had, and while
+ * the stream is being captured, they run field by field (the _nnz entry points
  * below have no such limit). The same holds for dcpse_apply_transpose_f32 and
  * _f64. */
 dcpse_status dcpse_apply_f32(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr, const int32_t* col,

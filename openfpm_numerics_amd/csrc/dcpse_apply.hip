@@ -800,13 +800,14 @@ static dcpse_status apply_impl(dcpse_ctx* ctx, int64_t n_rows, const int64_t* ro
         fil = static_cast<T*>(given->scratch);
         width = room >= 16 ? 16 : room >= 8 ? 8 : room >= 4 ? 4 : 0;
     } else if (particle_major && !captured(ctx->stream)) {
+        const size_t room = pass_width(nfields);
         Workspace ws;
-        dcpse_status st = reserve_workspace(ctx, (size_t)n_rows * 16 * sizeof(T) + 256, &ws);
-        if (st) return st;
-        use.emplace(ctx);
-        fil = ws.take<T>((size_t)n_rows * 16);
-        if (!fil) return fail(ctx, DCPSE_ERR_INVALID, "apply workspace sizing error");
-        width = 16;
+        if (reserve_workspace(ctx, (size_t)n_rows * room * sizeof(T) + 256, &ws) == DCPSE_OK) {
+            use.emplace(ctx);
+            fil = ws.take<T>((size_t)n_rows * room);
+            if (!fil) return fail(ctx, DCPSE_ERR_INVALID, "apply workspace sizing error");
+            width = (int)room;
+        }  // no room: field by field
     }
     while (width > 0 && nfields - b0 >= kBatchMin) {
         const int nf = std::min(nfields - b0, width), pass = pass_width(nf);

@@ -242,10 +242,21 @@ dcpse_status reserve_workspace(dcpse_ctx* ctx, size_t bytes, Workspace* w) {
         if (ctx->ws_queued) DCPSE_HIP_CHECK(ctx, hipEventSynchronize(ctx->ws_event));
         DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->ws) DCPSE_HIP_CHECK(ctx, hipFree(ctx->ws));
+        // nothing is left if the larger one cannot be had
+        const size_t grown = std::max(bytes, ctx->ws_size * 2);
         ctx->ws = nullptr;
-        size_t nb = std::max(bytes, ctx->ws_size * 2);
-        DCPSE_HIP_CHECK(ctx, hipMalloc(&ctx->ws, nb));
-        ctx->ws_size = nb;
+        ctx->ws_size = 0;
+        for (size_t nb : {grown, bytes}) {
+            const hipError_t e = hipMalloc(&ctx->ws, nb);
+            if (e == hipSuccess) {
+                ctx->ws_size = nb;
+                break;
+            }
+            (void)hipGetLastError();  // not the next launch's error
+            ctx->ws = nullptr;
+            if (nb == bytes)
+                return fail(ctx, DCPSE_ERR_HIP, "a workspace of %zu bytes: %s", bytes, hipGetErrorString(e));
+        }
     }
     w->base = static_cast<char*>(ctx->ws);
     w->cap = ctx->ws_size;
