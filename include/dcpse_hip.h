@@ -40,6 +40,7 @@
 #ifndef DCPSE_HIP_H
 #define DCPSE_HIP_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __cplusplus
@@ -281,7 +282,8 @@ dcpse_status dcpse_apply_transpose_f64(dcpse_ctx* ctx, int64_t n_cols, const int
 
 /* The same applies with what the host knows of the list and memory of the
  * caller's: nnz (row_ptr[n_rows]) picks the launch shape, so nothing is read
- * back; scratch (device, 16-byte aligned, scratch_bytes long, NULL for none)
+ * back (the entry points above read it at the first call on a row_ptr and
+ * n_rows and keep the shape for that address); scratch (device, 16-byte aligned, scratch_bytes long, NULL for none)
  * takes the particle-major copies of a batch instead of the context's
  * workspace: n_rows values per field of a pass, which has 4, 8 or 16 fields,
  * the smallest that holds the batch serving it best. With less, passes are

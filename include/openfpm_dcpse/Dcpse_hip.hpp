@@ -140,14 +140,16 @@ class Dcpse_hip : public openfpm_dcpse::field_operator<typename vector_type::pro
         prop_type* O[1] = {out};
         if constexpr (std::is_same<prop_type, float>::value) {
             const float* W[1] = {W32_.data()};
-            c.check(dcpse_apply_f32(c.get(), n, verletList_.devRowPtr(), verletList_.devCol(), 1, W, f, n_sup, 1,
-                                    f_self, n, O, n, alpha, beta),
-                    "dcpse_apply_f32");
+            c.check(dcpse_apply_nnz_f32(c.get(), n, (int64_t)verletList_.nnz(), verletList_.devRowPtr(),
+                                        verletList_.devCol(), 1, W, f, n_sup, 1, f_self, n, O, n, alpha, beta, nullptr,
+                                        0),
+                    "dcpse_apply_nnz_f32");
         } else {
             const double* W[1] = {w64()};
-            c.check(dcpse_apply_f64(c.get(), n, verletList_.devRowPtr(), verletList_.devCol(), 1, W, f, n_sup, 1,
-                                    f_self, n, O, n, alpha, beta),
-                    "dcpse_apply_f64");
+            c.check(dcpse_apply_nnz_f64(c.get(), n, (int64_t)verletList_.nnz(), verletList_.devRowPtr(),
+                                        verletList_.devCol(), 1, W, f, n_sup, 1, f_self, n, O, n, alpha, beta, nullptr,
+                                        0),
+                    "dcpse_apply_nnz_f64");
         }
     }
 
@@ -185,9 +187,9 @@ class Dcpse_hip : public openfpm_dcpse::field_operator<typename vector_type::pro
                 return;
             }
             const float* W[1] = {W32_.data()};
-            c.check(dcpse_apply_f32(c.get(), n, verletList_.devRowPtr(), verletList_.devCol(), 1, W, f, n, 1,
-                                    nullptr, n, O, n, alpha, beta),
-                    "dcpse_apply_f32");
+            c.check(dcpse_apply_nnz_f32(c.get(), n, (int64_t)verletList_.nnz(), verletList_.devRowPtr(),
+                                        verletList_.devCol(), 1, W, f, n, 1, nullptr, n, O, n, alpha, beta, nullptr, 0),
+                    "dcpse_apply_nnz_f32");
         } else {
             double* O[1] = {out};
             if (n > 0 && !s64_tried_ && ++n_apply64_ >= kSellAfter) build_sell64();
@@ -208,9 +210,9 @@ class Dcpse_hip : public openfpm_dcpse::field_operator<typename vector_type::pro
                 return;
             }
             const double* W[1] = {w64()};
-            c.check(dcpse_apply_f64(c.get(), n, verletList_.devRowPtr(), verletList_.devCol(), 1, W, f, n, 1,
-                                    nullptr, n, O, n, alpha, beta),
-                    "dcpse_apply_f64");
+            c.check(dcpse_apply_nnz_f64(c.get(), n, (int64_t)verletList_.nnz(), verletList_.devRowPtr(),
+                                        verletList_.devCol(), 1, W, f, n, 1, nullptr, n, O, n, alpha, beta, nullptr, 0),
+                    "dcpse_apply_nnz_f64");
         }
     }
 

@@ -703,16 +703,17 @@ static ApplyShape shape_of(dcpse_ctx* ctx, int64_t n_rows, int64_t nnz) {
 
 // The same where the caller gives no nnz: read once per (row_ptr, n_rows) and
 // cached in the context, so repeated applies of one operator never synchronise
-// the stream.
+// the stream. (Another list at the same address, with as many rows, gets the
+// shape of the first: another order of summation, and slower. The *_nnz entry
+// points have no such memory.)
 static ApplyShape auto_shape(dcpse_ctx* ctx, int64_t n_rows, const int64_t* row_ptr) {
     if (ctx->apply_group > 0) return {ctx->apply_group, ctx->apply_epl, ctx->apply_vec, 0.0};
     if (ctx->grp_rows == row_ptr && ctx->grp_n == n_rows) return {ctx->grp_g, ctx->grp_epl, ctx->grp_vec, ctx->grp_mean};
     int64_t nnz = 0;
-    ApplyShape sh{8, 8, 4, 0.0};
-    if (n_rows > 0 &&
-        hipMemcpyAsync(&nnz, row_ptr + n_rows, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream) == hipSuccess &&
-        hipStreamSynchronize(ctx->stream) == hipSuccess)
-        sh = shape_of(ctx, n_rows, nnz);
+    if (hipMemcpyAsync(&nnz, row_ptr + n_rows, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+        hipStreamSynchronize(ctx->stream) != hipSuccess)
+        return {8, 8, 4, 0.0};  // not kept: the next call looks again
+    const ApplyShape sh = shape_of(ctx, n_rows, nnz);
     ctx->grp_rows = row_ptr;
     ctx->grp_n = n_rows;
     ctx->grp_g = sh.G;
