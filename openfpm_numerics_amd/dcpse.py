@@ -28,7 +28,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .particles import ParticleSet, ParticleSubset, VerletList, sell_layout, sell_weights
+from .particles import ParticleSet, ParticleSubset, VerletList, capturing, sell_layout, sell_weights
 
 # support_options (src/DCPSE/SupportBuilder.hpp:13-19)
 RADIUS = 0
@@ -211,21 +211,28 @@ class Dcpse:
             W = torch.empty(max(vl.nnz, 1), dtype=torch.float64, device=K.device)
             _lib.context(K.device.index or 0).call("dcpse_scale_rows_f64", vl.n_rows, _lib.ptr(vl.row_ptr),
                                                    _lib.ptr(K), _lib.ptr(self.localEpsInvPow), _lib.ptr(W))
-            self._W[dtype] = W[:vl.nnz]
+            W = W[:vl.nnz]
+            if capturing():
+                return W
+            self._W[dtype] = W
         if dtype not in self._W:
             raise TypeError(f"no weights for {dtype}; use float32 or float64")
         return self._W[dtype]
 
     def sell_weights(self) -> torch.Tensor:
         """FP32 weights in the sliced-ELL layout of this operator's Verlet list."""
-        if self._W.get("sell") is None:
-            self._W["sell"] = sell_weights(self.verletList.row_ptr, self._W[torch.float32],
-                                           self.verletList.sell_slices(), self.verletList.n_rows)
-        return self._W["sell"]
+        sw = self._W.get("sell")
+        if sw is None:
+            sw = sell_weights(self.verletList.row_ptr, self._W[torch.float32], self.verletList.sell_slices(),
+                              self.verletList.n_rows)
+            if not capturing():
+                self._W["sell"] = sw
+        return sw
 
     def sell_weights64(self) -> torch.Tensor:
         """FP64 weights in the sliced-ELL layout of this operator's Verlet list."""
-        if self._W.get("sell64") is None:
+        sw = self._W.get("sell64")
+        if sw is None:
             vl = self.verletList
             slice_ptr, sell_row, n_slots = vl.sell_slices()
             sw = torch.empty(max(n_slots, 4), dtype=torch.float64, device=vl.row_ptr.device)
@@ -237,16 +244,20 @@ class Dcpse:
                 ctx.call("dcpse_sell_fill_weights_scaled_f64", vl.n_rows, _lib.ptr(vl.row_ptr),
                          _lib.ptr(self.calcKernels), _lib.ptr(self.localEpsInvPow), _lib.ptr(slice_ptr),
                          _lib.ptr(sell_row), _lib.ptr(sw))
-            self._W["sell64"] = sw
-        return self._W["sell64"]
+            if not capturing():
+                self._W["sell64"] = sw
+        return sw
 
     def sell_bundle16(self, dtype=torch.float32):
         """This operator alone as a 16-bit-offset bundle (see sell_bundle16)
         with FP32 or FP64 weights, built once per assembly."""
         key = "bundle16" if dtype == torch.float32 else "bundle16_64"
-        if self._W.get(key) is None:
-            self._W[key] = sell_bundle16([self], dtype)
-        return self._W[key]
+        b16 = self._W.get(key)
+        if b16 is None:
+            b16 = sell_bundle16([self], dtype)
+            if not capturing():
+                self._W[key] = b16
+        return b16
 
     def bundle16_suits(self) -> bool:
         """Whether the 16-bit bundle is the faster FP32 layout of this operator:
@@ -719,7 +730,7 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
     ctx = _lib.context(f.device.index or 0)
     if nb == 1 and USE_SELL and all([op._count_apply32(_FWD[f.dtype]) for op in ops]):
         plan = _SellPlan(ops, vl, f.dtype, fd is not None)
-        if fd is None and ops[0].same_set:
+        if fd is None and ops[0].same_set and not capturing():
             if len(ops[0]._plans) >= 8:
                 ops[0]._plans.clear()
             ops[0]._plans[key] = plan

@@ -179,6 +179,12 @@ def morton_order(pos: np.ndarray, box_lo, box_hi, bits: int | None = None) -> np
     return np.argsort(code, kind="stable")
 
 
+def capturing() -> bool:
+    """Whether the current stream is being captured into a graph: what is built
+    now has its values only when the graph is replayed, so nothing keeps it."""
+    return torch.cuda.is_current_stream_capturing()
+
+
 class VerletList:
     """Neighbour CSR in HBM: row_ptr int64[n+1], col int32[nnz]."""
 
@@ -277,11 +283,13 @@ class VerletList:
         """(slice_ptr, sell_row, sell_col): the sliced-ELL execution layout of
         this support with 32-bit columns, shared by every FP32 operator
         assembled on it; built on first use."""
-        if getattr(self, "_sell", None) is None:
+        layout = getattr(self, "_sell", None)
+        if layout is None:
             slice_ptr, sell_row, n_slots = self.sell_slices()
-            self._sell = (slice_ptr, sell_row, sell_cols(self.row_ptr, self.col, self.n_rows, slice_ptr, sell_row,
-                                                         n_slots))
-        return self._sell
+            layout = slice_ptr, sell_row, sell_cols(self.row_ptr, self.col, self.n_rows, slice_ptr, sell_row, n_slots)
+            if not capturing():
+                self._sell = layout
+        return layout
 
     def far16(self):
         """(exc_ptr, n_exc): the neighbours whose plain 16-bit offset does not fit,
