@@ -60,24 +60,29 @@ def _dcpse(op) -> Dcpse:
 _NAMES = {"bundle16": "bundle16_", "col16": "col16_", "sell": "sell_", "csr": ""}
 
 
-def _operator_args(d: Dcpse, dtype, layout: str):
-    """The library arguments that describe operator d on a layout, after n_rows."""
+def _operator(d: Dcpse, dtype, layout: str):
+    """The arrays and counts that describe operator d on a layout, as the library
+    takes them after n_rows; held by the caller until the call that uses them has
+    been made (inside a graph capture nothing else holds what is built for it)."""
     vl = d.verletList
-    p = _lib.ptr
     if layout == "bundle16":
         bundle, row16, exc_ptr, exc_col, exc_W, ne = d.sell_bundle16(dtype)
-        return p(vl.row_ptr), p(vl.sell_slices()[0]), p(row16), p(bundle), p(exc_ptr), p(exc_col), p(exc_W), ne
+        return [vl.row_ptr, vl.sell_slices()[0], row16, bundle, exc_ptr, exc_col, exc_W, ne]
     W = (d.sell_weights if dtype == torch.float32 else d.sell_weights64)
     if layout == "col16":
         c16 = d.col16()
         if c16 is None:
             raise ValueError("too many neighbours of this list do not fit 16-bit columns")
-        return (p(vl.row_ptr), *map(p, c16[:-1]), c16[-1], p(W()))
+        return [vl.row_ptr, *c16, W()]
     if layout == "sell":
-        return (p(vl.row_ptr), *map(p, vl.sell()), p(W()))
+        return [vl.row_ptr, *vl.sell(), W()]
     if layout == "csr":
-        return p(vl.row_ptr), p(vl.col), p(d.weights(dtype))
+        return [vl.row_ptr, vl.col, d.weights(dtype)]
     raise ValueError(f"unknown layout {layout!r}")
+
+
+def _args(held):
+    return [x if isinstance(x, int) else _lib.ptr(x) for x in held]
 
 
 def rk4(op, f: torch.Tensor, dt: float, n_steps: int, alpha: float = 1.0, layout: str = "auto",
@@ -112,8 +117,8 @@ def rk4(op, f: torch.Tensor, dt: float, n_steps: int, alpha: float = 1.0, layout
     p = _lib.ptr
     t = "f32" if f.dtype == torch.float32 else "f64"
     end = (float(alpha), float(dt), int(n_steps), p(f), p(work))
-    args = _operator_args(d, f.dtype, layout)
-    ctx.call(f"dcpse_rk4_{_NAMES[layout]}{t}", n, *args, *end)
+    held = _operator(d, f.dtype, layout)
+    ctx.call(f"dcpse_rk4_{_NAMES[layout]}{t}", n, *_args(held), *end)
     return f
 
 
@@ -129,6 +134,6 @@ def stage(op, u: torch.Tensor, alpha: float, y_a: torch.Tensor | None, ca: float
     p = _lib.ptr
     layout = _layout(d, u.dtype, layout, 1)
     t = "f32" if u.dtype == torch.float32 else "f64"
-    args = _operator_args(d, u.dtype, layout)
-    ctx.call(f"dcpse_stage_{_NAMES[layout]}{t}", vl.n_rows, *args, p(u), float(alpha), p(y_a), float(ca), p(out_a),
+    held = _operator(d, u.dtype, layout)
+    ctx.call(f"dcpse_stage_{_NAMES[layout]}{t}", vl.n_rows, *_args(held), p(u), float(alpha), p(y_a), float(ca), p(out_a),
              p(y_b), float(cb), p(out_b))

@@ -27,11 +27,13 @@ def _runs(A, name):
         "fused": lambda lap, dx, f: A.fused(dx, lap, f=f),
         "batch": lambda lap, dx, f: [dx(torch.stack([f, 2 * f, 3 * f, 4 * f]))],
         "rk4": lambda lap, dx, f: [A.rk4(dx, f.clone(), 1e-4, 2)],
+        "rk4_sell": lambda lap, dx, f: [A.rk4(dx, f.clone(), 1e-4, 2, layout="sell")],
+        "rk4_bundle16": lambda lap, dx, f: [A.rk4(dx, f.clone(), 1e-4, 2, layout="bundle16")],
     }[name]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("name", ["apply", "fused", "batch", "rk4"])
+@pytest.mark.parametrize("name", ["apply", "fused", "batch", "rk4", "rk4_sell", "rk4_bundle16"])
 def test_first_use_in_a_capture(cuda, name, dtype):
     import openfpm_numerics_amd as A
 
