@@ -274,6 +274,16 @@ class Dcpse:
         do not fit; else None."""
         return self.verletList.col16(BUNDLE16_MAX_EXC) if self.same_set else None
 
+    def sell_ready64(self) -> bool:
+        """Whether the FP64 sliced-ELL copy that suits this operator is built, so
+        that using it waits for nothing."""
+        vl = self.verletList
+        if not vl.counted("bundle16"):
+            return False
+        if self.bundle16_suits():
+            return self._W.get("bundle16_64") is not None
+        return self._W.get("sell64") is not None and vl.counted("col16") and (self.col16() or vl._sell) is not None
+
     def computeDifferentialOperator(self, f: torch.Tensor, out: torch.Tensor | None = None,
                                     f_domain: torch.Tensor | None = None, alpha=1.0, beta=0.0):
         """D f for a field (N,) or a batch of fields (B, N) over the support set."""

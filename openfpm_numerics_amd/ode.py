@@ -15,6 +15,7 @@ import torch
 from . import _lib
 from . import dcpse as _dcpse_module
 from .dcpse import Dcpse
+from .particles import capturing
 
 #: Neighbours up to which "auto" stays on the CSR kernel: its eight lanes per
 #: row keep a small set busy where the sliced-ELL layouts' one lane does not
@@ -22,30 +23,37 @@ from .dcpse import Dcpse
 #: in 2D 6.6 / 8.2, 131,000 in 2D 9.1 / 8.6; FP64 30,000 5.4 / 7.7, 90,000 8.3 /
 #: 8.2)
 CSR_MAX = {torch.float32: 3_600_000, torch.float64: 2_600_000}
-#: FP64 stages since assembly from which "auto" builds the sliced-ELL copy of a
+#: FP64 stages of one call from which "auto" runs on the sliced-ELL copy of a
 #: list of at least SELL64_LARGE neighbours, or of a smaller one, whose weights
-#: the last-level cache holds: it costs 0.2 to 0.5 ms and saves 20 us per stage
-#: at 77^3 particles, 3 us at 64^3
+#: the last-level cache holds: building it costs 0.2 to 0.5 ms and saves 20 us
+#: per stage at 77^3 particles, 3 us at 64^3
 SELL64_AFTER = 12
 SELL64_LARGE = 16_000_000
 SELL64_AFTER_SMALL = 64
 
 
+_NAMES = {"bundle16": "bundle16_", "col16": "col16_", "sell": "sell_", "csr": ""}
+
+
 def _layout(d: Dcpse, dtype, layout: str, stages: int) -> str:
-    """The layout a call of this many stages runs on."""
+    """The layout a call of this many stages runs on. In FP64 it follows from
+    the list and the call alone, so equal calls give equal bits; only a call
+    under graph capture, which may not wait for the copy's counts, runs on CSR
+    where the copy is not there."""
+    nnz = d.verletList.nnz
     if dtype == torch.float32:
         if layout != "auto":
             return layout
         d._n32["fwd"] += stages - 1
         ready = d._count_apply32("fwd")
     else:
-        if layout in ("bundle16", "col16", "sell", "csr"):
-            return layout
-        d._n32["stage64"] = d._n32.get("stage64", 0) + stages
-        after = SELL64_AFTER if d.verletList.nnz >= SELL64_LARGE else SELL64_AFTER_SMALL
-        ready = (d._n32["stage64"] >= max(after, _dcpse_module.SELL_AFTER) or d._W.get("bundle16_64") is not None
-                 or d._W.get("sell64") is not None)
-    if not ready or d.verletList.n_rows == 0 or d.verletList.nnz <= CSR_MAX[dtype]:
+        if layout in _NAMES:
+            return "csr" if capturing() and not d.verletList.counted(layout) else layout
+        after = SELL64_AFTER if nnz >= SELL64_LARGE else SELL64_AFTER_SMALL
+        ready = stages >= max(after, _dcpse_module.SELL_AFTER)
+    if not ready or d.verletList.n_rows == 0 or nnz <= CSR_MAX[dtype]:
+        return "csr"
+    if dtype == torch.float64 and capturing() and not d.sell_ready64():
         return "csr"
     return "bundle16" if d.bundle16_suits() else "col16" if d.col16() is not None else "sell"
 
@@ -55,9 +63,6 @@ def _dcpse(op) -> Dcpse:
     if not d.same_set:
         raise ValueError("time integration needs an operator whose support and domain sets are the same")
     return d
-
-
-_NAMES = {"bundle16": "bundle16_", "col16": "col16_", "sell": "sell_", "csr": ""}
 
 
 def _operator(d: Dcpse, dtype, layout: str):
@@ -92,12 +97,14 @@ def rk4(op, f: torch.Tensor, dt: float, n_steps: int, alpha: float = 1.0, layout
     float32 and float64 state run the kernels of their type on layout "bundle16"
     (sliced-ELL with 16-bit column offsets, the fewest bytes), "col16" (the
     list's 16-bit columns), "sell" (32-bit columns), "csr", or "auto": "csr" up
-    to ``CSR_MAX`` neighbours; above, the 4 n_steps stage applies count towards
-    the operator's ``dcpse.SELL_AFTER`` (FP64: ``SELL64_AFTER`` stages,
-    ``SELL64_AFTER_SMALL`` below ``SELL64_LARGE`` neighbours, or a copy that is
-    there) and run on "bundle16" once it is reached (its copy is then built;
-    "col16", then "sell", where too many neighbours do not fit,
-    ``dcpse.BUNDLE16_MAX_EXC``), on "csr" before.
+    to ``CSR_MAX`` neighbours; above, in FP32, the 4 n_steps stage applies count
+    towards the operator's ``dcpse.SELL_AFTER`` and run on "bundle16" once it is
+    reached (its copy is then built; "col16", then "sell", where too many
+    neighbours do not fit, ``dcpse.BUNDLE16_MAX_EXC``), on "csr" before; in FP64
+    a call of at least ``SELL64_AFTER`` stages (``SELL64_AFTER_SMALL`` below
+    ``SELL64_LARGE`` neighbours, ``dcpse.SELL_AFTER`` if that is larger) runs on
+    it, a shorter one on "csr", as does one being captured before the copy was
+    built.
     ``work`` (3N of f's dtype) may be passed to avoid an allocation per call.
     """
     d = _dcpse(op)

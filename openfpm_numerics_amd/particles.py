@@ -304,6 +304,12 @@ class VerletList:
             self._far16 = (exc_ptr, int(n_exc[0]))
         return self._far16
 
+    def counted(self, layout: str) -> bool:
+        """Whether what a layout ("csr", "sell", "bundle16", "col16") of this list
+        needs counted is counted, so that its first use waits for nothing."""
+        known = {"sell": self._slices, "bundle16": self._far16, "col16": self._col16}
+        return layout not in known or known[layout] is not None
+
     def col16(self, max_far: float):
         """The 16-bit columns of the sliced-ELL layout (one particle set; see
         dcpse_sell_fill_col16), shared by every operator on this list: the
