@@ -1535,9 +1535,11 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
         for (int d = 0; d < dim; ++d)
             if ((periodic >> d) & 1u) grouped = grouped && box_hi[d] - box_lo[d] > (kHomeEdge + 2.1) * rmax;
         int K = (int)std::min(dim == 3 ? 8.0 : 16.0, std::ceil(2.0 * spread - 1e-9));
-        for (; grouped && K >= 1; --K) {
-            if ((st = make_grid(ctx, dim, box_lo, box_hi, periodic, rmax, K, &g))) return st;
-            if (g.ncell <= 8 * n_sup + 4096 || K == 1) break;
+        for (; grouped; --K) {
+            // (one cell per cut-off needs three cut-offs of a periodic
+            // dimension, the scans of a wavefront per particle 2.5)
+            grouped = make_grid(ctx, dim, box_lo, box_hi, periodic, rmax, K, &g) == DCPSE_OK;
+            if (!grouped || g.ncell <= 8 * n_sup + 4096 || K == 1) break;
         }
         nws = dim == 3 ? 8 : 4;
     }
