@@ -1402,6 +1402,14 @@ static void launch_groups(int dim, int nws, F launch) {
     else width(std::integral_constant<int, 3>());
 }
 
+// Home cells of a set too sparse to fill them. A home cell takes 24 bytes and a
+// few passes; up to this many groups are faster than a wavefront per particle
+// (300,000 particles of 47 neighbours in one corner, us with groups / without:
+// 4.8M cells 459 / 1268, 19M 863 / 1708, 38M 1385 / 2049) and the memory is no
+// more than that of the cells make_grid allows (6.7e7 of 12 bytes); a box of 500
+// cut-offs a side would have 2e8.
+constexpr double kMaxHomeCells = 3.4e7;
+
 // The home levels of a set with cut-offs in [rmin, rmax]: a level for every
 // halving, as long as their cells number a few per particle.
 static void make_levels(int dim, const double* box_lo, const double* box_hi, unsigned periodic, double rmin,
@@ -1428,8 +1436,8 @@ static void make_levels(int dim, const double* box_lo, const double* box_hi, uns
         }
         if (total + cells > 4.0 * (double)n + 4096.0 && l > 0) break;
         total += cells;
-        if (total > 1e9) {  // (level 0 of a sparse set: not worth grouping)
-            h->n = 0;
+        if (total > std::min(std::max(kMaxHomeCells, 4.0 * (double)n + 4096.0), 1e9)) {
+            h->n = 0;  // level 0 of a large and nearly empty box
             return;
         }
         g.ncell = (int64_t)cells;

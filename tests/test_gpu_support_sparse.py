@@ -38,3 +38,30 @@ def test_narrow_periodic_strip(cuda, dim, across):
     rp, col = _brute(pos, rc, [0.0] * dim, hi, bc)
     assert len(col) > n // 4
     assert np.array_equal(vl.row_ptr.cpu().numpy(), rp) and np.array_equal(vl.col.cpu().numpy(), col)
+
+
+def test_memory_of_a_nearly_empty_box(cuda):
+    """500 cut-offs a side: no more memory than the cells of a search without
+    groups (6.7e7 of 12 bytes, and as much again for a workspace that doubled)."""
+    from openfpm_numerics_amd import _lib
+
+    n, side = 2000, 500.0
+    rng = np.random.default_rng(0)
+    pos = rng.uniform(240.0, 246.0, (n, 3))
+    rc = rng.uniform(0.9, 1.0, n)
+    rc[0] = 1.0
+    soa = torch.as_tensor(pos.T.copy(), device=cuda)
+    rcd = torch.as_tensor(rc, device=cuda)
+    lo, hi = np.zeros(3), np.full(3, side)
+    rp = torch.empty(n + 1, dtype=torch.int64, device=cuda)
+    nnz = np.zeros(1, np.int64)
+    ctx, p = _lib.Context(cuda.index or 0), _lib.ptr
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    args = (3, p(soa), n, None)
+    ctx.call("dcpse_support_count", *args, n, p(rcd), 1, p(lo), p(hi), 0, p(rp), p(nnz))
+    assert free - torch.cuda.mem_get_info()[0] < 2 * 12 * 6.7e7 + 64e6
+    col = torch.empty(int(nnz[0]), dtype=torch.int32, device=cuda)
+    ctx.call("dcpse_support_fill_counted", *args, None, n, p(rcd), 1, p(lo), p(hi), 0, p(rp), p(col))
+    want = _brute(pos, rc, lo, hi, [0, 0, 0])
+    assert np.array_equal(rp.cpu().numpy(), want[0]) and np.array_equal(col.cpu().numpy(), want[1])
