@@ -133,9 +133,10 @@ int32_t dcpse_rhs(int32_t dim, const uint32_t* beta, uint32_t order, double* b, 
  * count: writes row_ptr[0..n_dom] (device int64) and *nnz (host; this call
  * synchronises the stream). fill: writes col[nnz] (device int32), for the
  * same arguments as the count and unchanged positions. With one set and one
- * cut-off, the context keeps the count's cell list and per-particle take
- * masks (about 64 bytes per particle) and a fill that directly follows a
- * count with the same arguments gathers its rows from them. */
+ * cut-off, the context keeps the count's cell list, candidate lists and
+ * per-particle take masks, and a fill that directly follows a count with the
+ * same arguments writes its rows from them; with a cut-off per particle only
+ * dcpse_support_fill_counted does, and this fill searches again. */
 dcpse_status dcpse_support_count(dcpse_ctx* ctx, int32_t dim,
                                  const double* pos_sup, int64_t n_sup,
                                  const double* pos_dom, int64_t n_dom,
@@ -178,9 +179,10 @@ dcpse_status dcpse_support_count_one(dcpse_ctx* ctx, int32_t dim,
                                      const double* box_lo, const double* box_hi, uint32_t periodic_mask,
                                      int64_t* row_ptr, int64_t* nnz);
 /* dcpse_support_fill (dom_ids NULL) or _fill_subset as the next call on this
- * context after the count with the same arguments and data: the extremes of
- * the cut-offs are those of the count instead of being reduced and read back
- * again. */
+ * context after the count with the same arguments and data, unchanged in
+ * place: the extremes of the cut-offs are those of the count instead of being
+ * reduced and read back again, and the rows of one set are written from what
+ * the count kept. After a count of other arguments it searches again. */
 dcpse_status dcpse_support_fill_counted(dcpse_ctx* ctx, int32_t dim,
                                         const double* pos_sup, int64_t n_sup,
                                         const double* pos_dom, const int32_t* dom_ids, int64_t n_dom,

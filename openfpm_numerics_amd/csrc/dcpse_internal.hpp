@@ -22,6 +22,7 @@ struct dcpse_support_cache {
     int64_t n = 0;
     double rcut = 0.0, rmin = 0.0;  // largest and smallest cut-off
     int rcut_pp = 0;      // a cut-off per particle
+    const double* rcuts = nullptr;
     double lo[3] = {0.0, 0.0, 0.0}, hi[3] = {0.0, 0.0, 0.0};
     unsigned periodic = 0;
     int nws = 0;          // mask words per particle

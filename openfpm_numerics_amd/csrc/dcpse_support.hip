@@ -1567,10 +1567,13 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
     const int64_t max_groups = !compact ? n_home : pp ? std::min(n_sup, n_sup / 4 + 4096) : n_sup;
 
     // the fill of one set reuses the cell list, candidate lists and take masks
-    // of the count just before it when the arguments match
+    // of the count just before it when the arguments match; with a cut-off per
+    // particle, whose values the key does not hold, only where the caller says
+    // that they are the count's
     const bool count_pass = col == nullptr;
     const bool cached = grouped && !count_pass && sc.valid && sc.dim == dim && sc.pos == pos_sup &&
                         sc.n == n_sup && sc.rcut == rmax && sc.rmin == rmin && sc.rcut_pp == rcut_pp &&
+                        (!rcut_pp || (continues && sc.rcuts == rcut)) &&
                         sc.periodic == periodic && sc.nws == nws &&
                         std::equal(box_lo, box_lo + dim, sc.lo) && std::equal(box_hi, box_hi + dim, sc.hi);
     sc.valid = false;
@@ -1759,6 +1762,7 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
             sc.rcut = rmax;
             sc.rmin = rmin;
             sc.rcut_pp = rcut_pp;
+            sc.rcuts = rcut;
             sc.periodic = periodic;
             sc.nws = nws;
             for (int d = 0; d < 3; ++d) {
