@@ -19,8 +19,10 @@ dcpse_status dcpse_ctx_create(dcpse_ctx** out, int32_t device) {
     dcpse_ctx* ctx = new dcpse_ctx();
     ctx->device = device;
     hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
+    if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0) {
         ctx->num_cus = prop.multiProcessorCount;
+        ctx->sup.keep = prop.totalGlobalMem / 16;
+    }
     // the device's default (null) stream until the caller binds another one
     ctx->stream = nullptr;
     if (noalloc_scratch_init(ctx) != DCPSE_OK) {

@@ -13,8 +13,8 @@
 // support count of one set; the fill that follows with the same arguments
 // writes its rows from them instead of repeating the distance tests.
 struct dcpse_support_cache {
-    void* buf = nullptr;  // grow-only device buffer
-    size_t cap = 0;
+    void* buf = nullptr;  // device buffer, kept up to `keep` bytes
+    size_t cap = 0, keep = ~size_t(0);
     bool valid = false;
     bool spill = false;   // some particles are left to the position kernel
     int dim = 0;

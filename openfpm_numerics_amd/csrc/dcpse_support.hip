@@ -1789,6 +1789,11 @@ static dcpse_status support_pass(dcpse_ctx* ctx, int dim, const double* pos_sup,
         DCPSE_LAUNCH_CHECK(ctx);
         DCPSE_HIP_CHECK(ctx, hipStreamSynchronize(s));
         const int32_t ovf = (int32_t)ctx->host[0];
+        if (sc.cap > sc.keep) {  // a large set's lists are not kept (25M particles and more)
+            (void)hipFree(sc.buf);
+            sc.buf = nullptr;
+            sc.cap = 0;
+        }
         if (ovf & 3)
             return fail(ctx, DCPSE_ERR_INVALID,
                         "support fill disagrees with row_ptr (positions or rcut changed since count?)");

@@ -65,3 +65,34 @@ def test_memory_of_a_nearly_empty_box(cuda):
     ctx.call("dcpse_support_fill_counted", *args, None, n, p(rcd), 1, p(lo), p(hi), 0, p(rp), p(col))
     want = _brute(pos, rc, lo, hi, [0, 0, 0])
     assert np.array_equal(rp.cpu().numpy(), want[0]) and np.array_equal(col.cpu().numpy(), want[1])
+
+
+def test_large_lists_are_given_back(cuda):
+    """The candidate lists of 30M particles with a cut-off each (650 bytes per
+    particle, more than a sixteenth of the memory) go with the fill; those of a
+    small set stay for the next count, and both searches repeat."""
+    from openfpm_numerics_amd import _lib
+
+    ctx, p = _lib.Context(cuda.index or 0), _lib.ptr
+    lo, hi = np.zeros(3), np.ones(3)
+    kept = []
+    for n in (30_000_000, 100_000):
+        gen = torch.Generator("cuda").manual_seed(n)
+        soa = torch.rand((3, n), generator=gen, dtype=torch.float64, device=cuda)
+        h = (1.0 / n) ** (1 / 3)
+        rc = h * (1.0 + 0.2 * torch.rand(n, generator=gen, dtype=torch.float64, device=cuda))
+        rp = torch.empty(n + 1, dtype=torch.int64, device=cuda)
+        nnz = np.zeros(1, np.int64)
+        args = (3, p(soa), n, None)
+        box = (p(lo), p(hi), 7, p(rp))
+        ctx.call("dcpse_support_count", *args, n, p(rc), 1, *box, p(nnz))
+        cols = [torch.full((int(nnz[0]),), -1, dtype=torch.int32, device=cuda) for _ in range(2)]
+        torch.cuda.synchronize()
+        held = torch.cuda.mem_get_info()[0]
+        ctx.call("dcpse_support_fill_counted", *args, None, n, p(rc), 1, *box, p(cols[0]))
+        kept.append(torch.cuda.mem_get_info()[0] - held)
+        ctx.call("dcpse_support_fill", *args, n, p(rc), 1, *box, p(cols[1]))
+        assert torch.equal(*cols)
+        del soa, rc, rp, cols
+    assert kept[0] > torch.cuda.get_device_properties(cuda).total_memory // 16
+    assert kept[1] == 0
