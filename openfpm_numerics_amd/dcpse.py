@@ -23,6 +23,7 @@ import ctypes as C
 import math
 import os
 import struct
+import weakref
 
 import numpy as np
 import torch
@@ -617,7 +618,8 @@ class _SellPlan:
     the library function and its arguments up to the field, and the tensors
     they point into. It counts as long as the kernels, the list and the module's
     settings are those it was made from (tokens: an assembly, a load and a new
-    list bring new ones; the other operators' are part of its key)."""
+    list bring new ones; the other operators' are part of its key) and the other
+    operators' weights, which only they hold, are there."""
 
     def __init__(self, ops, vl, dtype, n_domain: bool):
         p = _lib.ptr
@@ -629,7 +631,7 @@ class _SellPlan:
         self.n, self.n_rows = vl.n_cols, vl.n_rows
         self.outs_type = C.c_void_p * len(ops)
         self.domain = True  # the function takes the field on the domain
-        c16 = None
+        self.others = ()
         if len(ops) == 1 and ops[0].bundle16_suits():
             # one operator: its 16-bit-offset bundle, built once per assembly
             *keep, ne = ops[0].sell_bundle16(dtype)
@@ -639,23 +641,32 @@ class _SellPlan:
             args = (p(vl.row_ptr), p(slice_ptr), p(row16), 1, p(bundle), p(exc_ptr), p(exc_col), p(exc_W), ne)
         else:
             W = [op.sell_weights() if dtype == torch.float32 else op.sell_weights64() for op in ops]
+            self.built = W  # inside a graph capture the operators do not hold them
             c16 = None if n_domain or (vl.nnz <= COL16_MIN and not vl._col16) else ops[0].col16()
             self.W = _lib.ptr_array(W)
             if c16 is not None:
-                name, keep, self.domain = "dcpse_apply_col16_", [vl.row_ptr, *c16[:-1], *W], False
+                name, keep, self.domain = "dcpse_apply_col16_", [vl.row_ptr, *c16[:-1], W[0]], False
                 args = (p(vl.row_ptr), *map(p, c16[:-1]), c16[-1], len(ops), self.W)
             else:  # 32-bit columns
-                name, keep = "dcpse_apply_sell_", [vl.row_ptr, *vl.sell(), *W]
+                name, keep = "dcpse_apply_sell_", [vl.row_ptr, *vl.sell(), W[0]]
                 args = (*map(p, keep[:4]), len(ops), self.W)
         self.name = name + t
         self.keep = keep
         self.fn = getattr(self.ctx.lib, self.name)
         self.args = (self.ctx.h, self.n_rows, *args)
 
+    def keep_for_later(self):
+        """The other operators' weights are theirs: those of an operator that is
+        assembled again or dropped are not held by this one's plans."""
+        if "built" in self.__dict__:
+            self.others = tuple(weakref.ref(W) for W in self.built[1:])
+            del self.built
+        return self
+
     def counts_for(self, ops, vl) -> bool:
         tokens = self.tokens
         return (tokens[0] is vl._gen and self.max_exc == BUNDLE16_MAX_EXC
-                and ops[0]._gen is tokens[1])
+                and ops[0]._gen is tokens[1] and all([W() is not None for W in self.others]))
 
     def __call__(self, f, fd, outs, alpha, beta):
         self.ctx.bind_current_stream()
@@ -740,11 +751,11 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
     ctx = _lib.context(f.device.index or 0)
     if nb == 1 and USE_SELL and all([op._count_apply32(_FWD[f.dtype]) for op in ops]):
         plan = _SellPlan(ops, vl, f.dtype, fd is not None)
+        plan(f2, _lib.ptr(fd), outs, alpha, beta)
         if fd is None and ops[0].same_set and not capturing():
             if len(ops[0]._plans) >= 8:
                 ops[0]._plans.clear()
-            ops[0]._plans[key] = plan
-        plan(f2, _lib.ptr(fd), outs, alpha, beta)
+            ops[0]._plans[key] = plan.keep_for_later()
         return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
     W = [op.weights(f.dtype) for op in ops]
     name = "dcpse_apply_nnz_f32" if f.dtype == torch.float32 else "dcpse_apply_nnz_f64"
