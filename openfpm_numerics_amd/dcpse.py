@@ -283,7 +283,10 @@ class Dcpse:
             return False
         if self.bundle16_suits():
             return self._W.get("bundle16_64") is not None
-        return self._W.get("sell64") is not None and vl.counted("col16") and (self.col16() or vl._sell) is not None
+        if self._W.get("sell64") is None or vl._far_col16 is None:
+            return False
+        refused = vl._far_col16 > BUNDLE16_MAX_EXC * max(vl.nnz, 1)
+        return (vl._sell if refused else vl._col16) is not None
 
     def computeDifferentialOperator(self, f: torch.Tensor, out: torch.Tensor | None = None,
                                     f_domain: torch.Tensor | None = None, alpha=1.0, beta=0.0):
@@ -625,7 +628,7 @@ class _SellPlan:
         p = _lib.ptr
         t = "f32" if dtype == torch.float32 else "f64"
         self.tokens = (vl._gen, ops[0]._gen)
-        self.max_exc = BUNDLE16_MAX_EXC
+        self.settings = (BUNDLE16_MAX_EXC, COL16_MIN)
         self.device = vl.row_ptr.device
         self.ctx = _lib.context(self.device.index or 0)
         self.n, self.n_rows = vl.n_cols, vl.n_rows
@@ -642,7 +645,7 @@ class _SellPlan:
         else:
             W = [op.sell_weights() if dtype == torch.float32 else op.sell_weights64() for op in ops]
             self.built = W  # inside a graph capture the operators do not hold them
-            c16 = None if n_domain or (vl.nnz <= COL16_MIN and not vl._col16) else ops[0].col16()
+            c16 = None if n_domain or vl.nnz <= COL16_MIN else ops[0].col16()
             self.W = _lib.ptr_array(W)
             if c16 is not None:
                 name, keep, self.domain = "dcpse_apply_col16_", [vl.row_ptr, *c16[:-1], W[0]], False
@@ -665,7 +668,7 @@ class _SellPlan:
 
     def counts_for(self, ops, vl) -> bool:
         tokens = self.tokens
-        return (tokens[0] is vl._gen and self.max_exc == BUNDLE16_MAX_EXC
+        return (tokens[0] is vl._gen and self.settings == (BUNDLE16_MAX_EXC, COL16_MIN)
                 and ops[0]._gen is tokens[1] and all([W() is not None for W in self.others]))
 
     def __call__(self, f, fd, outs, alpha, beta):

@@ -95,6 +95,7 @@ class ParticleSet:
         vl._slices = None
         vl._far16 = None
         vl._col16 = None
+        vl._far_col16 = None
         return vl
 
 
@@ -200,6 +201,7 @@ class VerletList:
         self._slices = None
         self._far16 = None
         self._col16 = None
+        self._far_col16 = None  # far neighbours of the 16-bit columns, once counted
         self._gen = object()  # token of these neighbours
         self.map_ctr = -1
 
@@ -315,7 +317,11 @@ class VerletList:
         dcpse_sell_fill_col16), shared by every operator on this list: the
         arguments (slice_ptr, sell_row16, col16, base, exc_ptr, exc_col,
         exc_slot, n_exc); None where more than the share max_far of the
-        neighbours would be listed as far. Built on first use."""
+        neighbours would be listed as far. Built on first use; the count of far
+        neighbours stays known where the columns are not kept."""
+        most = max_far * max(self.nnz, 1)
+        if getattr(self, "_far_col16", None) is not None and self._far_col16 > most:
+            return None
         if getattr(self, "_col16", None) is None:
             dev = self.row_ptr.device
             ctx = _lib.context(dev.index or 0)
@@ -327,18 +333,17 @@ class VerletList:
             ctx.call("dcpse_sell_fill_col16", self.n_rows, _lib.ptr(self.row_ptr), _lib.ptr(self.col),
                      _lib.ptr(slice_ptr), _lib.ptr(sell_row), _lib.ptr(col16), _lib.ptr(base), _lib.ptr(exc_ptr),
                      n_exc.ctypes.data)
-            ne = int(n_exc[0])
-            if ne > max_far * max(self.nnz, 1):
-                self._col16 = False
-            else:
-                sell_row16 = torch.empty_like(sell_row)
-                exc_col = torch.empty(max(ne, 1), dtype=torch.int32, device=dev)
-                exc_slot = torch.empty(max(ne, 1), dtype=torch.int32, device=dev)
-                ctx.call("dcpse_sell_fill_col16_far", self.n_rows, _lib.ptr(self.row_ptr), _lib.ptr(self.col),
-                         _lib.ptr(slice_ptr), _lib.ptr(sell_row), _lib.ptr(base), _lib.ptr(exc_ptr), ne,
-                         _lib.ptr(sell_row16), _lib.ptr(exc_col), _lib.ptr(exc_slot))
-                self._col16 = (slice_ptr, sell_row16, col16, base, exc_ptr, exc_col, exc_slot, ne)
-        return self._col16 or None
+            ne = self._far_col16 = int(n_exc[0])
+            if ne > most:
+                return None
+            sell_row16 = torch.empty_like(sell_row)
+            exc_col = torch.empty(max(ne, 1), dtype=torch.int32, device=dev)
+            exc_slot = torch.empty(max(ne, 1), dtype=torch.int32, device=dev)
+            ctx.call("dcpse_sell_fill_col16_far", self.n_rows, _lib.ptr(self.row_ptr), _lib.ptr(self.col),
+                     _lib.ptr(slice_ptr), _lib.ptr(sell_row), _lib.ptr(base), _lib.ptr(exc_ptr), ne,
+                     _lib.ptr(sell_row16), _lib.ptr(exc_col), _lib.ptr(exc_slot))
+            self._col16 = (slice_ptr, sell_row16, col16, base, exc_ptr, exc_col, exc_slot, ne)
+        return self._col16
 
 
 def sell_slices(row_ptr: torch.Tensor, n_rows: int):
