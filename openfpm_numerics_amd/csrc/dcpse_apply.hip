@@ -313,7 +313,7 @@ struct BatchRow {
     int len, lenv;  // nonzeros; those taken in chunks of 4 (0: all by the tail)
     int g, h;       // lane of its part, part
     vf4a fp;
-    // the chunks' columns and weights, read ahead while they fit 32 registers
+    // the chunks' columns and weights, read ahead while they fit 48 registers
     static constexpr bool AHEAD = 2 * EL * GP * NCH <= 48;
     vq q[AHEAD ? GP * NCH : 1];
     vw w[AHEAD ? GP * NCH : 1];

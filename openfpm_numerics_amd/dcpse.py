@@ -61,8 +61,11 @@ SELL_AFTER = 1
 #: does not fit those either, the 32-bit sliced-ELL layout.
 BUNDLE16_MAX_EXC = 0.01
 #: Neighbours above which several operators in one pass take the list's 16-bit
-#: columns: below, the 32-bit ones are as fast (8.2 and 8.4 us a stage with 3.8M
-#: neighbours, caches hold them) and 35 us quicker to build.
+#: columns, which cost 30 to 45 us more to build than the 32-bit ones. us per
+#: apply of two operators with 32-bit / 16-bit columns, FP32 and FP64: 2M
+#: neighbours 9.2 / 9.1 and 11.8 / 11.1, 4M 13.8 / 12.1 and 19.0 / 17.5, 8M 21.5 /
+#: 19.4 and 32.4 / 30.8, 16M 37.4 / 32.5 and 69 / 60 (2D; three operators and 3D
+#: alike): paid for after some 60, 25, 15 and 8 applies
 COL16_MIN = 4_000_000
 _FILE_VERSION = 1
 
