@@ -631,7 +631,7 @@ class _SellPlan:
         p = _lib.ptr
         t = "f32" if dtype == torch.float32 else "f64"
         self.tokens = (vl._gen, ops[0]._gen)
-        self.settings = (BUNDLE16_MAX_EXC, COL16_MIN)
+        self.max_exc, self.col16_min = BUNDLE16_MAX_EXC, COL16_MIN
         self.device = vl.row_ptr.device
         self.ctx = _lib.context(self.device.index or 0)
         self.n, self.n_rows = vl.n_cols, vl.n_rows
@@ -671,8 +671,8 @@ class _SellPlan:
 
     def counts_for(self, ops, vl) -> bool:
         tokens = self.tokens
-        return (tokens[0] is vl._gen and self.settings == (BUNDLE16_MAX_EXC, COL16_MIN)
-                and ops[0]._gen is tokens[1] and all([W() is not None for W in self.others]))
+        return (tokens[0] is vl._gen and ops[0]._gen is tokens[1] and self.max_exc == BUNDLE16_MAX_EXC
+                and self.col16_min == COL16_MIN and (not self.others or all([W() is not None for W in self.others])))
 
     def __call__(self, f, fd, outs, alpha, beta):
         self.ctx.bind_current_stream()
