@@ -25,11 +25,15 @@ from .particles import capturing
 CSR_MAX = {torch.float32: 3_600_000, torch.float64: 2_600_000}
 #: FP64 stages of one call from which "auto" runs on the sliced-ELL copy of a
 #: list of at least SELL64_LARGE neighbours, or of a smaller one, whose weights
-#: the last-level cache holds: building it costs 0.2 to 0.5 ms and saves 20 us
-#: per stage at 77^3 particles, 3 us at 64^3
-SELL64_AFTER = 12
-SELL64_LARGE = 16_000_000
-SELL64_AFTER_SMALL = 64
+#: and columns (12 bytes a neighbour on CSR) the 256 MB last-level cache holds.
+#: us per stage CSR / "bundle16" and for building the copy: 4M neighbours 11.4 /
+#: 9.8, 80; 8.7M 21.1 / 21.7, 100; 15M 32.0 / 28.8, 115; 18M 38.5 / 35.2, 125; 28M
+#: 89 / 64, 180; 45M 142 / 112, 240: paid for by some 50, -, 36, 37, 7 and 8
+#: stages. A single ``stage`` counts as SELL64_AFTER: it is one of a longer
+#: integration, which the caller drives
+SELL64_AFTER = 8
+SELL64_LARGE = 20_000_000
+SELL64_AFTER_SMALL = 40
 
 
 _NAMES = {"bundle16": "bundle16_", "col16": "col16_", "sell": "sell_", "csr": ""}
@@ -133,13 +137,14 @@ def stage(op, u: torch.Tensor, alpha: float, y_a: torch.Tensor | None, ca: float
           y_b: torch.Tensor | None, cb: float, out_b: torch.Tensor | None, layout: str = "auto"):
     """One fused stage: k = alpha * D u; out_a = y_a + ca k; out_b = y_b + cb k (outputs may be None).
 
-    Layouts as for rk4; "auto" counts one apply towards ``dcpse.SELL_AFTER``."""
+    Layouts as for rk4; "auto" counts one apply towards ``dcpse.SELL_AFTER`` in
+    FP32 and runs as a call of ``SELL64_AFTER`` stages in FP64."""
     d = _dcpse(op)
     vl = d.verletList
     ctx = _lib.context(u.device.index or 0)
     ctx.bind_current_stream()
     p = _lib.ptr
-    layout = _layout(d, u.dtype, layout, 1)
+    layout = _layout(d, u.dtype, layout, 1 if u.dtype == torch.float32 else SELL64_AFTER)
     t = "f32" if u.dtype == torch.float32 else "f64"
     held = _operator(d, u.dtype, layout)
     ctx.call(f"dcpse_stage_{_NAMES[layout]}{t}", vl.n_rows, *_args(held), p(u), float(alpha), p(y_a), float(ca), p(out_a),

@@ -32,7 +32,7 @@ def small(monkeypatch):
 
 def test_equal_calls_equal_bits(cuda, small):
     lap, f = _operator(cuda)
-    first = {steps: small.rk4(lap, f.clone(), 1e-6, steps) for steps in (1, 15, 16, 20)}
+    first = {steps: small.rk4(lap, f.clone(), 1e-6, steps) for steps in (1, 9, 10, 20)}
     one = torch.empty_like(f)
     small.stage(lap, f, 1.0, f, 0.5, one, None, 0.0, None)
     for use in (lambda: None, lambda: lap(f), lambda: small.rk4(lap, f.clone(), 1e-6, 100)):
@@ -42,6 +42,24 @@ def test_equal_calls_equal_bits(cuda, small):
         again = torch.empty_like(f)
         small.stage(lap, f, 1.0, f, 0.5, again, None, 0.0, None)
         assert torch.equal(again, one)
+
+
+def test_single_stages_of_large_lists(cuda, small, monkeypatch):
+    """On the copy from the first stage on, unless copies are deferred."""
+    from openfpm_numerics_amd import dcpse
+
+    monkeypatch.setattr(small, "SELL64_LARGE", 0)
+    lap, f = _operator(cuda)
+    outs = [torch.empty_like(f) for _ in range(3)]
+    small.stage(lap, f, 1.0, f, 0.5, outs[0], None, 0.0, None)
+    assert lap.dcpse._W.get("bundle16_64") is not None
+    small.stage(lap, f, 1.0, f, 0.5, outs[1], None, 0.0, None)
+    small.stage(lap, f, 1.0, f, 0.5, outs[2], None, 0.0, None, layout="bundle16")
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    monkeypatch.setattr(dcpse, "SELL_AFTER", 1000)
+    lap, f = _operator(cuda)
+    small.stage(lap, f, 1.0, f, 0.5, outs[0], None, 0.0, None)
+    assert lap.dcpse._W.get("bundle16_64") is None
 
 
 def test_deferred_copies(cuda, small, monkeypatch):
