@@ -175,7 +175,7 @@ class Dcpse_hip : public openfpm_dcpse::field_operator<typename vector_type::pro
         if constexpr (std::is_same<prop_type, float>::value) {
             float* O[1] = {out};
             // the sliced-ELL copy from the kSellAfter-th apply since assembly
-            // on (building it costs what some 50 applies save)
+            // on (building it costs what some 20 applies save)
             if (n > 0 && !b16_tried_ && ++n_apply32_ >= kSellAfter) build_bundle16();
             if (b16_) {
                 c.check(dcpse_apply_sell_bundle16_f32(c.get(), n, verletList_.devRowPtr(),

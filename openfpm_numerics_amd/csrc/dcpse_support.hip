@@ -6,9 +6,9 @@
 // src/DCPSE/SupportBuilder.cuh:15-61. Unlike that builder (one thread per
 // particle, host-side serial prefix sum, size_t keys, 4 host round trips), the
 // whole CSR is built on the device: a cell grid by counting sort, then one
-// wavefront per cell (one set, one cut-off) or per particle over the
-// neighbouring cells' particles, flattened into one candidate list and sorted
-// in registers, so every row comes out in ascending particle index
+// wavefront per group of neighbouring particles (one set) or per particle over
+// the neighbouring cells' particles, flattened into one candidate list and
+// sorted in registers, so every row comes out in ascending particle index
 // (deterministic, independent of atomic ordering).
 #include <algorithm>
 #include <climits>
