@@ -430,10 +430,10 @@ class Dcpse:
                      _lib.ptr(sell_colT), _lib.ptr(sell_WT), _lib.ptr(diag), _lib.ptr(g2), _lib.ptr(o), alpha, beta)
             return o.reshape(g.shape)
         name = "dcpse_apply_transpose_nnz_f32" if g.dtype == torch.float32 else "dcpse_apply_transpose_nnz_f64"
-        scratch = _batch_scratch(g2)
+        scratch, at, size = _batch_scratch(g2)
         ctx.call(name, n, self.verletList.nnz, _lib.ptr(rowT), _lib.ptr(colT), _lib.ptr(WT), _lib.ptr(diag),
-                 _lib.ptr(g2), n, nb, _lib.ptr(o), n, alpha, beta, _lib.ptr(scratch), _nbytes(scratch))
-        return o.reshape(g.shape)
+                 _lib.ptr(g2), n, nb, _lib.ptr(o), n, alpha, beta, at, size)
+        return o if out is None and g.dim() == 2 else o.reshape(g.shape)
 
     # ---- persistence (Dcpse.hpp:302-379) -------------------------------------------
     def save(self, file: str, rank: int = 0):
@@ -631,13 +631,13 @@ class _SellPlan:
         p = _lib.ptr
         t = "f32" if dtype == torch.float32 else "f64"
         self.tokens = (vl._gen, ops[0]._gen)
-        self.max_exc, self.col16_min = BUNDLE16_MAX_EXC, COL16_MIN
+        self.max_exc = BUNDLE16_MAX_EXC
         self.device = vl.row_ptr.device
         self.ctx = _lib.context(self.device.index or 0)
         self.n, self.n_rows = vl.n_cols, vl.n_rows
         self.outs_type = C.c_void_p * len(ops)
         self.domain = True  # the function takes the field on the domain
-        self.others = ()
+        self.weights = None  # beside a list's columns: (COL16_MIN, the other operators' weights)
         if len(ops) == 1 and ops[0].bundle16_suits():
             # one operator: its 16-bit-offset bundle, built once per assembly
             *keep, ne = ops[0].sell_bundle16(dtype)
@@ -647,7 +647,7 @@ class _SellPlan:
             args = (p(vl.row_ptr), p(slice_ptr), p(row16), 1, p(bundle), p(exc_ptr), p(exc_col), p(exc_W), ne)
         else:
             W = [op.sell_weights() if dtype == torch.float32 else op.sell_weights64() for op in ops]
-            self.built = W  # inside a graph capture the operators do not hold them
+            self.weights = COL16_MIN, W  # inside a graph capture the operators do not hold them
             c16 = None if n_domain or vl.nnz <= COL16_MIN else ops[0].col16()
             self.W = _lib.ptr_array(W)
             if c16 is not None:
@@ -664,15 +664,22 @@ class _SellPlan:
     def keep_for_later(self):
         """The other operators' weights are theirs: those of an operator that is
         assembled again or dropped are not held by this one's plans."""
-        if "built" in self.__dict__:
-            self.others = tuple(weakref.ref(W) for W in self.built[1:])
-            del self.built
+        if self.weights is not None:
+            self.weights = self.weights[0], [weakref.ref(W) for W in self.weights[1][1:]]
         return self
 
     def counts_for(self, ops, vl) -> bool:
         tokens = self.tokens
-        return (tokens[0] is vl._gen and ops[0]._gen is tokens[1] and self.max_exc == BUNDLE16_MAX_EXC
-                and self.col16_min == COL16_MIN and (not self.others or all([W() is not None for W in self.others])))
+        if tokens[0] is not vl._gen or ops[0]._gen is not tokens[1] or self.max_exc != BUNDLE16_MAX_EXC:
+            return False
+        if self.weights is not None:
+            least, others = self.weights
+            if least != COL16_MIN:
+                return False
+            for W in others:
+                if W() is None:
+                    return False
+        return True
 
     def __call__(self, f, fd, outs, alpha, beta):
         self.ctx.bind_current_stream()
@@ -689,22 +696,20 @@ _FWD = {torch.float32: "fwd", torch.float64: "fwd64"}
 
 
 def _batch_scratch(f2: torch.Tensor):
-    """Memory for the particle-major copies of a batch (B, N) of 3 or more
-    fields, as wide as its widest pass (4, 8 or 16 fields); None for fewer, or
-    where there is no room, and the batch then runs field by field. It comes
-    from torch's allocator, so each stream, and a graph being captured, has
-    its own."""
+    """(tensor, address, bytes) of memory for the particle-major copies of a
+    batch (B, N) of 3 or more fields, as wide as its widest pass (4, 8 or 16
+    fields); none for fewer, or where there is no room, and the batch then runs
+    field by field. It comes from torch's allocator, so each stream, and a graph
+    being captured, has its own; held until the call has been made."""
     nb, n = f2.shape
     if nb < 3:
-        return None
+        return None, None, 0
+    width = 4 if nb <= 4 else 8 if nb <= 8 else 16
     try:
-        return torch.empty((4 if nb <= 4 else 8 if nb <= 8 else 16) * n, dtype=f2.dtype, device=f2.device)
+        scratch = f2.new_empty(width * n)
     except torch.cuda.OutOfMemoryError:
-        return None
-
-
-def _nbytes(t) -> int:
-    return 0 if t is None else t.numel() * t.element_size()
+        return None, None, 0
+    return scratch, scratch.data_ptr(), width * n * f2.element_size()
 
 
 def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = None, alpha=1.0, beta=0.0):
@@ -729,7 +734,8 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
     plan = ops[0]._plans.get(key)
     if (plan is not None and outs is None and f_domain is None and USE_SELL and type(f) is torch.Tensor
             and f.dim() == 1 and f.is_contiguous() and f.shape[0] == plan.n and f.device == plan.device
-            and plan.counts_for(ops, vl) and all([op._n32[_FWD[f.dtype]] + 1 >= SELL_AFTER for op in ops])):
+            and plan.counts_for(ops, vl)
+            and (SELL_AFTER <= 1 or all([op._n32[_FWD[f.dtype]] + 1 >= SELL_AFTER for op in ops]))):
         for op in ops:
             op._n32[_FWD[f.dtype]] += 1
         outs = [torch.empty_like(f) for _ in ops]
@@ -748,7 +754,8 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
     elif not ops[0].same_set:
         raise ValueError("two-set operators need f_domain (the field on the domain particles)")
     n_rows = vl.n_rows
-    if outs is None:
+    made = outs is None
+    if made:
         outs = [torch.empty((nb, n_rows), dtype=f.dtype, device=f.device) for _ in ops]
     else:
         outs = [o.reshape(nb, n_rows) for o in outs]
@@ -768,11 +775,11 @@ def apply_ops(ops, f: torch.Tensor, outs=None, f_domain: torch.Tensor | None = N
     if len(ops) > 1 and nb > 1:
         res = [apply_ops([op], f, [o], f_domain, alpha, beta)[0] for op, o in zip(ops, outs)]
         return [r.reshape(*f.shape[:-1], n_rows) for r in res]
-    scratch = _batch_scratch(f2) if fd is None else None
+    scratch, at, size = _batch_scratch(f2) if fd is None else (None, None, 0)
     ctx.call(name, n_rows, vl.nnz, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), len(ops), _lib.ptr_array(W),
              _lib.ptr(f2), n, nb, _lib.ptr(fd), n_rows if fd is not None else n, _lib.ptr_array(outs), n_rows,
-             alpha, beta, _lib.ptr(scratch), _nbytes(scratch))
-    return [o.reshape(*f.shape[:-1], n_rows) for o in outs]
+             alpha, beta, at, size)
+    return outs if made and f.dim() == 2 else [o.reshape(*f.shape[:-1], n_rows) for o in outs]
 
 
 def sell_bundle(ops) -> torch.Tensor:
@@ -875,14 +882,13 @@ class PreparedApply:
             self.args = (self.ctx.h, vl.n_rows, _lib.ptr(vl.row_ptr), _lib.ptr(slice_ptr), _lib.ptr(sell_row),
                          _lib.ptr(sell_col), len(ops), self.W, _lib.ptr(f2), None, self.O, alpha, beta)
         else:
-            scratch = _batch_scratch(f2) if len(ops) == 1 else None
+            scratch, at, size = _batch_scratch(f2) if len(ops) == 1 else (None, None, 0)
             self._keep = (ops, f, outs, [op.weights(f.dtype) for op in ops], scratch)
             self.fn = (self.ctx.lib.dcpse_apply_nnz_f32 if f.dtype == torch.float32
                        else self.ctx.lib.dcpse_apply_nnz_f64)
             self.W = _lib.ptr_array(self._keep[3])
             self.args = (self.ctx.h, vl.n_rows, vl.nnz, _lib.ptr(vl.row_ptr), _lib.ptr(vl.col), len(ops), self.W,
-                         _lib.ptr(f2), n, nb, None, n, self.O, vl.n_rows, alpha, beta, _lib.ptr(scratch),
-                         _nbytes(scratch))
+                         _lib.ptr(f2), n, nb, None, n, self.O, vl.n_rows, alpha, beta, at, size)
         lib = self.ctx.lib
         self.layout = next((name for fn, name in ((lib.dcpse_apply_sell_f32, "sell"),
                                                   (lib.dcpse_apply_sell_bundle_f32, "sell_bundle"),
